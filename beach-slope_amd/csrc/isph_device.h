@@ -329,9 +329,44 @@ __device__ __forceinline__ int quadrant(double x, double y, double xl, double xr
 }
 
 // ---------------------------------------------------------------------
+// The last six levels of the halving tree, v[l] += v[l + s] for s = 32..1
+// over a wavefront (the result in lane 0): half-wave and row exchanges, then
+// row shifts, a few cycles a level where a shuffle goes through the LDS
+// crossbar.  Lane 0's operands, and so its bits, are those of the shuffles.
+// ---------------------------------------------------------------------
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double wave_tree(double v) {
+  {
+    const long long b = __double_as_longlong(v);
+    const auto lo = __builtin_amdgcn_permlane32_swap((int)b, (int)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((int)(b >> 32), (int)(b >> 32), false, false);
+    v = __longlong_as_double(((long long)hi[0] << 32) | (unsigned int)lo[0]) +
+        __longlong_as_double(((long long)hi[1] << 32) | (unsigned int)lo[1]);
+  }
+  {
+    const long long b = __double_as_longlong(v);
+    const auto lo = __builtin_amdgcn_permlane16_swap((int)b, (int)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((int)(b >> 32), (int)(b >> 32), false, false);
+    v = __longlong_as_double(((long long)hi[0] << 32) | (unsigned int)lo[0]) +
+        __longlong_as_double(((long long)hi[1] << 32) | (unsigned int)lo[1]);
+  }
+  v = v + dpp_f64<0x108>(v);  // row_shl: lane l reads lane l + 8 of its row of 16
+  v = v + dpp_f64<0x104>(v);
+  v = v + dpp_f64<0x102>(v);
+  v = v + dpp_f64<0x101>(v);
+  return v;
+}
+
+// ---------------------------------------------------------------------
 // deterministic block reduction: halving tree v[t] += v[t+s], s = 128..1.
-// The first two levels go through LDS, the last six through wavefront
-// shuffles inside wave 0; the result is identical to the LDS tree.
+// The first two levels go through LDS, the last six run inside wave 0
+// (wave_tree); the result is identical to the LDS tree.
 // ---------------------------------------------------------------------
 __device__ __forceinline__ double block_tree(double val, double* lds) {
   const int t = threadIdx.x;
@@ -341,9 +376,7 @@ __device__ __forceinline__ double block_tree(double val, double* lds) {
   __syncthreads();
   double v = 0.0;
   if (t < 64) {
-    v = lds[t] + lds[t + 64];
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) v = v + __shfl_down(v, s, 64);
+    v = wave_tree(lds[t] + lds[t + 64]);
   }
   __syncthreads();
   return v;  // valid in thread 0
@@ -366,10 +399,7 @@ __device__ __forceinline__ void block_tree_n(double (&v)[N], double* lds) {
   if (t < 64) {
 #pragma unroll
     for (int k = 0; k < N; k++) {
-      double a = lds[k * RED_BLOCK + t] + lds[k * RED_BLOCK + t + 64];
-#pragma unroll
-      for (int s = 32; s >= 1; s >>= 1) a = a + __shfl_down(a, s, 64);
-      v[k] = a;
+      v[k] = wave_tree(lds[k * RED_BLOCK + t] + lds[k * RED_BLOCK + t + 64]);
     }
   }
   __syncthreads();

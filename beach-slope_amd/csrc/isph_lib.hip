@@ -21,6 +21,7 @@
 #include "isph_solver.h"
 #include "isph_mg.h"
 #include "isph_batch.h"
+#include "isph_persist.h"
 #include "isph_buffer.h"
 #include "isph_wcsph.h"
 
@@ -93,6 +94,7 @@ struct isph_ctx {
   // previous precision solve: iterations to the first stop, and after it
   // (chunk sizing only; the results do not depend on the chunks)
   int pred_first = 0, pred_after = 0;
+  PersArg ps{};            // resident FP64 solve: its exchange slots and windows
   bool in_batch = false;   // a member of a batch: its form (precision, WCSPH) is fixed
   int tshape[TK_N] = {TS_P256, TS_P256, TS_P256, TS_P256, TS_P256,
                      TS_P256, TS_P256, TS_P256, TS_P256};  // tuned launch shapes
@@ -181,6 +183,75 @@ static void fill_devparams(isph_ctx* c) {
   d.wo = host_wo(P.h, d.k1, d.k2);
 }
 
+// ---------------------------------------------------------------------
+// the resident FP64 solve (isph_persist.h): its launch shape and launches
+// ---------------------------------------------------------------------
+#define RES_MAX_WG 256          // workgroups of a launch, at most one per CU
+#define RES_WLIST (RES_MAX_WG * (8 * 1024 / PS_CHUNK))
+#define RES_ITERS 1024          // iterations of one launch at most
+
+struct ResPlan {
+  int T = 0, R = 0, W = 0, nbw = 0, G = 0;
+  size_t lds = 0;
+  const void* setup = nullptr;
+  const void* solve = nullptr;
+};
+
+template <int T, int R, int W, int KR>
+static void res_shape(ResPlan& p, int nblk) {
+  p.T = T;
+  p.R = R;
+  p.W = W;  // window elements per thread
+  p.lds = (size_t)ps_lds_bytes<T, R, W>(nblk);
+  p.setup = reinterpret_cast<const void*>(&k_ps_setup<T>);
+  p.solve = reinterpret_cast<const void*>(&k_bicg_resident<T, R, W, KR>);
+}
+
+// The launch shape for nblk row blocks: one workgroup per CU at most, the
+// smallest workgroup whose threads hold its rows.  False where the device
+// cannot hold the grid resident; the solve then runs launch by launch.
+static bool res_plan(int nblk, ResPlan* out) {
+  int dev = 0, cus = 0, coop = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
+      !coop || nblk < 1 || nblk > PS_MAX_CHUNKS / 4)
+    return false;
+  ResPlan p;
+  const int wg = std::min(cus, RES_MAX_WG);
+  p.nbw = (nblk + wg - 1) / wg;
+  p.G = (nblk + p.nbw - 1) / p.nbw;
+  if (p.nbw <= 1) res_shape<256, 1, 8, 32>(p, nblk);
+  else if (p.nbw <= 2) res_shape<512, 1, 6, 32>(p, nblk);
+  else if (p.nbw <= 4) res_shape<1024, 1, 4, 0>(p, nblk);
+  else if (p.nbw <= 8) res_shape<1024, 2, 5, 0>(p, nblk);
+  else if (p.nbw <= 12) res_shape<1024, 3, 6, 0>(p, nblk);
+  else return false;
+  int per_cu = 0;
+  if (hipFuncSetAttribute(p.solve, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds) !=
+          hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, p.solve, p.T, p.lds) != hipSuccess ||
+      (int64_t)per_cu * cus < p.G) {
+    (void)hipGetLastError();
+    return false;
+  }
+  *out = p;
+  return true;
+}
+
+static hipError_t res_setup(const ResPlan& p, Dev& D, PersArg& Q, hipStream_t st) {
+  Q.lidx = D.aoff;
+  Q.wcap = p.W * p.T / PS_CHUNK;
+  Q.nbw = p.nbw;
+  void* args[] = {&D, &Q};
+  return hipLaunchKernel(p.setup, dim3(p.G), dim3(p.T), args, 0, st);
+}
+static hipError_t res_launch(const ResPlan& p, Dev& D, PersArg& Q, int iters, unsigned ep,
+                             hipStream_t st) {
+  void* args[] = {&D, &Q, &iters, &ep};
+  return hipLaunchCooperativeKernel(p.solve, dim3(p.G), dim3(p.T), args, p.lds, st);
+}
+
 extern "C" int64_t isph_footprint_bytes(int64_t n_cap, int64_t n_solid_cap, int32_t cellx,
                                         int32_t celly, int32_t precision) {
   const int64_t ncell = (int64_t)cellx * celly;
@@ -191,11 +262,13 @@ extern "C" int64_t isph_footprint_bytes(int64_t n_cap, int64_t n_solid_cap, int3
   per += 4 * 3;                                 // bin, rank, scan scratch
   per += 4 + ROW_CAP * (4 + 8) + 2 * 8;         // PPE rows, rhs, solution
   per += 6 * 8;                                 // FP64 solver vectors
-  // precision form: FP16 V-cycle matrix and packed column offsets, FP32
-  // vectors, level-0 multigrid vectors, setup rows
-  if (precision) per += 2 * 4 * ((ROW_CAP + 1) / 2) + 5 * 4 + 2 * 4 + 9 * 8;
+  per += 4 * ((ROW_CAP + 1) / 2);               // packed 16-bit columns
+  // precision form: FP16 V-cycle matrix, FP32 vectors, level-0 multigrid
+  // vectors, setup rows
+  if (precision) per += 4 * ((ROW_CAP + 1) / 2) + 5 * 4 + 2 * 4 + 9 * 8;
   int64_t b = per * n_cap + 4 * 8 * n_solid_cap + 4 * (ncell * (2 + 2 * NCLS) + 16);
   b += 5 * 8 * (n_cap / 256 + 2);               // reduction partials
+  b += 64 * (n_cap / 256 + 2);                  // exchange slots of the resident solve
   b += 8 * (2 * ncell + 2 * (ncell / 256 + 2)); // per-cell maxima and their block maxima
   // cell levels: stencil, x, b, r and 1/diagonal per unknown, the levels
   // holding 4/3 of the cell count
@@ -276,9 +349,12 @@ extern "C" int isph_create(const isph_params* params, int64_t n_cap, int64_t n_s
     rc |= ISPH_EHIP;
   rc |= dalloc(c, &D.sc, 1);
   rc |= dalloc(c, &c->d_bn2, 1);
+  rc |= dalloc(c, &D.aoff, N * ((ROW_CAP + 1) / 2));
+  rc |= dalloc(c, &c->ps.slots, 8 * (N / 256 + 2 + RES_MAX_WG));
+  rc |= dalloc(c, &c->ps.wlist, RES_WLIST);
+  rc |= dalloc(c, &c->ps.wcnt, RES_MAX_WG);
   if (params->precision) {
     rc |= dalloc(c, &D.av16, N * ((ROW_CAP + 1) / 2));
-    rc |= dalloc(c, &D.aoff, N * ((ROW_CAP + 1) / 2));
     float** ff[] = {&D.r32, &D.rh32, &D.pp32, &D.sv32, &D.d32};
     for (auto p : ff) rc |= dalloc(c, p, N);
     // cell hierarchy: level 1 is the cell grid, then 2x2 aggregation down to
@@ -1165,26 +1241,46 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
   return 0;
 }
 
-// run BiCGStab chunks until the device reports done; on a breakdown below
-// the iteration cap restart from the true residual, at most max_outer times
-static int bicg_loop(isph_ctx* c, int* iters_out, int* brk_out, int* conv_out,
-                     double* rel_out, int* restarts_out) {
+// run BiCGStab until the device reports done, in the resident form (plan
+// non-null) or in chunks of launches; on a breakdown below the iteration cap
+// restart from the true residual, at most max_outer times
+static int bicg_loop(isph_ctx* c, const ResPlan* plan, int* iters_out, int* brk_out,
+                     int* conv_out, double* rel_out, int* restarts_out) {
   const int n = c->n_hi;
   int chunk = 4, restarts = 0, prev = 0;
+  unsigned ep = 1;
   DevScalars s;
   for (int64_t it = 0;; ) {
-    for (int k = 0; k < chunk; k++) {
-      TIMED_LAUNCH(0, k_bicg_1, n, c->D);
-      FINALIZE(FIN_ALPHA, n);
-      TIMED_LAUNCH(1, k_bicg_2, n, c->D);
-      FINALIZE(FIN_OMEGA, n);
-      RLAUNCH(k_bicg_3, n, c->D);
-      FINALIZE(FIN_BETA, n);
-      RLAUNCH(k_bicg_4, n, c->D);
+    if (plan) {
+      // a refused launch (another process holds the device's cooperative
+      // queue) leaves the state as it was: the solve goes on launch by launch
+      if (res_launch(*plan, c->D, c->ps, RES_ITERS, ep, c->stream) == hipSuccess) {
+        chunk = RES_ITERS;
+        ep += 3u * (unsigned)chunk;
+      } else {
+        (void)hipGetLastError();
+        plan = nullptr;
+        chunk = 4;
+      }
+    }
+    if (!plan) {
+      for (int k = 0; k < chunk; k++) {
+        TIMED_LAUNCH(0, k_bicg_1, n, c->D);
+        FINALIZE(FIN_ALPHA, n);
+        TIMED_LAUNCH(1, k_bicg_2, n, c->D);
+        FINALIZE(FIN_OMEGA, n);
+        RLAUNCH(k_bicg_3, n, c->D);
+        FINALIZE(FIN_BETA, n);
+        RLAUNCH(k_bicg_4, n, c->D);
+      }
     }
     it += chunk;
     int rc = read_scalars(c, &s);
     if (rc) return rc;
+    if (plan && s.counter[PS_FLAG_ABORT]) {
+      set_err(c, "resident PPE solve: a grid-wide wait ran out");
+      return ISPH_EHIP;
+    }
     // the timed launches that did work: the chunk's leading iterations
     if (c->prof) timers_collect(c, s.iters - prev);
     prev = s.iters;
@@ -1210,6 +1306,11 @@ static int bicg_loop(isph_ctx* c, int* iters_out, int* brk_out, int* conv_out,
   *rel_out = s.rel;
   *restarts_out = restarts;
   return 0;
+}
+
+// the resident solve's flags
+__global__ void k_res_clear(Dev D) {
+  if (blockIdx.x == 0 && threadIdx.x < 4) D.sc->counter[threadIdx.x] = 0u;
 }
 
 static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
@@ -1249,15 +1350,21 @@ static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
       }
       st.rel_residual = (bnorm == 0.0) ? 0.0 : bnorm;
     } else {
+      // kernel timing brackets launches, so it takes the launch-per-phase form
+      ResPlan plan;
+      bool resident = !c->prof && res_plan(c->D.nblk, &plan);
+      hipLaunchKernelGGL(k_res_clear, dim3(1), dim3(64), 0, c->stream, c->D);
+      if (resident) HIPCHK(c, res_setup(plan, c->D, c->ps, c->stream));
       RLAUNCH(k_bicg_init, n, c->D);
       FINALIZE(FIN_INIT, n);
       DevScalars s;
       int rc = read_scalars(c, &s);
       if (rc) return rc;
+      if (s.counter[PS_FLAG_WIN]) resident = false;
       int it = 0, brk = 0, conv = s.conv, restarts = 0;
       double rel = s.rel;
       if (!s.done) {
-        rc = bicg_loop(c, &it, &brk, &conv, &rel, &restarts);
+        rc = bicg_loop(c, resident ? &plan : nullptr, &it, &brk, &conv, &rel, &restarts);
         if (rc) return rc;
       }
       st.iterations = it;
