@@ -10,6 +10,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -22,6 +23,7 @@
 #include "isph_mg.h"
 #include "isph_batch.h"
 #include "isph_persist.h"
+#include "isph_mgres.h"
 #include "isph_buffer.h"
 #include "isph_wcsph.h"
 
@@ -95,6 +97,8 @@ struct isph_ctx {
   // (chunk sizing only; the results do not depend on the chunks)
   int pred_first = 0, pred_after = 0;
   PersArg ps{};            // resident FP64 solve: its exchange slots and windows
+  ResDev rs{};             // resident precision solve: its words, slots and windows
+  bool loaded = false;     // the system came from isph_load_system (no cells behind its rows)
   bool in_batch = false;   // a member of a batch: its form (precision, WCSPH) is fixed
   int tshape[TK_N] = {TS_P256, TS_P256, TS_P256, TS_P256, TS_P256,
                      TS_P256, TS_P256, TS_P256, TS_P256};  // tuned launch shapes
@@ -190,6 +194,36 @@ static void fill_devparams(isph_ctx* c) {
 #define RES_WLIST (RES_MAX_WG * (8 * 1024 / PS_CHUNK))
 #define RES_ITERS 1024          // iterations of one launch at most
 
+// LDS of a resident workgroup at most; the kernels are allowed this much
+// whatever a launch needs, so contexts of several threads ask for the same
+#define RES_LDS_MAX (152 * 1024)
+
+// Workgroups of T threads and RES_LDS_MAX bytes of LDS of kernel fn that the
+// current device holds resident for a cooperative launch (0: none); asked
+// once per device and kernel
+static int resident_capacity(const void* fn, int T) {
+  static std::mutex mu;
+  static std::map<std::pair<int, const void*>, int> known;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  std::lock_guard<std::mutex> lock(mu);
+  const auto key = std::make_pair(dev, fn);
+  const auto at = known.find(key);
+  if (at != known.end()) return at->second;
+  int cus = 0, coop = 0, per_cu = 0, n = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) == hipSuccess &&
+      coop &&
+      hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS_MAX) ==
+          hipSuccess &&
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, T, RES_LDS_MAX) == hipSuccess)
+    n = per_cu * cus;
+  else
+    (void)hipGetLastError();
+  known[key] = n;
+  return n;
+}
+
 struct ResPlan {
   int T = 0, R = 0, W = 0, nbw = 0, G = 0;
   size_t lds = 0;
@@ -211,15 +245,9 @@ static void res_shape(ResPlan& p, int nblk) {
 // smallest workgroup whose threads hold its rows.  False where the device
 // cannot hold the grid resident; the solve then runs launch by launch.
 static bool res_plan(int nblk, ResPlan* out) {
-  int dev = 0, cus = 0, coop = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
-      !coop || nblk < 1 || nblk > PS_MAX_CHUNKS / 4)
-    return false;
+  if (nblk < 1 || nblk > PS_MAX_CHUNKS / 4) return false;
   ResPlan p;
-  const int wg = std::min(cus, RES_MAX_WG);
-  p.nbw = (nblk + wg - 1) / wg;
+  p.nbw = (nblk + RES_MAX_WG - 1) / RES_MAX_WG;
   p.G = (nblk + p.nbw - 1) / p.nbw;
   if (p.nbw <= 1) res_shape<256, 1, 8, 32>(p, nblk);
   else if (p.nbw <= 2) res_shape<512, 1, 6, 32>(p, nblk);
@@ -227,14 +255,7 @@ static bool res_plan(int nblk, ResPlan* out) {
   else if (p.nbw <= 8) res_shape<1024, 2, 5, 0>(p, nblk);
   else if (p.nbw <= 12) res_shape<1024, 3, 6, 0>(p, nblk);
   else return false;
-  int per_cu = 0;
-  if (hipFuncSetAttribute(p.solve, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds) !=
-          hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, p.solve, p.T, p.lds) != hipSuccess ||
-      (int64_t)per_cu * cus < p.G) {
-    (void)hipGetLastError();
-    return false;
-  }
+  if (p.lds > RES_LDS_MAX || resident_capacity(p.solve, p.T) < p.G) return false;
   *out = p;
   return true;
 }
@@ -266,13 +287,14 @@ extern "C" int64_t isph_footprint_bytes(int64_t n_cap, int64_t n_solid_cap, int3
   // precision form: FP16 V-cycle matrix, FP32 vectors, level-0 multigrid
   // vectors, setup rows
   if (precision) per += 4 * ((ROW_CAP + 1) / 2) + 5 * 4 + 2 * 4 + 9 * 8;
+  if (precision) per += 3 * 8 + 1;              // exchanged words, partial-sum slots
   int64_t b = per * n_cap + 4 * 8 * n_solid_cap + 4 * (ncell * (2 + 2 * NCLS) + 16);
   b += 5 * 8 * (n_cap / 256 + 2);               // reduction partials
   b += 64 * (n_cap / 256 + 2);                  // exchange slots of the resident solve
   b += 8 * (2 * ncell + 2 * (ncell / 256 + 2)); // per-cell maxima and their block maxima
   // cell levels: stencil, x, b, r and 1/diagonal per unknown, the levels
   // holding 4/3 of the cell count
-  if (precision) b += 4 * 13 * ((4 * ncell) / 3 + MG_MAX_LEVELS) + 8 * MG_DENSE_MAX * MG_DENSE_MAX;
+  if (precision) b += (4 * 13 + 16) * ((4 * ncell) / 3 + MG_MAX_LEVELS) + 8 * MG_DENSE_MAX * MG_DENSE_MAX;
   return b + (1 << 20);
 }
 
@@ -378,6 +400,15 @@ extern "C" int isph_create(const isph_params* params, int64_t n_cap, int64_t n_s
     rc |= dalloc(c, &G.rowst, 9 * N);
     rc |= dalloc(c, &G.d0, N);
     rc |= dalloc(c, &G.x0, N);
+    rc |= dalloc(c, &c->rs.slots, 10 * (N / 256 + 2));
+    rc |= dalloc(c, &c->rs.mail, RES_MAX_WG * RS_MAIL);
+    rc |= dalloc(c, &c->rs.x0w, N);
+    rc |= dalloc(c, &c->rs.phw, N);
+    rc |= dalloc(c, &c->rs.r0w, N);
+    rc |= dalloc(c, &c->rs.bw, off);
+    rc |= dalloc(c, &c->rs.ew, off);
+    rc |= dalloc(c, &c->rs.wlist, RES_MAX_WG * RS_WCAP);
+    rc |= dalloc(c, &c->rs.wcnt, 2 * RES_MAX_WG);
     G.w = MG_OMEGA;
     G.cscale = MG_CSCALE;
   }
@@ -932,6 +963,7 @@ static int assemble_nocheck(isph_ctx* c) {
   hipLaunchKernelGGL(k_zero_nnz, dim3(1), dim3(64), 0, c->stream, c->D);
   TLAUNCH(TK_ASSEMBLE, k_ppe_assemble, c->n_hi, c->D);
   c->assembled = true;
+  c->loaded = false;
   return 0;
 }
 
@@ -959,6 +991,11 @@ struct BatchHost {
   std::vector<DevScalars> sc;
   int max_nmb = 0, max_nlev = 0;
   int co_lds = 0;                // LDS bytes of the coarse launch (largest scenario's)
+  ResDev* d_rs = nullptr;        // resident solve: scenario tables
+  std::vector<ResDev> rs;
+  int rs_T = 0, rs_grid = 0;     // its workgroups' size and number (0: launch by launch)
+  size_t rs_lds = 0;
+  const void *rs_setup = nullptr, *rs_solve = nullptr;
 };
 
 static void bh_free(BatchHost* b) {
@@ -967,6 +1004,7 @@ static void bh_free(BatchHost* b) {
   (void)hipFree(b->d_mgs);
   (void)hipFree(b->d_pre);
   (void)hipFree(b->d_sc);
+  (void)hipFree(b->d_rs);
   delete b;
 }
 
@@ -984,6 +1022,8 @@ static int bh_make(isph_ctx* const* ctxs, int S, BatchHost** out) {
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_mgs, sizeof(MgDev) * S);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_pre, sizeof(int) * b->pre.size());
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_sc, sizeof(DevScalars) * S);
+  if (e == hipSuccess) e = hipMalloc((void**)&b->d_rs, sizeof(ResDev) * S);
+  b->rs.resize(S);
   if (e != hipSuccess) {
     set_err(c, "batch tables: %s", hipGetErrorString(e));
     bh_free(b);
@@ -1012,6 +1052,8 @@ static int bh_make(isph_ctx* const* ctxs, int S, BatchHost** out) {
   return 0;
 }
 
+static void bh_plan(BatchHost* b);
+
 // refresh the scenario tables (state pointers swap at every rebin) and the
 // row prefix (the live count can shrink)
 static int bh_refresh(BatchHost* b) {
@@ -1029,7 +1071,74 @@ static int bh_refresh(BatchHost* b) {
                            c->stream));
   HIPCHK(c, hipMemcpyAsync(b->d_pre, b->pre.data(), sizeof(int) * b->pre.size(),
                            hipMemcpyHostToDevice, c->stream));
+  bh_plan(b);
+  if (b->rs_grid)
+    HIPCHK(c, hipMemcpyAsync(b->d_rs, b->rs.data(), sizeof(ResDev) * S, hipMemcpyHostToDevice,
+                             c->stream));
   return 0;
+}
+
+template <int T, int R>
+static int64_t rs_shape(BatchHost* b) {
+  b->rs_T = T;
+  b->rs_setup = reinterpret_cast<const void*>(&kb_rs_setup<T>);
+  b->rs_solve = reinterpret_cast<const void*>(&kb_pb_resident<T, R>);
+  return rs_row_lds<T, R>();
+}
+
+// The resident launch of b's scenarios: the fewest row blocks per workgroup
+// with which every scenario's row workgroups and its coarse one fit the
+// device at one per CU, and the coarse workgroups' first levels.  Leaves
+// rs_grid 0 where the solve has to run launch by launch: kernel timing on,
+// more than 12 row blocks per workgroup, a loaded system, or a device that
+// cannot hold the grid.
+static void bh_plan(BatchHost* b) {
+  b->rs_grid = 0;
+  for (isph_ctx* c : b->ctx)
+    if (c->prof || c->loaded || c->D.nblk > PS_MAX_CHUNKS / 4) return;
+  int nbw = 0, grid = 0;
+  for (int k = 1; k <= 12 && !nbw; k++) {
+    grid = 0;
+    for (isph_ctx* c : b->ctx) grid += (c->D.nblk + k - 1) / k + 1;
+    if (grid <= RES_MAX_WG) nbw = k;
+  }
+  if (!nbw) return;
+  int64_t lds = nbw <= 2   ? rs_shape<512, 1>(b)
+                : nbw <= 4 ? rs_shape<1024, 1>(b)
+                : nbw <= 8 ? rs_shape<1024, 2>(b)
+                           : rs_shape<1024, 3>(b);
+  int wg0 = 0;
+  for (int s = 0; s < b->S; s++) {
+    isph_ctx* c = b->ctx[s];
+    ResDev& q = b->rs[s];
+    q = c->rs;
+    q.wg0 = wg0;
+    q.nbw = nbw;
+    q.G = (c->D.nblk + nbw - 1) / nbw;
+    wg0 += q.G + 1;
+    int l0 = 1;
+    while (l0 < c->G.nlev &&
+           (c->G.lev[l0].n > RS_CO_MAX || rs_coarse_lds(c->G, l0) > RES_LDS_MAX))
+      l0++;
+    q.m = l0 - 1;
+    lds = std::max(lds, rs_coarse_lds(c->G, l0));
+  }
+  if (lds > RES_LDS_MAX || resident_capacity(b->rs_solve, b->rs_T) < grid) return;
+  b->rs_lds = (size_t)lds;
+  b->rs_grid = grid;
+}
+
+static hipError_t bh_rs_setup(BatchHost* b, BatchDev B) {
+  const ResDev* rs = b->d_rs;
+  void* args[] = {&B, &rs};
+  return hipLaunchKernel(b->rs_setup, dim3(b->rs_grid), dim3(b->rs_T), args, 0,
+                         b->ctx[0]->stream);
+}
+static hipError_t bh_resident(BatchHost* b, BatchDev B, int iters, unsigned v0, unsigned ep) {
+  const ResDev* rs = b->d_rs;
+  void* args[] = {&B, &rs, &iters, &v0, &ep};
+  return hipLaunchCooperativeKernel(b->rs_solve, dim3(b->rs_grid), dim3(b->rs_T), args, b->rs_lds,
+                                    b->ctx[0]->stream);
 }
 
 static int bh_gather(BatchHost* b) {
@@ -1141,6 +1250,8 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
   // ||b||, then the FP64 start residual
   BLAUNCH(kb_pb_bnorm, grow, 256, B);
   BLAUNCH(kb_pfinalize, S, 256, B, (int)PFIN_BNORM, 0, 0);
+  bool resident = b->rs_grid > 0;
+  if (resident) HIPCHK(c, bh_rs_setup(b, B));
   BLAUNCH(kb_pb_resid, grow, 256, B, 1);
   BLAUNCH(kb_pfinalize, S, 256, B, (int)PFIN_RESID, 1, 0);
   rc = bh_gather(b);
@@ -1153,6 +1264,17 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
       if (rc) return rc;
     }
   }
+  // the packed columns are window positions in the resident form; back to
+  // offsets where the solve cannot run resident after all
+  bool positions = resident;
+  auto to_launches = [&]() -> int {
+    resident = false;
+    if (positions) BLAUNCH(kb_mg_setup0, grow, 256, B);
+    positions = false;
+    return 0;
+  };
+  for (int s = 0; s < S && resident; s++)
+    if (b->sc[s].counter[PS_FLAG_WIN] && (rc = to_launches())) return rc;
   // packed 16-bit column offsets unless some scenario's rows need int32
   bool off16 = true;
   for (int s = 0; s < S; s++) off16 = off16 && !b->sc[s].far;
@@ -1182,6 +1304,7 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
     return p;
   };
   int chunk = 4, seq = 0;
+  unsigned vtag = 1, ep = 1;  // numbers of the resident form's V-cycles and reductions
   bool guessed = false;  // the chunk just run was sized from the last solve
   if (const int p = predicted(false); p > 0) {
     chunk = p;
@@ -1192,14 +1315,31 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
       set_err(c, "precision solve: scenarios did not finish");
       return ISPH_ENOCONV;
     }
-    rc = off16 ? bh_iterate<true>(b, B, grow, chunk, seq)
-               : bh_iterate<false>(b, B, grow, chunk, seq);
-    if (rc) return rc;
+    if (resident) {
+      if (bh_resident(b, B, RES_ITERS, vtag, ep) == hipSuccess) {
+        vtag += 2u * RES_ITERS;
+        ep += 2u * RES_ITERS;
+      } else {  // refused (another process holds the cooperative queue): nothing ran
+        (void)hipGetLastError();
+        rc = to_launches();
+        if (rc) return rc;
+      }
+    }
+    if (!resident) {
+      rc = off16 ? bh_iterate<true>(b, B, grow, chunk, seq)
+                 : bh_iterate<false>(b, B, grow, chunk, seq);
+      if (rc) return rc;
+    }
     // FP64 check of every scenario whose iteration stopped in this chunk
     BLAUNCH(kb_pb_resid, grow, 256, B, 2);
     BLAUNCH(kb_pfinalize, S, 256, B, (int)PFIN_RESID, 2, 0);
     rc = bh_gather(b);
     if (rc) return rc;
+    for (int s = 0; s < S; s++)
+      if (resident && b->sc[s].counter[PS_FLAG_ABORT]) {
+        set_err(b->ctx[s], "resident PPE solve: a wait ran out");
+        return ISPH_EHIP;
+      }
     // the timed launches that did work: the chunk's leading iterations
     int worked = 0, restarted = 0;
     for (int s = 0; s < S; s++) {
@@ -1903,6 +2043,7 @@ extern "C" int isph_load_system(isph_ctx* c, int32_t n, const int32_t* len, cons
   HIPCHK(c, hipMemcpy(c->D.sc, &s, sizeof s, hipMemcpyHostToDevice));
   set_nhi(c, n);
   c->assembled = true;
+  c->loaded = true;
   return 0;
 }
 
@@ -2269,6 +2410,7 @@ static int ph_step(isph_batch* b, std::vector<isph_solve_stats>& pst, int* worst
   for (isph_ctx* c : b->ctx) {
     c->have_nbr = true;
     c->assembled = true;
+    c->loaded = false;
   }
   // the solves: the precision-form scenarios together, FP64 ones in turn
   if (b->pb) {

@@ -983,6 +983,8 @@ __device__ __forceinline__ void pb_finalize(const Dev& D, int op, int init, int 
       S->fin = 0;
       S->rel = 0.0;
       S->stop_seq = -1;
+#pragma unroll
+      for (int k = 0; k < 4; k++) S->counter[k] = 0u;  // the resident solve's flags
       if (bn == 0.0 || !isfinite(bn)) {
         S->fin = 1;
         S->done = 1;

@@ -1,0 +1,1094 @@
+// isph_mgres.h -- the precision-form BiCGStab (isph_mg.h) of any number of
+// scenarios as one resident launch.
+//
+// The launch-per-phase form takes 18 to 26 dependent launches per iteration,
+// and below a few hundred thousand rows almost all of an iteration is their
+// latency: 92 us at 7,485 rows, 116 us at 22k, 140 us at 137k, where the data
+// of an iteration needs 1, 2 and 12 us.  Here the phases of an iteration
+// meet through memory words instead: every value that another workgroup
+// needs travels as one 64-bit word, the float in its low half and the number
+// of the V-cycle in its high half, and the reader polls the word itself.  No
+// phase waits for more than the words it reads.
+//
+// Work split.  A scenario's row blocks (256 rows) lie in runs of nbw blocks on
+// its row workgroups (1024 threads, up to R rows per thread); one more
+// workgroup per scenario runs the coarse levels, with their stencils and the
+// dense inverse in LDS for the whole solve, and forms the dot products.
+// Windows, row positions and the polling rules are those of isph_persist.h.
+//   level 0   x0 (and ph, sh) of the window's rows by words; the products
+//             gather from LDS
+//   restrict  a cell's rows are summed by the workgroup holding its first
+//             row; rows of the next workgroup arrive by words
+//   levels 1..m   aggregates (down) and cells (up) in equal runs per
+//             workgroup; right-hand sides and corrections by words
+//   levels m+1..  the coarse workgroup
+// The arithmetic and its order are those of the launch-per-phase bodies, so
+// every iterate, scalar and count has the same bits.
+//
+// A word is rewritten one V-cycle later; the dot product between the two has
+// collected partial sums that every reader published after its reads.
+#pragma once
+#include "isph_batch.h"
+#include "isph_persist.h"
+
+#define RS_W 6                      // window elements per thread
+#define RS_WCAP (RS_W * 1024 / PS_CHUNK)
+// Unknowns of the coarse workgroup's first level at most; their stencils stay
+// in registers.  A level more on the row workgroups costs two more hops of
+// ~1.2 us a V-cycle, a level of 1-4 unknowns per thread more in the one
+// workgroup 2-4 us: 1,024 against 2,560 unknowns took 51.0 against 55.8 us
+// per iteration at 7,485 rows and 73.7 against 77.4 at 22k; 300 took 52.4
+// and 74.7.
+#define RS_CO_MAX 1024
+#define RS_PER(T) ((RS_CO_MAX + (T)-1) / (T))
+#define RS_MAIL 16                  // words of a workgroup's mail line
+#define RS_TAIL 256                 // rows of the next workgroups in a workgroup's last cell
+
+struct ResDev {
+  int wg0, G;                 // first workgroup; row workgroups (the coarse one is wg0 + G)
+  int nbw;                    // row blocks per workgroup
+  int m;                      // cell levels 1..m on the row workgroups
+  unsigned long long* slots;  // 10 words per row block
+  unsigned long long* mail;   // RS_MAIL words per workgroup
+  unsigned long long *x0w, *phw, *r0w;  // a word per row: x0, V-cycle result, r0
+  unsigned long long *bw, *ew;          // a word per cell of every level: b, e
+  int32_t* wlist;             // per workgroup: RS_WCAP window chunks
+  int32_t* wcnt;              // per workgroup: their count, and the slot of its own first chunk
+};
+
+// A pointer read from a table, in the global address space (else its
+// accesses are flat ones)
+template <typename V>
+__device__ __forceinline__ V* glob(V* p) {
+  return (V*)(__attribute__((address_space(1))) V*)p;
+}
+template <typename A>
+__device__ __forceinline__ A ld_table(const A* p) {
+  return *(const A*)(const __attribute__((address_space(1))) A*)p;
+}
+
+// One tagged float; the wait is bounded and ends early once a wait of the
+// workgroup has run out
+__device__ __forceinline__ float rs_wait(const unsigned long long* p, unsigned tag,
+                                         volatile int* bad, unsigned long long w) {
+  if ((unsigned)(w >> 32) != tag) {
+    int spin = 0;
+    do {
+      w = ld_agent(p);
+      if (++spin >= PS_SPIN || ((spin & 1023) == 0 && *bad)) {
+        *bad = 1;
+        break;
+      }
+    } while ((unsigned)(w >> 32) != tag);
+  }
+  return __uint_as_float((uint32_t)w);
+}
+// N words together: ld(k) reads word k (a word of the tag itself where lane
+// needs none); all are read again until every one carries the number
+template <int N, typename LD>
+__device__ __forceinline__ void rs_poll(unsigned tag, volatile int* bad, LD ld,
+                                        float (&out)[N]) {
+  for (int spin = 0;;) {
+    unsigned long long w[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) w[k] = ld(k);
+    bool all = true;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      all = all && (unsigned)(w[k] >> 32) == tag;
+      out[k] = __uint_as_float((uint32_t)w[k]);
+    }
+    if (all) return;
+    if (++spin >= PS_SPIN || ((spin & 1023) == 0 && *bad)) {
+      *bad = 1;
+      return;
+    }
+  }
+}
+__device__ __forceinline__ void rs_put(unsigned long long* p, unsigned tag, float v) {
+  st_agent(p, ((unsigned long long)tag << 32) | __float_as_uint(v));
+}
+
+// The level table in LDS: a level's sizes by one LDS read (from memory every
+// use would be a load, a store of the loop before it being in the way)
+__device__ __forceinline__ MgLevel rs_level(const MgLevel* lev, int l) {
+  MgLevel L = lev[l];
+  L.ny = __builtin_amdgcn_readfirstlane(L.ny);
+  L.nx = __builtin_amdgcn_readfirstlane(L.nx);
+  L.n = __builtin_amdgcn_readfirstlane(L.n);
+  L.off = __builtin_amdgcn_readfirstlane(L.off);
+  return L;
+}
+
+// scenario of this workgroup
+__device__ __forceinline__ int rs_locate(const ResDev* rs, int S, int wg) {
+  int s = 0;
+  while (s + 1 < S && rs[s + 1].wg0 <= wg) s++;
+  return s;
+}
+
+// Windows, window positions (into D.aoff) and cleared words, one workgroup
+// per row workgroup of the solve
+template <int T>
+__global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
+  __shared__ uint16_t map[PS_MAX_CHUNKS];
+  __shared__ int cnt[T];
+  const int wcap = RS_W * T / PS_CHUNK;
+  const int s = rs_locate(rs, B.S, blockIdx.x), t = threadIdx.x;
+  const ResDev& Q = rs[s];
+  const Dev& D = B.devs[s];
+  const MgDev& G = B.mgs[s];
+  const int wg = blockIdx.x - Q.wg0;
+  if (wg >= Q.G) {  // the coarse workgroup's place
+    return;
+  }
+  const int n = D.sc->n, cap = D.cap, nblk = D.nblk;
+  const int nch = (n + PS_CHUNK - 1) / PS_CHUNK;
+  const int i0 = wg * Q.nbw * RED_BLOCK;
+  const int i1 = min(n, min(nblk, (wg + 1) * Q.nbw) * RED_BLOCK);
+  const int32_t* acol = glob(D.acol);
+  const int32_t* alen = glob(D.alen);
+  uint32_t* lidx = glob(D.aoff);
+  for (int b = wg * Q.nbw * 10 + t; b < min(nblk, (wg + 1) * Q.nbw) * 10; b += T)
+    Q.slots[b] = 0;
+  if (t < RS_MAIL) Q.mail[wg * RS_MAIL + t] = 0;
+  for (int i = i0 + t; i < i1; i += T) {
+    Q.x0w[i] = 0;
+    Q.phw[i] = 0;
+    Q.r0w[i] = 0;
+  }
+  const int tot = G.lev[G.nlev].off + G.lev[G.nlev].n;
+  for (int c = (int)((int64_t)tot * wg / Q.G) + t; c < (int)((int64_t)tot * (wg + 1) / Q.G);
+       c += T) {
+    Q.bw[c] = 0;
+    Q.ew[c] = 0;
+  }
+  for (int c = t; c < nch; c += T) map[c] = 0;
+  __syncthreads();
+  for (int i = i0 + t; i < i1; i += T) {
+    const int L = alen[i];
+    map[i / PS_CHUNK] = 1;  // its own rows, in order, whatever the columns
+    for (int k0 = 0; k0 < L; k0 += 8) {
+      int c[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) c[u] = acol[((k0 + u < L) ? k0 + u : k0) * cap + i];
+#pragma unroll
+      for (int u = 0; u < 8; u++) map[c[u] / PS_CHUNK] = 1;
+    }
+  }
+  __syncthreads();
+  const int per = (nch + T - 1) / T, c0 = t * per, c1 = min(nch, c0 + per);
+  int own = 0;
+  for (int c = c0; c < c1; c++) own += map[c];
+  cnt[t] = own;
+  __syncthreads();
+  for (int off = 1; off < T; off <<= 1) {
+    const int a = (t >= off) ? cnt[t - off] : 0;
+    __syncthreads();
+    cnt[t] += a;
+    __syncthreads();
+  }
+  const int total = cnt[T - 1];
+  // rows of the last cell in later workgroups (rs_rows_solve's tail)
+  int tail = 0;
+  if (i1 > i0 && i1 < n) {
+    const int k = D.cell[i1 - 1];
+    tail = D.cstart[k + 1] - i1;
+  }
+  if (total > wcap || tail > RS_TAIL) {  // the whole workgroup
+    if (t == 0) atomicOr(&D.sc->counter[PS_FLAG_WIN], 1u);
+    return;
+  }
+  int pos = cnt[t] - own;
+  for (int c = c0; c < c1; c++)
+    if (map[c]) {
+      Q.wlist[(size_t)wg * RS_WCAP + pos] = c;
+      if (c == i0 / PS_CHUNK) Q.wcnt[2 * wg + 1] = pos;
+      map[c] = (uint16_t)pos++;
+    }
+  if (t == 0) Q.wcnt[2 * wg] = total;
+  __syncthreads();
+  for (int i = i0 + t; i < i1; i += T) {
+    const int L = alen[i];
+    for (int k0 = 0; k0 < L; k0 += 8) {
+      int c[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) c[u] = acol[((k0 + u < L) ? k0 + u : k0) * cap + i];
+#pragma unroll
+      for (int u = 0; u < 8; u += 2) {
+        if (k0 + u >= L) break;
+        const uint32_t a = map[c[u] / PS_CHUNK] * PS_CHUNK + c[u] % PS_CHUNK;
+        const uint32_t b = map[c[u + 1] / PS_CHUNK] * PS_CHUNK + c[u + 1] % PS_CHUNK;
+        lidx[((k0 + u) >> 1) * cap + i] = a | (b << 16);
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------
+// rows
+// ---------------------------------------------------------------------
+// sum of the row's FP16 values times the window's floats, in entry order
+// (the order of ell_row_sum_h)
+template <bool FULL>
+__device__ __forceinline__ float rs_row_h8(const uint32_t*& ip, const uint32_t*& hp, int cap,
+                                           unsigned i, int k0, int L, int Lm, const float* X,
+                                           float acc) {
+  uint32_t w[4], h[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    w[q] = h[q] = 0u;
+    if (FULL || k0 + 2 * q < Lm) {
+      w[q] = *ps_at(ip, i);
+      h[q] = *ps_at(hp, i);
+    }
+    ip += cap;
+    hp += cap;
+  }
+  float g[8];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    w[q] = (k0 + 2 * q < L) ? w[q] : 0u;
+    g[2 * q] = X[w[q] & 0xffffu];
+    g[2 * q + 1] = X[w[q] >> 16];
+  }
+#pragma unroll
+  for (int u = 0; u < 8; u++) {
+    const unsigned short hb = (unsigned short)((u & 1) ? (h[u / 2] >> 16) : (h[u / 2] & 0xffffu));
+    const float a = acc + __half2float(__ushort_as_half(hb)) * g[u];
+    acc = (k0 + u < L) ? a : acc;
+  }
+  return acc;
+}
+__device__ __forceinline__ float rs_row_h(const uint32_t* ip, const uint32_t* hp, int cap,
+                                          unsigned i, int L, int Lm, const float* X) {
+  float acc = 0.0f;
+  int k0 = 0;
+#pragma unroll 1
+  for (; k0 + 8 <= Lm; k0 += 8) {
+    acc = rs_row_h8<true>(ip, hp, cap, i, k0, L, Lm, X, acc);
+  }
+  if (k0 < Lm) acc = rs_row_h8<false>(ip, hp, cap, i, k0, L, Lm, X, acc);
+  return acc;
+}
+// sum of the row's FP64 values times the window's floats, in entry order
+template <bool FULL>
+__device__ __forceinline__ double rs_row_d8(const uint32_t*& ip, const double*& vp, int cap,
+                                            unsigned i, int k0, int L, int Lm, const float* X,
+                                            double acc) {
+  uint32_t w[4];
+  double v[8];
+  float g[8];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    w[q] = 0u;
+    if (FULL || k0 + 2 * q < Lm) w[q] = *ps_at(ip, i);
+    ip += cap;
+  }
+#pragma unroll
+  for (int u = 0; u < 8; u++) {
+    v[u] = 0.0;
+    if (FULL || k0 + u < Lm) v[u] = *ps_at(vp, i);
+    vp += cap;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    w[q] = (k0 + 2 * q < L) ? w[q] : 0u;
+    g[2 * q] = X[w[q] & 0xffffu];
+    g[2 * q + 1] = X[w[q] >> 16];
+  }
+#pragma unroll
+  for (int u = 0; u < 8; u++) {
+    const double a = acc + v[u] * (double)g[u];
+    acc = (k0 + u < L) ? a : acc;
+  }
+  return acc;
+}
+__device__ __forceinline__ double rs_row_d(const uint32_t* ip, const double* vp, int cap,
+                                           unsigned i, int L, int Lm, const float* X) {
+  double acc = 0.0;
+  int k0 = 0;
+#pragma unroll 1
+  for (; k0 + 8 <= Lm; k0 += 8) {
+    acc = rs_row_d8<true>(ip, vp, cap, i, k0, L, Lm, X, acc);
+  }
+  if (k0 < Lm) acc = rs_row_d8<false>(ip, vp, cap, i, k0, L, Lm, X, acc);
+  return acc;
+}
+
+// ---------------------------------------------------------------------
+// dot products: the row workgroups publish their blocks' partial sums, the
+// coarse workgroup sums them in the order of final_tree2 and sends the sums
+// to each workgroup's mail line
+// ---------------------------------------------------------------------
+template <int T, int R, int NV>
+__device__ __forceinline__ bool rs_publish_wait(const ResDev& Q, int wg, int nblk, unsigned ep,
+                                                const double (&v)[NV][R], double* area,
+                                                double* res, volatile int* bad,
+                                                double (&out)[NV]) {
+  constexpr int S4 = T / 256;
+  const int t = threadIdx.x, wv = (t >> 6) & 3, l = t & 63, sub = t >> 8;
+  // tree j = k R + q of a block is summed by wavefront j mod 4 of its four;
+  // the other three leave their values in LDS
+#pragma unroll
+  for (int k = 0; k < NV; k++)
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      const int j = k * R + q, o = j & 3;
+      if (wv != o) area[(j * S4 + sub) * 192 + (wv < o ? wv : wv - 1) * 64 + l] = v[k][q];
+    }
+  __syncthreads();
+  unsigned long long* slots = glob(Q.slots);
+  const int b0 = wg * Q.nbw;
+#pragma unroll
+  for (int k = 0; k < NV; k++)
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      const int j = k * R + q, o = j & 3;
+      if (wv == o) {
+        const double* a = area + (j * S4 + sub) * 192 + l;
+        const double w0 = (o == 0) ? v[k][q] : a[0];
+        const double w1 = (o == 1) ? v[k][q] : a[(o < 1 ? 0 : 1) * 64];
+        const double w2 = (o == 2) ? v[k][q] : a[(o < 2 ? 1 : 2) * 64];
+        const double w3 = (o == 3) ? v[k][q] : a[2 * 64];
+        const double s = wave_tree((w0 + w2) + (w1 + w3));
+        const int lb = q * S4 + sub;
+        if (l == 0 && lb < Q.nbw && b0 + lb < nblk)
+          ps_publish(&slots[2 * ((size_t)k * nblk + b0 + lb)], ep, s);
+      }
+    }
+  if (t < 2 * NV) {
+    const unsigned long long* p = glob(Q.mail) + wg * RS_MAIL + t;
+    const float f = rs_wait(p, ep, bad, 0ull);
+    reinterpret_cast<uint32_t*>(res)[t] = __float_as_uint(f);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; k++) out[k] = res[k];
+  return !*bad;
+}
+
+template <int T, int NV>
+__device__ __forceinline__ bool rs_collect_send(const ResDev& Q, int nblk, unsigned ep,
+                                                double* col, double* res, volatile int* bad,
+                                                double (&out)[NV]) {
+  const int t = threadIdx.x, l = t & 63, wave = t >> 6;
+  const unsigned long long* slots = glob(Q.slots);
+  // thread t sums column t & 255 (blocks c, c + 256, ...) of one or two values
+  for (int e = t; e < NV * 256; e += T) {
+    const int k = e >> 8, c = e & 255;
+    const unsigned long long* p = slots + 2 * (size_t)k * nblk;
+    double a = 0.0;
+    for (int b0 = c; b0 < nblk; b0 += 4 * 256) {
+      unsigned long long w[4][2];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int b = min(b0 + 256 * u, nblk - 1);
+        w[u][0] = ld_agent(p + 2 * (size_t)b);
+        w[u][1] = ld_agent(p + 2 * (size_t)b + 1);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int b = b0 + 256 * u;
+        if (b < nblk) {
+          const uint32_t lo = __float_as_uint(rs_wait(p + 2 * (size_t)b, ep, bad, w[u][0]));
+          const uint32_t hi = __float_as_uint(rs_wait(p + 2 * (size_t)b + 1, ep, bad, w[u][1]));
+          a = a + __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+        }
+      }
+    }
+    col[e] = a;
+  }
+  __syncthreads();
+  if (wave < NV) {
+    const double* c = col + wave * 256;
+    const double s = wave_tree((c[l] + c[l + 128]) + (c[l + 64] + c[l + 192]));
+    if (l == 0) res[wave] = s;
+  }
+  __syncthreads();
+  if (*bad) return false;
+#pragma unroll
+  for (int k = 0; k < NV; k++) out[k] = res[k];
+  unsigned long long* mail = glob(Q.mail);
+  for (int e = t; e < Q.G * 2 * NV; e += T) {
+    const int g = e / (2 * NV), j = e - g * 2 * NV;
+    st_agent(&mail[g * RS_MAIL + j], ((unsigned long long)ep << 32) |
+                                         reinterpret_cast<const uint32_t*>(res)[j]);
+  }
+  return true;
+}
+
+// A scenario's hierarchy: the level table in LDS, uniform pointers
+struct RsMg {
+  const MgLevel* lev;
+  const float *sten, *rdg;
+  float w, c;
+};
+
+// The scalars of an iteration, formed alike by every workgroup of the scenario
+// (pb_finalize: PFIN_ALPHA, PFIN_OMEGA)
+struct RsScalars {
+  double rho, alpha, omega, beta, rr, rel;
+  int iters, conv, brk, done;
+  bool update;  // the stopped iteration's x and r update still applies
+};
+__device__ __forceinline__ void rs_alpha(RsScalars& z, double s0) {
+  z.alpha = z.rho / s0;
+  if (!isfinite(z.alpha)) {
+    z.brk = 1;
+    z.done = 1;
+  }
+}
+__device__ __forceinline__ void rs_omega(RsScalars& z, const double (&s)[5], double stop,
+                                         double bnorm, int max_iter) {
+  const double om = s[0] / s[1];
+  z.omega = om;
+  z.update = false;
+  if (!isfinite(om) || om == 0.0) {
+    z.brk = 1;
+    z.done = 1;
+    return;
+  }
+  z.update = true;
+  const double rr0 = s[4] - om * s[0], rr = (rr0 < 0.0) ? 0.0 : rr0;
+  const double rhon = s[3] - om * s[2];
+  z.iters++;
+  z.rr = rr;
+  z.rel = sqrt(rr) / bnorm;
+  if (sqrt(rr) <= stop) {
+    z.conv = 1;
+    z.done = 1;
+  } else if (rhon == 0.0 || !isfinite(rhon) || !isfinite(rr)) {
+    z.brk = 1;
+    z.done = 1;
+  } else {
+    z.beta = (rhon / z.rho) * (z.alpha / om);
+    z.rho = rhon;
+    if (z.iters >= max_iter) z.done = 1;
+  }
+}
+
+// ---------------------------------------------------------------------
+// cell levels on the row workgroups (mg_lvl_down, mg_lvl_up)
+// ---------------------------------------------------------------------
+// first item of workgroup w of G's equal runs over n items
+__device__ __forceinline__ int rs_part(int n, int w, int G) { return (int)((int64_t)n * w / G); }
+
+template <int T>
+__device__ __forceinline__ void rs_down(const RsMg& M, const ResDev& Q, int wg, int t,
+                                        int l, unsigned tag, volatile int* bad) {
+  const MgLevel L = rs_level(M.lev, l), C = rs_level(M.lev, l + 1);
+  const float w = M.w;
+  const float* st = M.sten + 9 * (size_t)L.off;
+  const float* rd = M.rdg + L.off;
+  unsigned long long* bw = glob(Q.bw);
+  const unsigned long long* bl = bw + L.off;
+  const int J0 = rs_part(C.n, wg, Q.G), J1 = rs_part(C.n, wg + 1, Q.G);
+  for (int e = t; e < 4 * (J1 - J0); e += T) {
+    const int J = J0 + (e >> 2), q = e & 3;
+    const int CJ = J / C.ny, CI = J - CJ * C.ny;
+    const int ci = 2 * CI + (q & 1), cj = 2 * CJ + (q >> 1);
+    const bool in = ci < L.ny && cj < L.nx;
+    const int I = in ? cj * L.ny + ci : 0;
+    int Nb[9];
+    mg_nbr9(L, in ? ci : 0, in ? cj : 0, I, Nb);
+    float sv[9], rv[9], bv[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      Nb[k] = Nb[k] >= 0 ? Nb[k] : (I | (1 << 30));  // bit 30: a term that is not added
+      sv[k] = *ps_at(st + (size_t)k * L.n, I);
+      rv[k] = *ps_at(rd, Nb[k] & ~(1 << 30));
+    }
+    rs_poll<9>(tag, bad, [&](int k) { return ld_agent(ps_at(bl, Nb[k] & ~(1 << 30))); }, bv);
+    float acc = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      const float tk = sv[k] * ((w * bv[k]) * rv[k]);
+      if (!(Nb[k] >> 30)) acc = acc + tk;
+    }
+    const float bI = bv[4];
+    const float res = in ? bI - acc : 0.0f;
+    const int lane = t & 63, base = lane & ~3;
+    const float r1 = __shfl(res, base + 1, 64), r2 = __shfl(res, base + 2, 64),
+                r3 = __shfl(res, base + 3, 64);
+    const int in_mask = __shfl((int)in, base + 1, 64) | (__shfl((int)in, base + 2, 64) << 1) |
+                        (__shfl((int)in, base + 3, 64) << 2);
+    if (q == 0) {
+      float s = 0.0f;
+      if (in) s = s + res;
+      if (in_mask & 1) s = s + r1;
+      if (in_mask & 2) s = s + r2;
+      if (in_mask & 4) s = s + r3;
+      rs_put(ps_at(bw + C.off, J), tag, s);
+    }
+  }
+}
+
+template <int T>
+__device__ __forceinline__ void rs_up(const RsMg& M, const ResDev& Q, int wg, int t,
+                                      int l, unsigned tag, volatile int* bad) {
+  const MgLevel L = rs_level(M.lev, l), C = rs_level(M.lev, l + 1);
+  const float w = M.w, c = M.c;
+  const float* st = M.sten + 9 * (size_t)L.off;
+  const float* rd = M.rdg + L.off;
+  const unsigned long long* bw = glob(Q.bw) + L.off;
+  unsigned long long* ew = glob(Q.ew);
+  const unsigned long long* ec = ew + C.off;
+  const int I0 = rs_part(L.n, wg, Q.G), I1 = rs_part(L.n, wg + 1, Q.G);
+  for (int I = I0 + t; I < I1; I += T) {
+    const int cj = I / L.ny, ci = I - cj * L.ny;
+    const int pI = (cj >> 1) * C.ny + (ci >> 1);
+    int Nb[9], Pa[9];
+    mg_nbr9(L, ci, cj, I, Nb);
+    mg_par9(C, ci, cj, Pa);
+    float sv[9], xv[9], xc[9];
+    unsigned has = 0;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      if (Nb[k] >= 0) has |= 1u << k;
+      else Nb[k] = I, Pa[k] = pI;  // read in place of a missing one; its term is not added
+      sv[k] = *ps_at(st + (size_t)k * L.n, I);
+    }
+    rs_poll<9>(tag, bad, [&](int k) { return ld_agent(ps_at(bw, Nb[k])); }, xv);
+    const float bI = xv[4], rI = *ps_at(rd, I);
+#pragma unroll
+    for (int k = 0; k < 9; k++) xv[k] = (w * xv[k]) * *ps_at(rd, Nb[k]);
+    rs_poll<9>(tag, bad, [&](int k) { return ld_agent(ps_at(ec, Pa[k])); }, xc);
+    float acc = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      xv[k] = xv[k] + c * xc[k];
+      const float tk = sv[k] * xv[k];
+      if ((has >> k) & 1) acc = acc + tk;
+    }
+    const float x1 = xv[4];
+    rs_put(ps_at(ew + L.off, I), tag, x1 + (w * (bI - acc)) * rI);
+  }
+}
+
+// ---------------------------------------------------------------------
+// the coarse workgroup (mg_coarse_block with its data kept in LDS and
+// registers over the solve)
+// ---------------------------------------------------------------------
+template <int T>
+__device__ __forceinline__ void rs_coarse_solve(const Dev& D, const MgDev& M, const ResDev& Q,
+                                                const MgLevel* lev,
+                                                int iters, unsigned v0, unsigned ep,
+                                                double* lds) {
+  constexpr int PER = RS_PER(T);
+  const int t0 = threadIdx.x;
+  DevScalars* Sc = glob(D.sc);
+  const int nblk = D.nblk, nl = M.nlev, l0 = Q.m + 1;
+  const float w = M.w, c = M.cscale;
+  double* col = lds;
+  double* res = lds + 5 * 256;
+  volatile int* bad = reinterpret_cast<int*>(res + 6);
+  const MgLevel L0 = rs_level(lev, l0), LD = rs_level(lev, nl);
+  const int base = L0.off;
+  const int S = LD.off + LD.n - base;
+  const int stb = (l0 < nl) ? rs_level(lev, l0 + 1).off : LD.off;
+  const int nst = 9 * (LD.off - stb), nrd = nst / 9, nd2 = LD.n * LD.n;
+  double* DI = res + 8;
+  float* X = reinterpret_cast<float*>(DI + nd2);
+  float* Bv = X + S;
+  float* R = X + 2 * S;
+  float* ST = X + 3 * S;
+  float* RD = ST + nst;
+  const float* sten = glob(M.sten);
+  const float* rdg = glob(M.rdg);
+  const double* dinv = glob(M.dense_inv);
+  if (t0 == 0) *bad = 0;
+  for (int e = t0; e < nd2; e += T) DI[e] = dinv[e];
+  for (int e = t0; e < nst; e += T) ST[e] = sten[9 * (size_t)stb + e];
+  for (int e = t0; e < nrd; e += T) RD[e] = rdg[stb + e];
+  float st0[PER][9], rd0[PER];
+  int ci0[PER], cj0[PER];
+#pragma unroll
+  for (int q = 0; q < PER; q++) {
+    const int I = t0 + q * T, Ic = (I < L0.n) ? I : 0;
+    const float* sg = sten + 9 * (size_t)L0.off;
+#pragma unroll
+    for (int k = 0; k < 9; k++) st0[q][k] = sg[k * L0.n + Ic];
+    rd0[q] = rdg[base + Ic];
+    cj0[q] = Ic / L0.ny;
+    ci0[q] = Ic - cj0[q] * L0.ny;
+  }
+  const unsigned long long* bw = glob(Q.bw) + base;
+  unsigned long long* ew = glob(Q.ew) + base;
+  RsScalars z;
+  z.rho = Sc->rho;
+  z.iters = Sc->iters;
+  z.conv = z.brk = z.done = 0;
+  z.alpha = z.omega = z.beta = z.rr = z.rel = 0.0;
+  const double bnorm = Sc->bnorm;
+  const double frac = (D.P.inner_tol > 0.0) ? D.P.inner_tol : PB_STOP_FRAC;
+  const double stop = frac * D.P.tol * bnorm;
+  const int max_iter = D.P.max_iter;
+  __syncthreads();
+  for (int it = 0; it < iters; it++) {
+#pragma unroll 1
+    for (int half = 0; half < 2; half++) {
+      const unsigned tag = v0 + 2 * it + half;
+      // (opaque: or the compiler holds every address formed from these in
+      // registers over the iterations)
+      int t = threadIdx.x;
+      asm volatile("" : "+v"(t));
+#pragma unroll
+      for (int q = 0; q < PER; q++) asm volatile("" : "+v"(ci0[q]), "+v"(cj0[q]));
+      // right-hand side of the first level
+      float bq[PER];
+      rs_poll<PER>(tag, bad, [&](int q) {
+        return (t + q * T < L0.n) ? ld_agent(ps_at(bw, t + q * T)) : (unsigned long long)tag << 32;
+      }, bq);
+#pragma unroll
+      for (int q = 0; q < PER; q++) {
+        const int I = t + q * T;
+        if (I < L0.n) {
+          Bv[I] = bq[q];
+          if (l0 < nl) X[I] = (w * bq[q]) * rd0[q];
+        }
+      }
+      __syncthreads();
+      for (int l = l0; l < nl; l++) {
+        const MgLevel L = rs_level(lev, l), C = rs_level(lev, l + 1);
+        float* x = X + (L.off - base);
+        const float* b = Bv + (L.off - base);
+        float* r = R + (L.off - base);
+        if (l == l0) {
+#pragma unroll
+          for (int q = 0; q < PER; q++) {
+            const int I = t + q * T;
+            __builtin_amdgcn_sched_barrier(0);  // one unknown's values in registers at a time
+            if (I < L.n) {
+              float acc = 0.0f, tk[9];
+              int Nb[9];
+              mg_nbr9(L, ci0[q], cj0[q], I, Nb);
+#pragma unroll
+              for (int k = 0; k < 9; k++) tk[k] = st0[q][k] * x[Nb[k] >= 0 ? Nb[k] : I];
+#pragma unroll
+              for (int k = 0; k < 9; k++)
+                if (Nb[k] >= 0) acc = acc + tk[k];
+              r[I] = bq[q] - acc;
+            }
+          }
+        } else {
+          const float* st = ST + 9 * (L.off - stb);
+          for (int I = t; I < L.n; I += T) {
+            const int cj = I / L.ny, ci = I - cj * L.ny;
+            float acc = 0.0f, tk[9];
+            int Nb[9];
+            mg_nbr9(L, ci, cj, I, Nb);
+#pragma unroll
+            for (int k = 0; k < 9; k++) tk[k] = st[k * L.n + I] * x[Nb[k] >= 0 ? Nb[k] : I];
+#pragma unroll
+            for (int k = 0; k < 9; k++)
+              if (Nb[k] >= 0) acc = acc + tk[k];
+            r[I] = b[I] - acc;
+          }
+        }
+        __syncthreads();
+        // restricted right-hand side, and its pre-smoothed iterate
+        float* bc = Bv + (C.off - base);
+        float* xn = X + (C.off - base);
+        for (int J = t; J < C.n; J += T) {
+          const int CJ = J / C.ny, CI = J - CJ * C.ny;
+          float s = 0.0f;
+#pragma unroll
+          for (int bb = 0; bb < 2; bb++)
+#pragma unroll
+            for (int a = 0; a < 2; a++) {
+              const int ci = 2 * CI + a, cj = 2 * CJ + bb;
+              if (ci < L.ny && cj < L.nx) s = s + r[cj * L.ny + ci];
+            }
+          bc[J] = s;
+          if (l + 1 < nl) xn[J] = (w * s) * RD[C.off - stb + J];
+        }
+        __syncthreads();
+      }
+      {
+        const float* b = Bv + (LD.off - base);
+        float* x = X + (LD.off - base);
+        for (int I = t; I < LD.n; I += T) {
+          double acc = 0.0;
+#pragma unroll 8
+          for (int J = 0; J < LD.n; J++) acc = acc + DI[J * LD.n + I] * (double)b[J];
+          x[I] = (float)acc;
+          if (l0 == nl) rs_put(&ew[I], tag, (float)acc);
+        }
+        __syncthreads();
+      }
+      for (int l = nl - 1; l >= l0; l--) {
+        const MgLevel L = rs_level(lev, l), C = rs_level(lev, l + 1);
+        const float* x = X + (L.off - base);
+        const float* b = Bv + (L.off - base);
+        const float* xc = (l + 1 == nl ? X : R) + (C.off - base);
+        float* out = R + (L.off - base);
+        if (l == l0) {
+#pragma unroll
+          for (int q = 0; q < PER; q++) {
+            const int I = t + q * T;
+            __builtin_amdgcn_sched_barrier(0);
+            if (I < L.n) {
+              const int ci = ci0[q], cj = cj0[q];
+              float acc = 0.0f, tk[9];
+              int Nb[9], Pa[9];
+              mg_nbr9(L, ci, cj, I, Nb);
+              mg_par9(C, ci, cj, Pa);
+              const int pI = (cj >> 1) * C.ny + (ci >> 1);
+#pragma unroll
+              for (int k = 0; k < 9; k++) {
+                const bool has = Nb[k] >= 0;
+                tk[k] = st0[q][k] * (x[has ? Nb[k] : I] + c * xc[has ? Pa[k] : pI]);
+              }
+#pragma unroll
+              for (int k = 0; k < 9; k++)
+                if (Nb[k] >= 0) acc = acc + tk[k];
+              const float x1 = x[I] + c * xc[pI];
+              rs_put(&ew[I], tag, x1 + (w * (bq[q] - acc)) * rd0[q]);
+            }
+          }
+        } else {
+          const float* st = ST + 9 * (L.off - stb);
+          for (int I = t; I < L.n; I += T) {
+            const int cj = I / L.ny, ci = I - cj * L.ny;
+            float acc = 0.0f, tk[9];
+            int Nb[9], Pa[9];
+            mg_nbr9(L, ci, cj, I, Nb);
+            mg_par9(C, ci, cj, Pa);
+            const int pI = (cj >> 1) * C.ny + (ci >> 1);
+#pragma unroll
+            for (int k = 0; k < 9; k++) {
+              const bool has = Nb[k] >= 0;
+              tk[k] = st[k * L.n + I] * (x[has ? Nb[k] : I] + c * xc[has ? Pa[k] : pI]);
+            }
+#pragma unroll
+            for (int k = 0; k < 9; k++)
+              if (Nb[k] >= 0) acc = acc + tk[k];
+            const float x1 = x[I] + c * xc[pI];
+            out[I] = x1 + (w * (b[I] - acc)) * RD[(L.off - stb) + I];
+          }
+        }
+        __syncthreads();
+      }
+      if (half == 0) {
+        double o[1];
+        if (!rs_collect_send<T, 1>(Q, nblk, ep++, col, res, bad, o)) return;
+        rs_alpha(z, o[0]);
+        if (z.done) break;
+      } else {
+        double o[5];
+        if (!rs_collect_send<T, 5>(Q, nblk, ep++, col, res, bad, o)) return;
+        rs_omega(z, o, stop, bnorm, max_iter);
+      }
+    }
+    if (z.done) break;
+  }
+  if (t0 == 0) {
+    Sc->rho = z.rho;
+    Sc->alpha = z.alpha;
+    Sc->omega = z.omega;
+    Sc->beta = z.beta;
+    Sc->rr = z.rr;
+    Sc->rel = z.rel;
+    Sc->iters = z.iters;
+    Sc->conv = z.conv;
+    Sc->brk = z.brk;
+    Sc->done = z.done;
+  }
+}
+
+// ---------------------------------------------------------------------
+// the row workgroups
+// ---------------------------------------------------------------------
+template <int T, int R>
+__device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, const ResDev& Q,
+                                              const MgLevel* lev,
+                                              int wg, int iters, unsigned v0, unsigned ep,
+                                              double* lds) {
+  constexpr int S4 = T / 256;
+  const int t = threadIdx.x, l = t & 63;
+  DevScalars* Sc = glob(D.sc);
+  const int n = Sc->n, nblk = D.nblk, cap = D.cap;
+  const int i0 = wg * Q.nbw * RED_BLOCK, i1 = min(n, min(nblk, (wg + 1) * Q.nbw) * RED_BLOCK);
+  double* area = lds;                      // 5 R S 192 doubles
+  double* res = lds + 5 * R * S4 * 192;
+  volatile int* bad = reinterpret_cast<int*>(res + 6);
+  float* X = reinterpret_cast<float*>(res + 8);  // the window
+  float* r0s = X + RS_W * T;                  // r0 of the workgroup's rows
+  if (t == 0) *bad = 0;
+  unsigned long long* x0w = glob(Q.x0w);
+  unsigned long long* phw = glob(Q.phw);
+  unsigned long long* r0w = glob(Q.r0w);
+  const MgLevel L1 = rs_level(lev, 1);
+  unsigned long long* b1w = glob(Q.bw) + L1.off;
+  const unsigned long long* e1w = glob(Q.ew) + L1.off;
+  const RsMg H{lev, glob(M.sten), glob(M.rdg), M.w, M.cscale};
+  const uint32_t* lidx = glob(D.aoff);
+  const uint32_t* av16 = glob(D.av16);
+  const double* aval = glob(D.aval);
+  const int32_t* cstart = glob(D.cstart);
+  const int32_t* cell = glob(D.cell);
+  double* sol = glob(D.sol);
+  const float mw = M.w, mc = M.cscale;
+  // this thread's rows: local row q T + t
+  const int32_t* wl = glob(Q.wlist) + (size_t)wg * RS_WCAP;
+  const int wn = glob(Q.wcnt)[2 * wg], s0 = glob(Q.wcnt)[2 * wg + 1];
+  int row[R], len[R], lmx[R];
+  float p[R], rh[R], d0[R];
+  double r[R];
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    const int i = i0 + q * T + t;
+    const bool in = i < i1;
+    row[q] = in ? i : -1;
+    len[q] = in ? glob(D.alen)[i] : 0;
+    lmx[q] = wave_max(len[q]);
+    p[q] = in ? glob(D.pp32)[i] : 0.0f;
+    rh[q] = in ? glob(D.rh32)[i] : 0.0f;
+    d0[q] = in ? glob(M.d0)[i] : 0.0f;
+    r[q] = in ? glob(D.r)[i] : 0.0;
+  }
+  // window elements: chunk (uniform per wavefront), cell of the row; own
+  // chunks hold the workgroup's rows at positions s0 * 64 + local row
+  const int oc0 = i0 / PS_CHUNK, oc1 = (i1 + PS_CHUNK - 1) / PS_CHUNK;
+  int wc[RS_W], wk[RS_W];
+#pragma unroll
+  for (int w = 0; w < RS_W; w++) {
+    const int s = w * (T / PS_CHUNK) + t / PS_CHUNK;
+    wc[w] = __builtin_amdgcn_readfirstlane((s < wn) ? wl[s] : -1);
+    const int g = wc[w] * PS_CHUNK + l;
+    wk[w] = (wc[w] >= 0 && g < n) ? cell[g] : -1;
+  }
+  // cells whose first row is here, with the empty ones up to the next
+  // workgroup's first; rows of a cell begun earlier are sent to its workgroup
+  auto first_owned = [&](int i) {
+    const int k = cell[i];
+    return cstart[k] == i ? k : k + 1;
+  };
+  const int K0 = wg == 0 ? 0 : (i0 >= n ? L1.n : first_owned(i0));
+  const int K1 = i1 >= n ? L1.n : first_owned(i1);
+  int head = 0;
+  if (i0 < n) {
+    const int k = cell[i0];
+    if (cstart[k] < i0) head = min(cstart[k + 1], i1) - i0;
+  }
+  const int tail = (K1 > K0 && i0 < i1 && i1 < n) ? cstart[K1] - i1 : 0;
+  int ca0 = 0, ca1 = 0;  // local rows of this thread's first cell
+  if (K0 + t < K1) {
+    ca0 = cstart[K0 + t] - i0;
+    ca1 = cstart[K0 + t + 1] - i0;
+  }
+  RsScalars z;
+  z.rho = Sc->rho;
+  z.iters = Sc->iters;
+  z.conv = z.brk = z.done = 0;
+  z.alpha = z.omega = z.beta = z.rr = z.rel = 0.0;
+  const double bnorm = Sc->bnorm;
+  const double frac = (D.P.inner_tol > 0.0) ? D.P.inner_tol : PB_STOP_FRAC;
+  const double stop = frac * D.P.tol * bnorm;
+  const int max_iter = D.P.max_iter;
+  double t1[R];
+  float ph[R], sh[R];
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    t1[q] = 0.0;
+    ph[q] = 0.0f;
+  }
+  __syncthreads();
+  bool ok = true;
+  for (int it = 0; it < iters && ok; it++) {
+#pragma unroll 1
+    for (int half = 0; half < 2; half++) {
+      const unsigned tag = v0 + 2 * it + half;
+      // (opaque: or the compiler holds every address formed from these in
+      // registers over the iterations)
+      int t = threadIdx.x;
+      asm volatile("" : "+v"(t));
+#pragma unroll
+      for (int q = 0; q < R; q++) asm volatile("" : "+v"(row[q]));
+#pragma unroll
+      for (int w = 0; w < RS_W; w++) asm volatile("" : "+v"(wk[w]));
+      const int l = t & 63;
+      // ---- V-cycle of v = p (half 0) or s, which is in r (half 1)
+      float v[R];
+#pragma unroll
+      for (int q = 0; q < R; q++) {
+        v[q] = half ? (float)r[q] : p[q];
+        if (row[q] >= 0) {
+          const float x0 = (mw * v[q]) * d0[q];
+          rs_put(ps_at(x0w, row[q]), tag, x0);
+          X[s0 * PS_CHUNK + q * T + t] = x0;
+        }
+      }
+      auto window = [&](const unsigned long long* words) {
+        float e[RS_W];
+        auto other = [&](int w) {
+          return wc[w] >= 0 && (wc[w] < oc0 || wc[w] >= oc1) && wk[w] >= 0;
+        };
+        rs_poll<RS_W>(tag, bad, [&](int w) {
+          return other(w) ? ld_agent(ps_at(words + (int64_t)wc[w] * PS_CHUNK, l))
+                          : (unsigned long long)tag << 32;
+        }, e);
+#pragma unroll
+        for (int w = 0; w < RS_W; w++)
+          if (other(w)) X[w * T + t] = e[w];
+      };
+      window(x0w);
+      __syncthreads();
+      // r0 = v - A x0
+#pragma unroll
+      for (int q = 0; q < R; q++) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (row[q] >= 0) {
+          const float acc = rs_row_h(lidx, av16, cap, row[q], len[q], lmx[q], X);
+          const float r0 = v[q] - acc;
+          r0s[q * T + t] = r0;
+          if (q * T + t < head) rs_put(ps_at(r0w, row[q]), tag, r0);
+        }
+      }
+      // the last cell's rows of the next workgroups follow this one's
+      if (t < tail) r0s[i1 - i0 + t] = rs_wait(ps_at(r0w + i1, t), tag, bad, 0ull);
+      __syncthreads();
+      // restriction to level 1, a cell per thread, rows in order
+      {
+        int a0 = ca0, a1 = ca1;
+        for (int K = K0 + t; K < K1; K += T) {
+          if (K != K0 + t) {
+            a0 = cstart[K] - i0;
+            a1 = cstart[K + 1] - i0;
+          }
+          float s = 0.0f;
+          for (int b0 = a0; b0 < a1; b0 += 8) {
+            float u8[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) u8[u] = r0s[min(b0 + u, a1 - 1)];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+              if (b0 + u < a1) s = s + u8[u];
+          }
+          rs_put(ps_at(b1w, K), tag, s);
+        }
+      }
+      for (int lv = 1; lv <= Q.m; lv++) rs_down<T>(H, Q, wg, t, lv, tag, bad);
+      for (int lv = Q.m; lv >= 1; lv--) rs_up<T>(H, Q, wg, t, lv, tag, bad);
+      // x1 = x0 + c e1 over the window; one wavefront waits for the first
+      // corrections before the others read theirs
+      if (t < 64 && wk[0] >= 0) (void)rs_wait(ps_at(e1w, wk[0]), tag, bad, 0ull);
+      __syncthreads();
+      {
+        float e[RS_W];
+        rs_poll<RS_W>(tag, bad, [&](int w) {
+          return wk[w] >= 0 ? ld_agent(ps_at(e1w, wk[w])) : (unsigned long long)tag << 32;
+        }, e);
+#pragma unroll
+        for (int w = 0; w < RS_W; w++)
+          if (wk[w] >= 0) X[w * T + t] = X[w * T + t] + mc * e[w];
+      }
+      __syncthreads();
+      // x = x1 + w (v - A x1) d
+      float y[R];
+#pragma unroll
+      for (int q = 0; q < R; q++) {
+        __builtin_amdgcn_sched_barrier(0);
+        y[q] = 0.0f;
+        if (row[q] >= 0) {
+          const float acc = rs_row_h(lidx, av16, cap, row[q], len[q], lmx[q], X);
+          y[q] = X[s0 * PS_CHUNK + q * T + t] + mw * (v[q] - acc) * d0[q];
+          rs_put(ps_at(phw, row[q]), tag, y[q]);
+        }
+      }
+      __syncthreads();  // the gathers of x1 are done
+#pragma unroll
+      for (int q = 0; q < R; q++)
+        if (row[q] >= 0) X[s0 * PS_CHUNK + q * T + t] = y[q];
+      window(phw);
+      __syncthreads();
+      // ---- the product, FP64
+      double acc[R];
+#pragma unroll
+      for (int q = 0; q < R; q++) {
+        __builtin_amdgcn_sched_barrier(0);
+        acc[q] = (row[q] >= 0) ? rs_row_d(lidx, aval, cap, row[q], len[q], lmx[q], X) : 0.0;
+      }
+      if (half == 0) {
+        double o[1], pv[1][R];
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+          t1[q] = acc[q];
+          ph[q] = y[q];
+          pv[0][q] = (row[q] >= 0) ? acc[q] * (double)rh[q] : 0.0;
+        }
+        ok = rs_publish_wait<T, R, 1>(Q, wg, nblk, ep++, pv, area, res, bad, o);
+        if (!ok) break;
+        rs_alpha(z, o[0]);
+        if (z.done) break;
+        // s = r - alpha t1
+#pragma unroll
+        for (int q = 0; q < R; q++) r[q] = r[q] - z.alpha * t1[q];
+      } else {
+        double o[5], pv[5][R];
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+          const bool in = row[q] >= 0;
+          const double sv = r[q], rd = (double)rh[q];
+          sh[q] = y[q];
+          pv[0][q] = in ? acc[q] * sv : 0.0;
+          pv[1][q] = in ? acc[q] * acc[q] : 0.0;
+          pv[2][q] = in ? acc[q] * rd : 0.0;
+          pv[3][q] = in ? sv * rd : 0.0;
+          pv[4][q] = in ? sv * sv : 0.0;
+        }
+        ok = rs_publish_wait<T, R, 5>(Q, wg, nblk, ep++, pv, area, res, bad, o);
+        if (!ok) break;
+        rs_omega(z, o, stop, bnorm, max_iter);
+        if (z.done && !z.update) break;
+        // x += alpha ph + omega sh ; r = s - omega t2 ; p = r + beta (p - omega t1)
+#pragma unroll
+        for (int q = 0; q < R; q++)
+          if (row[q] >= 0) {
+            double* xp = ps_at(sol, row[q]);
+            *xp = (*xp + z.alpha * (double)ph[q]) + z.omega * (double)sh[q];
+            r[q] = r[q] - z.omega * acc[q];
+            if (!z.done) p[q] = (float)(r[q] + z.beta * ((double)p[q] - z.omega * t1[q]));
+          }
+      }
+    }
+    if (z.done) break;
+  }
+  if (!ok) {
+    if (t == 0) atomicOr(&Sc->counter[PS_FLAG_ABORT], 1u);
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < R; q++)
+    if (row[q] >= 0) {
+      *ps_at(glob(D.r), row[q]) = r[q];
+      *ps_at(glob(D.pp32), row[q]) = p[q];
+    }
+}
+
+template <int T, int R>
+__host__ __device__ inline int64_t rs_row_lds() {
+  return 8 * (5 * R * (T / 256) * 192 + 8) + 4 * (RS_W * T + R * T + RS_TAIL);
+}
+__host__ __device__ inline int64_t rs_coarse_lds(const MgDev& G, int l0) {
+  return 8 * (5 * 256 + 8) + mg_coarse_lds_bytes(G, l0);
+}
+
+// up to `iters` iterations of every unfinished scenario
+template <int T, int R>
+__global__ void __launch_bounds__(T) kb_pb_resident(BatchDev B, const ResDev* rs, int iters,
+                                                       unsigned v0, unsigned ep) {
+  extern __shared__ double rs_lds[];
+  const int s = rs_locate(rs, B.S, blockIdx.x);
+  __shared__ MgLevel lev[MG_MAX_LEVELS];
+  const ResDev Q = rs[s];  // copies: fields of a table in memory are read anew after every store
+  const Dev& D = B.devs[s];
+  const MgDev& M = B.mgs[s];
+  const int wg = blockIdx.x - Q.wg0;
+  if (threadIdx.x < MG_MAX_LEVELS) lev[threadIdx.x] = M.lev[threadIdx.x];
+  __syncthreads();
+  if (D.sc->done) return;  // every workgroup of the scenario
+  if (wg == Q.G) rs_coarse_solve<T>(D, M, Q, lev, iters, v0, ep, rs_lds);
+  else rs_rows_solve<T, R>(D, M, Q, lev, wg, iters, v0, ep, rs_lds);
+}

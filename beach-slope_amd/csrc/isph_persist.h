@@ -47,7 +47,7 @@
 
 #define PS_CHUNK 64                 // rows per window chunk
 #define PS_MAX_CHUNKS 16384         // chunks of the largest system (2^20 rows)
-#define PS_SPIN (1 << 22)           // polls of one wait: seconds
+#define PS_SPIN (1 << 20)           // polls of one wait: about a second
 
 // DevScalars::counter slots of the resident solve
 #define PS_FLAG_WIN 0               // a window exceeds its capacity
