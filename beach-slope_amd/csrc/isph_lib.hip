@@ -252,7 +252,7 @@ static bool res_plan(int nblk, ResPlan* out) {
   if (p.nbw <= 1) res_shape<256, 1, 8, 32>(p, nblk);
   else if (p.nbw <= 2) res_shape<512, 1, 6, 32>(p, nblk);
   else if (p.nbw <= 4) res_shape<1024, 1, 4, 0>(p, nblk);
-  else if (p.nbw <= 8) res_shape<1024, 2, 5, 0>(p, nblk);
+  else if (p.nbw <= 8) res_shape<1024, 2, 6, 0>(p, nblk);
   else if (p.nbw <= 12) res_shape<1024, 3, 6, 0>(p, nblk);
   else return false;
   if (p.lds > RES_LDS_MAX || resident_capacity(p.solve, p.T) < p.G) return false;
@@ -261,7 +261,6 @@ static bool res_plan(int nblk, ResPlan* out) {
 }
 
 static hipError_t res_setup(const ResPlan& p, Dev& D, PersArg& Q, hipStream_t st) {
-  Q.lidx = D.aoff;
   Q.wcap = p.W * p.T / PS_CHUNK;
   Q.nbw = p.nbw;
   void* args[] = {&D, &Q};
@@ -282,7 +281,7 @@ extern "C" int64_t isph_footprint_bytes(int64_t n_cap, int64_t n_solid_cap, int3
   per += 4 + 4 * NBR_CAP;                       // neighbour list
   per += 4 * 3;                                 // bin, rank, scan scratch
   per += 4 + ROW_CAP * (4 + 8) + 2 * 8;         // PPE rows, rhs, solution
-  per += 6 * 8;                                 // FP64 solver vectors
+  per += 7 * 8;                                 // FP64 solver vectors
   per += 4 * ((ROW_CAP + 1) / 2);               // packed 16-bit columns
   // precision form: FP16 V-cycle matrix, FP32 vectors, level-0 multigrid
   // vectors, setup rows
@@ -373,8 +372,9 @@ extern "C" int isph_create(const isph_params* params, int64_t n_cap, int64_t n_s
   rc |= dalloc(c, &c->d_bn2, 1);
   rc |= dalloc(c, &D.aoff, N * ((ROW_CAP + 1) / 2));
   rc |= dalloc(c, &c->ps.slots, 8 * (N / 256 + 2 + RES_MAX_WG));
+  rc |= dalloc(c, &c->ps.rhi, N);
   rc |= dalloc(c, &c->ps.wlist, RES_WLIST);
-  rc |= dalloc(c, &c->ps.wcnt, RES_MAX_WG);
+  rc |= dalloc(c, &c->ps.wcnt, 2 * RES_MAX_WG);
   if (params->precision) {
     rc |= dalloc(c, &D.av16, N * ((ROW_CAP + 1) / 2));
     float** ff[] = {&D.r32, &D.rh32, &D.pp32, &D.sv32, &D.d32};
@@ -1494,7 +1494,16 @@ static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
       ResPlan plan;
       bool resident = !c->prof && res_plan(c->D.nblk, &plan);
       hipLaunchKernelGGL(k_res_clear, dim3(1), dim3(64), 0, c->stream, c->D);
-      if (resident) HIPCHK(c, res_setup(plan, c->D, c->ps, c->stream));
+      if (resident) {
+        PersArg& Q = c->ps;
+        auto words = [](double* p) { return reinterpret_cast<unsigned long long*>(p); };
+        Q.tlo = words(c->D.t1);
+        Q.thi = words(c->D.t2);
+        Q.rlo = words(c->D.sv);
+        Q.lidx = c->D.aoff;
+        Q.ls = c->D.cap;
+        HIPCHK(c, res_setup(plan, c->D, Q, c->stream));
+      }
       RLAUNCH(k_bicg_init, n, c->D);
       FINALIZE(FIN_INIT, n);
       DevScalars s;
@@ -2638,9 +2647,10 @@ extern "C" int isph_batch_destroy(isph_batch* b) {
 // ---------------------------------------------------------------------
 // allocation-free FP64 solve (isph_ppe_solve_noalloc)
 // ---------------------------------------------------------------------
-// Scratch of the allocation-free solve, one static device array per GPU:
-// six BiCGStab vectors of ISPH_NOALLOC_MAX_ROWS doubles (r, rh, p, t1, s,
-// t2), the block partials of two dot products, then the solver scalars and
+// Scratch of the allocation-free solve, one static device array per GPU: room
+// for six BiCGStab vectors of ISPH_NOALLOC_MAX_ROWS doubles (r, rh, p, t1, s,
+// t2; a smaller system's vectors, then what the resident form exchanges and
+// its window positions), the block partials of two dot products, then the solver scalars and
 // the squared right-hand-side norm.  Host code never uses the array's name
 // as an address: scratch_base() looks up each device's own copy once, with
 // that device current, and every kernel argument is derived from it.
@@ -2776,16 +2786,43 @@ extern "C" int isph_ppe_solve_noalloc(int32_t n, int32_t ld, const int32_t* row_
   D.aval = const_cast<double*>(val);
   D.b = const_cast<double*>(rhs);
   D.sol = x;
-  D.r = base;
-  D.rh = base + NA_ROWS;
-  D.pp = base + 2 * NA_ROWS;
-  D.t1 = base + 3 * NA_ROWS;
-  D.sv = base + 4 * NA_ROWS;
-  D.t2 = base + 5 * NA_ROWS;
   D.part = base + 6 * NA_ROWS;
   D.sc = reinterpret_cast<DevScalars*>(base + 6 * NA_ROWS + NA_PART);
+  // The six vectors lie one behind the other at the length of this system, so
+  // a system of up to about 270k rows leaves room behind them for what the
+  // resident form needs; a larger one runs launch by launch.
+  const size_t nv = ((size_t)n + 31) & ~(size_t)31;
+  D.r = base;
+  D.rh = base + nv;
+  D.pp = base + 2 * nv;
+  D.t1 = base + 3 * nv;
+  D.sv = base + 4 * nv;
+  D.t2 = base + 5 * nv;
+  ResPlan plan;
+  PersArg Q{};
+  bool resident = res_plan(grid_of(n), &plan);
+  if (resident) {
+    auto words = [](double* p) { return reinterpret_cast<unsigned long long*>(p); };
+    Q.tlo = words(D.t1);
+    Q.thi = words(D.t2);
+    Q.rlo = words(D.sv);
+    size_t at = 6 * nv;  // in doubles
+    auto take = [&](size_t doubles) {
+      double* p = base + at;
+      at += (doubles + 31) & ~(size_t)31;
+      return p;
+    };
+    Q.rhi = words(take(nv));
+    Q.slots = words(take(8 * ((size_t)grid_of(n) + RES_MAX_WG)));
+    Q.wlist = reinterpret_cast<int32_t*>(take(RES_WLIST / 2));
+    Q.wcnt = reinterpret_cast<int32_t*>(take(RES_MAX_WG));
+    Q.lidx = reinterpret_cast<uint32_t*>(take(((ROW_CAP + 1) / 2) * nv / 2));
+    Q.ls = (int)nv;
+    resident = at <= 6 * NA_ROWS;
+  }
   double* d_bn2 = base + 6 * NA_ROWS + NA_PART + NA_SC_DOUBLES - 1;
   const int rg = row_grid(n), nb = grid_of(n);
+  hipError_t e0 = hipSuccess;
   // clear the scalars the previous call left; check the rows; ||b||^2
   NA_LAUNCH(k_na_begin, 1, D.sc, n);
   NA_LAUNCH(k_na_check, grid_of(n), D);
@@ -2807,17 +2844,35 @@ extern "C" int isph_ppe_solve_noalloc(int32_t n, int32_t ld, const int32_t* row_
     }
     out.rel_residual = (bnorm == 0.0) ? 0.0 : bnorm;
   } else {
-    // the FP64 iteration of isph_ppe_solve: same launches, same chunked
-    // polling, same restarts from the true residual after a breakdown
+    // the FP64 iteration of isph_ppe_solve: the same two forms, the same
+    // restarts from the true residual after a breakdown
     NA_LAUNCH(k_na_set_bnorm, 1, D.sc, bnorm);
+    if (resident) {
+      e0 = res_setup(plan, D, Q, st);
+      if (e0 != hipSuccess)
+        return na_fail(ISPH_EHIP, "isph_ppe_solve_noalloc: window set-up: %s",
+                       hipGetErrorString(e0));
+    }
     NA_LAUNCH(k_bicg_init, rg, D);
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, st, D, (int)FIN_INIT, nb,
                        (double*)nullptr);
     rc = na_read(st, D.sc, &s, nullptr);
     if (rc) return rc;
+    if (s.counter[PS_FLAG_WIN]) resident = false;
     int restarts = 0, chunk = 4;
+    unsigned ep = 1;
     for (int64_t it = 0; !s.done;) {
-      for (int k = 0; k < chunk; k++) {
+      if (resident) {
+        if (res_launch(plan, D, Q, RES_ITERS, ep, st) == hipSuccess) {
+          chunk = RES_ITERS;
+          ep += 3u * RES_ITERS;
+        } else {  // refused: nothing ran
+          (void)hipGetLastError();
+          resident = false;
+          chunk = 4;
+        }
+      }
+      for (int k = 0; k < chunk && !resident; k++) {
         NA_LAUNCH(k_bicg_1, rg, D);
         hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, st, D, (int)FIN_ALPHA, nb,
                            (double*)nullptr);
@@ -2832,6 +2887,8 @@ extern "C" int isph_ppe_solve_noalloc(int32_t n, int32_t ld, const int32_t* row_
       it += chunk;
       rc = na_read(st, D.sc, &s, nullptr);
       if (rc) return rc;
+      if (resident && s.counter[PS_FLAG_ABORT])
+        return na_fail(ISPH_EHIP, "isph_ppe_solve_noalloc: a grid-wide wait ran out");
       if (s.done) {
         if (s.brk && !s.conv && s.iters < max_iter && restarts < max_outer) {
           restarts++;

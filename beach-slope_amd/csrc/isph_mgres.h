@@ -499,7 +499,7 @@ __device__ __forceinline__ void rs_down(const RsMg& M, const ResDev& Q, int wg, 
       sv[k] = *ps_at(st + (size_t)k * L.n, I);
       rv[k] = *ps_at(rd, Nb[k] & ~(1 << 30));
     }
-    rs_poll<9>(tag, bad, [&](int k) { return ld_agent(ps_at(bl, Nb[k] & ~(1 << 30))); }, bv);
+    rs_poll<9>(tag, bad, [&](int k) { return ld_word(bl, Nb[k] & ~(1 << 30)); }, bv);
     float acc = 0.0f;
 #pragma unroll
     for (int k = 0; k < 9; k++) {
@@ -549,11 +549,11 @@ __device__ __forceinline__ void rs_up(const RsMg& M, const ResDev& Q, int wg, in
       else Nb[k] = I, Pa[k] = pI;  // read in place of a missing one; its term is not added
       sv[k] = *ps_at(st + (size_t)k * L.n, I);
     }
-    rs_poll<9>(tag, bad, [&](int k) { return ld_agent(ps_at(bw, Nb[k])); }, xv);
+    rs_poll<9>(tag, bad, [&](int k) { return ld_word(bw, Nb[k]); }, xv);
     const float bI = xv[4], rI = *ps_at(rd, I);
 #pragma unroll
     for (int k = 0; k < 9; k++) xv[k] = (w * xv[k]) * *ps_at(rd, Nb[k]);
-    rs_poll<9>(tag, bad, [&](int k) { return ld_agent(ps_at(ec, Pa[k])); }, xc);
+    rs_poll<9>(tag, bad, [&](int k) { return ld_word(ec, Pa[k]); }, xc);
     float acc = 0.0f;
 #pragma unroll
     for (int k = 0; k < 9; k++) {
@@ -638,7 +638,7 @@ __device__ __forceinline__ void rs_coarse_solve(const Dev& D, const MgDev& M, co
       // right-hand side of the first level
       float bq[PER];
       rs_poll<PER>(tag, bad, [&](int q) {
-        return (t + q * T < L0.n) ? ld_agent(ps_at(bw, t + q * T)) : (unsigned long long)tag << 32;
+        return (t + q * T < L0.n) ? ld_word(bw, t + q * T) : (unsigned long long)tag << 32;
       }, bq);
 #pragma unroll
       for (int q = 0; q < PER; q++) {
@@ -926,7 +926,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
           return wc[w] >= 0 && (wc[w] < oc0 || wc[w] >= oc1) && wk[w] >= 0;
         };
         rs_poll<RS_W>(tag, bad, [&](int w) {
-          return other(w) ? ld_agent(ps_at(words + (int64_t)wc[w] * PS_CHUNK, l))
+          return other(w) ? ld_word(words + (int64_t)wc[w] * PS_CHUNK, l)
                           : (unsigned long long)tag << 32;
         }, e);
 #pragma unroll
@@ -978,7 +978,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
       {
         float e[RS_W];
         rs_poll<RS_W>(tag, bad, [&](int w) {
-          return wk[w] >= 0 ? ld_agent(ps_at(e1w, wk[w])) : (unsigned long long)tag << 32;
+          return wk[w] >= 0 ? ld_word(e1w, wk[w]) : (unsigned long long)tag << 32;
         }, e);
 #pragma unroll
         for (int w = 0; w < RS_W; w++)

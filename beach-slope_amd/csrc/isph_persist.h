@@ -20,22 +20,21 @@
 // and a strip on each side, since rows are sorted by cell) and rewrites each
 // column as a 16-bit position in that window.  The products gather from the
 // window in LDS.  A workgroup's threads keep r, t1 and p of the window's
-// elements in registers: r and t1 are read after the reduction that follows
-// their production, and p = r + beta (p - omega t1) is formed for the window
-// by the same expression as at its owner, so p is never exchanged.  Rows
-// whose window does not fit (wlist's capacity) leave the flag set and the
-// solve runs launch by launch.
+// elements in registers: t1 and r of other workgroups' rows are read while
+// the reduction after their production is under way, and
+// p = r + beta (p - omega t1) is formed for the window by the same expression
+// as at its owner, so p is never exchanged.  Rows whose window does not fit
+// (wlist's capacity) leave the flag set and the solve runs launch by launch.
 //
-// Visibility between workgroups.  Exchanged data (r, t1, the partial sums)
-// is written and read with relaxed agent-scope atomics, which write through
-// and read past the per-XCD caches; every wave waits for its stores
-// (s_waitcnt) before the workgroup's barrier, after which one lane publishes
-// the block's partial sums.  A published word carries 32 bits of the value
-// and the reduction's number, so a reader polls the data itself: there is no
-// counter and no fence (an agent-scope release writes the XCD's L2 back:
-// 8.3 us per barrier of 256 workgroups against 2.4 us for this one).  Two
-// sets of words alternate: a set is written again only after the reduction
-// between has completed, which every reader of it has passed.
+// Visibility between workgroups.  Exchanged values (r, t1, the partial sums)
+// are doubles in two 64-bit words, each with 32 bits of the value and the
+// number of the reduction it belongs to, written and read with relaxed
+// agent-scope atomics, which write through and read past the per-XCD caches.
+// A reader polls the data itself, so there is no counter, no wait for stores
+// and no fence (an agent-scope release writes the XCD's L2 back: 8.3 us per
+// barrier of 256 workgroups against 2.4 us for an exchange of words).  A word
+// is written again only after a reduction that its readers took part in after
+// their reads; the partial sums, read within one, alternate between two sets.
 //
 // Progress.  The launch is cooperative (all workgroups resident); every wait
 // is bounded (PS_SPIN polls) and a wait that ends without its data makes the
@@ -55,9 +54,13 @@
 
 struct PersArg {
   unsigned long long* slots;  // two sets of 4 words per row block, 8 per workgroup
-  uint32_t* lidx;             // window positions, slots 2w and 2w+1 of row i at [w * cap + i]
+  // the words of t1 and r (several rows per thread: of s and p), one array
+  // per half
+  unsigned long long *tlo, *thi, *rlo, *rhi;
+  uint32_t* lidx;             // window positions, slots 2w and 2w+1 of row i at [w * ls + i]
+  int ls;                     // leading dimension of lidx
   int32_t* wlist;             // per workgroup: its chunks, ascending (wcap entries)
-  int32_t* wcnt;              // per workgroup: their count
+  int32_t* wcnt;              // per workgroup: their count, and the slot of its own first chunk
   int wcap;                   // window capacity in chunks
   int nbw;                    // row blocks per workgroup
 };
@@ -69,6 +72,21 @@ __device__ __forceinline__ void st_agent(V* p, V v) {
 template <typename V>
 __device__ __forceinline__ V ld_agent(const V* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Element i of an array through its uniform base and a 32-bit byte offset,
+// so that every array shares one offset register
+template <typename V>
+__device__ __forceinline__ V* ps_at(V* base, unsigned i) {
+  typedef typename std::conditional<std::is_const<V>::value, const char, char>::type Byte;
+  return reinterpret_cast<V*>(reinterpret_cast<Byte*>(base) + (i * (unsigned)sizeof(V)));
+}
+
+// An exchanged word polled in a loop: the index is opaque, so the loop holds
+// one offset per word and not a 64-bit address
+__device__ __forceinline__ unsigned long long ld_word(const unsigned long long* base, unsigned i) {
+  asm volatile("" : "+v"(i));
+  return ld_agent(ps_at(base, i));
 }
 
 // Windows of the workgroups' rows (one workgroup each, as the solve), the
@@ -87,10 +105,12 @@ __global__ void __launch_bounds__(T) k_ps_setup(Dev D, PersArg Q) {
       Q.slots[4 * ((size_t)D.nblk + b) + q] = 0;
     }
   if (t < 8) Q.slots[8 * ((size_t)D.nblk + wg) + t] = 0;
+  for (int i = i0 + t; i < i1; i += T) Q.tlo[i] = Q.thi[i] = Q.rlo[i] = Q.rhi[i] = 0;
   for (int c = t; c < nch; c += T) map[c] = 0;
   __syncthreads();
   for (int i = i0 + t; i < i1; i += T) {
     const int L = D.alen[i];
+    map[i / PS_CHUNK] = 1;  // its own rows, in order, whatever the columns
     for (int k0 = 0; k0 < L; k0 += 8) {
       int c[8];
 #pragma unroll
@@ -117,7 +137,7 @@ __global__ void __launch_bounds__(T) k_ps_setup(Dev D, PersArg Q) {
   if (total > Q.wcap) {  // the whole workgroup
     if (t == 0) {
       atomicOr(&D.sc->counter[PS_FLAG_WIN], 1u);
-      Q.wcnt[wg] = 0;
+      Q.wcnt[2 * wg] = 0;
     }
     return;
   }
@@ -125,9 +145,10 @@ __global__ void __launch_bounds__(T) k_ps_setup(Dev D, PersArg Q) {
   for (int c = c0; c < c1; c++)
     if (map[c]) {
       Q.wlist[(size_t)wg * Q.wcap + pos] = c;
+      if (c == i0 / PS_CHUNK) Q.wcnt[2 * wg + 1] = pos;
       map[c] = (uint16_t)pos++;
     }
-  if (t == 0) Q.wcnt[wg] = total;
+  if (t == 0) Q.wcnt[2 * wg] = total;
   __syncthreads();
   for (int i = i0 + t; i < i1; i += T) {
     const int L = D.alen[i];
@@ -140,7 +161,7 @@ __global__ void __launch_bounds__(T) k_ps_setup(Dev D, PersArg Q) {
         if (k0 + u >= L) break;
         const uint32_t a = map[c[u] / PS_CHUNK] * PS_CHUNK + c[u] % PS_CHUNK;
         const uint32_t b = map[c[u + 1] / PS_CHUNK] * PS_CHUNK + c[u + 1] % PS_CHUNK;
-        Q.lidx[((k0 + u) >> 1) * cap + i] = a | (b << 16);
+        Q.lidx[(size_t)((k0 + u) >> 1) * Q.ls + i] = a | (b << 16);
       }
     }
   }
@@ -154,14 +175,14 @@ __device__ __forceinline__ double lane0(double v) {
 }
 
 // LDS of the resident solve in doubles: the window, then an area shared by
-// the block trees and the gathered partials, then the column sums, then (R >
-// 1) p and t1 of the workgroup's rows
+// the block trees and the gathered partials, then the column sums, then (one
+// row per thread) t1, later r, of the workgroup's rows
 template <int T, int R>
 __host__ __device__ constexpr int ps_tree_doubles() { return 2 * R * (T / 256) * 192; }
 template <int T, int R, int W>
 __host__ __device__ inline int64_t ps_lds_bytes(int nblk) {
   const int64_t a = ps_tree_doubles<T, R>(), b = 2 * (int64_t)nblk;
-  return 8 * ((int64_t)W * T + (a > b ? a : b) + 2 * 256 + 2 + (R > 1 ? 2 * R * T : 0)) + 16;
+  return 8 * ((int64_t)W * T + (a > b ? a : b) + 2 * 256 + 2 + (R > 1 ? 0 : T));
 }
 
 // One word of reduction ep, polled until it carries the number; false when
@@ -178,16 +199,15 @@ __device__ __forceinline__ bool ps_wait(const unsigned long long* p, unsigned ep
 // double is two words, low half first, so out is the doubles' array.  The
 // workgroup reads each word once, 64 consecutive ones per wavefront (four
 // cache lines), several in flight per thread.
-template <int T>
+template <int T, int G>
 __device__ __forceinline__ bool ps_collect(const unsigned long long* set, int words, unsigned ep,
                                            uint32_t* out) {
-  constexpr int G = 4;
   for (int w0 = threadIdx.x; w0 < words; w0 += G * T) {
     uint32_t lo[G];
     unsigned long long w[G];
     bool all = false;
 #pragma unroll
-    for (int u = 0; u < G; u++) w[u] = ld_agent(&set[min(w0 + u * T, words - 1)]);
+    for (int u = 0; u < G; u++) w[u] = ld_word(set, min(w0 + u * T, words - 1));
     all = true;
 #pragma unroll
     for (int u = 0; u < G; u++) {
@@ -210,55 +230,52 @@ __device__ __forceinline__ void ps_publish(unsigned long long* p, unsigned ep, d
 }
 
 // Grid-wide sums of NV values per row in the order of block_tree and
-// final_tree2.  Every vector store of the caller's before this call is
-// visible to every workgroup after it.  Returns false when a wait ran out.
+// final_tree2; `mid` runs between the publication of this workgroup's partial
+// sums and the wait for the others'.  Returns false when a wait ran out.
 //
 // Up to 256 row blocks (one per workgroup, T = 256) every workgroup collects
 // all partials itself: one exchange.  With more, the readers' requests for
 // the same lines would take longer than a second exchange (24 us against 4 at
 // 809 blocks): workgroup 0 collects the partials and sends the sums to a line
 // of each workgroup's own.
-template <int T, int R, int NV>
+template <int T, int R, int NV, typename MID>
 __device__ __forceinline__ bool ps_reduce(const PersArg& Q, int nblk, int b0, unsigned ep,
                                           const double (&v)[NV][R], double* area, double* col,
-                                          int* bad, double (&out)[NV]) {
+                                          int* bad, double (&out)[NV], MID mid) {
   constexpr int S = T / 256;
   const int t = threadIdx.x, wv = (t >> 6) & 3, l = t & 63, sub = t >> 8;
-  if (wv) {
+  // tree j = k R + q of a block is summed by wavefront j mod 4 of its four;
+  // the other three leave their values in LDS
 #pragma unroll
-    for (int k = 0; k < NV; k++)
-#pragma unroll
-      for (int q = 0; q < R; q++)
-        area[((k * R + q) * S + sub) * 192 + (wv - 1) * 64 + l] = v[k][q];
-  }
-  __syncthreads();
-  double s[NV][R];
-  if (wv == 0) {
-#pragma unroll
-    for (int q = 0; q < R; q++)
-#pragma unroll
-      for (int k = 0; k < NV; k++) {
-        const double* a = area + ((k * R + q) * S + sub) * 192;
-        s[k][q] = wave_tree((v[k][q] + a[64 + l]) + (a[l] + a[128 + l]));
-      }
-  }
-  __builtin_amdgcn_s_waitcnt(0);  // this wave's vector stores have completed
-  __syncthreads();                // ... and every wave's; the trees are read
-  // two sets of slots of 4 words per block, used with NV doubles each
-  unsigned long long* set = Q.slots + (size_t)(ep & 1) * 4 * nblk;
-  if (wv == 0 && l == 0) {
+  for (int k = 0; k < NV; k++)
 #pragma unroll
     for (int q = 0; q < R; q++) {
-      const int lb = q * S + sub;
-      if (lb < Q.nbw && b0 + lb < nblk) {
+      const int j = k * R + q, o = j & 3;
+      if (wv != o) area[(j * S + sub) * 192 + (wv < o ? wv : wv - 1) * 64 + l] = v[k][q];
+    }
+  __syncthreads();
+  // two sets of slots of 4 words per block, used with NV doubles each
+  unsigned long long* set = Q.slots + (size_t)(ep & 1) * 4 * nblk;
 #pragma unroll
-        for (int k = 0; k < NV; k++)
-          ps_publish(&set[2 * (size_t)(NV * (b0 + lb) + k)], ep, s[k][q]);
+  for (int k = 0; k < NV; k++)
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      const int j = k * R + q, o = j & 3;
+      if (wv == o) {
+        const double* a = area + (j * S + sub) * 192 + l;
+        const double w0 = (o == 0) ? v[k][q] : a[0];
+        const double w1 = (o == 1) ? v[k][q] : a[(o < 1 ? 0 : 1) * 64];
+        const double w2 = (o == 2) ? v[k][q] : a[(o < 2 ? 1 : 2) * 64];
+        const double w3 = (o == 3) ? v[k][q] : a[2 * 64];
+        const double s = wave_tree((w0 + w2) + (w1 + w3));
+        const int lb = q * S + sub;
+        if (l == 0 && lb < Q.nbw && b0 + lb < nblk)
+          ps_publish(&set[2 * (size_t)(NV * (b0 + lb) + k)], ep, s);
       }
     }
-  }
+  mid();
   if (T == 256) {
-    if (!ps_collect<T>(set, 2 * NV * nblk, ep, reinterpret_cast<uint32_t*>(col))) *bad = 1;
+    if (!ps_collect<T, 4>(set, 2 * NV * nblk, ep, reinterpret_cast<uint32_t*>(col))) *bad = 1;
     __syncthreads();
     // every wavefront sums for itself: lane l holds columns l, l + 64, ...
 #pragma unroll
@@ -274,7 +291,9 @@ __device__ __forceinline__ bool ps_reduce(const PersArg& Q, int nblk, int b0, un
   unsigned long long* mail = Q.slots + (size_t)8 * nblk;  // 8 words per workgroup
   double* res = col + 512;
   if (blockIdx.x == 0) {
-    if (!ps_collect<T>(set, 2 * NV * nblk, ep, reinterpret_cast<uint32_t*>(area))) *bad = 1;
+    __syncthreads();  // the trees are read; the area takes the partials
+    if (!ps_collect<T, 4>(set, 2 * NV * nblk, ep, reinterpret_cast<uint32_t*>(area)))
+      *bad = 1;
     __syncthreads();
     if (t < 256) {
 #pragma unroll
@@ -308,14 +327,6 @@ __device__ __forceinline__ bool ps_reduce(const PersArg& Q, int nblk, int b0, un
   return !*bad;
 }
 
-// Element i of an array through its uniform base and a 32-bit byte offset,
-// so that every array shares one offset register
-template <typename V>
-__device__ __forceinline__ V* ps_at(V* base, unsigned i) {
-  typedef typename std::conditional<std::is_const<V>::value, const char, char>::type Byte;
-  return reinterpret_cast<V*>(reinterpret_cast<Byte*>(base) + (i * (unsigned)sizeof(V)));
-}
-
 // A thread's first KR row entries, held in registers for the whole launch
 // (KR 0: none); ps_row reads the rest from memory
 template <int KR>
@@ -324,32 +335,34 @@ struct PsRow {
   uint32_t w[KR ? KR / 2 : 1];
 };
 
-// Eight entries k0.. of row i: their positions and values (those below the
-// wavefront's longest row Lm; FULL: all eight are), gathers and products
-template <bool FULL>
-__device__ __forceinline__ double ps_row8(const uint32_t* ip, const double* vp, int cap,
-                                          unsigned i, int k0, int L, int Lm, const double* win,
-                                          double acc) {
-  uint32_t w[4];
-  double v[8], g[8];
+// U entries k0.. of row i: their positions and values (those below the
+// wavefront's longest row Lm; FULL: all are), gathers and products
+template <int U, bool FULL>
+__device__ __forceinline__ double ps_entries(const uint32_t*& ip, const double*& vp, int ls,
+                                             int cap, unsigned i, int k0, int L, int Lm,
+                                             const double* win, double acc) {
+  uint32_t w[U / 2];
+  double v[U], g[U];
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
+  for (int q = 0; q < U / 2; q++) {
     w[q] = 0u;
-    if (FULL || k0 + 2 * q < Lm) w[q] = *ps_at(ip + (size_t)q * cap, i);
+    if (FULL || k0 + 2 * q < Lm) w[q] = *ps_at(ip, i);
+    ip += ls;
   }
 #pragma unroll
-  for (int u = 0; u < 8; u++) {
+  for (int u = 0; u < U; u++) {
     v[u] = 0.0;
-    if (FULL || k0 + u < Lm) v[u] = *ps_at(vp + (size_t)u * cap, i);
+    if (FULL || k0 + u < Lm) v[u] = *ps_at(vp, i);
+    vp += cap;
   }
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
+  for (int q = 0; q < U / 2; q++) {
     w[q] = (k0 + 2 * q < L) ? w[q] : 0u;  // a shorter row's slots hold no position
     g[2 * q] = win[w[q] & 0xffffu];
     g[2 * q + 1] = win[w[q] >> 16];
   }
 #pragma unroll
-  for (int u = 0; u < 8; u++) {
+  for (int u = 0; u < U; u++) {
     const double a = acc + v[u] * g[u];
     acc = (k0 + u < L) ? a : acc;
   }
@@ -359,8 +372,8 @@ __device__ __forceinline__ double ps_row8(const uint32_t* ip, const double* vp, 
 // y_i = sum_k A_ik win[pos(k)] in row order (the order of ell_row_sum).  The
 // loop runs to the wavefront's longest row (Lm, uniform), so the slots' bases
 // are scalars.
-template <int KR>
-__device__ __forceinline__ double ps_row(const PsRow<KR>& M, const uint32_t* idx,
+template <int U, int KR>
+__device__ __forceinline__ double ps_row(const PsRow<KR>& M, const uint32_t* idx, int ls,
                                          const double* val, int cap, unsigned i, int L, int Lm,
                                          const double* win) {
   double acc = 0.0;
@@ -379,16 +392,13 @@ __device__ __forceinline__ double ps_row(const PsRow<KR>& M, const uint32_t* idx
       acc = (k0 + u < L) ? a : acc;
     }
   }
-  const uint32_t* ip = idx + (size_t)(KR / 2) * cap;
+  const uint32_t* ip = idx + (size_t)(KR / 2) * ls;
   const double* vp = val + (size_t)KR * cap;
   int k0 = KR;
 #pragma unroll 1
-  for (; k0 + 8 <= Lm; k0 += 8) {
-    acc = ps_row8<true>(ip, vp, cap, i, k0, L, Lm, win, acc);
-    ip += (size_t)4 * cap;
-    vp += (size_t)8 * cap;
-  }
-  if (k0 < Lm) acc = ps_row8<false>(ip, vp, cap, i, k0, L, Lm, win, acc);
+  for (; k0 + U <= Lm; k0 += U)
+    acc = ps_entries<U, true>(ip, vp, ls, cap, i, k0, L, Lm, win, acc);
+  if (k0 < Lm) acc = ps_entries<U, false>(ip, vp, ls, cap, i, k0, L, Lm, win, acc);
   return acc;
 }
 __device__ __forceinline__ int wave_max(int v) {
@@ -398,145 +408,234 @@ __device__ __forceinline__ int wave_max(int v) {
 }
 
 // up to `iters` BiCGStab iterations from the state in D.sol, D.r, D.rh, D.pp
-// and the scalars (k_bicg_init or a previous launch); leaves the state there
+// and the scalars (k_bicg_init or a previous launch); leaves the state there.
+//
+// One row per thread: the window's p, r and t1 stay in registers as above.
+// Several rows per thread: those registers hold the rows' own vectors, so p
+// and s themselves are exchanged, straight into the window in LDS (two more
+// hops of ~1.5 us in an iteration of 40 us and more, where 150 spilled
+// registers took 20).
 template <int T, int R, int W, int KR>
 __global__ void __launch_bounds__(T) k_bicg_resident(Dev D, PersArg Q, int iters, unsigned ep) {
   constexpr int S = T / 256;
-  // With several rows per thread the 128 registers of a 1024-thread
-  // workgroup do not hold every vector: p and t1 of the rows sit in LDS
-  // slots of their thread, r, rh and x are read from memory where used (by
-  // their own thread only; r past the caches, as it is exchanged).
-  constexpr bool XREG = R == 1;
+  constexpr bool ONE = R == 1;
+  constexpr int U = ONE ? 8 : 4;   // row entries in flight per thread
+  constexpr int WR = ONE ? W : 1;  // window elements in registers
   extern __shared__ double ps_lds[];
-  const int t = threadIdx.x, sub = t >> 8, wg = blockIdx.x;
+  __shared__ int bad_[1];
+  int* bad = bad_;
+  const int wg = blockIdx.x;
   DevScalars* Sc = D.sc;
   const int n = Sc->n, nblk = D.nblk, cap = D.cap, b0 = wg * Q.nbw;
   const int ta = ps_tree_doubles<T, R>();
   double* win = ps_lds;
   double* area = win + W * T;
   double* col = area + (ta > 2 * nblk ? ta : 2 * nblk);
-  double* lp = col + 514;
-  double* lt = lp + R * T;
-  int* bad = reinterpret_cast<int*>(XREG ? lp : lt + R * T);
-  if (t == 0) *bad = 0;
+  double* own = col + 514;  // one row per thread: its t1, then r
   double rho = Sc->rho;
   const double bnorm = Sc->bnorm, tol = D.P.tol;
   const int max_iter = D.P.max_iter;
   int it = Sc->iters;
   int row[R], len[R], lmx[R];
-  double r[R], rh[R], pv[R], x[R], tv[R];
+  double r[R], rh[R], p[R], x[R], t1[R];
   PsRow<KR> M[R];
-  auto P = [&](int q) -> double& {
-    if constexpr (XREG) return pv[q];
-    else return lp[q * T + t];
-  };
-  auto T1 = [&](int q) -> double& {
-    if constexpr (XREG) return tv[q];
-    else return lt[q * T + t];
-  };
-#pragma unroll
-  for (int q = 0; q < R; q++) {
-    const int lb = q * S + sub, i = (b0 + lb) * RED_BLOCK + (t & 255);
-    const bool in = lb < Q.nbw && i < n;
-    row[q] = in ? i : -1;
-    len[q] = in ? D.alen[i] : 0;
-    lmx[q] = wave_max(len[q]);
-    r[q] = (in && XREG) ? D.r[i] : 0.0;
-    rh[q] = (in && XREG) ? D.rh[i] : 0.0;
-    x[q] = (in && XREG) ? D.sol[i] : 0.0;
-    P(q) = in ? D.pp[i] : 0.0;
-#pragma unroll
-    for (int k = 0; k < KR; k++) {
-      M[q].v[k] = (k < len[q]) ? D.aval[k * cap + i] : 0.0;
-      if (k % 2 == 0) M[q].w[k / 2] = (k < len[q]) ? Q.lidx[(k / 2) * cap + i] : 0u;
-    }
-  }
   // the window's elements of this thread: element e = w T + t is row
   // 64 c + (t & 63) with c the chunk of its wavefront (-1: none)
-  const int wn = Q.wcnt[wg], l = t & 63;
   int wc[W];
-  double rw[W], pw[W], tw[W];
+  double rw[WR], pw[WR], tw[WR];
+  const int oc0 = b0 * (RED_BLOCK / PS_CHUNK), oc1 = oc0 + Q.nbw * (RED_BLOCK / PS_CHUNK);
+  const int wn = Q.wcnt[2 * wg], s0 = Q.wcnt[2 * wg + 1];
+  {
+    const int t = threadIdx.x, sub = t >> 8, l = t & 63;
+    if (t == 0) *bad = 0;
 #pragma unroll
-  for (int w = 0; w < W; w++) {
-    const int s = w * (T / PS_CHUNK) + t / PS_CHUNK;
-    wc[w] = __builtin_amdgcn_readfirstlane((s < wn) ? Q.wlist[(size_t)wg * Q.wcap + s] : -1);
-    const int g = wc[w] * PS_CHUNK + l;
-    const bool in = wc[w] >= 0 && g < n;
-    rw[w] = in ? D.r[g] : 0.0;
-    pw[w] = in ? D.pp[g] : 0.0;
+    for (int q = 0; q < R; q++) {
+      const int lb = q * S + sub, i = (b0 + lb) * RED_BLOCK + (t & 255);
+      const bool in = lb < Q.nbw && i < n;
+      row[q] = in ? i : -1;
+      len[q] = in ? D.alen[i] : 0;
+      lmx[q] = wave_max(len[q]);
+      r[q] = in ? D.r[i] : 0.0;
+      p[q] = in ? D.pp[i] : 0.0;
+      rh[q] = (in && ONE) ? D.rh[i] : 0.0;
+      x[q] = (in && ONE) ? D.sol[i] : 0.0;
+#pragma unroll
+      for (int k = 0; k < KR; k++) {
+        M[q].v[k] = (k < len[q]) ? D.aval[k * cap + i] : 0.0;
+        if (k % 2 == 0) M[q].w[k / 2] = (k < len[q]) ? Q.lidx[(size_t)(k / 2) * Q.ls + i] : 0u;
+      }
+    }
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+      const int s = w * (T / PS_CHUNK) + t / PS_CHUNK;
+      wc[w] = __builtin_amdgcn_readfirstlane((s < wn) ? Q.wlist[(size_t)wg * Q.wcap + s] : -1);
+      if (ONE) {
+        const int g = wc[w] * PS_CHUNK + l;
+        const bool in = wc[w] >= 0 && g < n;
+        rw[w] = in ? D.r[g] : 0.0;
+        pw[w] = in ? D.pp[g] : 0.0;
+      }
+    }
   }
   __syncthreads();
   int conv = 0, brk = 0, done = 0;
   double alpha = 0.0, omega = 0.0, beta = 0.0, rr = 0.0, rel = 0.0;
   bool ok = true;
   for (int k = 0; k < iters; k++) {
-    // (the row numbers are opaque to the compiler here, or it would hold
-    // every array's address of every row in registers across iterations)
+    // (opaque: or the compiler holds every address formed from these in
+    // registers over the iterations)
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
 #pragma unroll
     for (int q = 0; q < R; q++) asm volatile("" : "+v"(row[q]));
-    // t1 = A p ; alpha = rho / (t1 . rh)
+    const int l = t & 63;
+    // a value of this thread's row q to the other workgroups, as words of e
+    auto put = [&](unsigned long long* lo, unsigned long long* hi, int q, unsigned e, double v) {
+      const unsigned long long tag = (unsigned long long)e << 32;
+      const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+      if (row[q] >= 0) {
+        st_agent(ps_at(lo, row[q]), (b & 0xffffffffull) | tag);
+        st_agent(ps_at(hi, row[q]), (b >> 32) | tag);
+      }
+    };
+    // N of the window's elements from w0 on: other workgroups' rows from their
+    // words of e (o[j]; own rows' entries are left)
+    auto get = [&]<int N>(const unsigned long long* lo, const unsigned long long* hi, unsigned e,
+                          int w0, double (&o)[N]) {
+      for (int spin = 0;;) {
+        unsigned long long a[N], b[N];
+        bool all = true;
 #pragma unroll
-    for (int w = 0; w < W; w++) win[w * T + t] = pw[w];
+        for (int j = 0; j < N; j++) {
+          const int c = wc[w0 + j];
+          a[j] = b[j] = (unsigned long long)e << 32;
+          if (c >= 0 && (c < oc0 || c >= oc1) && l < n - c * PS_CHUNK) {
+            a[j] = ld_word(lo + (int64_t)c * PS_CHUNK, l);
+            b[j] = ld_word(hi + (int64_t)c * PS_CHUNK, l);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+          all = all && (unsigned)(a[j] >> 32) == e && (unsigned)(b[j] >> 32) == e;
+          o[j] = __longlong_as_double((long long)((a[j] & 0xffffffffull) | (b[j] << 32)));
+        }
+        if (all) break;
+        if (++spin >= PS_SPIN || ((spin & 1023) == 0 && *(volatile int*)bad)) {
+          *bad = 1;
+          break;
+        }
+      }
+    };
+    // several rows per thread: v of every row into the window
+    auto exchange = [&](unsigned long long* lo, unsigned long long* hi, unsigned e,
+                        const double (&v)[R]) {
+#pragma unroll
+      for (int q = 0; q < R; q++) {
+        put(lo, hi, q, e, v[q]);
+        if (row[q] >= 0) win[s0 * PS_CHUNK + q * T + t] = v[q];
+      }
+#pragma unroll
+      for (int w0 = 0; w0 < W; w0 += 2) {
+        double o[2];
+        static_assert(ONE || W % 2 == 0, "window elements are read two at a time");
+        get(lo, hi, e, w0, o);
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          const int c = wc[w0 + j];
+          if (c >= 0 && (c < oc0 || c >= oc1)) win[(w0 + j) * T + t] = o[j];
+        }
+      }
+    };
+    // one row per thread: the window's v, own rows' from LDS
+    auto window = [&](const unsigned long long* lo, const unsigned long long* hi, unsigned e,
+                      double (&o)[WR]) {
+      get(lo, hi, e, 0, o);
+#pragma unroll
+      for (int w = 0; w < WR; w++)
+        if (wc[w] >= oc0 && wc[w] < oc1) o[w] = own[(wc[w] - oc0) * PS_CHUNK + l];
+    };
+    // t1 = A p ; alpha = rho / (t1 . rh)
+    if constexpr (ONE) {
+#pragma unroll
+      for (int w = 0; w < W; w++) win[w * T + t] = pw[w];
+    } else {
+      exchange(Q.rlo, Q.rhi, ep, p);
+    }
     __syncthreads();
     double v1[1][R], o1[1];
 #pragma unroll
     for (int q = 0; q < R; q++) {
       __builtin_amdgcn_sched_barrier(0);  // one row's loads in registers at a time
-      if (!XREG) rh[q] = (row[q] >= 0) ? *ps_at(D.rh, row[q]) : 0.0;
-      double t1 = 0.0;
-      if (row[q] >= 0) {
-        t1 = ps_row<KR>(M[q], Q.lidx, D.aval, cap, row[q], len[q], lmx[q], win);
-        st_agent(ps_at(D.t1, row[q]), t1);
+      if (!ONE) rh[q] = (row[q] >= 0) ? *ps_at(D.rh, row[q]) : 0.0;
+      t1[q] = (row[q] >= 0)
+                  ? ps_row<U, KR>(M[q], Q.lidx, Q.ls, D.aval, cap, row[q], len[q], lmx[q], win)
+                  : 0.0;
+      if constexpr (ONE) {
+        own[t] = t1[q];
+        put(Q.tlo, Q.thi, q, ep, t1[q]);
       }
-      T1(q) = t1;
-      v1[0][q] = (row[q] >= 0) ? t1 * rh[q] : 0.0;
+      v1[0][q] = (row[q] >= 0) ? t1[q] * rh[q] : 0.0;
     }
-    ok = ps_reduce<T, R, 1>(Q, nblk, b0, ep++, v1, area, col, bad, o1);
+    ok = ps_reduce<T, R, 1>(Q, nblk, b0, ep, v1, area, col, bad, o1, [&]() {
+      if constexpr (ONE) window(Q.tlo, Q.thi, ep, tw);
+    });
+    ep++;
     if (!ok) break;
-    // s = r - alpha t1 ; t2 = A s ; omega = (t2 . s) / (t2 . t2)
-#pragma unroll
-    for (int w = 0; w < W; w++) {
-      // uniform base of the chunk, one lane offset
-      const double* c = D.t1 + (int64_t)wc[w] * PS_CHUNK;
-      tw[w] = (wc[w] >= 0 && l < n - wc[w] * PS_CHUNK) ? ld_agent(c + (unsigned)l) : 0.0;
-    }
+    // s = r - alpha t1 (in r) ; t2 = A s ; omega = (t2 . s) / (t2 . t2)
     alpha = rho / o1[0];
 #pragma unroll
-    for (int w = 0; w < W; w++) win[w * T + t] = rw[w] - alpha * tw[w];
+    for (int q = 0; q < R; q++) r[q] = r[q] - alpha * t1[q];
+    if constexpr (ONE) {
+#pragma unroll
+      for (int w = 0; w < W; w++) win[w * T + t] = rw[w] - alpha * tw[w];
+    } else {
+      exchange(Q.tlo, Q.thi, ep, r);
+    }
     __syncthreads();
-    double s[R], t2[R], v2[2][R], o2[2];
+    double t2[R], v2[2][R], o2[2];
 #pragma unroll
     for (int q = 0; q < R; q++) {
       __builtin_amdgcn_sched_barrier(0);
-      if (!XREG) r[q] = (row[q] >= 0) ? ld_agent(ps_at(D.r, row[q])) : 0.0;
-      t2[q] = (row[q] >= 0) ? ps_row<KR>(M[q], Q.lidx, D.aval, cap, row[q], len[q], lmx[q], win) : 0.0;
-      s[q] = r[q] - alpha * T1(q);
-      v2[0][q] = (row[q] >= 0) ? t2[q] * s[q] : 0.0;
+      t2[q] = (row[q] >= 0)
+                  ? ps_row<U, KR>(M[q], Q.lidx, Q.ls, D.aval, cap, row[q], len[q], lmx[q], win)
+                  : 0.0;
+      v2[0][q] = (row[q] >= 0) ? t2[q] * r[q] : 0.0;
       v2[1][q] = (row[q] >= 0) ? t2[q] * t2[q] : 0.0;
     }
-    ok = ps_reduce<T, R, 2>(Q, nblk, b0, ep++, v2, area, col, bad, o2);
+    ok = ps_reduce<T, R, 2>(Q, nblk, b0, ep, v2, area, col, bad, o2, [&]() {
+      if constexpr (!ONE) {
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+          rh[q] = (row[q] >= 0) ? *ps_at(D.rh, row[q]) : 0.0;
+          x[q] = (row[q] >= 0) ? *ps_at(D.sol, row[q]) : 0.0;
+        }
+      }
+    });
+    ep++;
     if (!ok) break;
     omega = o2[0] / o2[1];
     // x = (x + alpha p) + omega s ; r = s - omega t2 ; rho' = r . rh ; rr = r . r
 #pragma unroll
     for (int q = 0; q < R; q++) {
-      if (!XREG) {
-        rh[q] = (row[q] >= 0) ? *ps_at(D.rh, row[q]) : 0.0;
-        x[q] = (row[q] >= 0) ? *ps_at(D.sol, row[q]) : 0.0;
-      }
-      x[q] = (x[q] + alpha * P(q)) + omega * s[q];
-      r[q] = s[q] - omega * t2[q];
-      if (row[q] >= 0) {
-        st_agent(ps_at(D.r, row[q]), r[q]);
-        if (!XREG) *ps_at(D.sol, row[q]) = x[q];
+      x[q] = (x[q] + alpha * p[q]) + omega * r[q];
+      if (!ONE && row[q] >= 0) *ps_at(D.sol, row[q]) = x[q];
+      r[q] = r[q] - omega * t2[q];
+      p[q] = p[q] - omega * t1[q];
+      if constexpr (ONE) {
+        own[t] = r[q];
+        put(Q.rlo, Q.rhi, q, ep, r[q]);
       }
       v2[0][q] = (row[q] >= 0) ? r[q] * rh[q] : 0.0;
       v2[1][q] = (row[q] >= 0) ? r[q] * r[q] : 0.0;
-      P(q) = P(q) - omega * T1(q);
     }
+    if constexpr (ONE) {
 #pragma unroll
-    for (int w = 0; w < W; w++) pw[w] = pw[w] - omega * tw[w];
-    ok = ps_reduce<T, R, 2>(Q, nblk, b0, ep++, v2, area, col, bad, o2);
+      for (int w = 0; w < W; w++) pw[w] = pw[w] - omega * tw[w];
+    }
+    ok = ps_reduce<T, R, 2>(Q, nblk, b0, ep, v2, area, col, bad, o2, [&]() {
+      if constexpr (ONE) window(Q.rlo, Q.rhi, ep, rw);
+    });
+    ep++;
     if (!ok) break;
     // FIN_BETA
     it++;
@@ -557,22 +656,20 @@ __global__ void __launch_bounds__(T) k_bicg_resident(Dev D, PersArg Q, int iters
     }
     if (done) break;
     // p = r + beta (p - omega t1), here and over the window
+    if constexpr (ONE) {
 #pragma unroll
-    for (int w = 0; w < W; w++) {
-      // uniform base of the chunk, one lane offset
-      const double* c = D.r + (int64_t)wc[w] * PS_CHUNK;
-      rw[w] = (wc[w] >= 0 && l < n - wc[w] * PS_CHUNK) ? ld_agent(c + (unsigned)l) : 0.0;
+      for (int w = 0; w < W; w++) pw[w] = rw[w] + beta * pw[w];
     }
 #pragma unroll
-    for (int w = 0; w < W; w++) pw[w] = rw[w] + beta * pw[w];
-#pragma unroll
-    for (int q = 0; q < R; q++) P(q) = r[q] + beta * P(q);
+    for (int q = 0; q < R; q++) p[q] = r[q] + beta * p[q];
   }
+  const int t = threadIdx.x;
 #pragma unroll
   for (int q = 0; q < R; q++)
     if (row[q] >= 0) {
-      if (XREG) *ps_at(D.sol, row[q]) = x[q];
-      *ps_at(D.pp, row[q]) = P(q);
+      if (ONE) D.sol[row[q]] = x[q];
+      D.pp[row[q]] = p[q];
+      D.r[row[q]] = r[q];
     }
   if (t == 0 && !ok) atomicOr(&Sc->counter[PS_FLAG_ABORT], 1u);
   if (wg == 0 && t == 0 && ok) {
