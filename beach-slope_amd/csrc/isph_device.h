@@ -35,6 +35,8 @@ struct DevParams {
   double cs;        // incr*h1 = 4h (setup.f90:120-123)
   double k1, k2;    // 10/(28*3.14 h^2), 1/(3*3.14 h^2), real4 products (kernel.f90:61-62)
   double two_h, lim2, wo;
+  // correctly rounded reciprocals of h, h^2 and h^3 (div_by), and 12 / h^2
+  double yh, yhh, yhhh, c12;
   // weakly compressible variant: sound speed, Tait exponent, delta-SPH
   // coefficient, still-water level of the hydrostatic density
   double c0, gam, delt, swl;
@@ -234,16 +236,32 @@ __device__ __forceinline__ A ell_row_sum_any(const Dev& D, const VAL* __restrict
 // ---------------------------------------------------------------------
 // kernel.f90 restatement (device)
 // ---------------------------------------------------------------------
+// a / b from y = 1 / b rounded to nearest, with the division's own bits: two
+// steps q + (a - b q) y, the first of which makes q faithful and the second,
+// by Markstein's theorem (P. W. Markstein, IBM J. Res. Dev. 34, 1990: exact
+// FMA residual, y correctly rounded, q faithful), correctly rounded.  For
+// operands whose quotient and residual are normal numbers: here b is a power
+// of the smoothing length and a a multiple of a power of r <= 2h (a
+// subnormal a, r below 1e-102, differs from the division in bits that the
+// sum it goes into drops).  Five FMAs where the division takes eleven
+// instructions, one of them at a quarter of their rate.
+__device__ __forceinline__ double div_by(double a, double b, double y) {
+  double q = a * y;
+  q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
 // Wab, kernel.f90:34-66 (hWab, kernel.f90:164-184, is identical).
 __device__ __forceinline__ double d_wab(double r, const DevParams& P) {
   const double h = P.h;
+  const double q = div_by(r, h, P.yh);  // r / h
   double t1, t2;
   if (r < h) {
-    t1 = (4.0 - ((6.0 * (r * r)) / (h * h))) + ((3.0 * ((r * r) * r)) / ((h * h) * h));
-    const double q = r / h;
-    t2 = (((q * q) * q) - ((6.0 * r) / h)) + 6.0;
+    t1 = (4.0 - div_by(6.0 * (r * r), h * h, P.yhh)) +
+         div_by(3.0 * ((r * r) * r), (h * h) * h, P.yhhh);
+    t2 = (((q * q) * q) - div_by(6.0 * r, h, P.yh)) + 6.0;
   } else {
-    const double a = 2.0 - r / h;
+    const double a = 2.0 - q;
     t1 = (a * a) * a;
     t2 = t1;
   }
@@ -257,29 +275,29 @@ __device__ __forceinline__ double d_wab(double r, const DevParams& P) {
 //   else:   t1 = t2 = ((3 / (r h)) (2 - r / h)^2) (-d)
 //   W'     = (0.1 t1) k1 + (0.9 t2) k2,
 // rounded as written; the bracketed factors depend on r alone, so they are
-// formed once (their divisions are most of the pair's FP64 work) and
-// multiply both components, which gives each component the same bits.  The
-// lanes of a wavefront take both branches, so the divisions of the two
-// branches share instructions: lane by lane the first divides 9r by h^3 or
-// r by h, the second 3r by h^3 or 3 by r h, each its own branch's operands.
+// formed once and multiply both components, which gives each component the
+// same bits.  Of their five divisions one is left: those by powers of h are
+// div_by, and 6 / (r h) is twice 3 / (r h), exactly.  The lanes of a
+// wavefront take both branches, so 9r / h^3 and r / h share instructions, each
+// lane with its own branch's operands.
 __device__ __forceinline__ void d_wabd2(double dx, double dy, double r, const DevParams& P,
                                         double& kx, double& ky) {
   const double h = P.h;
   const bool nr = r < h;
   const double hhh = (h * h) * h, rh = r * h;
-  const double qa = (nr ? 9.0 * r : r) / (nr ? hhh : h);      // 9r / h^3  |  r / h
-  const double qb = (nr ? 3.0 * r : 3.0) / (nr ? hhh : rh);   // 3r / h^3  |  3 / (r h)
+  const double qa = div_by(nr ? 9.0 * r : r, nr ? hhh : h, nr ? P.yhhh : P.yh);
+  const double g = 3.0 / rh;
   double t1x, t2x, t1y, t2y;
   if (nr) {
-    const double f1 = qa - (12.0 / (h * h));
-    const double f2 = qb - (6.0 / rh);
+    const double f1 = qa - P.c12;
+    const double f2 = div_by(3.0 * r, hhh, P.yhhh) - (2.0 * g);
     t1x = f1 * dx;
     t2x = f2 * dx;
     t1y = f1 * dy;
     t2y = f2 * dy;
   } else {
     const double a = 2.0 - qa;
-    const double f = qb * (a * a);
+    const double f = g * (a * a);
     t1x = f * (-dx);
     t2x = t1x;
     t1y = f * (-dy);

@@ -185,6 +185,10 @@ static void fill_devparams(isph_ctx* c) {
   d.two_h = 2 * P.h;
   d.lim2 = (d.two_h * d.two_h) * (1.0 + 1e-9);
   d.wo = host_wo(P.h, d.k1, d.k2);
+  d.yh = 1.0 / P.h;
+  d.yhh = 1.0 / (P.h * P.h);
+  d.yhhh = 1.0 / ((P.h * P.h) * P.h);
+  d.c12 = 12.0 / (P.h * P.h);
 }
 
 // ---------------------------------------------------------------------
