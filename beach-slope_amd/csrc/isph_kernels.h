@@ -18,6 +18,126 @@
   const int i = blockIdx.x * blockDim.x + threadIdx.x; \
   const int n = D.sc->n;
 
+// ---------------------------------------------------------------------
+// Lanes per particle.  The neighbour-sum kernels run with one lane per
+// particle (LPP 1) or eight (LPP 8).  A particle's walk over its ~20
+// neighbours is a serial chain of loads and FP64 operations: with few
+// particles the chip waits on that chain (one wavefront per SIMD and less), and
+// eight lanes that each take every eighth pair cut it to three rounds.  The
+// pairs' addends are computed in parallel; every lane of the group then adds
+// them in list order, so sums have the bits of the serial walk.  The lanes of
+// a group leave every loop together.
+// ---------------------------------------------------------------------
+// value of lane U of each group of eight lanes
+template <int U>
+__device__ __forceinline__ double bcast8(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_ds_swizzle((int)b, (U << 5) | 0x18);
+  const int hi = __builtin_amdgcn_ds_swizzle((int)(b >> 32), (U << 5) | 0x18);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+// the group's eight bits of a ballot
+__device__ __forceinline__ unsigned bits8(bool v) {
+  return (unsigned)(__ballot(v) >> (threadIdx.x & 56)) & 0xffu;
+}
+// LDS accesses of this wavefront before the call are done before those after
+__device__ __forceinline__ void wave_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// S sums over the pairs of a group of eight lanes, each pair with Q addends
+// (a[s * Q + q]) to each: lane s of the group holds sum s, and adds the
+// group's addends to it in pair order out of LDS.  Rows are 16 bytes longer
+// than the addends, so the lanes' 16-byte reads fall on different banks.
+template <int S, int Q>
+struct Fold8 {
+  static constexpr int ROW = 8 * Q + 2;
+  double* w;        // where this lane's addends go
+  const double* r;  // this lane's sum's addends
+  double acc = 0.0;
+  __device__ __forceinline__ Fold8(int sub) {
+    __shared__ __align__(16) double buf[RED_BLOCK / 8][S * ROW];
+    double* g = buf[threadIdx.x >> 3];
+    w = g + Q * sub;
+    r = g + ROW * (S < 8 ? min(sub, S - 1) : sub);
+  }
+  // lanes without a pair bring zeros (a sum that starts at +0 never is -0,
+  // so adding +0 leaves it alone)
+  __device__ __forceinline__ void add(const double (&a)[S * Q]) {
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+      for (int q = 0; q < Q; q++) w[s * ROW + q] = a[s * Q + q];
+    wave_lds();
+    double2 v[4 * Q];
+#pragma unroll
+    for (int k = 0; k < 4 * Q; k++) v[k] = ((const double2*)r)[k];
+#pragma unroll
+    for (int k = 0; k < 4 * Q; k++) {
+      acc = acc + v[k].x;
+      acc = acc + v[k].y;
+    }
+    wave_lds();
+  }
+  template <int U>
+  __device__ __forceinline__ void get(double (&sum)[S]) const {
+    if constexpr (U < S) {
+      sum[U] = bcast8<U>(acc);
+      get<U + 1>(sum);
+    }
+  }
+};
+
+// Walk over the cnt neighbours of particle i: load(j) reads the fields of
+// neighbour j, term(f, a) forms the pair's Q addends to each of the S sums
+// (which start at 0); they are added in list order.  With one lane, two
+// neighbours' fields are requested before either is used.
+template <int LPP, int S, int Q, typename LOAD, typename TERM>
+__device__ __forceinline__ void walk_pairs(const int32_t* nbr, int cap, int i, int sub, int cnt,
+                                           LOAD load, TERM term, double (&sum)[S]) {
+  typedef decltype(load(0)) F;
+  if constexpr (LPP == 1) {
+#pragma unroll
+    for (int s = 0; s < S; s++) sum[s] = 0.0;
+    auto pair = [&](const F& f) {
+      double a[S * Q];
+      term(f, a);
+#pragma unroll
+      for (int s = 0; s < S; s++)
+#pragma unroll
+        for (int q = 0; q < Q; q++) sum[s] = sum[s] + a[s * Q + q];
+    };
+    for (int k0 = 0; k0 < cnt; k0 += 2) {
+      int jb[2];
+#pragma unroll
+      for (int q = 0; q < 2; q++) jb[q] = (k0 + q < cnt) ? nbr[(k0 + q) * cap + i] : i;
+      const F f0 = load(jb[0]), f1 = load(jb[1]);
+      pair(f0);
+      if (k0 + 1 >= cnt) break;
+      pair(f1);
+    }
+  } else {
+    Fold8<S, Q> fold(sub);
+    for (int k0 = 0; k0 < cnt; k0 += 8) {
+      const bool on = k0 + sub < cnt;
+      const F f = load(on ? nbr[(k0 + sub) * cap + i] : i);
+      double a[S * Q];
+#pragma unroll
+      for (int m = 0; m < S * Q; m++) a[m] = 0.0;
+      if (on) term(f, a);
+      fold.add(a);
+    }
+    fold.template get<0>(sum);
+  }
+}
+
+// particle and lane of its group
+#define PIDX_L(LPP)                                                  \
+  const int g_ = blockIdx.x * blockDim.x + threadIdx.x;              \
+  const int i = (LPP) == 1 ? g_ : g_ / (LPP), sub = (LPP) == 1 ? 0 : g_ % (LPP); \
+  const int n = D.sc->n;
+
 __global__ void k_fill_i32(int32_t* a, int len, int val) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < len) a[i] = val;
@@ -279,6 +399,35 @@ __global__ void k_scan_add(int32_t* out, const int32_t* tile_sums, int len) {
 // ---------------------------------------------------------------------
 // neighbour / nsearch2, search.f90:13-399
 // ---------------------------------------------------------------------
+// the search's results of particle i from its position, neighbour count and
+// the gradient-correction sums
+__device__ __forceinline__ void neighbour_store(const Dev& D, const int i, int cnt, double xi,
+                                                double yi, double m0, double m1, double m2,
+                                                double m3) {
+  const DevParams& P = D.P;
+  D.ncnt[i] = cnt;
+  D.xnb[i] = xi;
+  D.ynb[i] = yi;
+  uint8_t fl = D.flags[i] & (uint8_t)~F_FREE;
+  double gv = 0.0;
+  if (D.tid[i] == TID_FLUID) {
+    D.vic[i] = 0;
+    gv = m0 + m3;
+    // invertmat2D, functions.f90:62-96 (1e-5 is a real4 literal)
+    const double det = m0 * m3 - m1 * m2;
+    double c1, c2, c3, c4;
+    if ((fabs(det) >= (double)1e-5f) && !isnan(det) && isfinite(det)) {
+      c1 = m3 / det; c2 = (-m1) / det; c3 = (-m2) / det; c4 = m0 / det;
+    } else {
+      c1 = 1.0; c2 = 0.0; c3 = 0.0; c4 = 1.0;
+    }
+    D.cf1[i] = c1; D.cf2[i] = c2; D.cf3[i] = c3; D.cf4[i] = c4;
+    if ((gv <= P.fs_thresh) && !(fl & F_BUFFER)) fl |= F_FREE;
+  }
+  D.gradvx[i] = gv;
+  D.flags[i] = fl;
+}
+
 // The search for particle i.  POS(j, x, y) gives particle j's position,
 // MR(j, m, rho) its mass and density: read from global memory by the
 // per-particle kernel, from the workgroup's LDS tile by the tiled one; the
@@ -365,27 +514,7 @@ __device__ __forceinline__ void neighbour_core(const Dev& D, const int i, POS po
       m3 = m3 + k2 * r3;
     }
   }
-  D.ncnt[i] = cnt;
-  D.xnb[i] = xi;
-  D.ynb[i] = yi;
-  uint8_t fl = D.flags[i] & (uint8_t)~F_FREE;
-  double gv = 0.0;
-  if (D.tid[i] == TID_FLUID) {
-    D.vic[i] = 0;
-    gv = m0 + m3;
-    // invertmat2D, functions.f90:62-96 (1e-5 is a real4 literal)
-    const double det = m0 * m3 - m1 * m2;
-    double c1, c2, c3, c4;
-    if ((fabs(det) >= (double)1e-5f) && !isnan(det) && isfinite(det)) {
-      c1 = m3 / det; c2 = (-m1) / det; c3 = (-m2) / det; c4 = m0 / det;
-    } else {
-      c1 = 1.0; c2 = 0.0; c3 = 0.0; c4 = 1.0;
-    }
-    D.cf1[i] = c1; D.cf2[i] = c2; D.cf3[i] = c3; D.cf4[i] = c4;
-    if ((gv <= P.fs_thresh) && !(fl & F_BUFFER)) fl |= F_FREE;
-  }
-  D.gradvx[i] = gv;
-  D.flags[i] = fl;
+  neighbour_store(D, i, cnt, xi, yi, m0, m1, m2, m3);
 }
 
 __device__ __forceinline__ void neighbour_body(const Dev& D, const int i, const int n) {
@@ -397,6 +526,89 @@ __device__ __forceinline__ void neighbour_body(const Dev& D, const int i, const 
 __global__ void __launch_bounds__(256) k_neighbour(Dev D) {
   PIDX();
   neighbour_body(D, i, n);
+}
+
+// The search with eight lanes per particle: eight candidates are tested at
+// once (32 positions in flight), the accepted ones take their list positions
+// by a ballot, and the pairs of the list, kept in LDS, are shared out.
+__device__ __forceinline__ void neighbour_body8(const Dev& D, const int i, const int sub,
+                                                const int n) {
+  __shared__ int32_t list[RED_BLOCK / 8][NBR_CAP];
+  int32_t* mine = list[threadIdx.x >> 3];
+  if (i >= n) return;
+  const DevParams& P = D.P;
+  const int cap = D.cap;
+  const double xi = D.x[i], yi = D.y[i];
+  int ci, cj;
+  double xl, xr, yb, yt;
+  cell_bounds(D.cell[i], P, ci, cj, xl, xr, yb, yt);
+  const int q = quadrant(xi, yi, xl, xr, yb, yt);
+  const int r0 = ci - ((q == 2 || q == 3) ? 1 : 0);
+  const int c0 = cj - ((q == 0 || q == 3) ? 1 : 0);
+  const int ka = c0 * P.celly + r0, kb = ka + P.celly;
+  const int ja = D.cstart[ka], ea = D.cstart[ka + 2], jc = D.cstart[kb], ec = D.cstart[kb + 2];
+  int cnt = 0;
+  constexpr int NB = 4;
+#pragma unroll 1
+  for (int half = 0; half < 2; half++) {
+    const int jb = half ? jc : ja, je = half ? ec : ea;
+    for (int b0 = jb; b0 < je; b0 += 8 * NB) {
+      double cx[NB], cy[NB];
+#pragma unroll
+      for (int u = 0; u < NB; u++) {
+        const int j = min(b0 + 8 * u + sub, je - 1);
+        cx[u] = D.x[j];
+        cy[u] = D.y[j];
+      }
+#pragma unroll
+      for (int u = 0; u < NB; u++) {
+        const int j = b0 + 8 * u + sub;
+        const double dx = xi - cx[u], dy = yi - cy[u];
+        const double d2 = (dx * dx) + (dy * dy);
+        const bool in = j < je && j != i && !(d2 > P.lim2) && sqrt(d2) < P.two_h;
+        const unsigned hit = bits8(in);
+        const int at = cnt + __popc(hit & ((1u << sub) - 1u));
+        if (in && at < NBR_CAP) {
+          D.nbr[at * cap + i] = j;
+          mine[at] = j;
+        }
+        cnt += __popc(hit);
+      }
+    }
+  }
+  if (cnt > NBR_CAP) {
+    // the step fails with ISPH_ECAP; the sums below cover the stored entries
+    if (sub == 0) atomicOr(&D.sc->err, ERR_NBR_CAP);
+    cnt = NBR_CAP;
+  }
+  // the list's entries were written by other lanes of this wavefront
+  wave_lds();
+  Fold8<4, 1> fold(sub);
+  for (int k0 = 0; k0 < cnt; k0 += 8) {
+    double a[4] = {0.0, 0.0, 0.0, 0.0};
+    if (k0 + sub < cnt) {
+      const int j = mine[k0 + sub];
+      const double xj = D.x[j], yj = D.y[j], mj = D.m[j], rj = D.rho[j];
+      const double dx = xi - xj, dy = yi - yj;
+      const double r = sqrt((dx * dx) + (dy * dy));
+      double k1, k2;
+      d_wabd2(dx, dy, r, P, k1, k2);
+      const double r1 = (mj * (xj - xi)) / rj;
+      const double r3 = (mj * (yj - yi)) / rj;
+      a[0] = k1 * r1;
+      a[1] = k2 * r1;
+      a[2] = k1 * r3;
+      a[3] = k2 * r3;
+    }
+    fold.add(a);
+  }
+  double m[4];
+  fold.get<0>(m);
+  if (sub == 0) neighbour_store(D, i, cnt, xi, yi, m[0], m[1], m[2], m[3]);
+}
+__global__ void __launch_bounds__(256) k_neighbour8(Dev D) {
+  PIDX_L(8);
+  neighbour_body8(D, i, sub, n);
 }
 
 // ---------------------------------------------------------------------
@@ -482,12 +694,16 @@ __global__ void __launch_bounds__(256) k_neighbour_tile8(Dev D) {
 // ---------------------------------------------------------------------
 // effpor + porsearch, porous.f90:32-224
 // ---------------------------------------------------------------------
-__device__ __forceinline__ void effpor_body(const Dev& D, const int i, const int n) {
+template <int LPP>
+__device__ __forceinline__ void effpor_body(const Dev& D, const int i, const int n,
+                                            const int sub = 0) {
   if (i >= n) return;
   const DevParams& P = D.P;
-  D.resist[i] = 0.0;
   if (D.tid[i] != TID_FLUID) {
-    D.por[i] = 1.0;  // non-fluid porosity keeps its default (particle.f90:62-64)
+    if (sub == 0) {
+      D.resist[i] = 0.0;
+      D.por[i] = 1.0;  // non-fluid porosity keeps its default (particle.f90:62-64)
+    }
     return;
   }
   int ci, cj;
@@ -503,39 +719,66 @@ __device__ __forceinline__ void effpor_body(const Dev& D, const int i, const int
   else { di[1] = -1; di[2] = -1; dj[2] = -1; dj[3] = -1; }
   const double por = P.por;
   double sf = 0.0;
-  // eight solids' positions requested before any is tested, then the mass
-  // and density of those within reach requested before any is used (the sum
-  // stays in solid order)
-  constexpr int NB_SOL = 8;
-  for (int cb = 0; cb < 4; cb++) {
-    const int k = (cj + dj[cb]) * P.celly + (ci + di[cb]);
-    const int qe = D.sstart[k + 1];
-    for (int s0 = D.sstart[k]; s0 < qe; s0 += NB_SOL) {
-      double sx[NB_SOL], sy[NB_SOL], d2[NB_SOL], sm[NB_SOL], sr[NB_SOL];
+  if constexpr (LPP == 1) {
+    // eight solids' positions requested before any is tested, then the mass
+    // and density of those within reach requested before any is used (the sum
+    // stays in solid order)
+    constexpr int NB_SOL = 8;
+    for (int cb = 0; cb < 4; cb++) {
+      const int k = (cj + dj[cb]) * P.celly + (ci + di[cb]);
+      const int qe = D.sstart[k + 1];
+      for (int s0 = D.sstart[k]; s0 < qe; s0 += NB_SOL) {
+        double sx[NB_SOL], sy[NB_SOL], d2[NB_SOL], sm[NB_SOL], sr[NB_SOL];
 #pragma unroll
-      for (int u = 0; u < NB_SOL; u++) {
-        const int s = (s0 + u < qe) ? s0 + u : s0;
-        sx[u] = D.sx[s];
-        sy[u] = D.sy[s];
-      }
+        for (int u = 0; u < NB_SOL; u++) {
+          const int s = (s0 + u < qe) ? s0 + u : s0;
+          sx[u] = D.sx[s];
+          sy[u] = D.sy[s];
+        }
 #pragma unroll
-      for (int u = 0; u < NB_SOL; u++) {
-        const double dx = x - sx[u], dy = y - sy[u];
-        d2[u] = (dx * dx) + (dy * dy);
-        // certainly beyond 2h (or past the cell's solids): nothing to read
-        const bool in = (s0 + u < qe) && !(d2[u] > P.lim2);
-        const int s = in ? s0 + u : s0;
-        sm[u] = in ? D.sm[s] : 0.0;
-        sr[u] = in ? D.srho[s] : 1.0;
-      }
+        for (int u = 0; u < NB_SOL; u++) {
+          const double dx = x - sx[u], dy = y - sy[u];
+          d2[u] = (dx * dx) + (dy * dy);
+          // certainly beyond 2h (or past the cell's solids): nothing to read
+          const bool in = (s0 + u < qe) && !(d2[u] > P.lim2);
+          const int s = in ? s0 + u : s0;
+          sm[u] = in ? D.sm[s] : 0.0;
+          sr[u] = in ? D.srho[s] : 1.0;
+        }
 #pragma unroll
-      for (int u = 0; u < NB_SOL; u++) {
-        if (s0 + u >= qe) break;
-        if (d2[u] > P.lim2) continue;  // no square root
-        const double r = sqrt(d2[u]);
-        if (r < P.two_h) sf = sf + ((((1.0 - por * 1.0) * d_wab(r, P)) * sm[u]) / sr[u]);
+        for (int u = 0; u < NB_SOL; u++) {
+          if (s0 + u >= qe) break;
+          if (d2[u] > P.lim2) continue;  // no square root
+          const double r = sqrt(d2[u]);
+          if (r < P.two_h) sf = sf + ((((1.0 - por * 1.0) * d_wab(r, P)) * sm[u]) / sr[u]);
+        }
       }
     }
+  } else {
+    // the four cells' ranges in one trip, then eight solids at a time
+    Fold8<1, 1> fold(sub);
+    int sb[4], se[4];
+#pragma unroll
+    for (int cb = 0; cb < 4; cb++) {
+      const int k = (cj + dj[cb]) * P.celly + (ci + di[cb]);
+      sb[cb] = D.sstart[k];
+      se[cb] = D.sstart[k + 1];
+    }
+#pragma unroll
+    for (int cb = 0; cb < 4; cb++)
+      for (int s0 = sb[cb]; s0 < se[cb]; s0 += 8) {
+        const int s = min(s0 + sub, se[cb] - 1);
+        const double dx = x - D.sx[s], dy = y - D.sy[s], ms = D.sm[s], rs = D.srho[s];
+        const double d2 = (dx * dx) + (dy * dy);
+        double a[1] = {0.0};
+        if (s0 + sub < se[cb] && !(d2 > P.lim2)) {
+          const double r = sqrt(d2);
+          if (r < P.two_h) a[0] = (((1.0 - por * 1.0) * d_wab(r, P)) * ms) / rs;
+        }
+        fold.add(a);
+      }
+    if (sub != 0) return;
+    sf = fold.acc;
   }
   if (sf > (1.0 - por)) sf = 1.0 - por;
   const double nn = 1.0 - sf;
@@ -550,107 +793,105 @@ __device__ __forceinline__ void effpor_body(const Dev& D, const int i, const int
   const double b = (((fch * sp) * sqrt(P.lamk)) * (1.0 - nn)) / (sqrt(n3) * P.d50);
   D.resist[i] = a - b;
 }
-__global__ void k_effpor(Dev D) {
-  PIDX();
-  effpor_body(D, i, n);
+template <int LPP>
+__global__ void __launch_bounds__(256) k_effpor(Dev D) {
+  PIDX_L(LPP);
+  effpor_body<LPP>(D, i, n, sub);
 }
 
 // ---------------------------------------------------------------------
 // eddyvis, turbulence.f90:12-110
 // ---------------------------------------------------------------------
-__device__ __forceinline__ void eddyvis_body(const Dev& D, const int i, const int n) {
+template <int LPP>
+__device__ __forceinline__ void eddyvis_body(const Dev& D, const int i, const int n,
+                                             const int sub = 0) {
   if (i >= n) return;
   if (D.tid[i] != TID_FLUID) {
-    D.nut[i] = 0.0;
-    D.tke[i] = 0.0;
+    if (sub == 0) {
+      D.nut[i] = 0.0;
+      D.tke[i] = 0.0;
+    }
     return;
   }
   const DevParams& P = D.P;
-  const int cap = D.cap, cnt = D.ncnt[i];
   const double c1 = D.cf1[i], c2 = D.cf2[i], c3 = D.cf3[i], c4 = D.cf4[i];
   const double xi = D.xnb[i], yi = D.ynb[i];
   const double ui = D.u[i] / D.por[i], vi = D.v[i] / D.por[i];
-  double t1 = 0.0, t2 = 0.0, t3 = 0.0;
-  // neighbours two at a time: both neighbours' fields are requested before
-  // either is used (the sums stay in list order)
-  for (int k0 = 0; k0 < cnt; k0 += 2) {
-    int jb[2];
-    double xb[2], yb[2], nb[2], mb[2], rb[2], ub[2], vb[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) jb[q] = (k0 + q < cnt) ? D.nbr[(k0 + q) * cap + i] : i;
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int j = jb[q];
-      xb[q] = D.xnb[j]; yb[q] = D.ynb[j]; nb[q] = D.por[j]; mb[q] = D.m[j];
-      rb[q] = D.rho[j]; ub[q] = D.u[j]; vb[q] = D.v[j];
-    }
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      if (k0 + q >= cnt) break;
-      const Klt z = d_klt(xi - xb[q], yi - yb[q], P);
-      const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
-      const double nj = nb[q], mj = mb[q], rj = rb[q];
-      const double du = (ub[q] / nj) - ui, dv = (vb[q] / nj) - vi;
-      t1 = t1 + ((mj * du) * gx) / rj;
-      t2 = t2 + ((mj * dv) * gy) / rj;
-      t3 = t3 + ((0.50 * mj) * ((du * gy) + (dv * gx))) / rj;
-    }
-  }
+  double t[3];
+  struct F {
+    double x, y, n, m, r, u, v;
+  };
+  walk_pairs<LPP, 3, 1>(
+      D.nbr, D.cap, i, sub, D.ncnt[i],
+      [&](int j) {
+        return F{D.xnb[j], D.ynb[j], D.por[j], D.m[j], D.rho[j], D.u[j], D.v[j]};
+      },
+      [&](const F& f, double (&a)[3]) {
+        const Klt z = d_klt(xi - f.x, yi - f.y, P);
+        const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
+        const double du = (f.u / f.n) - ui, dv = (f.v / f.n) - vi;
+        a[0] = ((f.m * du) * gx) / f.r;
+        a[1] = ((f.m * dv) * gy) / f.r;
+        a[2] = ((0.50 * f.m) * ((du * gy) + (dv * gx))) / f.r;
+      },
+      t);
+  if (sub != 0) return;
+  const double t1 = t[0], t2 = t[1], t3 = t[2];
   const double t4 = sqrt((2 * ((t1 * t1) + (t2 * t2))) + ((2 * t3) * (2 * t3)));
   const double dl = P.dl;
   D.nut[i] = ((0.150 * dl) * (0.150 * dl)) * t4;
   D.tke[i] = (0.080 / 1.0) * ((dl * t4) * (dl * t4));
 }
-__global__ void k_eddyvis(Dev D) {
-  PIDX();
-  eddyvis_body(D, i, n);
+template <int LPP>
+__global__ void __launch_bounds__(256) k_eddyvis(Dev D) {
+  PIDX_L(LPP);
+  eddyvis_body<LPP>(D, i, n, sub);
 }
 
 // ---------------------------------------------------------------------
 // int_vel, integrator.f90:459-703 (pass 1: varts of free particles)
 // ---------------------------------------------------------------------
-__device__ __forceinline__ void int_vel_varts_body(const Dev& D, const int i, const int n) {
+template <int LPP>
+__device__ __forceinline__ void int_vel_varts_body(const Dev& D, const int i, const int n,
+                                                   const int sub = 0) {
   if (i >= n || !(D.flags[i] & F_FREE)) return;
   const DevParams& P = D.P;
-  const int cap = D.cap, cnt = D.ncnt[i];
   const double c1 = D.cf1[i], c2 = D.cf2[i], c3 = D.cf3[i], c4 = D.cf4[i];
   const double xi = D.xnb[i], yi = D.ynb[i];
   const double ui = D.u[i] / D.por[i], vi = D.v[i] / D.por[i];
-  double t1 = 0.0, t2 = 0.0;
-  // neighbours two at a time: both neighbours' fields are requested before
-  // either is used (the sums stay in list order)
-  for (int k0 = 0; k0 < cnt; k0 += 2) {
-    int jb[2];
-    double xb[2], yb[2], nb[2], mb[2], rb[2], ub[2], vb[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) jb[q] = (k0 + q < cnt) ? D.nbr[(k0 + q) * cap + i] : i;
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int j = jb[q];
-      xb[q] = D.xnb[j]; yb[q] = D.ynb[j]; nb[q] = D.por[j]; mb[q] = D.m[j];
-      rb[q] = D.rho[j]; ub[q] = D.u[j]; vb[q] = D.v[j];
-    }
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      if (k0 + q >= cnt) break;
-      const Klt z = d_klt(xi - xb[q], yi - yb[q], P);
-      const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
-      const double nj = nb[q], vj = mb[q] / rb[q];
-      t1 = t1 + (((ub[q] / nj) - ui) * gx) * vj;
-      t2 = t2 + (((vb[q] / nj) - vi) * gy) * vj;
-    }
-  }
+  double t[2];
+  struct F {
+    double x, y, n, m, r, u, v;
+  };
+  walk_pairs<LPP, 2, 1>(
+      D.nbr, D.cap, i, sub, D.ncnt[i],
+      [&](int j) {
+        return F{D.xnb[j], D.ynb[j], D.por[j], D.m[j], D.rho[j], D.u[j], D.v[j]};
+      },
+      [&](const F& f, double (&a)[2]) {
+        const Klt z = d_klt(xi - f.x, yi - f.y, P);
+        const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
+        const double vj = f.m / f.r;
+        a[0] = (((f.u / f.n) - ui) * gx) * vj;
+        a[1] = (((f.v / f.n) - vi) * gy) * vj;
+      },
+      t);
+  if (sub != 0) return;
+  const double t1 = t[0], t2 = t[1];
   const double uu = D.u[i], vv = D.v[i];
   D.varts[i] = (((1.0 * (P.dl * P.dl)) * sqrt((t1 * t1) + (t2 * t2))) * sqrt((uu * uu) + (vv * vv))) /
                ((D.sc->umax + (double)1e-6f) * D.por[i]);
 }
-__global__ void k_int_vel_varts(Dev D) {
-  PIDX();
-  int_vel_varts_body(D, i, n);
+template <int LPP>
+__global__ void __launch_bounds__(256) k_int_vel_varts(Dev D) {
+  PIDX_L(LPP);
+  int_vel_varts_body<LPP>(D, i, n, sub);
 }
 
 // pass 2: intermediate velocity (viscous + SPS + tke terms, Darcy-Forchheimer)
-__device__ __forceinline__ void int_vel_body(const Dev& D, const int i, const int n) {
+template <int LPP>
+__device__ __forceinline__ void int_vel_body(const Dev& D, const int i, const int n,
+                                             const int sub = 0) {
   if (i >= n) return;
   const DevParams& P = D.P;
   const double dt = D.sc->dt;
@@ -658,7 +899,6 @@ __device__ __forceinline__ void int_vel_body(const Dev& D, const int i, const in
   const double ni = D.por[i];
   if (D.tid[i] == TID_FLUID && !buf) {
     const double eps6 = (double)1e-6f;
-    const int cap = D.cap, cnt = D.ncnt[i];
     const double c1 = D.cf1[i], c2 = D.cf2[i], c3 = D.cf3[i], c4 = D.cf4[i];
     const double xnbi = D.xnb[i], ynbi = D.ynb[i];
     const double xi = D.x[i], yi = D.y[i], ui = D.u[i], vi = D.v[i];
@@ -667,76 +907,72 @@ __device__ __forceinline__ void int_vel_body(const Dev& D, const int i, const in
     const double vartsi = freei ? D.varts[i] : 0.0;
     const double nuti = D.nut[i], tkei = D.tke[i];
     const double cmu_wall = visi * (1.0 / r0i);
-    double us = 0.0, vs = 0.0;
-    // neighbours two at a time: both neighbours' unconditional fields are
-    // requested before either is used (the sums stay in list order)
-    for (int k0 = 0; k0 < cnt; k0 += 2) {
-    int jb[2], tb[2];
-    uint8_t fb[2];
-    double xnb_[2], ynb_[2], mb[2], rb[2], xb[2], yb[2], ub[2], vb[2], kb[2], r0b[2], ntb[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) jb[q] = (k0 + q < cnt) ? D.nbr[(k0 + q) * cap + i] : i;
+    double t[2];
     // rho0 and nu_t of the neighbour are used by fluid neighbours only (most
     // of them): read with the other fields rather than after the type test
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int j = jb[q];
-      xnb_[q] = D.xnb[j]; ynb_[q] = D.ynb[j]; tb[q] = D.tid[j]; fb[q] = D.flags[j];
-      mb[q] = D.m[j]; rb[q] = D.rho[j]; xb[q] = D.x[j]; yb[q] = D.y[j];
-      ub[q] = D.u[j]; vb[q] = D.v[j]; kb[q] = D.tke[j]; r0b[q] = D.rho0[j]; ntb[q] = D.nut[j];
-    }
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      if (k0 + q >= cnt) break;
-      const int j = jb[q];
-      const Klt z = d_klt(xnbi - xnb_[q], ynbi - ynb_[q], P);
-      const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
-      const int tj = tb[q];
-      double cmu;
-      if (tj == TID_FLUID) {
-        const double r0j = r0b[q], visj = d_vis(r0j);
-        cmu = (((2 * visi) * visj) * ((1.0 / r0i) * (1.0 / r0j))) / ((visi / r0i) + (visj / r0j));
-      } else {
-        cmu = cmu_wall;
-      }
-      double vart;
-      if (freei) vart = vartsi;
-      else if ((fb[q] & F_FREE) && !buf) vart = (d_wab(z.r, P) * D.varts[j]) / P.wo;
-      else vart = 0.0;
-      const double pvol = mb[q] / rb[q];
-      const double pd = 1.0 / ((z.r * z.r) + P.lam);
-      const double dxij = xi - xb[q], dyij = yi - yb[q];
-      const double uj = ub[q], vj = vb[q];
-      double a1 = ((((2 * pvol) * (ui - uj)) * dxij) * gx) * pd;
-      double a2 = ((((2 * pvol) * (ui - uj)) * dyij) * gy) * pd;
-      us = us + (a1 + a2) * (cmu + vart);
-      // the SPS viscosity of the pair (the harmonic mean is the same value
-      // in both components, so it is divided once)
-      double nutj = 0.0, hm = 0.0;
-      bool low = false;
-      if (tj > 2) {
-        nutj = ntb[q];
-        low = (nuti < eps6) && (nutj < eps6);
-        if (!low) hm = ((2 * nuti) * nutj) / (nuti + nutj);
-      }
-      if (tj > 2) {
-        if (low) us = us + ((a1 + a2) * (nuti + nutj)) * 0.50;
-        else us = us + (a1 + a2) * hm;
-      }
-      a1 = ((((2 * pvol) * (vi - vj)) * dxij) * gx) * pd;
-      a2 = ((((2 * pvol) * (vi - vj)) * dyij) * gy) * pd;
-      vs = vs + (a1 + a2) * (cmu + vart);
-      if (tj > 2) {
-        if (low) vs = vs + ((a1 + a2) * (nuti + nutj)) * 0.50;
-        else vs = vs + (a1 + a2) * hm;
-      }
-      const double dk = pvol * (kb[q] - tkei);
-      double tk = dk * gx;
-      us = us - ((tk * ni) * 2.0) / 3;
-      tk = dk * gy;
-      vs = vs - ((tk * ni) * 2.0) / 3;
-    }
-    }
+    struct F {
+      double xn, yn, m, r, x, y, u, v, k, r0, nt;
+      int j, t;
+      uint8_t f;
+    };
+    // the addends to us (a[0..2]) and vs (a[3..5]): viscous, SPS (0 for a wall
+    // neighbour), kinetic energy
+    walk_pairs<LPP, 2, 3>(
+        D.nbr, D.cap, i, sub, D.ncnt[i],
+        [&](int j) {
+          return F{D.xnb[j], D.ynb[j], D.m[j], D.rho[j], D.x[j],    D.y[j], D.u[j],
+                   D.v[j],   D.tke[j], D.rho0[j], D.nut[j], j, D.tid[j], D.flags[j]};
+        },
+        [&](const F& f, double (&a)[6]) {
+          const Klt z = d_klt(xnbi - f.xn, ynbi - f.yn, P);
+          const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
+          double cmu;
+          if (f.t == TID_FLUID) {
+            const double visj = d_vis(f.r0);
+            cmu = (((2 * visi) * visj) * ((1.0 / r0i) * (1.0 / f.r0))) /
+                  ((visi / r0i) + (visj / f.r0));
+          } else {
+            cmu = cmu_wall;
+          }
+          double vart;
+          if (freei) vart = vartsi;
+          else if ((f.f & F_FREE) && !buf) vart = (d_wab(z.r, P) * D.varts[f.j]) / P.wo;
+          else vart = 0.0;
+          const double pvol = f.m / f.r;
+          const double pd = 1.0 / ((z.r * z.r) + P.lam);
+          const double dxij = xi - f.x, dyij = yi - f.y;
+          double a1 = ((((2 * pvol) * (ui - f.u)) * dxij) * gx) * pd;
+          double a2 = ((((2 * pvol) * (ui - f.u)) * dyij) * gy) * pd;
+          const double au = a1 + a2;
+          a1 = ((((2 * pvol) * (vi - f.v)) * dxij) * gx) * pd;
+          a2 = ((((2 * pvol) * (vi - f.v)) * dyij) * gy) * pd;
+          const double av = a1 + a2;
+          a[0] = au * (cmu + vart);
+          a[3] = av * (cmu + vart);
+          a[1] = 0.0;
+          a[4] = 0.0;
+          if (f.t > 2) {
+            // the SPS viscosity of the pair (the harmonic mean is the same
+            // value in both components, so it is divided once)
+            const bool low = (nuti < eps6) && (f.nt < eps6);
+            if (low) {
+              a[1] = (au * (nuti + f.nt)) * 0.50;
+              a[4] = (av * (nuti + f.nt)) * 0.50;
+            } else {
+              const double hm = ((2 * nuti) * f.nt) / (nuti + f.nt);
+              a[1] = au * hm;
+              a[4] = av * hm;
+            }
+          }
+          const double dk = pvol * (f.k - tkei);
+          double tk = dk * gx;
+          a[2] = -(((tk * ni) * 2.0) / 3);
+          tk = dk * gy;
+          a[5] = -(((tk * ni) * 2.0) / 3);
+        },
+        t);
+    if (sub != 0) return;
+    double us = t[0], vs = t[1];
     const double den = 1.0 - ((dt * D.resist[i]) * ni);
     us = (ui + (dt * us)) / den;
     vs = (vi + (dt * vs)) / den;
@@ -744,14 +980,15 @@ __device__ __forceinline__ void int_vel_body(const Dev& D, const int i, const in
     D.us[i] = us;
     D.vs[i] = vs;
   }
-  if (buf) {
+  if (buf && sub == 0) {
     D.us[i] = D.u[i];
     D.vs[i] = (P.g * ni) * dt;
   }
 }
+template <int LPP>
 __global__ void __launch_bounds__(256) k_int_vel(Dev D) {
-  PIDX();
-  int_vel_body(D, i, n);
+  PIDX_L(LPP);
+  int_vel_body<LPP>(D, i, n, sub);
 }
 
 // ---------------------------------------------------------------------
@@ -761,115 +998,139 @@ __global__ void __launch_bounds__(256) k_int_vel(Dev D) {
 // Raw values are written first, then divided by the diagonal (Jacobi,
 // isph.f90:432-440) once the diagonal is known.
 // ---------------------------------------------------------------------
-__device__ __forceinline__ int ppe_assemble_row(const Dev& D, int i) {
+// the fields of the row's own particle
+struct PpeRow {
+  int tid;
+  bool free;
+  double n, rho, m, rhon, x, y, us, vs, xn, yn, c1, c2, c3, c4, dt, rhoref;
+};
+__device__ __forceinline__ PpeRow ppe_row(const Dev& D, int i) {
+  PpeRow R;
+  R.tid = D.tid[i];
+  R.free = (D.flags[i] & F_FREE) != 0;
+  R.n = D.por[i]; R.rho = D.rho[i]; R.m = D.m[i];
+  R.rhon = R.rho * (1.0 / R.n);
+  R.x = D.x[i]; R.y = D.y[i]; R.us = D.us[i]; R.vs = D.vs[i];
+  R.xn = D.xnb[i]; R.yn = D.ynb[i];
+  R.c1 = D.cf1[i]; R.c2 = D.cf2[i]; R.c3 = D.cf3[i]; R.c4 = D.cf4[i];
+  R.dt = D.sc->dt;
+  R.rhoref = D.P.rho * D.P.rel_den;
+  return R;
+}
+// a neighbour's fields
+struct PpeNbr {
+  double n, r, m, x, y, xn, yn, us, vs;
+  int j, t;
+};
+__device__ __forceinline__ PpeNbr ppe_nbr(const Dev& D, int j) {
+  return PpeNbr{D.por[j], D.rho[j], D.m[j], D.x[j], D.y[j], D.xnb[j], D.ynb[j],
+                D.us[j],  D.vs[j],  j,      D.tid[j]};
+}
+// The pair's entry val and its addends to the diagonal and the right side;
+// true when the row holds the entry (the addends are 0 otherwise).
+__device__ __forceinline__ bool ppe_pair(const Dev& D, const PpeRow& R, const PpeNbr& f,
+                                         double& val, double& dg, double& rs) {
   const DevParams& P = D.P;
+  const int tj = f.t, j = f.j;
+  const double nj = f.n, rhoj = f.r;
+  const double rho_j = rhoj * (1.0 / nj);
+  const double pvol = f.m * (1.0 / rhoj);
+  const double ddx = f.x - R.x, ddy = f.y - R.y;
+  const double dd = sqrt((ddx * ddx) + (ddy * ddy));
+  const double pd = 1.0 / ((dd * dd) + P.lam);
+  const Klt z = d_klt(R.xn - f.xn, R.yn - f.yn, P);
+  const double dx = R.x - f.x, dy = R.y - f.y;
+  bool wr = false;
+  double t1, t2;
+  val = dg = rs = 0.0;
+  if (R.tid == TID_FLUID) {
+    const double lamp = (R.free && tj == TID_FLUID) ? (1.0 + D.rho0[j] / R.rhoref) : 1.0;
+    const double rho_ij = (((2 * rhoj) * R.rho) * (1.0 / (nj * R.n))) *
+                          (1.0 / ((rhoj * (1.0 / nj)) + (R.rho * (1.0 / R.n))));
+    const double gx = R.c1 * z.k1 + R.c2 * z.k2, gy = R.c3 * z.k1 + R.c4 * z.k2;
+    t1 = (((2 * pvol) * gx) * dx) * pd;
+    t2 = (((2 * pvol) * gy) * dy) * pd;
+    val = -(t1 + t2);
+    wr = true;
+    dg = (t1 + t2) * lamp;
+    if (tj == TID_FLUID) {
+      t1 = (pvol * (((f.us * rho_ij) / nj) - ((R.us * rho_ij) / R.n))) * gx;
+      t2 = (pvol * (((f.vs * rho_ij) / nj) - ((R.vs * rho_ij) / R.n))) * gy;
+    } else {
+      t1 = (pvol * (((f.us * R.rhon) / R.n) - ((R.us * R.rhon) / R.n))) * gx;
+      t2 = (pvol * (((f.vs * R.rhon) / R.n) - ((R.vs * R.rhon) / R.n))) * gy;
+    }
+    rs = (t1 + t2) / R.dt;
+  } else if (R.tid == TID_GHOST) {
+    if (tj <= 2) {
+      t1 = (((2 * pvol) * z.k1) * dx) * pd;
+      t2 = (((2 * pvol) * z.k2) * dy) * pd;
+      val = -(t1 + t2);
+      wr = true;
+      dg = t1 + t2;
+    }
+  } else if (R.tid == TID_FIXED) {
+    if (tj == TID_FLUID) {
+      const double gxj = D.cf1[j] * z.k1 + D.cf2[j] * z.k2;
+      const double gyj = D.cf3[j] * z.k1 + D.cf4[j] * z.k2;
+      t1 = ((((2 * R.m) * gxj) * dx) * pd) / R.rho;
+      t2 = ((((2 * R.m) * gyj) * dy) * pd) / R.rho;
+      val = -(t1 + t2);
+      wr = true;
+      dg = t1 + t2;
+      t1 = ((R.m * (((f.us * rho_j) / nj) - ((R.us * rho_j) / R.n))) * gxj) / R.rho;
+      t2 = ((R.m * (((f.vs * rho_j) / nj) - ((R.vs * rho_j) / R.n))) * gyj) / R.rho;
+      rs = (t1 + t2) / R.dt;
+    } else if (tj <= 2) {
+      t1 = (((2 * pvol) * z.k1) * dx) * pd;
+      t2 = (((2 * pvol) * z.k2) * dy) * pd;
+      val = -(t1 + t2);
+      wr = true;
+      dg = t1 + t2;
+    }
+  }
+  return wr;
+}
+
+__device__ __forceinline__ int ppe_assemble_row(const Dev& D, int i) {
   const int cap = D.cap, cnt = D.ncnt[i];
-  const double dt = D.sc->dt;
-  const int tidi = D.tid[i];
-  const bool freei = (D.flags[i] & F_FREE) != 0;
-  const double ni = D.por[i], rhoi = D.rho[i], mi = D.m[i];
-  const double rho_i = rhoi * (1.0 / ni);
-  const double xi = D.x[i], yi = D.y[i], usi = D.us[i], vsi = D.vs[i];
-  const double xnbi = D.xnb[i], ynbi = D.ynb[i];
-  const double c1 = D.cf1[i], c2 = D.cf2[i], c3 = D.cf3[i], c4 = D.cf4[i];
-  const double rhoref = P.rho * P.rel_den;
+  const PpeRow R = ppe_row(D, i);
   double diag = 0.0, rhs = 0.0;
   int L = 0, dpos = 0;
   bool before = true, first_written = false;
   // neighbours two at a time: both neighbours' common fields are requested
   // before either is used (entries and sums stay in list order)
   for (int k0 = 0; k0 < cnt; k0 += 2) {
-  int jb[2], tb[2];
-  double nb_[2], rb_[2], mb_[2], xb_[2], yb_[2], xnb_[2], ynb_[2], usb[2], vsb[2];
+    int jb[2];
 #pragma unroll
-  for (int q = 0; q < 2; q++) jb[q] = (k0 + q < cnt) ? D.nbr[(k0 + q) * cap + i] : i;
+    for (int q = 0; q < 2; q++) jb[q] = (k0 + q < cnt) ? D.nbr[(k0 + q) * cap + i] : i;
+    const PpeNbr fb[2] = {ppe_nbr(D, jb[0]), ppe_nbr(D, jb[1])};
 #pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int j = jb[q];
-    tb[q] = D.tid[j]; nb_[q] = D.por[j]; rb_[q] = D.rho[j]; mb_[q] = D.m[j];
-    xb_[q] = D.x[j]; yb_[q] = D.y[j]; xnb_[q] = D.xnb[j]; ynb_[q] = D.ynb[j];
-    usb[q] = D.us[j]; vsb[q] = D.vs[j];
-  }
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int k = k0 + q;
-    if (k >= cnt) break;
-    const int j = jb[q];
-    if (before && j > i) {
-      // reserve the diagonal slot (and the ghost-row slot-1 value)
-      before = false;
-      dpos = L;
-      L += 1 + ((tidi == TID_GHOST && k > 0 && !first_written) ? 1 : 0);
-    }
-    const int tj = tb[q];
-    const double nj = nb_[q], rhoj = rb_[q];
-    const double rho_j = rhoj * (1.0 / nj);
-    const double pvol = mb_[q] * (1.0 / rhoj);
-    const double xj = xb_[q], yj = yb_[q];
-    const double ddx = xj - xi, ddy = yj - yi;
-    const double dd = sqrt((ddx * ddx) + (ddy * ddy));
-    const double pd = 1.0 / ((dd * dd) + P.lam);
-    const Klt z = d_klt(xnbi - xnb_[q], ynbi - ynb_[q], P);
-    const double dx = xi - xj, dy = yi - yj;
-    bool wr = false;
-    double val = 0.0, t1, t2;
-    if (tidi == TID_FLUID) {
-      const double lamp = (freei && tj == TID_FLUID) ? (1.0 + D.rho0[j] / rhoref) : 1.0;
-      const double rho_ij = (((2 * rhoj) * rhoi) * (1.0 / (nj * ni))) *
-                            (1.0 / ((rhoj * (1.0 / nj)) + (rhoi * (1.0 / ni))));
-      const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
-      t1 = (((2 * pvol) * gx) * dx) * pd;
-      t2 = (((2 * pvol) * gy) * dy) * pd;
-      val = -(t1 + t2);
-      wr = true;
-      diag = diag + (t1 + t2) * lamp;
-      if (tj == TID_FLUID) {
-        t1 = (pvol * (((usb[q] * rho_ij) / nj) - ((usi * rho_ij) / ni))) * gx;
-        t2 = (pvol * (((vsb[q] * rho_ij) / nj) - ((vsi * rho_ij) / ni))) * gy;
-      } else {
-        t1 = (pvol * (((usb[q] * rho_i) / ni) - ((usi * rho_i) / ni))) * gx;
-        t2 = (pvol * (((vsb[q] * rho_i) / ni) - ((vsi * rho_i) / ni))) * gy;
+    for (int q = 0; q < 2; q++) {
+      const int k = k0 + q;
+      if (k >= cnt) break;
+      const int j = jb[q];
+      if (before && j > i) {
+        // reserve the diagonal slot (and the ghost-row slot-1 value)
+        before = false;
+        dpos = L;
+        L += 1 + ((R.tid == TID_GHOST && k > 0 && !first_written) ? 1 : 0);
       }
-      rhs = rhs + (t1 + t2) / dt;
-    } else if (tidi == TID_GHOST) {
-      if (tj <= 2) {
-        t1 = (((2 * pvol) * z.k1) * dx) * pd;
-        t2 = (((2 * pvol) * z.k2) * dy) * pd;
-        val = -(t1 + t2);
-        wr = true;
-        diag = diag + (t1 + t2);
-      }
-    } else if (tidi == TID_FIXED) {
-      if (tj == TID_FLUID) {
-        const double gxj = D.cf1[j] * z.k1 + D.cf2[j] * z.k2;
-        const double gyj = D.cf3[j] * z.k1 + D.cf4[j] * z.k2;
-        t1 = ((((2 * mi) * gxj) * dx) * pd) / rhoi;
-        t2 = ((((2 * mi) * gyj) * dy) * pd) / rhoi;
-        val = -(t1 + t2);
-        wr = true;
-        diag = diag + (t1 + t2);
-        t1 = ((mi * (((D.us[j] * rho_j) / nj) - ((usi * rho_j) / ni))) * gxj) / rhoi;
-        t2 = ((mi * (((D.vs[j] * rho_j) / nj) - ((vsi * rho_j) / ni))) * gyj) / rhoi;
-        rhs = rhs + (t1 + t2) / dt;
-      } else if (tj <= 2) {
-        t1 = (((2 * pvol) * z.k1) * dx) * pd;
-        t2 = (((2 * pvol) * z.k2) * dy) * pd;
-        val = -(t1 + t2);
-        wr = true;
-        diag = diag + (t1 + t2);
+      double val, dg, rs;
+      const bool wr = ppe_pair(D, R, fb[q], val, dg, rs);
+      diag = diag + dg;
+      rhs = rhs + rs;
+      if (k == 0) first_written = wr;
+      if (wr) {
+        D.acol[L * cap + i] = j;
+        D.aval[L * cap + i] = val;
+        L++;
       }
     }
-    if (k == 0) first_written = wr;
-    if (wr) {
-      D.acol[L * cap + i] = j;
-      D.aval[L * cap + i] = val;
-      L++;
-    }
-  }
   }
   if (before) {
     dpos = L;
-    L += 1 + ((tidi == TID_GHOST && cnt > 0 && !first_written) ? 1 : 0);
+    L += 1 + ((R.tid == TID_GHOST && cnt > 0 && !first_written) ? 1 : 0);
   }
   // A particle with no neighbours gets the identity row, so p = 0 (its rhs
   // is 0): the diagonal value 1 the reference leaves commented out at
@@ -879,7 +1140,7 @@ __device__ __forceinline__ int ppe_assemble_row(const Dev& D, int i) {
   if (!(isfinite(t1) && t1 != 0.0)) atomicOr(&D.sc->err, ERR_DIAG);
   D.acol[dpos * cap + i] = i;
   D.aval[dpos * cap + i] = diag / t1;
-  const bool quirk = (tidi == TID_GHOST && cnt > 0 && D.nbr[i] < i && !first_written);
+  const bool quirk = (R.tid == TID_GHOST && cnt > 0 && D.nbr[i] < i && !first_written);
   if (quirk) {
     D.acol[(dpos + 1) * cap + i] = i;
     D.aval[(dpos + 1) * cap + i] = 1.0 / t1;
@@ -893,16 +1154,87 @@ __device__ __forceinline__ int ppe_assemble_row(const Dev& D, int i) {
   return L;
 }
 
+// The row with eight lanes: a round's entries take their positions by
+// ballots (the diagonal, and the ghost row's slot-1 value, before the first
+// column beyond i), the raw row is kept in LDS, and the lanes share out its
+// division and its stores.
+__device__ __forceinline__ int ppe_assemble_row8(const Dev& D, int i, int sub) {
+  __shared__ double sval[RED_BLOCK / 8][ROW_CAP];
+  __shared__ int32_t scol[RED_BLOCK / 8][ROW_CAP];
+  double* rv = sval[threadIdx.x >> 3];
+  int32_t* rc = scol[threadIdx.x >> 3];
+  const int cap = D.cap, cnt = D.ncnt[i];
+  const PpeRow R = ppe_row(D, i);
+  Fold8<2, 1> fold(sub);
+  int L = 0, dpos = 0;
+  bool before = true, first_written = false;
+  for (int k0 = 0; k0 < cnt; k0 += 8) {
+    const bool on = k0 + sub < cnt;
+    const int j = on ? D.nbr[(k0 + sub) * cap + i] : i;
+    const PpeNbr f = ppe_nbr(D, j);
+    double val = 0.0, a[2] = {0.0, 0.0};
+    const bool wr = on && ppe_pair(D, R, f, val, a[0], a[1]);
+    const unsigned written = bits8(wr), after = bits8(on && j > i);
+    if (k0 == 0) first_written = written & 1u;
+    int skip = 0, first = 8;  // slots reserved before lane `first` of this round
+    if (before && after) {
+      before = false;
+      first = __ffs((int)after) - 1;
+      skip = 1 + ((R.tid == TID_GHOST && k0 + first > 0 && !first_written) ? 1 : 0);
+      dpos = L + __popc(written & ((1u << first) - 1u));
+    }
+    if (wr) {
+      const int at = L + __popc(written & ((1u << sub) - 1u)) + (sub >= first ? skip : 0);
+      rc[at] = j;
+      rv[at] = val;
+    }
+    L += __popc(written) + skip;
+    fold.add(a);
+  }
+  double sum[2];
+  fold.get<0>(sum);
+  double diag = sum[0];
+  const bool ghost1 = R.tid == TID_GHOST && cnt > 0 && !first_written;
+  if (before) {
+    dpos = L;
+    L += 1 + (ghost1 ? 1 : 0);
+  }
+  if (cnt == 0) diag = 1.0;  // the identity row, as above
+  const double t1 = diag;
+  if (sub == 0 && !(isfinite(t1) && t1 != 0.0)) atomicOr(&D.sc->err, ERR_DIAG);
+  const bool quirk = ghost1 && D.nbr[i] < i;
+  wave_lds();
+  for (int k = sub; k < L; k += 8) {
+    const bool d = k == dpos, q = quirk && k == dpos + 1;
+    D.acol[k * cap + i] = (d || q) ? i : rc[k];
+    D.aval[k * cap + i] = (d ? diag : q ? 1.0 : rv[k]) / t1;
+  }
+  if (sub == 0) {
+    D.alen[i] = L;
+    D.b[i] = sum[1] / t1;
+  }
+  return L;
+}
+
 // the stored entries are counted per workgroup: one atomic per workgroup
 // rather than one per row on a single address
-__device__ __forceinline__ void ppe_assemble_body(const Dev& D, const int i, const int n) {
-  const int L = (i < n) ? ppe_assemble_row(D, i) : 0;
+template <int LPP>
+__device__ __forceinline__ void ppe_assemble_body(const Dev& D, const int i, const int n,
+                                                  const int sub = 0) {
+  int L = 0;
+  if constexpr (LPP == 1) {
+    if (i < n) L = ppe_assemble_row(D, i);
+  } else {
+    if (i < n) L = ppe_assemble_row8(D, i, sub);
+    if (sub != 0) L = 0;
+  }
   const unsigned long long s = block_sum_u64((unsigned long long)L);
   if (threadIdx.x == 0 && s != 0) atomicAdd(&D.sc->nnz, s);
 }
+template <int LPP>
 __global__ void __launch_bounds__(256) k_ppe_assemble(Dev D) {
-  PIDX();
-  ppe_assemble_body(D, i, n);
+  PIDX_L(LPP);
+  ppe_assemble_body<LPP>(D, i, n, sub);
 }
 
 // ---------------------------------------------------------------------
@@ -914,71 +1246,64 @@ __device__ __forceinline__ unsigned long long max_bits(double v) {
   return (a == a) ? (unsigned long long)__double_as_longlong(a) : 0ull;
 }
 
-__device__ __forceinline__ void comp_vel_row(const Dev& D, int i) {
+template <int LPP>
+__device__ __forceinline__ void comp_vel_row(const Dev& D, int i, int sub) {
   const DevParams& P = D.P;
   const double dt = D.sc->dt;
   const bool buf = (D.flags[i] & F_BUFFER) != 0;
   if (D.tid[i] == TID_FLUID && !buf) {
-    const int cap = D.cap, cnt = D.ncnt[i];
     const double c1 = D.cf1[i], c2 = D.cf2[i], c3 = D.cf3[i], c4 = D.cf4[i];
     const double xnbi = D.xnb[i], ynbi = D.ynb[i];
     const double ni = D.por[i], rhoi = D.rho[i], pi = D.p[i];
-    double u = 0.0, v = 0.0;
-    // neighbours two at a time: both neighbours' fields are requested before
-    // either is used (the sums stay in list order)
-    for (int k0 = 0; k0 < cnt; k0 += 2) {
-      int jb[2];
-      double xb[2], yb[2], nb[2], rb[2], pb[2], mb[2];
-      int tb[2];
-#pragma unroll
-      for (int q = 0; q < 2; q++) jb[q] = (k0 + q < cnt) ? D.nbr[(k0 + q) * cap + i] : i;
-#pragma unroll
-      for (int q = 0; q < 2; q++) {
-        const int j = jb[q];
-        xb[q] = D.xnb[j]; yb[q] = D.ynb[j]; nb[q] = D.por[j]; rb[q] = D.rho[j];
-        pb[q] = D.p[j]; mb[q] = D.m[j]; tb[q] = D.tid[j];
-      }
-#pragma unroll
-      for (int q = 0; q < 2; q++) {
-      if (k0 + q >= cnt) break;
-      const Klt z = d_klt(xnbi - xb[q], ynbi - yb[q], P);
-      const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
-      const double nj = nb[q], rhoj = rb[q], pj = pb[q];
-      const double V = mb[q] / rhoj;
-      double t1;
-      if (tb[q] == TID_FLUID) {
-        const double a = ((pj * rhoi) / ni) + ((pi * rhoj) / nj);
-        const double den = rhoi * ((rhoi / ni) + (rhoj / nj));
-        t1 = (2 * (((V * (ni * ni)) * a) * gx)) / den;
-        u = u - t1 * dt;
-        t1 = (2 * (((V * (ni * ni)) * a) * gy)) / den;
-        v = v - t1 * dt;
-      } else {
-        t1 = (((V * (ni * ni)) * (pj + pi)) * gx) / rhoi;
-        u = u - t1 * dt;
-        t1 = (((V * (ni * ni)) * (pj + pi)) * gy) / rhoi;
-        v = v - t1 * dt;
-      }
-      }
-    }
-    u = D.us[i] + u;
-    v = D.vs[i] + v;
+    double t[2];
+    struct F {
+      double x, y, n, r, p, m;
+      int t;
+    };
+    walk_pairs<LPP, 2, 1>(
+        D.nbr, D.cap, i, sub, D.ncnt[i],
+        [&](int j) {
+          return F{D.xnb[j], D.ynb[j], D.por[j], D.rho[j], D.p[j], D.m[j], D.tid[j]};
+        },
+        [&](const F& f, double (&a)[2]) {
+          const Klt z = d_klt(xnbi - f.x, ynbi - f.y, P);
+          const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
+          const double V = f.m / f.r;
+          double t1, t2;
+          if (f.t == TID_FLUID) {
+            const double q = ((f.p * rhoi) / ni) + ((pi * f.r) / f.n);
+            const double den = rhoi * ((rhoi / ni) + (f.r / f.n));
+            t1 = (2 * (((V * (ni * ni)) * q) * gx)) / den;
+            t2 = (2 * (((V * (ni * ni)) * q) * gy)) / den;
+          } else {
+            t1 = (((V * (ni * ni)) * (f.p + pi)) * gx) / rhoi;
+            t2 = (((V * (ni * ni)) * (f.p + pi)) * gy) / rhoi;
+          }
+          a[0] = -(t1 * dt);
+          a[1] = -(t2 * dt);
+        },
+        t);
+    if (sub != 0) return;
+    const double u = D.us[i] + t[0], v = D.vs[i] + t[1];
     D.u[i] = u;
     D.v[i] = v;
     D.vel[i] = sqrt((u * u) + (v * v)) / ni;
   }
-  if (buf) {
+  if (buf && sub == 0) {
     D.u[i] = D.us[i];
     D.v[i] = 0.0;
   }
 }
 
-__device__ __forceinline__ void comp_vel_body(const Dev& D, const int i, const int n) {
-  if (i < n) comp_vel_row(D, i);
+template <int LPP>
+__device__ __forceinline__ void comp_vel_body(const Dev& D, const int i, const int n,
+                                              const int sub = 0) {
+  if (i < n) comp_vel_row<LPP>(D, i, sub);
 }
+template <int LPP>
 __global__ void __launch_bounds__(256) k_comp_vel(Dev D) {
-  PIDX();
-  comp_vel_body(D, i, n);
+  PIDX_L(LPP);
+  comp_vel_body<LPP>(D, i, n, sub);
 }
 
 // The per-cell maxima of comp_vel (integrator.f90:831-841): a cell that
@@ -1077,7 +1402,9 @@ __global__ void k_freesurf(Dev D) {
 // -csh*h^2*frac*gradW*V; the stored shift is the capped one, the velocity
 // correction uses the uncapped shift.
 // ---------------------------------------------------------------------
-__device__ __forceinline__ void opt2_shift_body(const Dev& D, const int i, const int n) {
+template <int LPP>
+__device__ __forceinline__ void opt2_shift_body(const Dev& D, const int i, const int n,
+                                                const int sub = 0) {
   if (i >= n) return;
   if (!(D.tid[i] == TID_FLUID && !(D.flags[i] & F_BUFFER))) return;
   const int cnt = D.ncnt[i];
@@ -1086,48 +1413,42 @@ __device__ __forceinline__ void opt2_shift_body(const Dev& D, const int i, const
     // (part_shift.f90:32-35) but stores them only for count > 0
     // (part_shift.f90:38-161), so its apply step (part_shift.f90:179-182)
     // would add the slot's saved position and intermediate velocity.
-    D.xs[i] = 0.0;
-    D.ys[i] = 0.0;
-    D.us[i] = 0.0;
-    D.vs[i] = 0.0;
+    if (sub == 0) {
+      D.xs[i] = 0.0;
+      D.ys[i] = 0.0;
+      D.us[i] = 0.0;
+      D.vs[i] = 0.0;
+    }
     return;
   }
   const DevParams& P = D.P;
-  const int cap = D.cap;
   const double c1 = D.cf1[i], c2 = D.cf2[i], c3 = D.cf3[i], c4 = D.cf4[i];
   const double xnbi = D.xnb[i], ynbi = D.ynb[i];
   const double frac = (D.flags[i] & F_FREE) ? 0.01 : 1.0;
   const double coef = (P.csh * (P.h * P.h)) * frac;
   const double ui = D.u[i], vi = D.v[i];
-  double xsa = 0.0, ysa = 0.0, a1 = 0.0, a2 = 0.0, b1 = 0.0, b2 = 0.0;
-  // neighbours two at a time: both neighbours' fields are requested before
-  // either is used (the sums stay in list order)
-  for (int k0 = 0; k0 < cnt; k0 += 2) {
-    int jb[2];
-    double xb[2], yb[2], mb[2], rb[2], ub[2], vb[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) jb[q] = (k0 + q < cnt) ? D.nbr[(k0 + q) * cap + i] : i;
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int j = jb[q];
-      xb[q] = D.xnb[j]; yb[q] = D.ynb[j]; mb[q] = D.m[j]; rb[q] = D.rho[j];
-      ub[q] = D.u[j]; vb[q] = D.v[j];
-    }
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      if (k0 + q >= cnt) break;
-      const Klt z = d_klt(xnbi - xb[q], ynbi - yb[q], P);
-      const double V = mb[q] / rb[q];
-      xsa = xsa - ((coef * z.k1) * V);
-      ysa = ysa - ((coef * z.k2) * V);
-      const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
-      const double du = ub[q] - ui, dv = vb[q] - vi;
-      a1 = a1 + (gx * du) * V;
-      a2 = a2 + (gy * du) * V;
-      b1 = b1 + (gx * dv) * V;
-      b2 = b2 + (gy * dv) * V;
-    }
-  }
+  double t[6];
+  struct F {
+    double x, y, m, r, u, v;
+  };
+  walk_pairs<LPP, 6, 1>(
+      D.nbr, D.cap, i, sub, cnt,
+      [&](int j) { return F{D.xnb[j], D.ynb[j], D.m[j], D.rho[j], D.u[j], D.v[j]}; },
+      [&](const F& f, double (&a)[6]) {
+        const Klt z = d_klt(xnbi - f.x, ynbi - f.y, P);
+        const double V = f.m / f.r;
+        a[0] = -((coef * z.k1) * V);
+        a[1] = -((coef * z.k2) * V);
+        const double gx = c1 * z.k1 + c2 * z.k2, gy = c3 * z.k1 + c4 * z.k2;
+        const double du = f.u - ui, dv = f.v - vi;
+        a[2] = (gx * du) * V;
+        a[3] = (gy * du) * V;
+        a[4] = (gx * dv) * V;
+        a[5] = (gy * dv) * V;
+      },
+      t);
+  if (sub != 0) return;
+  const double xsa = t[0], ysa = t[1], a1 = t[2], a2 = t[3], b1 = t[4], b2 = t[5];
   const double capv = P.maxshift * P.dl;
   const double ax = fabs(xsa), ay = fabs(ysa);
   D.xs[i] = (xsa == 0.0) ? 0.0 : (((capv < ax) ? capv : ax) * xsa) / ax;
@@ -1135,9 +1456,10 @@ __device__ __forceinline__ void opt2_shift_body(const Dev& D, const int i, const
   D.us[i] = a1 * xsa + a2 * ysa;
   D.vs[i] = b1 * xsa + b2 * ysa;
 }
+template <int LPP>
 __global__ void __launch_bounds__(256) k_opt2_shift(Dev D) {
-  PIDX();
-  opt2_shift_body(D, i, n);
+  PIDX_L(LPP);
+  opt2_shift_body<LPP>(D, i, n, sub);
 }
 
 __device__ __forceinline__ void shift_apply_body(const Dev& D, const int i, const int n) {
@@ -1234,75 +1556,76 @@ __global__ void __launch_bounds__(256) k_timestep(Dev D) {
 // scalart_anisotropic / scalarupdate, scalar.f90:242-397.  The neighbour
 // list (and its r) is from the last neighbour search; positions are current.
 // ---------------------------------------------------------------------
-__device__ __forceinline__ void scalart_body(const Dev& D, const int i, const int n) {
+template <int LPP>
+__device__ __forceinline__ void scalart_body(const Dev& D, const int i, const int n,
+                                             const int sub = 0) {
   if (i >= n || D.tid[i] != TID_FLUID) return;
   const DevParams& P = D.P;
   const double al = 0.0025, at = 0.00025, Dm = (double)1e-9f, thr = 0.7;
   const double eps6 = (double)1e-6f;
   const double dt = D.sc->dt;
   const double capv = (0.12 * (P.dl * P.dl)) / dt;
-  const int cap = D.cap, cnt = D.ncnt[i];
   const double xnbi = D.xnb[i], ynbi = D.ynb[i], xi = D.x[i], yi = D.y[i];
   const double ui = D.u[i], vi_ = D.v[i], ni = D.por[i], ci1 = D.c[i];
   const double nuti = D.nut[i], vol0i = D.vol0[i];
   const double vi = sqrt((ui * ui) + (vi_ * vi_)) / ni;
-  double cd = 0.0;
-  // neighbours two at a time: both neighbours' fields are requested before
-  // either is used (the sum stays in list order)
-  for (int k0 = 0; k0 < cnt; k0 += 2) {
-  int tb[2];
-  double xnb_[2], ynb_[2], ub[2], vb[2], nb[2], cb[2], xb[2], yb[2], nutb[2];
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int j = (k0 + q < cnt) ? D.nbr[(k0 + q) * cap + i] : i;
-    tb[q] = D.tid[j]; xnb_[q] = D.xnb[j]; ynb_[q] = D.ynb[j]; ub[q] = D.u[j]; vb[q] = D.v[j];
-    nb[q] = D.por[j]; cb[q] = D.c[j]; xb[q] = D.x[j]; yb[q] = D.y[j]; nutb[q] = D.nut[j];
-  }
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    if (k0 + q >= cnt) break;
-    if (tb[q] != TID_FLUID) continue;
-    const double ex = xnbi - xnb_[q], ey = ynbi - ynb_[q];
-    const double r = sqrt((ex * ex) + (ey * ey));
-    const double uj = ub[q], vj_ = vb[q], nj = nb[q], c2 = cb[q];
-    const double dx = xi - xb[q], dy = yi - yb[q];
-    double t1x;
-    if ((ni < thr) && (nj < thr)) {
-      const double vj = sqrt((uj * uj) + (vj_ * vj_)) / nj;
-      const double Dxxi = ui / ((sqrt((al * vi) + Dm) * vi) * ni);
-      const double Dxyi = vi_ / ((sqrt((al * vi) + Dm) * vi) * ni);
-      const double Dyxi = (-vi_) / ((sqrt((at * vi) + Dm) * vi) * ni);
-      const double Dyyi = ui / ((sqrt((at * vi) + Dm) * vi) * ni);
-      const double Dxxj = uj / ((sqrt((al * vj) + Dm) * vj) * nj);
-      const double Dxyj = vj_ / ((sqrt((al * vj) + Dm) * vj) * nj);
-      const double Dyxj = (-vj_) / ((sqrt((at * vj) + Dm) * vj) * nj);
-      const double Dyyj = uj / ((sqrt((at * vj) + Dm) * vj) * nj);
-      const double pd = 1.0 / r;
-      const double A = ((((Dxxi + Dxxj) * dx) * pd) * 0.5) + ((((Dxyi + Dxyj) * dy) * pd) * 0.5);
-      const double B = ((((Dyxi + Dyxj) * dx) * pd) * 0.5) + ((((Dyyi + Dyyj) * dy) * pd) * 0.5);
-      t1x = (A * A) + (B * B);
-      t1x = 1.0 / t1x;
-      t1x = (t1x <= capv) ? t1x : capv;
-    } else {
-      const double nutj = nutb[q];
-      const double Dxxi = Dm + nuti / P.tschmidt;
-      const double Dxxj = Dm + nutj / P.tschmidt;
-      if ((nuti < eps6) && (nutj < eps6)) t1x = (Dxxi + Dxxj) * 0.50;
-      else t1x = ((2 * Dxxi) * Dxxj) / (Dxxi + Dxxj);
-    }
-    const double t3 = (vol0i * (ni + nj)) / (ni * nj);
-    double hwx, hwy;
-    d_wabd2(dx, dy, r, P, hwx, hwy);
-    const double den = (r * r) + P.lam;
-    cd = (cd + (((((((t1x * 1.0) * t3) * (ci1 - c2)) * dx) * hwx) / den))) +
-         (((((((t1x * 1.0) * t3) * (ci1 - c2)) * dy) * hwy) / den));
-  }
-  }
-  D.cdiff[i] = cd;
+  double cd[1];
+  struct F {
+    double xn, yn, u, v, n, c, x, y, nt;
+    int t;
+  };
+  // a wall neighbour adds nothing (0 twice: cd is never -0)
+  walk_pairs<LPP, 1, 2>(
+      D.nbr, D.cap, i, sub, D.ncnt[i],
+      [&](int j) {
+        return F{D.xnb[j], D.ynb[j], D.u[j], D.v[j], D.por[j], D.c[j],
+                 D.x[j],   D.y[j],   D.nut[j], D.tid[j]};
+      },
+      [&](const F& f, double (&a)[2]) {
+        a[0] = 0.0;
+        a[1] = 0.0;
+        if (f.t != TID_FLUID) return;
+        const double ex = xnbi - f.xn, ey = ynbi - f.yn;
+        const double r = sqrt((ex * ex) + (ey * ey));
+        const double uj = f.u, vj_ = f.v, nj = f.n, c2 = f.c;
+        const double dx = xi - f.x, dy = yi - f.y;
+        double t1x;
+        if ((ni < thr) && (nj < thr)) {
+          const double vj = sqrt((uj * uj) + (vj_ * vj_)) / nj;
+          const double Dxxi = ui / ((sqrt((al * vi) + Dm) * vi) * ni);
+          const double Dxyi = vi_ / ((sqrt((al * vi) + Dm) * vi) * ni);
+          const double Dyxi = (-vi_) / ((sqrt((at * vi) + Dm) * vi) * ni);
+          const double Dyyi = ui / ((sqrt((at * vi) + Dm) * vi) * ni);
+          const double Dxxj = uj / ((sqrt((al * vj) + Dm) * vj) * nj);
+          const double Dxyj = vj_ / ((sqrt((al * vj) + Dm) * vj) * nj);
+          const double Dyxj = (-vj_) / ((sqrt((at * vj) + Dm) * vj) * nj);
+          const double Dyyj = uj / ((sqrt((at * vj) + Dm) * vj) * nj);
+          const double pd = 1.0 / r;
+          const double A = ((((Dxxi + Dxxj) * dx) * pd) * 0.5) + ((((Dxyi + Dxyj) * dy) * pd) * 0.5);
+          const double B = ((((Dyxi + Dyxj) * dx) * pd) * 0.5) + ((((Dyyi + Dyyj) * dy) * pd) * 0.5);
+          t1x = (A * A) + (B * B);
+          t1x = 1.0 / t1x;
+          t1x = (t1x <= capv) ? t1x : capv;
+        } else {
+          const double Dxxi = Dm + nuti / P.tschmidt;
+          const double Dxxj = Dm + f.nt / P.tschmidt;
+          if ((nuti < eps6) && (f.nt < eps6)) t1x = (Dxxi + Dxxj) * 0.50;
+          else t1x = ((2 * Dxxi) * Dxxj) / (Dxxi + Dxxj);
+        }
+        const double t3 = (vol0i * (ni + nj)) / (ni * nj);
+        double hwx, hwy;
+        d_wabd2(dx, dy, r, P, hwx, hwy);
+        const double den = (r * r) + P.lam;
+        a[0] = ((((((t1x * 1.0) * t3) * (ci1 - c2)) * dx) * hwx) / den);
+        a[1] = ((((((t1x * 1.0) * t3) * (ci1 - c2)) * dy) * hwy) / den);
+      },
+      cd);
+  if (sub == 0) D.cdiff[i] = cd[0];
 }
+template <int LPP>
 __global__ void __launch_bounds__(256) k_scalart(Dev D) {
-  PIDX();
-  scalart_body(D, i, n);
+  PIDX_L(LPP);
+  scalart_body<LPP>(D, i, n, sub);
 }
 
 // stime < 0: use the sub-step length dtsol from the last timestep

@@ -81,7 +81,7 @@ struct isph_ctx {
                        {"mg_up", 0},     {"pfinalize", 2}, {"mg_restrict0", 2}};
   Dev D;
   hipStream_t stream = nullptr;
-  int64_t cap = 0, scap = 0;
+  int64_t cap = 0, scap = 0, ns = 0;  // particle and solid capacities, solids
   int n_hi = 0;          // host-side upper bound of the live particle count
   int ncell = 0;
   int device = 0;
@@ -658,6 +658,7 @@ extern "C" int isph_upload_solids(isph_ctx* c, int64_t ns, const double* x, cons
     HIPCHK(c, hipMemcpy(D.srho, br.data(), 8 * ns, hipMemcpyHostToDevice));
   }
   HIPCHK(c, hipMemcpy(D.sstart, cs.data(), 4 * (c->ncell + 1), hipMemcpyHostToDevice));
+  c->ns = ns;
   return 0;
 }
 
@@ -736,17 +737,52 @@ extern "C" int isph_set_scalars(isph_ctx* c, const isph_scalars* in) {
     }                                                                                \
   } while (0)
 
-// launch of a tuned particle kernel with the context's block size for it
-#define TLAUNCH(tk, kern, nthreads, ...)                                             \
+// Whether neighbour-sum kernel tk runs eight lanes per particle.  That
+// shortens a particle's chain of loads and operations and costs the fold of
+// the sums through LDS, so it wins until the chip is full of one-lane
+// wavefronts.  Both sides in us, one lane / eight, on porous flumes:
+//   particles      20k      80k      160k     320k     640k
+//   neighbour    43/16    58/37    74/65   107/111  200/210
+//   effpor       48/14    49/26    60/37    77/56   112/103
+//   eddyvis      17/9     25/22    34/37    54/64    95/121
+//   varts        16/7     18/8     22/9     23/10    31/13
+//   int_vel      25/13    38/33    54/58    88/101  160/197
+//   assemble     50/20    70/46    88/77   154/141  275/267
+//   comp_vel     17/8     29/24    39/40    58/70   105/132
+//   opt2_shift   14/8     20/19    28/31    42/55    76/103
+//   scalart      29/13    40/35    55/58    95/105  148/200
+// effpor's walk is over ~50 solids and the longest of them; without solids
+// there is no walk (4.8/6 at 40k, 5/7 at 80k).  varts, which skips all but the
+// free surface, and the assembly run eight lanes always.
+// The weakly compressible step keeps one lane: its dam break compresses past
+// the list's capacity after about a thousand steps, and a faster step reaches
+// that inside the run that it would have to be compared over.
+static bool lanes8(const isph_ctx* c, int tk) {
+  if (c->wcsph) return false;
+  switch (tk) {
+    case TK_EFFPOR: return c->ns > 0 || c->n_hi <= 32768;
+    case TK_NEIGHBOUR: return c->n_hi <= 262144;
+    default: return c->n_hi <= 102400;
+  }
+}
+
+// launch over the particles with block size b_ and LPP lanes per particle
+#define NLAUNCH(kern, lpp, b_)                                                  \
   do {                                                                               \
-    const int b_ = ts_block[c->tshape[tk]];                                          \
-    hipLaunchKernelGGL(kern, dim3(std::max(1, ((nthreads) + b_ - 1) / b_)), dim3(b_), 0, \
-                       c->stream, __VA_ARGS__);                                      \
+    const int64_t t_ = (lpp) * (int64_t)c->n_hi;                                     \
+    const dim3 g_((unsigned)std::max<int64_t>(1, (t_ + (b_) - 1) / (b_)));           \
+    hipLaunchKernelGGL(kern, g_, dim3(b_), 0, c->stream, c->D);                      \
     hipError_t e_ = hipGetLastError();                                               \
     if (e_ != hipSuccess) {                                                          \
-      set_err(c, "launch of %s failed: %s", #kern, hipGetErrorString(e_));          \
+      set_err(c, "launch of %s failed: %s", #kern, hipGetErrorString(e_));           \
       return ISPH_EHIP;                                                              \
     }                                                                                \
+  } while (0)
+// launch of a tuned particle kernel with the context's block size for it
+#define TLAUNCH(tk, kern)                                                            \
+  do {                                                                               \
+    if (lanes8(c, tk)) NLAUNCH(kern<8>, 8, ts_block[c->tshape[tk]]);                 \
+    else NLAUNCH(kern<1>, 1, ts_block[c->tshape[tk]]);                               \
   } while (0)
 
 static std::pair<hipEvent_t, hipEvent_t> timer_pair(KTimer& t) {
@@ -922,7 +958,8 @@ static int launch_neighbour(isph_ctx* c) {
     }
     return 0;
   }
-  TLAUNCH(TK_NEIGHBOUR, k_neighbour, c->n_hi, c->D);
+  if (lanes8(c, TK_NEIGHBOUR)) NLAUNCH(k_neighbour8, 8, ts_block[sh]);
+  else NLAUNCH(k_neighbour, 1, ts_block[sh]);
   return 0;
 }
 
@@ -942,20 +979,20 @@ extern "C" int isph_neighbour(isph_ctx* c) {
 
 extern "C" int isph_effpor(isph_ctx* c) {
   if (!c) return ISPH_EARG;
-  TLAUNCH(TK_EFFPOR, k_effpor, c->n_hi, c->D);
+  TLAUNCH(TK_EFFPOR, k_effpor);
   return 0;
 }
 extern "C" int isph_eddyvis(isph_ctx* c) {
   if (!c) return ISPH_EARG;
   if (!c->have_nbr) { set_err(c, "eddyvis before neighbour"); return ISPH_ESTATE; }
-  TLAUNCH(TK_EDDYVIS, k_eddyvis, c->n_hi, c->D);
+  TLAUNCH(TK_EDDYVIS, k_eddyvis);
   return 0;
 }
 extern "C" int isph_int_vel(isph_ctx* c) {
   if (!c) return ISPH_EARG;
   if (!c->have_nbr) { set_err(c, "int_vel before neighbour"); return ISPH_ESTATE; }
-  TLAUNCH(TK_VARTS, k_int_vel_varts, c->n_hi, c->D);
-  TLAUNCH(TK_INTVEL, k_int_vel, c->n_hi, c->D);
+  NLAUNCH(k_int_vel_varts<8>, 8, ts_block[c->tshape[TK_VARTS]]);
+  TLAUNCH(TK_INTVEL, k_int_vel);
   return 0;
 }
 
@@ -965,7 +1002,7 @@ __global__ void k_zero_nnz(Dev D) {
 
 static int assemble_nocheck(isph_ctx* c) {
   hipLaunchKernelGGL(k_zero_nnz, dim3(1), dim3(64), 0, c->stream, c->D);
-  TLAUNCH(TK_ASSEMBLE, k_ppe_assemble, c->n_hi, c->D);
+  NLAUNCH(k_ppe_assemble<8>, 8, ts_block[c->tshape[TK_ASSEMBLE]]);
   c->assembled = true;
   c->loaded = false;
   return 0;
@@ -1555,7 +1592,7 @@ extern "C" int isph_ppesolve(isph_ctx* c, isph_solve_stats* stats) {
 
 extern "C" int isph_comp_vel(isph_ctx* c) {
   if (!c) return ISPH_EARG;
-  TLAUNCH(TK_COMPVEL, k_comp_vel, c->n_hi, c->D);
+  TLAUNCH(TK_COMPVEL, k_comp_vel);
   LAUNCH(k_cell_max, c->ncell, c->D, c->ncell, 0);
   return 0;
 }
@@ -1571,7 +1608,7 @@ extern "C" int isph_freesurf(isph_ctx* c) {
 }
 extern "C" int isph_opt2_shift(isph_ctx* c) {
   if (!c) return ISPH_EARG;
-  TLAUNCH(TK_SHIFT, k_opt2_shift, c->n_hi, c->D);
+  TLAUNCH(TK_SHIFT, k_opt2_shift);
   LAUNCH(k_shift_apply, c->n_hi, c->D);
   return 0;
 }
@@ -1590,7 +1627,7 @@ extern "C" int isph_timestep(isph_ctx* c) {
 extern "C" int isph_scalart_anisotropic(isph_ctx* c) {
   if (!c) return ISPH_EARG;
   if (!c->have_nbr) { set_err(c, "scalar transport before neighbour"); return ISPH_ESTATE; }
-  TLAUNCH(TK_SCALART, k_scalart, c->n_hi, c->D);
+  TLAUNCH(TK_SCALART, k_scalart);
   return 0;
 }
 
@@ -1604,8 +1641,8 @@ extern "C" int isph_init_state(isph_ctx* c) {
   if (!c) return ISPH_EARG;
   int rc = isph_neighbour(c);
   if (rc) return rc;
-  TLAUNCH(TK_EFFPOR, k_effpor, c->n_hi, c->D);
-  TLAUNCH(TK_EDDYVIS, k_eddyvis, c->n_hi, c->D);
+  TLAUNCH(TK_EFFPOR, k_effpor);
+  TLAUNCH(TK_EDDYVIS, k_eddyvis);
   LAUNCH(k_cell_max, c->ncell, c->D, c->ncell, 1);
   rc = isph_timestep(c);
   if (rc) return rc;
@@ -1846,7 +1883,7 @@ static int step_pre(isph_ctx* c) {
   }
   hipLaunchKernelGGL(k_advance_t, dim3(1), dim3(64), 0, c->stream, c->D);
   for (int q = 0; q < s.solsteps; q++) {
-    TLAUNCH(TK_SCALART, k_scalart, c->n_hi, c->D);
+    TLAUNCH(TK_SCALART, k_scalart);
     LAUNCH(k_scalarupdate, c->n_hi, c->D, -1.0);
   }
   rc = buffer_clock(c, s.t, s.t + s.dt);  // the device's t + dt, the same double sum
@@ -1860,10 +1897,10 @@ static int step_pre(isph_ctx* c) {
   if (rc) return rc;
   rc = neighbour_nocheck(c);
   if (rc) return rc;
-  TLAUNCH(TK_EFFPOR, k_effpor, c->n_hi, c->D);
-  TLAUNCH(TK_EDDYVIS, k_eddyvis, c->n_hi, c->D);
-  TLAUNCH(TK_VARTS, k_int_vel_varts, c->n_hi, c->D);
-  TLAUNCH(TK_INTVEL, k_int_vel, c->n_hi, c->D);
+  TLAUNCH(TK_EFFPOR, k_effpor);
+  TLAUNCH(TK_EDDYVIS, k_eddyvis);
+  NLAUNCH(k_int_vel_varts<8>, 8, ts_block[c->tshape[TK_VARTS]]);
+  TLAUNCH(TK_INTVEL, k_int_vel);
   if (c->wcsph) {
     // continuity and the Tait law in place of the pressure Poisson solve
     LAUNCH(k_calmasscons, c->n_hi, c->D);
@@ -1881,7 +1918,7 @@ static int step_pre(isph_ctx* c) {
 
 // check: read the error bits now (else the next step_pre's scalar read does)
 static int step_post(isph_ctx* c, bool check) {
-  TLAUNCH(TK_COMPVEL, k_comp_vel, c->n_hi, c->D);
+  TLAUNCH(TK_COMPVEL, k_comp_vel);
   LAUNCH(k_cell_max, c->ncell, c->D, c->ncell, 0);
   LAUNCH(k_comp_pos, c->n_hi, c->D);
   int rc = rebin(c, 1);
@@ -1889,13 +1926,13 @@ static int step_post(isph_ctx* c, bool check) {
   rc = neighbour_nocheck(c);
   if (rc) return rc;
   LAUNCH(k_freesurf, c->n_hi, c->D);
-  TLAUNCH(TK_EFFPOR, k_effpor, c->n_hi, c->D);
-  TLAUNCH(TK_SHIFT, k_opt2_shift, c->n_hi, c->D);
+  TLAUNCH(TK_EFFPOR, k_effpor);
+  TLAUNCH(TK_SHIFT, k_opt2_shift);
   LAUNCH(k_shift_apply, c->n_hi, c->D);
   if (!c->wcsph) LAUNCH(k_densityupdate, c->n_hi, c->D);
   rc = isph_timestep(c);
   if (rc) return rc;
-  TLAUNCH(TK_EDDYVIS, k_eddyvis, c->n_hi, c->D);
+  TLAUNCH(TK_EDDYVIS, k_eddyvis);
   return check ? check_err_flags(c) : 0;
 }
 
@@ -2985,14 +3022,14 @@ extern "C" int isph_autotune(isph_ctx* c, int32_t trials, int32_t* shape, double
       auto launch = [&]() -> int {
         switch (tk) {
           case TK_NEIGHBOUR: return launch_neighbour(c);
-          case TK_EFFPOR: TLAUNCH(tk, k_effpor, c->n_hi, c->D); break;
-          case TK_EDDYVIS: TLAUNCH(tk, k_eddyvis, c->n_hi, c->D); break;
-          case TK_VARTS: TLAUNCH(tk, k_int_vel_varts, c->n_hi, c->D); break;
-          case TK_INTVEL: TLAUNCH(tk, k_int_vel, c->n_hi, c->D); break;
-          case TK_ASSEMBLE: TLAUNCH(tk, k_ppe_assemble, c->n_hi, c->D); break;
-          case TK_COMPVEL: TLAUNCH(tk, k_comp_vel, c->n_hi, c->D); break;
-          case TK_SHIFT: TLAUNCH(tk, k_opt2_shift, c->n_hi, c->D); break;
-          default: TLAUNCH(tk, k_scalart, c->n_hi, c->D); break;
+          case TK_EFFPOR: TLAUNCH(tk, k_effpor); break;
+          case TK_EDDYVIS: TLAUNCH(tk, k_eddyvis); break;
+          case TK_VARTS: NLAUNCH(k_int_vel_varts<8>, 8, ts_block[c->tshape[tk]]); break;
+          case TK_INTVEL: TLAUNCH(tk, k_int_vel); break;
+          case TK_ASSEMBLE: NLAUNCH(k_ppe_assemble<8>, 8, ts_block[c->tshape[tk]]); break;
+          case TK_COMPVEL: TLAUNCH(tk, k_comp_vel); break;
+          case TK_SHIFT: TLAUNCH(tk, k_opt2_shift); break;
+          default: TLAUNCH(tk, k_scalart); break;
         }
         return 0;
       };

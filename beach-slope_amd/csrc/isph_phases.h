@@ -107,7 +107,7 @@ __global__ void kb_clear_err(PhaseBatch B) {
 __global__ void __launch_bounds__(256) kb_scalart(PhaseBatch B, int q) {
   PH_PIDX(B);
   if (q >= D.sc->solsteps) return;
-  scalart_body(D, i, n);
+  scalart_body<1>(D, i, n);
 }
 __global__ void kb_scalarupdate(PhaseBatch B, int q) {
   PH_PIDX(B);
@@ -176,27 +176,27 @@ __global__ void __launch_bounds__(256) kb_neighbour_tile8(PhaseBatch B) {
 }
 __global__ void kb_effpor(PhaseBatch B) {
   PH_PIDX(B);
-  effpor_body(D, i, n);
+  effpor_body<1>(D, i, n);
 }
 __global__ void kb_eddyvis(PhaseBatch B) {
   PH_PIDX(B);
-  eddyvis_body(D, i, n);
+  eddyvis_body<1>(D, i, n);
 }
 __global__ void kb_int_vel_varts(PhaseBatch B) {
   PH_PIDX(B);
-  int_vel_varts_body(D, i, n);
+  int_vel_varts_body<1>(D, i, n);
 }
 __global__ void __launch_bounds__(256) kb_int_vel(PhaseBatch B) {
   PH_PIDX(B);
-  int_vel_body(D, i, n);
+  int_vel_body<1>(D, i, n);
 }
 __global__ void __launch_bounds__(256) kb_ppe_assemble(PhaseBatch B) {
   PH_PIDX(B);
-  ppe_assemble_body(D, i, n);
+  ppe_assemble_body<1>(D, i, n);
 }
 __global__ void __launch_bounds__(256) kb_comp_vel(PhaseBatch B) {
   PH_PIDX(B);
-  comp_vel_body(D, i, n);
+  comp_vel_body<1>(D, i, n);
 }
 __global__ void __launch_bounds__(256) kb_cell_max(PhaseBatch B, int init) {
   PH_IDX(B, PH_CELL);
@@ -212,7 +212,7 @@ __global__ void kb_freesurf(PhaseBatch B) {
 }
 __global__ void __launch_bounds__(256) kb_opt2_shift(PhaseBatch B) {
   PH_PIDX(B);
-  opt2_shift_body(D, i, n);
+  opt2_shift_body<1>(D, i, n);
 }
 __global__ void kb_shift_apply(PhaseBatch B) {
   PH_PIDX(B);
