@@ -1122,7 +1122,7 @@ static int bh_refresh(BatchHost* b) {
 template <int T, int R>
 static int64_t rs_shape(BatchHost* b) {
   b->rs_T = T;
-  b->rs_setup = reinterpret_cast<const void*>(&kb_rs_setup<T>);
+  b->rs_setup = reinterpret_cast<const void*>(&kb_rs_setup<T, R>);
   b->rs_solve = reinterpret_cast<const void*>(&kb_pb_resident<T, R>);
   return rs_row_lds<T, R>();
 }
@@ -1159,7 +1159,7 @@ static void bh_plan(BatchHost* b) {
     wg0 += q.G + 1;
     int l0 = 1;
     while (l0 < c->G.nlev &&
-           (c->G.lev[l0].n > RS_CO_MAX || rs_coarse_lds(c->G, l0) > RES_LDS_MAX))
+           (!rs_coarse_fits(c->G, l0) || rs_coarse_lds(c->G, l0) > RES_LDS_MAX))
       l0++;
     q.m = l0 - 1;
     lds = std::max(lds, rs_coarse_lds(c->G, l0));

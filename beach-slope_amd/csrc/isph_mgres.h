@@ -31,10 +31,11 @@
 #include "isph_batch.h"
 #include "isph_persist.h"
 
-#define RS_W 6                      // window elements per thread
-#define RS_WCAP (RS_W * 1024 / PS_CHUNK)
-// Unknowns of the coarse workgroup's first level at most; their stencils stay
-// in registers.  A level more on the row workgroups costs two more hops of
+// window elements per thread
+constexpr int rs_win(int T, int R) { return T == 512 && R > 1 ? 12 : 6; }
+#define RS_WCAP (6 * 1024 / PS_CHUNK)  // window chunks of a workgroup at most
+// Threads of the coarse workgroup's first level at most, four per unknown of
+// the next; their stencils stay in registers.  A level more on the row workgroups costs two more hops of
 // ~1.2 us a V-cycle, a level of 1-4 unknowns per thread more in the one
 // workgroup 2-4 us: 1,024 against 2,560 unknowns took 51.0 against 55.8 us
 // per iteration at 7,485 rows and 73.7 against 77.4 at 22k; 300 took 52.4
@@ -129,11 +130,11 @@ __device__ __forceinline__ int rs_locate(const ResDev* rs, int S, int wg) {
 
 // Windows, window positions (into D.aoff) and cleared words, one workgroup
 // per row workgroup of the solve
-template <int T>
+template <int T, int R>
 __global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
   __shared__ uint16_t map[PS_MAX_CHUNKS];
   __shared__ int cnt[T];
-  const int wcap = RS_W * T / PS_CHUNK;
+  const int wcap = rs_win(T, R) * T / PS_CHUNK;
   const int s = rs_locate(rs, B.S, blockIdx.x), t = threadIdx.x;
   const ResDev& Q = rs[s];
   const Dev& D = B.devs[s];
@@ -228,6 +229,53 @@ __global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
 // ---------------------------------------------------------------------
 // rows
 // ---------------------------------------------------------------------
+// The first entries of a workgroup's rows stay on the chip for the launch: read
+// from memory, a row's three batches of entries are three dependent trips of
+// ~0.5 us in each of the six products of an iteration.  512 threads with a row
+// each have the registers for them (and for their FP64 values); 1,024 with a
+// row each keep the positions and FP16 values in LDS; several rows per thread
+// stream them.  An iteration took 42.0 us before and 38.0 after at 7,485 rows,
+// 42.6 and 37.5 at 22k, 64.6 and 61.7 at 137k, 74.6 and 72.5 at 207k.
+constexpr int rs_reg_entries(int T, int R) { return T == 512 && R == 1 ? 24 : 0; }
+constexpr int rs_lds_entries(int T, int R) { return T * R == 1024 ? 22 : 0; }
+template <int T, int R>
+struct RsEntries {
+  static constexpr int KR = rs_reg_entries(T, R), KL = rs_lds_entries(T, R), K = KR + KL;
+  uint32_t rw[KR ? KR / 2 : 1], rv[KR ? KR / 2 : 1];  // positions, FP16 values
+  double rd[KR ? KR : 1];                             // FP64 values
+  uint32_t* lw;                                       // positions, then FP16 values
+  __device__ __forceinline__ void load(const uint32_t* ip, const uint32_t* hp, const double* vp,
+                                       int cap, unsigned i, int L, int t, uint32_t* lds) {
+    lw = lds;
+#pragma unroll
+    for (int q = 0; q < K / 2; q++) {
+      const bool in = 2 * q < L;
+      const uint32_t w = in ? *ps_at(ip + (size_t)q * cap, i) : 0u;
+      const uint32_t h = in ? *ps_at(hp + (size_t)q * cap, i) : 0u;
+      if (KR) {
+        rw[KR ? q : 0] = w;
+        rv[KR ? q : 0] = h;
+      } else {
+        lw[q * T + t] = w;
+        lw[(KL / 2 + q) * T + t] = h;
+      }
+    }
+    if (KR)
+#pragma unroll
+      for (int k = 0; k < KR; k++) rd[k] = k < L ? *ps_at(vp + (size_t)k * cap, i) : 0.0;
+  }
+  __device__ __forceinline__ uint32_t w(int q, int t) const {
+    return KR ? rw[KR ? q : 0] : lw[q * T + t];
+  }
+  __device__ __forceinline__ uint32_t h(int q, int t) const {
+    return KR ? rv[KR ? q : 0] : lw[(KL / 2 + q) * T + t];
+  }
+};
+
+__device__ __forceinline__ float rs_half(uint32_t h, int u) {
+  const unsigned short b = (unsigned short)((u & 1) ? (h >> 16) : (h & 0xffffu));
+  return __half2float(__ushort_as_half(b));
+}
 // sum of the row's FP16 values times the window's floats, in entry order
 // (the order of ell_row_sum_h)
 template <bool FULL>
@@ -254,16 +302,38 @@ __device__ __forceinline__ float rs_row_h8(const uint32_t*& ip, const uint32_t*&
   }
 #pragma unroll
   for (int u = 0; u < 8; u++) {
-    const unsigned short hb = (unsigned short)((u & 1) ? (h[u / 2] >> 16) : (h[u / 2] & 0xffffu));
-    const float a = acc + __half2float(__ushort_as_half(hb)) * g[u];
+    const float a = acc + rs_half(h[u / 2], u) * g[u];
     acc = (k0 + u < L) ? a : acc;
   }
   return acc;
 }
-__device__ __forceinline__ float rs_row_h(const uint32_t* ip, const uint32_t* hp, int cap,
-                                          unsigned i, int L, int Lm, const float* X) {
+template <int T, int R>
+__device__ __forceinline__ float rs_row_h(const RsEntries<T, R>& E, const uint32_t* ip,
+                                          const uint32_t* hp, int cap, unsigned i, int t, int L,
+                                          int Lm, const float* X) {
+  constexpr int K = RsEntries<T, R>::K;
   float acc = 0.0f;
-  int k0 = 0;
+#pragma unroll
+  for (int k0 = 0; k0 < K; k0 += 8) {
+    if (k0 >= Lm) break;
+    float g[8], a[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      if (k0 + u >= K) continue;
+      const uint32_t w = E.w((k0 + u) / 2, t);
+      g[u] = X[(u & 1) ? w >> 16 : w & 0xffffu];
+      a[u] = rs_half(E.h((k0 + u) / 2, t), u);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      if (k0 + u >= K) continue;
+      const float s = acc + a[u] * g[u];
+      acc = (k0 + u < L) ? s : acc;
+    }
+  }
+  ip += (size_t)(K / 2) * cap;
+  hp += (size_t)(K / 2) * cap;
+  int k0 = K;
 #pragma unroll 1
   for (; k0 + 8 <= Lm; k0 += 8) {
     acc = rs_row_h8<true>(ip, hp, cap, i, k0, L, Lm, X, acc);
@@ -304,10 +374,36 @@ __device__ __forceinline__ double rs_row_d8(const uint32_t*& ip, const double*& 
   }
   return acc;
 }
-__device__ __forceinline__ double rs_row_d(const uint32_t* ip, const double* vp, int cap,
-                                           unsigned i, int L, int Lm, const float* X) {
+template <int T, int R>
+__device__ __forceinline__ double rs_row_d(const RsEntries<T, R>& E, const uint32_t* ip,
+                                           const double* vp, int cap, unsigned i, int t, int L,
+                                           int Lm, const float* X) {
+  constexpr int K = RsEntries<T, R>::K, KR = RsEntries<T, R>::KR;
   double acc = 0.0;
-  int k0 = 0;
+#pragma unroll
+  for (int k0 = 0; k0 < K; k0 += 8) {
+    if (k0 >= Lm) break;
+    float g[8];
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      if (k0 + u >= K) continue;
+      if (KR) v[u] = E.rd[KR ? k0 + u : 0];
+      else v[u] = (k0 + u < Lm) ? *ps_at(vp, i) : 0.0;
+      vp += cap;
+      const uint32_t w = E.w((k0 + u) / 2, t);
+      g[u] = X[(u & 1) ? w >> 16 : w & 0xffffu];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      if (k0 + u >= K) continue;
+      const double s = acc + v[u] * (double)g[u];
+      acc = (k0 + u < L) ? s : acc;
+    }
+  }
+  ip += (size_t)(K / 2) * cap;
+  int k0 = K;
+  if (K >= Lm) return acc;
 #pragma unroll 1
   for (; k0 + 8 <= Lm; k0 += 8) {
     acc = rs_row_d8<true>(ip, vp, cap, i, k0, L, Lm, X, acc);
@@ -321,13 +417,60 @@ __device__ __forceinline__ double rs_row_d(const uint32_t* ip, const double* vp,
 // coarse workgroup sums them in the order of final_tree2 and sends the sums
 // to each workgroup's mail line
 // ---------------------------------------------------------------------
+template <int T, int NV>
+__device__ __forceinline__ bool rs_collect(const ResDev& Q, int nblk, unsigned ep,
+                                                double* col, double* res, volatile int* bad,
+                                                double (&out)[NV]) {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  const int l = t & 63, wave = t >> 6;
+  const unsigned long long* slots = glob(Q.slots);
+  // thread t sums column t & 255 (blocks c, c + 256, ...) of one or two values
+  for (int e = t; e < NV * 256; e += T) {
+    const int k = e >> 8, c = e & 255;
+    const unsigned long long* p = slots + 2 * (size_t)k * nblk;
+    double a = 0.0;
+    for (int b0 = c; b0 < nblk; b0 += 4 * 256) {
+      unsigned long long w[4][2];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int b = min(b0 + 256 * u, nblk - 1);
+        w[u][0] = ld_agent(p + 2 * (size_t)b);
+        w[u][1] = ld_agent(p + 2 * (size_t)b + 1);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int b = b0 + 256 * u;
+        if (b < nblk) {
+          const uint32_t lo = __float_as_uint(rs_wait(p + 2 * (size_t)b, ep, bad, w[u][0]));
+          const uint32_t hi = __float_as_uint(rs_wait(p + 2 * (size_t)b + 1, ep, bad, w[u][1]));
+          a = a + __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+        }
+      }
+    }
+    col[e] = a;
+  }
+  __syncthreads();
+  if (wave < NV) {
+    const double* c = col + wave * 256;
+    const double s = wave_tree((c[l] + c[l + 128]) + (c[l + 64] + c[l + 192]));
+    if (l == 0) res[wave] = s;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; k++) out[k] = res[k];
+  return !*bad;
+}
+
 template <int T, int R, int NV>
 __device__ __forceinline__ bool rs_publish_wait(const ResDev& Q, int wg, int nblk, unsigned ep,
                                                 const double (&v)[NV][R], double* area,
                                                 double* res, volatile int* bad,
                                                 double (&out)[NV]) {
   constexpr int S4 = T / 256;
-  const int t = threadIdx.x, wv = (t >> 6) & 3, l = t & 63, sub = t >> 8;
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  const int wv = (t >> 6) & 3, l = t & 63, sub = t >> 8;
   // tree j = k R + q of a block is summed by wavefront j mod 4 of its four;
   // the other three leave their values in LDS
 #pragma unroll
@@ -372,43 +515,9 @@ template <int T, int NV>
 __device__ __forceinline__ bool rs_collect_send(const ResDev& Q, int nblk, unsigned ep,
                                                 double* col, double* res, volatile int* bad,
                                                 double (&out)[NV]) {
-  const int t = threadIdx.x, l = t & 63, wave = t >> 6;
-  const unsigned long long* slots = glob(Q.slots);
-  // thread t sums column t & 255 (blocks c, c + 256, ...) of one or two values
-  for (int e = t; e < NV * 256; e += T) {
-    const int k = e >> 8, c = e & 255;
-    const unsigned long long* p = slots + 2 * (size_t)k * nblk;
-    double a = 0.0;
-    for (int b0 = c; b0 < nblk; b0 += 4 * 256) {
-      unsigned long long w[4][2];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int b = min(b0 + 256 * u, nblk - 1);
-        w[u][0] = ld_agent(p + 2 * (size_t)b);
-        w[u][1] = ld_agent(p + 2 * (size_t)b + 1);
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int b = b0 + 256 * u;
-        if (b < nblk) {
-          const uint32_t lo = __float_as_uint(rs_wait(p + 2 * (size_t)b, ep, bad, w[u][0]));
-          const uint32_t hi = __float_as_uint(rs_wait(p + 2 * (size_t)b + 1, ep, bad, w[u][1]));
-          a = a + __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-        }
-      }
-    }
-    col[e] = a;
-  }
-  __syncthreads();
-  if (wave < NV) {
-    const double* c = col + wave * 256;
-    const double s = wave_tree((c[l] + c[l + 128]) + (c[l + 64] + c[l + 192]));
-    if (l == 0) res[wave] = s;
-  }
-  __syncthreads();
-  if (*bad) return false;
-#pragma unroll
-  for (int k = 0; k < NV; k++) out[k] = res[k];
+  if (!rs_collect<T, NV>(Q, nblk, ep, col, res, bad, out)) return false;
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
   unsigned long long* mail = glob(Q.mail);
   for (int e = t; e < Q.G * 2 * NV; e += T) {
     const int g = e / (2 * NV), j = e - g * 2 * NV;
@@ -432,8 +541,15 @@ struct RsScalars {
   int iters, conv, brk, done;
   bool update;  // the stopped iteration's x and r update still applies
 };
+// a value that is the same in every lane, out of the vector registers
+__device__ __forceinline__ double rs_uni(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readfirstlane((int)b);
+  const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
 __device__ __forceinline__ void rs_alpha(RsScalars& z, double s0) {
-  z.alpha = z.rho / s0;
+  z.alpha = rs_uni(z.rho / s0);
   if (!isfinite(z.alpha)) {
     z.brk = 1;
     z.done = 1;
@@ -441,7 +557,7 @@ __device__ __forceinline__ void rs_alpha(RsScalars& z, double s0) {
 }
 __device__ __forceinline__ void rs_omega(RsScalars& z, const double (&s)[5], double stop,
                                          double bnorm, int max_iter) {
-  const double om = s[0] / s[1];
+  const double om = rs_uni(s[0] / s[1]);
   z.omega = om;
   z.update = false;
   if (!isfinite(om) || om == 0.0) {
@@ -462,8 +578,8 @@ __device__ __forceinline__ void rs_omega(RsScalars& z, const double (&s)[5], dou
     z.brk = 1;
     z.done = 1;
   } else {
-    z.beta = (rhon / z.rho) * (z.alpha / om);
-    z.rho = rhon;
+    z.beta = rs_uni((rhon / z.rho) * (z.alpha / om));
+    z.rho = rs_uni(rhon);
     if (z.iters >= max_iter) z.done = 1;
   }
 }
@@ -473,6 +589,24 @@ __device__ __forceinline__ void rs_omega(RsScalars& z, const double (&s)[5], dou
 // ---------------------------------------------------------------------
 // first item of workgroup w of G's equal runs over n items
 __device__ __forceinline__ int rs_part(int n, int w, int G) { return (int)((int64_t)n * w / G); }
+
+// neighbours of cell (ci, cj): a bit for each that exists
+__device__ __forceinline__ unsigned rs_has(const MgLevel& L, int ci, int cj) {
+  const unsigned row = (ci > 0 ? 1u : 0u) | 2u | (ci + 1 < L.ny ? 4u : 0u);
+  return (cj > 0 ? row : 0u) | (row << 3) | (cj + 1 < L.nx ? row << 6 : 0u);
+}
+// neighbour k, the cell itself in place of a missing one (its term is not
+// added); formed anew at each use, for nine of them held over the polls are
+// nine registers
+__device__ __forceinline__ int rs_nbr(unsigned has, int I, int ny, int k) {
+  return I + (((has >> k) & 1) ? (k / 3 - 1) * ny + (k % 3 - 1) : 0);
+}
+// the coarser cell holding neighbour k of a cell at place q (row q & 1, column
+// q >> 1) of cell P
+__device__ __forceinline__ int rs_par(unsigned has, int P, int q, int ny, int k) {
+  const int di = ((q & 1) + k % 3 - 1) >> 1, dj = ((q >> 1) + k / 3 - 1) >> 1;
+  return P + (((has >> k) & 1) ? dj * ny + di : 0);
+}
 
 template <int T>
 __device__ __forceinline__ void rs_down(const RsMg& M, const ResDev& Q, int wg, int t,
@@ -490,21 +624,19 @@ __device__ __forceinline__ void rs_down(const RsMg& M, const ResDev& Q, int wg, 
     const int ci = 2 * CI + (q & 1), cj = 2 * CJ + (q >> 1);
     const bool in = ci < L.ny && cj < L.nx;
     const int I = in ? cj * L.ny + ci : 0;
-    int Nb[9];
-    mg_nbr9(L, in ? ci : 0, in ? cj : 0, I, Nb);
+    const unsigned has = in ? rs_has(L, ci, cj) : 0u;
     float sv[9], rv[9], bv[9];
 #pragma unroll
     for (int k = 0; k < 9; k++) {
-      Nb[k] = Nb[k] >= 0 ? Nb[k] : (I | (1 << 30));  // bit 30: a term that is not added
       sv[k] = *ps_at(st + (size_t)k * L.n, I);
-      rv[k] = *ps_at(rd, Nb[k] & ~(1 << 30));
+      rv[k] = *ps_at(rd, rs_nbr(has, I, L.ny, k));
     }
-    rs_poll<9>(tag, bad, [&](int k) { return ld_word(bl, Nb[k] & ~(1 << 30)); }, bv);
+    rs_poll<9>(tag, bad, [&](int k) { return ld_word(bl, rs_nbr(has, I, L.ny, k)); }, bv);
     float acc = 0.0f;
 #pragma unroll
     for (int k = 0; k < 9; k++) {
       const float tk = sv[k] * ((w * bv[k]) * rv[k]);
-      if (!(Nb[k] >> 30)) acc = acc + tk;
+      if ((has >> k) & 1) acc = acc + tk;
     }
     const float bI = bv[4];
     const float res = in ? bI - acc : 0.0f;
@@ -537,23 +669,18 @@ __device__ __forceinline__ void rs_up(const RsMg& M, const ResDev& Q, int wg, in
   const int I0 = rs_part(L.n, wg, Q.G), I1 = rs_part(L.n, wg + 1, Q.G);
   for (int I = I0 + t; I < I1; I += T) {
     const int cj = I / L.ny, ci = I - cj * L.ny;
-    const int pI = (cj >> 1) * C.ny + (ci >> 1);
-    int Nb[9], Pa[9];
-    mg_nbr9(L, ci, cj, I, Nb);
-    mg_par9(C, ci, cj, Pa);
-    float sv[9], xv[9], xc[9];
-    unsigned has = 0;
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-      if (Nb[k] >= 0) has |= 1u << k;
-      else Nb[k] = I, Pa[k] = pI;  // read in place of a missing one; its term is not added
-      sv[k] = *ps_at(st + (size_t)k * L.n, I);
-    }
-    rs_poll<9>(tag, bad, [&](int k) { return ld_word(bw, Nb[k]); }, xv);
+    const int P = (cj >> 1) * C.ny + (ci >> 1), q = (ci & 1) | ((cj & 1) << 1);
+    const unsigned has = rs_has(L, ci, cj);
+    float xv[9], xc[9];
+    // (the words of this level are those that the way down polled)
+    rs_poll<9>(tag, bad, [&](int k) { return ld_word(bw, rs_nbr(has, I, L.ny, k)); }, xv);
     const float bI = xv[4], rI = *ps_at(rd, I);
 #pragma unroll
-    for (int k = 0; k < 9; k++) xv[k] = (w * xv[k]) * *ps_at(rd, Nb[k]);
-    rs_poll<9>(tag, bad, [&](int k) { return ld_word(ec, Pa[k]); }, xc);
+    for (int k = 0; k < 9; k++) xv[k] = (w * xv[k]) * *ps_at(rd, rs_nbr(has, I, L.ny, k));
+    float sv[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++) sv[k] = *ps_at(st + (size_t)k * L.n, I);
+    rs_poll<9>(tag, bad, [&](int k) { return ld_word(ec, rs_par(has, P, q, C.ny, k)); }, xc);
     float acc = 0.0f;
 #pragma unroll
     for (int k = 0; k < 9; k++) {
@@ -569,7 +696,89 @@ __device__ __forceinline__ void rs_up(const RsMg& M, const ResDev& Q, int wg, in
 // ---------------------------------------------------------------------
 // the coarse workgroup (mg_coarse_block with its data kept in LDS and
 // registers over the solve)
+//
+// Every V-cycle waits for this workgroup, so what counts is the length of its
+// chain.  A level takes one barrier down and one up: thread e has unknown
+// e & 3 of aggregate e >> 2, and the aggregate's residuals are summed by
+// shuffles.  Which unknown that is and which neighbours it has is worked out
+// once per solve (a word per thread and level), the first level's stencil,
+// diagonals and smoothed values stay in registers, and the pre-smoothed
+// values of the levels below are formed from b by their readers.
 // ---------------------------------------------------------------------
+// unknown of level L (coarsened to C) of thread e, and its neighbours: bits 0-9
+// and 10-18 (0 where the aggregate has no such unknown)
+__device__ __forceinline__ int rs_co_info(const MgLevel& L, const MgLevel& C, int e) {
+  const int J = e >> 2;
+  if (J >= C.n) return 0;
+  const int CJ = J / C.ny, CI = J - CJ * C.ny;
+  const int ci = 2 * CI + (e & 1), cj = 2 * CJ + ((e >> 1) & 1);
+  if (ci >= L.ny || cj >= L.nx) return 0;
+  const int I = cj * L.ny + ci;
+  int Nb[9], has = 0;
+  mg_nbr9(L, ci, cj, I, Nb);
+#pragma unroll
+  for (int k = 0; k < 9; k++) has |= (Nb[k] >= 0) << k;
+  return I | (has << 10);
+}
+// neighbour k of the unknown, itself in place of a missing one
+__device__ __forceinline__ int rs_co_nbr(int info, int ny, int k) {
+  const int I = info & 1023;
+  return ((info >> (10 + k)) & 1) ? I + (k / 3 - 1) * ny + (k % 3 - 1) : I;
+}
+// the level-C unknown holding neighbour k, for thread e
+__device__ __forceinline__ int rs_co_par(int info, int e, int cny, int k) {
+  const int di = ((e & 1) + k % 3 - 1) >> 1, dj = (((e >> 1) & 1) + k / 3 - 1) >> 1;
+  return ((info >> (10 + k)) & 1) ? (e >> 2) + dj * cny + di : e >> 2;
+}
+// x of the pre-smoothing sweep at the unknown and its neighbours
+__device__ __forceinline__ void rs_co_x(int info, int ny, float w, const float* b,
+                                        const float (&rd)[9], float (&x)[9], float& bI) {
+  float bv[9];
+#pragma unroll
+  for (int k = 0; k < 9; k++) bv[k] = b[rs_co_nbr(info, ny, k)];
+#pragma unroll
+  for (int k = 0; k < 9; k++) x[k] = (w * bv[k]) * rd[k];
+  bI = bv[4];
+}
+// residual of x, summed over the aggregate by its first thread
+__device__ __forceinline__ float rs_co_down(int info, int t, const float (&st)[9],
+                                            const float (&x)[9], float bI) {
+  float acc = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    const float tk = st[k] * x[k];
+    if ((info >> (10 + k)) & 1) acc = acc + tk;
+  }
+  const int in = (info >> 14) & 1;
+  const float res = in ? bI - acc : 0.0f;
+  const int base = t & 60;
+  const float r1 = __shfl(res, base + 1, 64), r2 = __shfl(res, base + 2, 64),
+              r3 = __shfl(res, base + 3, 64);
+  const int i1 = __shfl(in, base + 1, 64), i2 = __shfl(in, base + 2, 64),
+            i3 = __shfl(in, base + 3, 64);
+  float s = 0.0f;
+  if (in) s = s + res;
+  if (i1) s = s + r1;
+  if (i2) s = s + r2;
+  if (i3) s = s + r3;
+  return s;
+}
+// the unknown's value after the correction and the post-smoothing sweep
+__device__ __forceinline__ float rs_co_up(int info, int e, int cny, float w, float c,
+                                          const float* xc, const float (&st)[9],
+                                          const float (&x)[9], float bI, float rI) {
+  float xv[9];
+#pragma unroll
+  for (int k = 0; k < 9; k++) xv[k] = x[k] + c * xc[rs_co_par(info, e, cny, k)];
+  float acc = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    const float tk = st[k] * xv[k];
+    if ((info >> (10 + k)) & 1) acc = acc + tk;
+  }
+  return xv[4] + (w * (bI - acc)) * rI;
+}
+
 template <int T>
 __device__ __forceinline__ void rs_coarse_solve(const Dev& D, const MgDev& M, const ResDev& Q,
                                                 const MgLevel* lev,
@@ -584,34 +793,45 @@ __device__ __forceinline__ void rs_coarse_solve(const Dev& D, const MgDev& M, co
   double* res = lds + 5 * 256;
   volatile int* bad = reinterpret_cast<int*>(res + 6);
   const MgLevel L0 = rs_level(lev, l0), LD = rs_level(lev, nl);
+  const MgLevel C0 = rs_level(lev, l0 < nl ? l0 + 1 : nl);
   const int base = L0.off;
   const int S = LD.off + LD.n - base;
-  const int stb = (l0 < nl) ? rs_level(lev, l0 + 1).off : LD.off;
-  const int nst = 9 * (LD.off - stb), nrd = nst / 9, nd2 = LD.n * LD.n;
+  const int stb = C0.off;
+  const int nst = l0 < nl ? 9 * (LD.off - stb) : 0, nrd = nst / 9;
+  const int nd8 = (LD.n + 7) & ~7;  // rows of the inverse, to a multiple of 8 with zeros
   double* DI = res + 8;
-  float* X = reinterpret_cast<float*>(DI + nd2);
-  float* Bv = X + S;
-  float* R = X + 2 * S;
-  float* ST = X + 3 * S;
+  float* Bv = reinterpret_cast<float*>(DI + nd8 * LD.n);  // S, and zeros after the last level
+  float* R = Bv + S + 8;
+  float* ST = R + S;
   float* RD = ST + nst;
+  int* IN = reinterpret_cast<int*>(RD + nrd);
   const float* sten = glob(M.sten);
   const float* rdg = glob(M.rdg);
   const double* dinv = glob(M.dense_inv);
   if (t0 == 0) *bad = 0;
-  for (int e = t0; e < nd2; e += T) DI[e] = dinv[e];
+  if (t0 < 8) Bv[S + t0] = 0.0f;
+  for (int e = t0; e < nd8 * LD.n; e += T) DI[e] = e < LD.n * LD.n ? dinv[e] : 0.0;
   for (int e = t0; e < nst; e += T) ST[e] = sten[9 * (size_t)stb + e];
   for (int e = t0; e < nrd; e += T) RD[e] = rdg[stb + e];
-  float st0[PER][9], rd0[PER];
-  int ci0[PER], cj0[PER];
+  {
+    int* in = IN;
+    for (int l = l0 + 1; l < nl; l++) {
+      const MgLevel L = rs_level(lev, l), C = rs_level(lev, l + 1);
+      for (int e = t0; e < 4 * C.n; e += T) in[e] = rs_co_info(L, C, e);
+      in += 4 * C.n;
+    }
+  }
+  float st0[PER][9], rd0[PER][9];
+  int inf0[PER];
 #pragma unroll
   for (int q = 0; q < PER; q++) {
-    const int I = t0 + q * T, Ic = (I < L0.n) ? I : 0;
+    inf0[q] = l0 < nl ? rs_co_info(L0, C0, t0 + q * T) : 0;
     const float* sg = sten + 9 * (size_t)L0.off;
 #pragma unroll
-    for (int k = 0; k < 9; k++) st0[q][k] = sg[k * L0.n + Ic];
-    rd0[q] = rdg[base + Ic];
-    cj0[q] = Ic / L0.ny;
-    ci0[q] = Ic - cj0[q] * L0.ny;
+    for (int k = 0; k < 9; k++) {
+      st0[q][k] = sg[k * L0.n + (inf0[q] & 1023)];
+      rd0[q][k] = rdg[base + rs_co_nbr(inf0[q], L0.ny, k)];
+    }
   }
   const unsigned long long* bw = glob(Q.bw) + base;
   unsigned long long* ew = glob(Q.ew) + base;
@@ -634,140 +854,112 @@ __device__ __forceinline__ void rs_coarse_solve(const Dev& D, const MgDev& M, co
       int t = threadIdx.x;
       asm volatile("" : "+v"(t));
 #pragma unroll
-      for (int q = 0; q < PER; q++) asm volatile("" : "+v"(ci0[q]), "+v"(cj0[q]));
+      for (int q = 0; q < PER; q++) asm volatile("" : "+v"(inf0[q]));
       // right-hand side of the first level
-      float bq[PER];
-      rs_poll<PER>(tag, bad, [&](int q) {
-        return (t + q * T < L0.n) ? ld_word(bw, t + q * T) : (unsigned long long)tag << 32;
-      }, bq);
+      float x0[PER][9], b0[PER];
+      if (l0 < nl) {
+        rs_poll<PER>(tag, bad, [&](int q) {
+          return (inf0[q] >> 14) & 1 ? ld_word(bw, inf0[q] & 1023)
+                                     : (unsigned long long)tag << 32;
+        }, b0);
 #pragma unroll
-      for (int q = 0; q < PER; q++) {
-        const int I = t + q * T;
-        if (I < L0.n) {
-          Bv[I] = bq[q];
-          if (l0 < nl) X[I] = (w * bq[q]) * rd0[q];
-        }
+        for (int q = 0; q < PER; q++)
+          if ((inf0[q] >> 14) & 1) Bv[inf0[q] & 1023] = b0[q];
+      } else if (t < LD.n) {
+        Bv[t] = rs_wait(bw + t, tag, bad, 0ull);
       }
       __syncthreads();
-      for (int l = l0; l < nl; l++) {
-        const MgLevel L = rs_level(lev, l), C = rs_level(lev, l + 1);
-        float* x = X + (L.off - base);
-        const float* b = Bv + (L.off - base);
-        float* r = R + (L.off - base);
-        if (l == l0) {
+      if (l0 < nl) {
+        float* bc = Bv + (C0.off - base);
 #pragma unroll
-          for (int q = 0; q < PER; q++) {
-            const int I = t + q * T;
-            __builtin_amdgcn_sched_barrier(0);  // one unknown's values in registers at a time
-            if (I < L.n) {
-              float acc = 0.0f, tk[9];
-              int Nb[9];
-              mg_nbr9(L, ci0[q], cj0[q], I, Nb);
-#pragma unroll
-              for (int k = 0; k < 9; k++) tk[k] = st0[q][k] * x[Nb[k] >= 0 ? Nb[k] : I];
-#pragma unroll
-              for (int k = 0; k < 9; k++)
-                if (Nb[k] >= 0) acc = acc + tk[k];
-              r[I] = bq[q] - acc;
-            }
-          }
-        } else {
-          const float* st = ST + 9 * (L.off - stb);
-          for (int I = t; I < L.n; I += T) {
-            const int cj = I / L.ny, ci = I - cj * L.ny;
-            float acc = 0.0f, tk[9];
-            int Nb[9];
-            mg_nbr9(L, ci, cj, I, Nb);
-#pragma unroll
-            for (int k = 0; k < 9; k++) tk[k] = st[k * L.n + I] * x[Nb[k] >= 0 ? Nb[k] : I];
-#pragma unroll
-            for (int k = 0; k < 9; k++)
-              if (Nb[k] >= 0) acc = acc + tk[k];
-            r[I] = b[I] - acc;
-          }
+        for (int q = 0; q < PER; q++) {
+          const int e = t + q * T;
+          rs_co_x(inf0[q], L0.ny, w, Bv, rd0[q], x0[q], b0[q]);
+          const float s = rs_co_down(inf0[q], t, st0[q], x0[q], b0[q]);
+          if (!(e & 3) && (e >> 2) < C0.n) bc[e >> 2] = s;
         }
         __syncthreads();
-        // restricted right-hand side, and its pre-smoothed iterate
+      }
+      const int* in = IN;
+      for (int l = l0 + 1; l < nl; l++) {
+        const MgLevel L = rs_level(lev, l), C = rs_level(lev, l + 1);
+        const float* st = ST + 9 * (L.off - stb);
         float* bc = Bv + (C.off - base);
-        float* xn = X + (C.off - base);
-        for (int J = t; J < C.n; J += T) {
-          const int CJ = J / C.ny, CI = J - CJ * C.ny;
-          float s = 0.0f;
+        for (int e = t; e < 4 * C.n; e += T) {
+          const int info = in[e];
+          float sv[9], rv[9], x[9], bI;
 #pragma unroll
-          for (int bb = 0; bb < 2; bb++)
-#pragma unroll
-            for (int a = 0; a < 2; a++) {
-              const int ci = 2 * CI + a, cj = 2 * CJ + bb;
-              if (ci < L.ny && cj < L.nx) s = s + r[cj * L.ny + ci];
-            }
-          bc[J] = s;
-          if (l + 1 < nl) xn[J] = (w * s) * RD[C.off - stb + J];
+          for (int k = 0; k < 9; k++) {
+            sv[k] = st[k * L.n + (info & 1023)];
+            rv[k] = RD[L.off - stb + rs_co_nbr(info, L.ny, k)];
+          }
+          rs_co_x(info, L.ny, w, Bv + (L.off - base), rv, x, bI);
+          const float s = rs_co_down(info, t, sv, x, bI);
+          if (!(e & 3)) bc[e >> 2] = s;
         }
+        in += 4 * C.n;
         __syncthreads();
       }
-      {
+      if (t < LD.n) {
+        // eight rows of the inverse requested before the last eight are used
         const float* b = Bv + (LD.off - base);
-        float* x = X + (LD.off - base);
-        for (int I = t; I < LD.n; I += T) {
-          double acc = 0.0;
-#pragma unroll 8
-          for (int J = 0; J < LD.n; J++) acc = acc + DI[J * LD.n + I] * (double)b[J];
-          x[I] = (float)acc;
-          if (l0 == nl) rs_put(&ew[I], tag, (float)acc);
+        const double* di = DI + t;
+        double acc = 0.0, dv[8];
+        float bv[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          dv[u] = di[u * LD.n];
+          bv[u] = b[u];
+        }
+        for (int J = 8; J < nd8; J += 8) {
+          double dn[8];
+          float bn[8];
+#pragma unroll
+          for (int u = 0; u < 8; u++) {
+            dn[u] = di[(J + u) * LD.n];
+            bn[u] = b[J + u];
+          }
+#pragma unroll
+          for (int u = 0; u < 8; u++) {
+            acc = acc + dv[u] * (double)bv[u];
+            dv[u] = dn[u];
+            bv[u] = bn[u];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) acc = acc + dv[u] * (double)bv[u];
+        if (l0 == nl) rs_put(&ew[t], tag, (float)acc);
+        R[LD.off - base + t] = (float)acc;
+      }
+      __syncthreads();
+      for (int l = nl - 1; l > l0; l--) {
+        const MgLevel L = rs_level(lev, l), C = rs_level(lev, l + 1);
+        const float* st = ST + 9 * (L.off - stb);
+        const float* xc = R + (C.off - base);
+        float* out = R + (L.off - base);
+        in -= 4 * C.n;
+        for (int e = t; e < 4 * C.n; e += T) {
+          const int info = in[e];
+          if (!((info >> 14) & 1)) continue;
+          float sv[9], rv[9], x[9], bI;
+#pragma unroll
+          for (int k = 0; k < 9; k++) {
+            sv[k] = st[k * L.n + (info & 1023)];
+            rv[k] = RD[L.off - stb + rs_co_nbr(info, L.ny, k)];
+          }
+          rs_co_x(info, L.ny, w, Bv + (L.off - base), rv, x, bI);
+          out[info & 1023] = rs_co_up(info, e, C.ny, w, c, xc, sv, x, bI, rv[4]);
         }
         __syncthreads();
       }
-      for (int l = nl - 1; l >= l0; l--) {
-        const MgLevel L = rs_level(lev, l), C = rs_level(lev, l + 1);
-        const float* x = X + (L.off - base);
-        const float* b = Bv + (L.off - base);
-        const float* xc = (l + 1 == nl ? X : R) + (C.off - base);
-        float* out = R + (L.off - base);
-        if (l == l0) {
+      if (l0 < nl) {
+        const float* xc = R + (C0.off - base);
 #pragma unroll
-          for (int q = 0; q < PER; q++) {
-            const int I = t + q * T;
-            __builtin_amdgcn_sched_barrier(0);
-            if (I < L.n) {
-              const int ci = ci0[q], cj = cj0[q];
-              float acc = 0.0f, tk[9];
-              int Nb[9], Pa[9];
-              mg_nbr9(L, ci, cj, I, Nb);
-              mg_par9(C, ci, cj, Pa);
-              const int pI = (cj >> 1) * C.ny + (ci >> 1);
-#pragma unroll
-              for (int k = 0; k < 9; k++) {
-                const bool has = Nb[k] >= 0;
-                tk[k] = st0[q][k] * (x[has ? Nb[k] : I] + c * xc[has ? Pa[k] : pI]);
-              }
-#pragma unroll
-              for (int k = 0; k < 9; k++)
-                if (Nb[k] >= 0) acc = acc + tk[k];
-              const float x1 = x[I] + c * xc[pI];
-              rs_put(&ew[I], tag, x1 + (w * (bq[q] - acc)) * rd0[q]);
-            }
-          }
-        } else {
-          const float* st = ST + 9 * (L.off - stb);
-          for (int I = t; I < L.n; I += T) {
-            const int cj = I / L.ny, ci = I - cj * L.ny;
-            float acc = 0.0f, tk[9];
-            int Nb[9], Pa[9];
-            mg_nbr9(L, ci, cj, I, Nb);
-            mg_par9(C, ci, cj, Pa);
-            const int pI = (cj >> 1) * C.ny + (ci >> 1);
-#pragma unroll
-            for (int k = 0; k < 9; k++) {
-              const bool has = Nb[k] >= 0;
-              tk[k] = st[k * L.n + I] * (x[has ? Nb[k] : I] + c * xc[has ? Pa[k] : pI]);
-            }
-#pragma unroll
-            for (int k = 0; k < 9; k++)
-              if (Nb[k] >= 0) acc = acc + tk[k];
-            const float x1 = x[I] + c * xc[pI];
-            out[I] = x1 + (w * (b[I] - acc)) * RD[(L.off - stb) + I];
-          }
-        }
+        for (int q = 0; q < PER; q++)
+          if ((inf0[q] >> 14) & 1)
+            rs_put(&ew[inf0[q] & 1023], tag,
+                   rs_co_up(inf0[q], t + q * T, C0.ny, w, c, xc, st0[q], x0[q], b0[q],
+                            rd0[q][4]));
         __syncthreads();
       }
       if (half == 0) {
@@ -805,7 +997,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
                                               const MgLevel* lev,
                                               int wg, int iters, unsigned v0, unsigned ep,
                                               double* lds) {
-  constexpr int S4 = T / 256;
+  constexpr int S4 = T / 256, W = rs_win(T, R);
   const int t = threadIdx.x, l = t & 63;
   DevScalars* Sc = glob(D.sc);
   const int n = Sc->n, nblk = D.nblk, cap = D.cap;
@@ -814,7 +1006,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
   double* res = lds + 5 * R * S4 * 192;
   volatile int* bad = reinterpret_cast<int*>(res + 6);
   float* X = reinterpret_cast<float*>(res + 8);  // the window
-  float* r0s = X + RS_W * T;                  // r0 of the workgroup's rows
+  float* r0s = X + W * T;                  // r0 of the workgroup's rows
   if (t == 0) *bad = 0;
   unsigned long long* x0w = glob(Q.x0w);
   unsigned long long* phw = glob(Q.phw);
@@ -848,12 +1040,17 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
     d0[q] = in ? glob(M.d0)[i] : 0.0f;
     r[q] = in ? glob(D.r)[i] : 0.0;
   }
+  RsEntries<T, R> E[R];
+#pragma unroll
+  for (int q = 0; q < R; q++)
+    E[q].load(lidx, av16, aval, cap, max(row[q], 0), len[q], t,
+              reinterpret_cast<uint32_t*>(r0s + R * T + RS_TAIL) + q * E[0].KL * T);
   // window elements: chunk (uniform per wavefront), cell of the row; own
   // chunks hold the workgroup's rows at positions s0 * 64 + local row
   const int oc0 = i0 / PS_CHUNK, oc1 = (i1 + PS_CHUNK - 1) / PS_CHUNK;
-  int wc[RS_W], wk[RS_W];
+  int wc[W], wk[W];
 #pragma unroll
-  for (int w = 0; w < RS_W; w++) {
+  for (int w = 0; w < W; w++) {
     const int s = w * (T / PS_CHUNK) + t / PS_CHUNK;
     wc[w] = __builtin_amdgcn_readfirstlane((s < wn) ? wl[s] : -1);
     const int g = wc[w] * PS_CHUNK + l;
@@ -895,7 +1092,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
     ph[q] = 0.0f;
   }
   __syncthreads();
-  bool ok = true;
+  bool ok = true, pend = false;  // pend: the x update of the iteration before is to come
   for (int it = 0; it < iters && ok; it++) {
 #pragma unroll 1
     for (int half = 0; half < 2; half++) {
@@ -907,7 +1104,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
 #pragma unroll
       for (int q = 0; q < R; q++) asm volatile("" : "+v"(row[q]));
 #pragma unroll
-      for (int w = 0; w < RS_W; w++) asm volatile("" : "+v"(wk[w]));
+      for (int w = 0; w < W; w++) asm volatile("" : "+v"(wk[w]));
       const int l = t & 63;
       // ---- V-cycle of v = p (half 0) or s, which is in r (half 1)
       float v[R];
@@ -921,26 +1118,44 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
         }
       }
       auto window = [&](const unsigned long long* words) {
-        float e[RS_W];
         auto other = [&](int w) {
           return wc[w] >= 0 && (wc[w] < oc0 || wc[w] >= oc1) && wk[w] >= 0;
         };
-        rs_poll<RS_W>(tag, bad, [&](int w) {
-          return other(w) ? ld_word(words + (int64_t)wc[w] * PS_CHUNK, l)
-                          : (unsigned long long)tag << 32;
-        }, e);
 #pragma unroll
-        for (int w = 0; w < RS_W; w++)
-          if (other(w)) X[w * T + t] = e[w];
+        for (int w0 = 0; w0 < W; w0 += 6) {
+          float e[6];
+          rs_poll<6>(tag, bad, [&](int w) {
+            return other(w0 + w) ? ld_word(words + (int64_t)wc[w0 + w] * PS_CHUNK, l)
+                                 : (unsigned long long)tag << 32;
+          }, e);
+#pragma unroll
+          for (int w = 0; w < 6; w++)
+            if (other(w0 + w)) X[(w0 + w) * T + t] = e[w];
+        }
       };
+      // x += alpha ph + omega sh of the iteration before, while x0 is on its
+      // way (nothing of the iteration waits for it)
+      double xs[R];
+      if (pend) {
+#pragma unroll
+        for (int q = 0; q < R; q++)
+          if (row[q] >= 0) xs[q] = *ps_at(sol, row[q]);
+      }
       window(x0w);
+      if (pend) {
+#pragma unroll
+        for (int q = 0; q < R; q++)
+          if (row[q] >= 0)
+            *ps_at(sol, row[q]) = (xs[q] + z.alpha * (double)ph[q]) + z.omega * (double)sh[q];
+        pend = false;
+      }
       __syncthreads();
       // r0 = v - A x0
 #pragma unroll
       for (int q = 0; q < R; q++) {
         __builtin_amdgcn_sched_barrier(0);
         if (row[q] >= 0) {
-          const float acc = rs_row_h(lidx, av16, cap, row[q], len[q], lmx[q], X);
+          const float acc = rs_row_h<T, R>(E[q], lidx, av16, cap, row[q], t, len[q], lmx[q], X);
           const float r0 = v[q] - acc;
           r0s[q * T + t] = r0;
           if (q * T + t < head) rs_put(ps_at(r0w, row[q]), tag, r0);
@@ -975,14 +1190,15 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
       // corrections before the others read theirs
       if (t < 64 && wk[0] >= 0) (void)rs_wait(ps_at(e1w, wk[0]), tag, bad, 0ull);
       __syncthreads();
-      {
-        float e[RS_W];
-        rs_poll<RS_W>(tag, bad, [&](int w) {
-          return wk[w] >= 0 ? ld_word(e1w, wk[w]) : (unsigned long long)tag << 32;
+#pragma unroll
+      for (int w0 = 0; w0 < W; w0 += 6) {
+        float e[6];
+        rs_poll<6>(tag, bad, [&](int w) {
+          return wk[w0 + w] >= 0 ? ld_word(e1w, wk[w0 + w]) : (unsigned long long)tag << 32;
         }, e);
 #pragma unroll
-        for (int w = 0; w < RS_W; w++)
-          if (wk[w] >= 0) X[w * T + t] = X[w * T + t] + mc * e[w];
+        for (int w = 0; w < 6; w++)
+          if (wk[w0 + w] >= 0) X[(w0 + w) * T + t] = X[(w0 + w) * T + t] + mc * e[w];
       }
       __syncthreads();
       // x = x1 + w (v - A x1) d
@@ -992,7 +1208,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
         __builtin_amdgcn_sched_barrier(0);
         y[q] = 0.0f;
         if (row[q] >= 0) {
-          const float acc = rs_row_h(lidx, av16, cap, row[q], len[q], lmx[q], X);
+          const float acc = rs_row_h<T, R>(E[q], lidx, av16, cap, row[q], t, len[q], lmx[q], X);
           y[q] = X[s0 * PS_CHUNK + q * T + t] + mw * (v[q] - acc) * d0[q];
           rs_put(ps_at(phw, row[q]), tag, y[q]);
         }
@@ -1008,7 +1224,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
 #pragma unroll
       for (int q = 0; q < R; q++) {
         __builtin_amdgcn_sched_barrier(0);
-        acc[q] = (row[q] >= 0) ? rs_row_d(lidx, aval, cap, row[q], len[q], lmx[q], X) : 0.0;
+        acc[q] = (row[q] >= 0) ? rs_row_d<T, R>(E[q], lidx, aval, cap, row[q], t, len[q], lmx[q], X) : 0.0;
       }
       if (half == 0) {
         double o[1], pv[1][R];
@@ -1042,12 +1258,11 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
         if (!ok) break;
         rs_omega(z, o, stop, bnorm, max_iter);
         if (z.done && !z.update) break;
-        // x += alpha ph + omega sh ; r = s - omega t2 ; p = r + beta (p - omega t1)
+        pend = true;
+        // r = s - omega t2 ; p = r + beta (p - omega t1)
 #pragma unroll
         for (int q = 0; q < R; q++)
           if (row[q] >= 0) {
-            double* xp = ps_at(sol, row[q]);
-            *xp = (*xp + z.alpha * (double)ph[q]) + z.omega * (double)sh[q];
             r[q] = r[q] - z.omega * acc[q];
             if (!z.done) p[q] = (float)(r[q] + z.beta * ((double)p[q] - z.omega * t1[q]));
           }
@@ -1062,6 +1277,10 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
 #pragma unroll
   for (int q = 0; q < R; q++)
     if (row[q] >= 0) {
+      if (pend) {
+        double* xp = ps_at(sol, row[q]);
+        *xp = (*xp + z.alpha * (double)ph[q]) + z.omega * (double)sh[q];
+      }
       *ps_at(glob(D.r), row[q]) = r[q];
       *ps_at(glob(D.pp32), row[q]) = p[q];
     }
@@ -1069,10 +1288,24 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
 
 template <int T, int R>
 __host__ __device__ inline int64_t rs_row_lds() {
-  return 8 * (5 * R * (T / 256) * 192 + 8) + 4 * (RS_W * T + R * T + RS_TAIL);
+  return 8 * (5 * R * (T / 256) * 192 + 8) +
+         4 * (rs_win(T, R) * T + R * T + RS_TAIL + rs_lds_entries(T, R) * R * T);
+}
+// whether the coarse workgroup can take level l0 and those below
+__host__ __device__ inline bool rs_coarse_fits(const MgDev& G, int l0) {
+  return l0 == G.nlev || (4 * G.lev[l0 + 1].n <= RS_CO_MAX && G.lev[l0].n <= 1024);
 }
 __host__ __device__ inline int64_t rs_coarse_lds(const MgDev& G, int l0) {
-  return 8 * (5 * 256 + 8) + mg_coarse_lds_bytes(G, l0);
+  int64_t v = 8, st = 0, in = 0;
+  for (int l = l0; l <= G.nlev; l++) {
+    v += 2 * (int64_t)G.lev[l].n;
+    if (l > l0 && l < G.nlev) {
+      st += 10 * (int64_t)G.lev[l].n;
+      in += 4 * (int64_t)G.lev[l + 1].n;
+    }
+  }
+  const int64_t nd = G.lev[G.nlev].n;
+  return 8 * (5 * 256 + 8 + ((nd + 7) & ~7) * nd) + 4 * (v + st + in);
 }
 
 // up to `iters` iterations of every unfinished scenario

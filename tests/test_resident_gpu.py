@@ -68,6 +68,31 @@ def test_resident_solve_equals_launches(pkg, cases, nx, ny, iters, precision):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny", [(200, 40), (1400, 100)])
+def test_rows_longer_than_those_kept_on_the_chip(pkg, cases, nx, ny):
+    """Fluid pressed together by a quarter: rows of more than 24 entries, whose
+    ends the precision solve reads from memory."""
+    c = _tank(cases, nx, ny)
+    fl = c.parts["tid"] == 3
+    x0 = c.parts["x"][fl].min()
+    c.parts["x"][fl] = x0 + 0.75 * (c.parts["x"][fl] - x0)
+    c.params.update(precision=1, tol=1e-10, max_iter=60, max_outer=2)
+
+    def run(s):
+        rc, st = s.step(1, check=False)
+        longest = int(s.ppe()[0].max())
+        return rc, _stats(st), s.solution(), s.download(), longest
+
+    a, b = _both(pkg, c, run)
+    print(f"resident: n={c.n}, longest row {b[4]}", flush=True)
+    assert b[4] > 24
+    assert a[0] == b[0] and a[1] == b[1], (a[:2], b[:2])
+    assert np.array_equal(a[2], b[2])
+    for k in a[3]:
+        assert np.array_equal(a[3][k], b[3][k]), k
+
+
+@pytest.mark.gpu
 def test_far_columns_solve_launch_by_launch(pkg, cases):
     """Each row couples to rows all over the system: no window holds them."""
     c = cases.dam_break(dx=0.0025)
