@@ -22,7 +22,8 @@ enum {
   BK_DOWN = 2,                           // + l-1: 4 x level-(l+1) aggregates, l <= nmb
   BK_UP = 2 + MG_MAX_LEVELS,             // + l-1: level-l cells (x 4 on level 1), l <= nmb
   BK_COARSEN = 2 + 2 * MG_MAX_LEVELS,    // + l-1: level-(l+1) cells, l < nlev
-  BK_NKIND = 2 + 3 * MG_MAX_LEVELS
+  BK_STEN1 = 2 + 3 * MG_MAX_LEVELS,      // level-1 cells x 9
+  BK_NKIND
 };
 
 struct BatchDev {
@@ -74,14 +75,14 @@ __global__ void __launch_bounds__(256) kb_mg_setup0(BatchDev B) {
   mg_setup0_row(D, B.mgs[s_], vb_ * RED_BLOCK + threadIdx.x);
 }
 __global__ void __launch_bounds__(256) kb_mg_stencil1(BatchDev B) {
-  BATCH_CELLS(B, BK_CELL1);
+  BATCH_CELLS(B, BK_STEN1);
   mg_stencil1_cell(D, G, I_);
 }
 __global__ void __launch_bounds__(256) kb_mg_coarsen(BatchDev B, int l) {
   BATCH_CELLS(B, BK_COARSEN + l - 1);
   mg_coarsen_cell(G, l, I_);
 }
-__global__ void __launch_bounds__(MG_CO_THREADS) kb_mg_dense(BatchDev B) {
+__global__ void __launch_bounds__(MG_DENSE_THREADS) kb_mg_dense(BatchDev B) {
   mg_dense_block(B.mgs[blockIdx.x]);
 }
 

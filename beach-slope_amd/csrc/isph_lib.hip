@@ -1083,6 +1083,7 @@ static int bh_make(isph_ctx* const* ctxs, int S, BatchHost** out) {
       b->pre[(size_t)kind * (S + 1) + s + 1] = b->pre[(size_t)kind * (S + 1) + s] + blocks;
     };
     put(BK_CELL1, grid_of(G.lev[1].n));
+    put(BK_STEN1, grid_of(9 * G.lev[1].n));
     for (int l = 1; l < MG_MAX_LEVELS; l++) {
       put(BK_DOWN + l - 1, (l <= G.nmb) ? grid_of(4 * G.lev[l + 1].n) : 0);
       put(BK_UP + l - 1, (l <= G.nmb) ? grid_of((l == 1 ? 4 : 1) * G.lev[l].n) : 0);
@@ -1284,10 +1285,10 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
   const int grow = 8 * ((tot(BK_ROWS) + 7) / 8);
   // multigrid hierarchy from the assembled rows
   BLAUNCH(kb_mg_setup0, grow, 256, B);
-  BLAUNCH(kb_mg_stencil1, tot(BK_CELL1), 256, B);
+  BLAUNCH(kb_mg_stencil1, tot(BK_STEN1), 256, B);
   for (int l = 1; l < b->max_nlev; l++)
     if (tot(BK_COARSEN + l - 1) > 0) BLAUNCH(kb_mg_coarsen, tot(BK_COARSEN + l - 1), 256, B, l);
-  BLAUNCH(kb_mg_dense, S, MG_CO_THREADS, B);
+  BLAUNCH(kb_mg_dense, S, MG_DENSE_THREADS, B);
   // ||b||, then the FP64 start residual
   BLAUNCH(kb_pb_bnorm, grow, 256, B);
   BLAUNCH(kb_pfinalize, S, 256, B, (int)PFIN_BNORM, 0, 0);

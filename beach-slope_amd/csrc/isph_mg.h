@@ -29,8 +29,9 @@
 #define MG_MAX_LEVELS 24
 #define MG_DENSE_MAX 64
 #define MG_CO_THREADS 1024
-static_assert(MG_CO_THREADS % (2 * MG_DENSE_MAX) == 0,
-              "the dense inverse's update maps whole rows of 2 MG_DENSE_MAX columns");
+#define MG_DENSE_THREADS 512  // 256, 512, 1,024: 34, 31, 37 us (mg_dense_block)
+static_assert(MG_DENSE_MAX == 64 && MG_DENSE_THREADS % 64 == 0,
+              "the dense inverse maps a column to a lane and rows to wavefronts");
 // The first level of the coarse workgroup has at most MG_CO_PER unknowns per
 // thread: their stencils stay in registers for the whole cycle.
 #define MG_CO_PER 1
@@ -217,33 +218,29 @@ __device__ __forceinline__ void mg_setup0_row(const Dev& D, const MgDev& G, int 
   for (int q = 0; q < 9; q++) G.rowst[q * cap + i] = st[q];
 }
 
-// level 1, cell pass: the row sums of cell I's contiguous row range, in row
-// order; an empty cell gets an identity row
-__device__ __forceinline__ void mg_stencil1_cell(const Dev& D, const MgDev& G, int I) {
+// level 1, cell pass: the row sums of a cell's contiguous row range, in row
+// order; an empty cell gets an identity row.  A thread per cell and stencil
+// value (e = value * cells + cell): with one per cell the nine sums were four
+// to ten dependent trips of 36 loads on a chip nearly empty (28 us before,
+// 6 after at 22k rows; 56 and 24 at 653k).
+__device__ __forceinline__ void mg_stencil1_cell(const Dev& D, const MgDev& G, int e) {
   const MgLevel L = G.lev[1];
-  if (I >= L.n) return;
+  if (e >= 9 * L.n) return;
+  const int q = e / L.n, I = e - q * L.n;
   const int i0 = D.cstart[I], i1 = D.cstart[I + 1];
-  const int cap = D.cap;
-  float* st = G.sten + 9 * L.off;
-  double s[9];
+  const double* st = G.rowst + (size_t)q * D.cap;
+  double s = 0.0;
+  for (int b0 = i0; b0 < i1; b0 += 8) {
+    double v[8];
 #pragma unroll
-  for (int q = 0; q < 9; q++) s[q] = 0.0;
-  for (int b0 = i0; b0 < i1; b0 += 4) {  // four rows' loads in flight, sums in row order
-    double v[4][9];
+    for (int u = 0; u < 8; u++) v[u] = (b0 + u < i1) ? st[b0 + u] : 0.0;
 #pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-      for (int q = 0; q < 9; q++) v[u][q] = (b0 + u < i1) ? G.rowst[q * cap + b0 + u] : 0.0;
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-      if (b0 + u < i1)
-#pragma unroll
-        for (int q = 0; q < 9; q++) s[q] = s[q] + v[u][q];
+    for (int u = 0; u < 8; u++)
+      if (b0 + u < i1) s = s + v[u];
   }
-  if (i1 == i0) s[4] = 1.0;
-#pragma unroll
-  for (int q = 0; q < 9; q++) st[q * L.n + I] = (float)s[q];
-  G.rdg[L.off + I] = 1.0f / (float)s[4];
+  if (i1 == i0 && q == 4) s = 1.0;
+  (G.sten + 9 * L.off)[e] = (float)s;
+  if (q == 4) G.rdg[L.off + I] = 1.0f / (float)s;
 }
 
 // level l+1 cell I from level l: sum of the 2x2 children's stencils
@@ -289,79 +286,103 @@ __device__ __forceinline__ void mg_coarsen_cell(const MgDev& G, int l, int I) {
   G.rdg[C.off + I] = 1.0f / s[4];
 }
 
+// largest value of the wavefront, in every lane
+__device__ __forceinline__ double wave_fmax(double v) {
+  {
+    const long long b = __double_as_longlong(v);
+    const auto lo = __builtin_amdgcn_permlane32_swap((int)b, (int)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((int)(b >> 32), (int)(b >> 32), false, false);
+    v = fmax(__longlong_as_double(((long long)hi[0] << 32) | (unsigned int)lo[0]),
+             __longlong_as_double(((long long)hi[1] << 32) | (unsigned int)lo[1]));
+  }
+  {
+    const long long b = __double_as_longlong(v);
+    const auto lo = __builtin_amdgcn_permlane16_swap((int)b, (int)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((int)(b >> 32), (int)(b >> 32), false, false);
+    v = fmax(__longlong_as_double(((long long)hi[0] << 32) | (unsigned int)lo[0]),
+             __longlong_as_double(((long long)hi[1] << 32) | (unsigned int)lo[1]));
+  }
+  v = fmax(v, dpp_f64<0x128>(v));  // row_ror: lane l reads lane l + 8 of its row of 16, around
+  v = fmax(v, dpp_f64<0x124>(v));
+  v = fmax(v, dpp_f64<0x122>(v));
+  v = fmax(v, dpp_f64<0x121>(v));
+  return v;
+}
+__device__ __forceinline__ double lane_f64(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, l);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
 // Coarsest level (one workgroup): dense matrix and its explicit inverse by
-// Gauss-Jordan with partial pivoting on the augmented matrix [A | I], held in
-// LDS (MG_DENSE_MAX x 2 MG_DENSE_MAX doubles = 64 KB).  Per pivot column: one
-// wavefront finds the pivot (largest magnitude, first row on ties), the swap
-// is recorded, the pivot row scaled, and all other rows updated in parallel
-// from snapshots of the pivot row and column.
+// Gauss-Jordan with partial pivoting (largest magnitude, first row on ties).
+// Bound by the chain of a pivot step, 64 of them: column, search, quotient,
+// update, the next column.  So a step has one barrier: lane q of every
+// wavefront holds column q of its rows in registers, each wavefront searches
+// the pivot itself (swaps are recorded in perm, rows stay where they are) and
+// the updated matrix goes to the other of two copies in LDS, padded against
+// the column reads' bank conflicts.  The inverse grows in place: column c of
+// the pivot step holds the identity's column of the pivot row from then on,
+// with the values the augmented matrix [A | I] gets.  (The augmented form, the
+// search by shuffles in one wavefront and three barriers a step took 51 us for
+// a 20k-particle flume's coarsest level, this form 31.)
 __device__ __forceinline__ void mg_dense_block(const MgDev& G) {
-  __shared__ double A[MG_DENSE_MAX * 2 * MG_DENSE_MAX];
-  __shared__ double colc[MG_DENSE_MAX], prow[2 * MG_DENSE_MAX];
-  __shared__ int perm[MG_DENSE_MAX];  // row r of the swapped matrix is stored row perm[r]
-  __shared__ int piv;
+  constexpr int N = MG_DENSE_MAX, LD = N + 1, RW = N / (MG_DENSE_THREADS / 64);
+  __shared__ double A[2][N * LD];
+  __shared__ int rank[N];
   const MgLevel L = G.lev[G.nlev];
-  const int n = L.n, t = threadIdx.x, T = blockDim.x;
-  const int w2 = 2 * n;
+  const int n = L.n, t = threadIdx.x, q = t & 63;
+  const int r0 = __builtin_amdgcn_readfirstlane((t >> 6) * RW);  // this wavefront's rows
   const float* st = G.sten + 9 * L.off;
-  for (int e = t; e < n * w2; e += T) A[e] = 0.0;
+  for (int e = t; e < N * LD; e += MG_DENSE_THREADS) A[0][e] = 0.0;
   __syncthreads();
-  for (int I = t; I < n; I += T) {
+  for (int I = t; I < n; I += MG_DENSE_THREADS) {
     float v[9];  // every load before the first sum
 #pragma unroll
     for (int k = 0; k < 9; k++) v[k] = st[k * n + I];
     for (int k = 0; k < 9; k++) {
       const int J = mg_nbr(L, I, k);
-      if (J >= 0) A[I * w2 + J] += (double)v[k];
+      if (J >= 0) A[0][I * LD + J] += (double)v[k];
     }
-    A[I * w2 + n + I] = 1.0;
-    perm[I] = I;
   }
   __syncthreads();
-  // Row swaps are recorded in perm instead of moving the rows: the pivot
-  // search, its tie rule and every update are those of the swapped matrix,
-  // so the values are the same, with one barrier and one pass fewer per column.
+  double a[RW];
+#pragma unroll
+  for (int u = 0; u < RW; u++) a[u] = A[0][(r0 + u) * LD + q];
+  int perm = q;  // lane r: the stored row that is row r of the swapped matrix
   for (int c = 0; c < n; c++) {
-    if (t < 64) {
-      // lane r holds |A(r, c)| of swapped row r >= c (n <= 64 rows)
-      const bool cand = t >= c && t < n;
-      const int ph = cand ? perm[t] : 0;
-      double bv = cand ? fabs(A[ph * w2 + c]) : -1.0;
-      int br = t;
-      for (int off = 32; off >= 1; off >>= 1) {
-        const double ov = __shfl_down(bv, off, 64);
-        const int orow = __shfl_down(br, off, 64);
-        if (ov > bv || (ov == bv && orow < br)) { bv = ov; br = orow; }
-      }
-      if (t == 0) {
-        const int pc = perm[c], pb = perm[br];
-        perm[c] = pb;
-        perm[br] = pc;
-        piv = pb;
-      }
-    }
-    __syncthreads();
-    const int pr = piv;  // stored row of the pivot
-    const double pv = A[pr * w2 + c];
-    for (int e = t; e < w2; e += T) prow[e] = (pv != 0.0) ? A[pr * w2 + e] / pv : 0.0;
-    for (int r = t; r < n; r += T) colc[r] = A[r * w2 + c];
-    __syncthreads();
-    // thread t updates column t mod 2 MG_DENSE_MAX of stored rows t / (2 MG_DENSE_MAX),
-    // + T / (2 MG_DENSE_MAX), ... (no division in the loop)
-    {
-      const int q = t & (2 * MG_DENSE_MAX - 1), rs = T / (2 * MG_DENSE_MAX);
-      if (q < w2)
-        for (int r = t / (2 * MG_DENSE_MAX); r < n; r += rs)
-          A[r * w2 + q] = (r == pr) ? prow[q] : A[r * w2 + q] - colc[r] * prow[q];
+    const double* M = A[c & 1];
+    const double col = M[q * LD + c];     // stored row q
+    const double cp = M[perm * LD + c];   // swapped row q
+    const bool cand = q >= c && q < n;
+    const double key = cand ? fabs(cp) : -1.0;
+    const double big = wave_fmax(key);
+    const unsigned long long at = __ballot(cand && key == big);
+    const int br = at ? (int)__builtin_ctzll(at) : c;  // (no lane: every candidate is NaN)
+    const int pr = __builtin_amdgcn_readlane(perm, br), pc = __builtin_amdgcn_readlane(perm, c);
+    if (q == c) perm = pr;
+    else if (q == br) perm = pc;
+    const double pv = lane_f64(col, pr);
+    const double x = (q == c) ? 1.0 : M[pr * LD + q];
+    const double prow = (pv != 0.0) ? x / pv : 0.0;
+#pragma unroll
+    for (int u = 0; u < RW; u++) {
+      const double f = lane_f64(col, r0 + u);
+      a[u] = (r0 + u == pr) ? prow : ((q == c) ? 0.0 : a[u]) - f * prow;
+      A[(c + 1) & 1][(r0 + u) * LD + q] = a[u];
     }
     __syncthreads();
   }
-  // stored transposed, inv(r, cc) at [cc * n + r], so the coarse solve's
-  // threads (one per row r) read consecutive addresses
-  for (int e = t; e < n * n; e += T) {
-    const int cc = e / n, r = e - cc * n;
-    G.dense_inv[e] = A[perm[r] * w2 + n + cc];
-  }
+  // Lane c's perm is the pivot row of step c: row c of the inverse, and the
+  // identity's column that column c holds.  Stored transposed, inv(r, cc) at
+  // [cc * n + r], so the coarse solve's threads (one per row r) read
+  // consecutive addresses.
+  if (t < n) rank[perm] = t;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < RW; u++)
+    if (q < n && r0 + u < n) G.dense_inv[perm * n + rank[r0 + u]] = a[u];
 }
 
 // ---------------------------------------------------------------------
