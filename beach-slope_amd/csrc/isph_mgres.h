@@ -231,13 +231,22 @@ __global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
 // ---------------------------------------------------------------------
 // The first entries of a workgroup's rows stay on the chip for the launch: read
 // from memory, a row's three batches of entries are three dependent trips of
-// ~0.5 us in each of the six products of an iteration.  512 threads with a row
-// each have the registers for them (and for their FP64 values); 1,024 with a
-// row each keep the positions and FP16 values in LDS; several rows per thread
-// stream them.  An iteration took 42.0 us before and 38.0 after at 7,485 rows,
-// 42.6 and 37.5 at 22k, 64.6 and 61.7 at 137k, 74.6 and 72.5 at 207k.
+// ~0.5 us in each of the six products of an iteration, and above ~250k rows
+// the traffic itself is what bounds them.  512 threads with a row each have
+// the registers (for the FP64 values too); 1,024 threads keep positions and
+// FP16 values in the LDS that the window leaves: 22, 14 and 8 entries of each
+// row at 1, 2 and 3 rows per thread.  An iteration took 42.0 us before and
+// 38.0 after at 7,485 rows, 42.6 and 37.5 at 22k, 64.6 and 61.7 at 137k, 93.7
+// and 87.4 at 310k, 104.8 and 95.7 at 413k, 139.8 and 133.2 at 653k.
 constexpr int rs_reg_entries(int T, int R) { return T == 512 && R == 1 ? 24 : 0; }
-constexpr int rs_lds_entries(int T, int R) { return T * R == 1024 ? 22 : 0; }
+constexpr int rs_lds_entries(int T, int R) {
+  return T != 1024 ? 0 : R == 1 ? 22 : R == 2 ? 14 : 8;
+}
+// words of the window with the rows' r0, which the reductions' area shares
+constexpr int rs_work_words(int T, int R) {
+  const int area = 2 * 5 * (T / 256) * 192, window = rs_win(T, R) * T + R * T + RS_TAIL;
+  return area > window ? area : window;
+}
 template <int T, int R>
 struct RsEntries {
   static constexpr int KR = rs_reg_entries(T, R), KL = rs_lds_entries(T, R), K = KR + KL;
@@ -471,25 +480,26 @@ __device__ __forceinline__ bool rs_publish_wait(const ResDev& Q, int wg, int nbl
   int t = threadIdx.x;
   asm volatile("" : "+v"(t));
   const int wv = (t >> 6) & 3, l = t & 63, sub = t >> 8;
-  // tree j = k R + q of a block is summed by wavefront j mod 4 of its four;
-  // the other three leave their values in LDS
-#pragma unroll
-  for (int k = 0; k < NV; k++)
-#pragma unroll
-    for (int q = 0; q < R; q++) {
-      const int j = k * R + q, o = j & 3;
-      if (wv != o) area[(j * S4 + sub) * 192 + (wv < o ? wv : wv - 1) * 64 + l] = v[k][q];
-    }
-  __syncthreads();
+  // A block's trees are summed by its four wavefronts in turn, the other three
+  // leaving their values in LDS, the rows of a thread one after the other: the
+  // area (5 KB per four wavefronts for the five products) takes the place of
+  // the window, and what it leaves free holds row entries.
   unsigned long long* slots = glob(Q.slots);
   const int b0 = wg * Q.nbw;
 #pragma unroll
-  for (int k = 0; k < NV; k++)
+  for (int q = 0; q < R; q++) {
+    __syncthreads();  // the window's or the last values' readers are through
 #pragma unroll
-    for (int q = 0; q < R; q++) {
-      const int j = k * R + q, o = j & 3;
+    for (int k = 0; k < NV; k++) {
+      const int o = (k * R + q) & 3;
+      if (wv != o) area[(k * S4 + sub) * 192 + (wv < o ? wv : wv - 1) * 64 + l] = v[k][q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      const int o = (k * R + q) & 3;
       if (wv == o) {
-        const double* a = area + (j * S4 + sub) * 192 + l;
+        const double* a = area + (k * S4 + sub) * 192 + l;
         const double w0 = (o == 0) ? v[k][q] : a[0];
         const double w1 = (o == 1) ? v[k][q] : a[(o < 1 ? 0 : 1) * 64];
         const double w2 = (o == 2) ? v[k][q] : a[(o < 2 ? 1 : 2) * 64];
@@ -500,6 +510,7 @@ __device__ __forceinline__ bool rs_publish_wait(const ResDev& Q, int wg, int nbl
           ps_publish(&slots[2 * ((size_t)k * nblk + b0 + lb)], ep, s);
       }
     }
+  }
   if (t < 2 * NV) {
     const unsigned long long* p = glob(Q.mail) + wg * RS_MAIL + t;
     const float f = rs_wait(p, ep, bad, 0ull);
@@ -1002,9 +1013,9 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
   DevScalars* Sc = glob(D.sc);
   const int n = Sc->n, nblk = D.nblk, cap = D.cap;
   const int i0 = wg * Q.nbw * RED_BLOCK, i1 = min(n, min(nblk, (wg + 1) * Q.nbw) * RED_BLOCK);
-  double* area = lds;                      // 5 R S 192 doubles
-  double* res = lds + 5 * R * S4 * 192;
+  double* res = lds;
   volatile int* bad = reinterpret_cast<int*>(res + 6);
+  double* area = res + 8;  // 5 S4 192 doubles, in the window's place
   float* X = reinterpret_cast<float*>(res + 8);  // the window
   float* r0s = X + W * T;                  // r0 of the workgroup's rows
   if (t == 0) *bad = 0;
@@ -1044,7 +1055,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
 #pragma unroll
   for (int q = 0; q < R; q++)
     E[q].load(lidx, av16, aval, cap, max(row[q], 0), len[q], t,
-              reinterpret_cast<uint32_t*>(r0s + R * T + RS_TAIL) + q * E[0].KL * T);
+              reinterpret_cast<uint32_t*>(X) + rs_work_words(T, R) + q * E[0].KL * T);
   // window elements: chunk (uniform per wavefront), cell of the row; own
   // chunks hold the workgroup's rows at positions s0 * 64 + local row
   const int oc0 = i0 / PS_CHUNK, oc1 = (i1 + PS_CHUNK - 1) / PS_CHUNK;
@@ -1288,8 +1299,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
 
 template <int T, int R>
 __host__ __device__ inline int64_t rs_row_lds() {
-  return 8 * (5 * R * (T / 256) * 192 + 8) +
-         4 * (rs_win(T, R) * T + R * T + RS_TAIL + rs_lds_entries(T, R) * R * T);
+  return 8 * 8 + 4 * (rs_work_words(T, R) + rs_lds_entries(T, R) * R * T);
 }
 // whether the coarse workgroup can take level l0 and those below
 __host__ __device__ inline bool rs_coarse_fits(const MgDev& G, int l0) {
