@@ -179,10 +179,17 @@ __device__ __forceinline__ double lane0(double v) {
 // row per thread) t1, later r, of the workgroup's rows
 template <int T, int R>
 __host__ __device__ constexpr int ps_tree_doubles() { return 2 * R * (T / 256) * 192; }
+// row positions and values kept in LDS: what the window leaves of it
+constexpr int ps_lds_pos(int T, int R) { return T != 1024 ? 0 : R == 3 ? 16 : 22; }
+constexpr int ps_lds_val(int T, int R) { return T == 1024 && R == 1 ? 7 : 0; }
 template <int T, int R, int W>
 __host__ __device__ inline int64_t ps_lds_bytes(int nblk) {
-  const int64_t a = ps_tree_doubles<T, R>(), b = 2 * (int64_t)nblk;
-  return 8 * ((int64_t)W * T + (a > b ? a : b) + 2 * 256 + 2 + (R > 1 ? 0 : T));
+  const int64_t a = ps_tree_doubles<T, R>(), b = 2 * (int64_t)nblk, w = (int64_t)W * T;
+  const int64_t area = a > b ? a : b, own = 2 * 256 + 2 + (R > 1 ? 0 : T);
+  if (T == 1024)  // the area shares the window's place; row entries
+    return 8 * ((w > area ? w : area) + own + ps_lds_val(T, R) * R * T) +
+           4 * (ps_lds_pos(T, R) / 2 * R * T);
+  return 8 * (w + area + own);
 }
 
 // One word of reduction ep, polled until it carries the number; false when
@@ -243,7 +250,10 @@ __device__ __forceinline__ bool ps_reduce(const PersArg& Q, int nblk, int b0, un
                                           const double (&v)[NV][R], double* area, double* col,
                                           int* bad, double (&out)[NV], MID mid) {
   constexpr int S = T / 256;
-  const int t = threadIdx.x, wv = (t >> 6) & 3, l = t & 63, sub = t >> 8;
+  int t = threadIdx.x;
+  if (T == 1024) asm volatile("" : "+v"(t));  // (opaque: no addresses held over the iterations)
+  const int wv = (t >> 6) & 3, l = t & 63, sub = t >> 8;
+  if (T == 1024) __syncthreads();  // the area is in the window's place
   // tree j = k R + q of a block is summed by wavefront j mod 4 of its four;
   // the other three leave their values in LDS
 #pragma unroll
@@ -401,6 +411,54 @@ __device__ __forceinline__ double ps_row(const PsRow<KR>& M, const uint32_t* idx
   if (k0 < Lm) acc = ps_entries<U, false>(ip, vp, ls, cap, i, k0, L, Lm, win, acc);
   return acc;
 }
+// The same with the first KP positions and KV values of every row in LDS
+// (lw, lv: those of this row), where 1,024 threads have no registers for them:
+// what an iteration streams is most of its time there.  Without / with them, us
+// per iteration: 20.3 / 19.0 at 136k rows, 26.5 / 20.9 at 207k, 39.3 / 36.9 at
+// 307k, 44.9 / 40.5 at 409k, 63.0 / 59.0 at 653k.
+template <int U, int KP, int KV, int T>
+__device__ __forceinline__ double ps_row_lds(const uint32_t* lw, const double* lv, int t,
+                                             const uint32_t* idx, int ls, const double* val,
+                                             int cap, unsigned i, int L, int Lm,
+                                             const double* win) {
+  double acc = 0.0;
+  const double* vp = val + (size_t)KV * cap;
+#pragma unroll
+  for (int k0 = 0; k0 < KP; k0 += U) {
+    if (k0 >= Lm) break;
+    double v[U], g[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (k0 + u >= KP) continue;
+      if (k0 + u < KV) {
+        v[u] = lv[(k0 + u) * T + t];
+      } else {
+        v[u] = (k0 + u < Lm) ? *ps_at(vp, i) : 0.0;
+        vp += cap;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (k0 + u >= KP) continue;
+      const uint32_t w = lw[((k0 + u) / 2) * T + t];
+      g[u] = win[(u & 1) ? (w >> 16) : (w & 0xffffu)];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (k0 + u >= KP) continue;
+      const double a = acc + v[u] * g[u];
+      acc = (k0 + u < L) ? a : acc;
+    }
+  }
+  const uint32_t* ip = idx + (size_t)(KP / 2) * ls;
+  int k0 = KP;
+#pragma unroll 1
+  for (; k0 + U <= Lm; k0 += U)
+    acc = ps_entries<U, true>(ip, vp, ls, cap, i, k0, L, Lm, win, acc);
+  if (k0 < Lm) acc = ps_entries<U, false>(ip, vp, ls, cap, i, k0, L, Lm, win, acc);
+  return acc;
+}
+
 __device__ __forceinline__ int wave_max(int v) {
 #pragma unroll
   for (int s = 32; s >= 1; s >>= 1) v = max(v, __shfl_xor(v, s, 64));
@@ -419,7 +477,9 @@ template <int T, int R, int W, int KR>
 __global__ void __launch_bounds__(T) k_bicg_resident(Dev D, PersArg Q, int iters, unsigned ep) {
   constexpr int S = T / 256;
   constexpr bool ONE = R == 1;
-  constexpr int U = ONE ? 8 : 4;   // row entries in flight per thread
+  // row entries in flight per thread (several rows: 4, 6, 8 took 37.8, 36.9,
+  // 36.4 us an iteration at 307k rows and 59.0, 59.0, 59.2 at 653k)
+  constexpr int U = ONE ? 8 : 6;
   constexpr int WR = ONE ? W : 1;  // window elements in registers
   extern __shared__ double ps_lds[];
   __shared__ int bad_[1];
@@ -429,9 +489,14 @@ __global__ void __launch_bounds__(T) k_bicg_resident(Dev D, PersArg Q, int iters
   const int n = Sc->n, nblk = D.nblk, cap = D.cap, b0 = wg * Q.nbw;
   const int ta = ps_tree_doubles<T, R>();
   double* win = ps_lds;
-  double* area = win + W * T;
-  double* col = area + (ta > 2 * nblk ? ta : 2 * nblk);
+  // 1,024 threads: the reductions' area in the window's place, for row entries
+  const int tn = ta > 2 * nblk ? ta : 2 * nblk;
+  double* area = (T == 1024) ? win : win + W * T;
+  double* col = (T == 1024) ? win + (W * T > tn ? W * T : tn) : area + tn;
   double* own = col + 514;  // one row per thread: its t1, then r
+  constexpr int KP = ps_lds_pos(T, R), KV = ps_lds_val(T, R);
+  double* lv = own + (ONE ? T : 0);
+  uint32_t* lw = reinterpret_cast<uint32_t*>(lv + KV * R * T);
   double rho = Sc->rho;
   const double bnorm = Sc->bnorm, tol = D.P.tol;
   const int max_iter = D.P.max_iter;
@@ -464,6 +529,13 @@ __global__ void __launch_bounds__(T) k_bicg_resident(Dev D, PersArg Q, int iters
         M[q].v[k] = (k < len[q]) ? D.aval[k * cap + i] : 0.0;
         if (k % 2 == 0) M[q].w[k / 2] = (k < len[q]) ? Q.lidx[(size_t)(k / 2) * Q.ls + i] : 0u;
       }
+#pragma unroll
+      for (int k = 0; k < KP; k += 2)
+        lw[(q * KP / 2 + k / 2) * T + t] =
+            (k < len[q]) ? Q.lidx[(size_t)(k / 2) * Q.ls + i] : 0u;
+#pragma unroll
+      for (int k = 0; k < KV; k++)
+        lv[(q * KV + k) * T + t] = (k < len[q]) ? D.aval[k * cap + i] : 0.0;
     }
 #pragma unroll
     for (int w = 0; w < W; w++) {
@@ -554,6 +626,13 @@ __global__ void __launch_bounds__(T) k_bicg_resident(Dev D, PersArg Q, int iters
       for (int w = 0; w < WR; w++)
         if (wc[w] >= oc0 && wc[w] < oc1) o[w] = own[(wc[w] - oc0) * PS_CHUNK + l];
     };
+    auto product = [&](int q) -> double {
+      if constexpr (KP > 0)
+        return ps_row_lds<U, KP, KV, T>(lw + q * KP / 2 * T, lv + q * KV * T, t, Q.lidx, Q.ls,
+                                        D.aval, cap, row[q], len[q], lmx[q], win);
+      else
+        return ps_row<U, KR>(M[q], Q.lidx, Q.ls, D.aval, cap, row[q], len[q], lmx[q], win);
+    };
     // t1 = A p ; alpha = rho / (t1 . rh)
     if constexpr (ONE) {
 #pragma unroll
@@ -567,9 +646,7 @@ __global__ void __launch_bounds__(T) k_bicg_resident(Dev D, PersArg Q, int iters
     for (int q = 0; q < R; q++) {
       __builtin_amdgcn_sched_barrier(0);  // one row's loads in registers at a time
       if (!ONE) rh[q] = (row[q] >= 0) ? *ps_at(D.rh, row[q]) : 0.0;
-      t1[q] = (row[q] >= 0)
-                  ? ps_row<U, KR>(M[q], Q.lidx, Q.ls, D.aval, cap, row[q], len[q], lmx[q], win)
-                  : 0.0;
+      t1[q] = (row[q] >= 0) ? product(q) : 0.0;
       if constexpr (ONE) {
         own[t] = t1[q];
         put(Q.tlo, Q.thi, q, ep, t1[q]);
@@ -596,9 +673,7 @@ __global__ void __launch_bounds__(T) k_bicg_resident(Dev D, PersArg Q, int iters
 #pragma unroll
     for (int q = 0; q < R; q++) {
       __builtin_amdgcn_sched_barrier(0);
-      t2[q] = (row[q] >= 0)
-                  ? ps_row<U, KR>(M[q], Q.lidx, Q.ls, D.aval, cap, row[q], len[q], lmx[q], win)
-                  : 0.0;
+      t2[q] = (row[q] >= 0) ? product(q) : 0.0;
       v2[0][q] = (row[q] >= 0) ? t2[q] * r[q] : 0.0;
       v2[1][q] = (row[q] >= 0) ? t2[q] * t2[q] : 0.0;
     }

@@ -68,15 +68,16 @@ def test_resident_solve_equals_launches(pkg, cases, nx, ny, iters, precision):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("nx,ny", [(200, 40), (1400, 100)])
-def test_rows_longer_than_those_kept_on_the_chip(pkg, cases, nx, ny):
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nx,ny", [(200, 40), (1400, 100), (2200, 160)])
+def test_rows_longer_than_those_kept_on_the_chip(pkg, cases, nx, ny, precision):
     """Fluid pressed together by a quarter: rows of more than 24 entries, whose
-    ends the precision solve reads from memory."""
+    ends the solves read from memory."""
     c = _tank(cases, nx, ny)
     fl = c.parts["tid"] == 3
     x0 = c.parts["x"][fl].min()
     c.parts["x"][fl] = x0 + 0.75 * (c.parts["x"][fl] - x0)
-    c.params.update(precision=1, tol=1e-10, max_iter=60, max_outer=2)
+    c.params.update(precision=precision, tol=1e-10, max_iter=60, max_outer=2)
 
     def run(s):
         rc, st = s.step(1, check=False)
