@@ -31,9 +31,8 @@
 #include "isph_batch.h"
 #include "isph_persist.h"
 
-// window elements per thread
-constexpr int rs_win(int T, int R) { return T == 512 && R > 1 ? 12 : 6; }
-#define RS_WCAP (6 * 1024 / PS_CHUNK)  // window chunks of a workgroup at most
+#define RS_W 6                      // window elements per thread
+#define RS_WCAP (RS_W * 1024 / PS_CHUNK)  // window chunks of a workgroup at most
 // Threads of the coarse workgroup's first level at most, four per unknown of
 // the next; their stencils stay in registers.  A level more on the row workgroups costs two more hops of
 // ~1.2 us a V-cycle, a level of 1-4 unknowns per thread more in the one
@@ -42,6 +41,13 @@ constexpr int rs_win(int T, int R) { return T == 512 && R > 1 ? 12 : 6; }
 // and 74.7.
 #define RS_CO_MAX 1024
 #define RS_PER(T) ((RS_CO_MAX + (T)-1) / (T))
+// Cells of its window that a thread forms the level-1 correction of, with one
+// row per thread; 0: the cells' own workgroups do, and send it.  Forming it in
+// every window repeats work and saves an exchange: 45.7 us an iteration with
+// the exchange, 43.4 without at 22k rows, 61.8 and 57.5 at 137k, 72.2 and 67.3
+// at 207k; with two and three rows per thread 88.3 and 92.1 at 307k, 133.1 and
+// 134.1 at 653k.
+constexpr int rs_cells(int R) { return R == 1 ? 2 : 0; }
 #define RS_MAIL 16                  // words of a workgroup's mail line
 #define RS_TAIL 256                 // rows of the next workgroups in a workgroup's last cell
 
@@ -134,7 +140,7 @@ template <int T, int R>
 __global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
   __shared__ uint16_t map[PS_MAX_CHUNKS];
   __shared__ int cnt[T];
-  const int wcap = rs_win(T, R) * T / PS_CHUNK;
+  const int wcap = RS_W * T / PS_CHUNK;
   const int s = rs_locate(rs, B.S, blockIdx.x), t = threadIdx.x;
   const ResDev& Q = rs[s];
   const Dev& D = B.devs[s];
@@ -208,6 +214,20 @@ __global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
       map[c] = (uint16_t)pos++;
     }
   if (t == 0) Q.wcnt[2 * wg] = total;
+  if (rs_cells(R) > 0) {
+    // the window's cells (a chunk's rows lie in cell order), of which
+    // rs_rows_solve takes rs_cells per thread
+    if (t == 0) cnt[0] = 0;
+    __syncthreads();
+    int mine = 0;
+    for (int p = t; p < total * PS_CHUNK; p += T) {
+      const int g = Q.wlist[(size_t)wg * RS_WCAP + p / PS_CHUNK] * PS_CHUNK + p % PS_CHUNK;
+      if (g < n && (g % PS_CHUNK == 0 || D.cell[g] != D.cell[g - 1])) mine++;
+    }
+    atomicAdd(&cnt[0], mine);
+    __syncthreads();
+    if (cnt[0] > rs_cells(R) * T && t == 0) atomicOr(&D.sc->counter[PS_FLAG_WIN], 1u);
+  }
   __syncthreads();
   for (int i = i0 + t; i < i1; i += T) {
     const int L = alen[i];
@@ -244,7 +264,7 @@ constexpr int rs_lds_entries(int T, int R) {
 }
 // words of the window with the rows' r0, which the reductions' area shares
 constexpr int rs_work_words(int T, int R) {
-  const int area = 2 * 5 * (T / 256) * 192, window = rs_win(T, R) * T + R * T + RS_TAIL;
+  const int area = 2 * 5 * (T / 256) * 192, window = RS_W * T + R * T + RS_TAIL;
   return area > window ? area : window;
 }
 template <int T, int R>
@@ -667,41 +687,47 @@ __device__ __forceinline__ void rs_down(const RsMg& M, const ResDev& Q, int wg, 
   }
 }
 
-template <int T>
-__device__ __forceinline__ void rs_up(const RsMg& M, const ResDev& Q, int wg, int t,
-                                      int l, unsigned tag, volatile int* bad) {
-  const MgLevel L = rs_level(M.lev, l), C = rs_level(M.lev, l + 1);
+// value of level-L cell I after the correction from level C and the
+// post-smoothing sweep, from the words of both levels
+__device__ __forceinline__ float rs_up_cell(const RsMg& M, const ResDev& Q, const MgLevel& L,
+                                            const MgLevel& C, int I, unsigned tag,
+                                            volatile int* bad) {
   const float w = M.w, c = M.c;
   const float* st = M.sten + 9 * (size_t)L.off;
   const float* rd = M.rdg + L.off;
   const unsigned long long* bw = glob(Q.bw) + L.off;
-  unsigned long long* ew = glob(Q.ew);
-  const unsigned long long* ec = ew + C.off;
-  const int I0 = rs_part(L.n, wg, Q.G), I1 = rs_part(L.n, wg + 1, Q.G);
-  for (int I = I0 + t; I < I1; I += T) {
-    const int cj = I / L.ny, ci = I - cj * L.ny;
-    const int P = (cj >> 1) * C.ny + (ci >> 1), q = (ci & 1) | ((cj & 1) << 1);
-    const unsigned has = rs_has(L, ci, cj);
-    float xv[9], xc[9];
-    // (the words of this level are those that the way down polled)
-    rs_poll<9>(tag, bad, [&](int k) { return ld_word(bw, rs_nbr(has, I, L.ny, k)); }, xv);
-    const float bI = xv[4], rI = *ps_at(rd, I);
+  const unsigned long long* ec = glob(Q.ew) + C.off;
+  const int cj = I / L.ny, ci = I - cj * L.ny;
+  const int P = (cj >> 1) * C.ny + (ci >> 1), q = (ci & 1) | ((cj & 1) << 1);
+  const unsigned has = rs_has(L, ci, cj);
+  float xv[9], xc[9];
+  // (the words of this level are those that the way down polled)
+  rs_poll<9>(tag, bad, [&](int k) { return ld_word(bw, rs_nbr(has, I, L.ny, k)); }, xv);
+  const float bI = xv[4], rI = *ps_at(rd, I);
 #pragma unroll
-    for (int k = 0; k < 9; k++) xv[k] = (w * xv[k]) * *ps_at(rd, rs_nbr(has, I, L.ny, k));
-    float sv[9];
+  for (int k = 0; k < 9; k++) xv[k] = (w * xv[k]) * *ps_at(rd, rs_nbr(has, I, L.ny, k));
+  float sv[9];
 #pragma unroll
-    for (int k = 0; k < 9; k++) sv[k] = *ps_at(st + (size_t)k * L.n, I);
-    rs_poll<9>(tag, bad, [&](int k) { return ld_word(ec, rs_par(has, P, q, C.ny, k)); }, xc);
-    float acc = 0.0f;
+  for (int k = 0; k < 9; k++) sv[k] = *ps_at(st + (size_t)k * L.n, I);
+  rs_poll<9>(tag, bad, [&](int k) { return ld_word(ec, rs_par(has, P, q, C.ny, k)); }, xc);
+  float acc = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 9; k++) {
-      xv[k] = xv[k] + c * xc[k];
-      const float tk = sv[k] * xv[k];
-      if ((has >> k) & 1) acc = acc + tk;
-    }
-    const float x1 = xv[4];
-    rs_put(ps_at(ew + L.off, I), tag, x1 + (w * (bI - acc)) * rI);
+  for (int k = 0; k < 9; k++) {
+    xv[k] = xv[k] + c * xc[k];
+    const float tk = sv[k] * xv[k];
+    if ((has >> k) & 1) acc = acc + tk;
   }
+  return xv[4] + (w * (bI - acc)) * rI;
+}
+
+template <int T>
+__device__ __forceinline__ void rs_up(const RsMg& M, const ResDev& Q, int wg, int t,
+                                      int l, unsigned tag, volatile int* bad) {
+  const MgLevel L = rs_level(M.lev, l), C = rs_level(M.lev, l + 1);
+  unsigned long long* ew = glob(Q.ew) + L.off;
+  const int I0 = rs_part(L.n, wg, Q.G), I1 = rs_part(L.n, wg + 1, Q.G);
+  for (int I = I0 + t; I < I1; I += T)
+    rs_put(ps_at(ew, I), tag, rs_up_cell(M, Q, L, C, I, tag, bad));
 }
 
 // ---------------------------------------------------------------------
@@ -1008,7 +1034,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
                                               const MgLevel* lev,
                                               int wg, int iters, unsigned v0, unsigned ep,
                                               double* lds) {
-  constexpr int S4 = T / 256, W = rs_win(T, R);
+  constexpr int S4 = T / 256, W = RS_W;
   const int t = threadIdx.x, l = t & 63;
   DevScalars* Sc = glob(D.sc);
   const int n = Sc->n, nblk = D.nblk, cap = D.cap;
@@ -1019,6 +1045,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
   float* X = reinterpret_cast<float*>(res + 8);  // the window
   float* r0s = X + W * T;                  // r0 of the workgroup's rows
   if (t == 0) *bad = 0;
+  float* E1 = X + rs_work_words(T, R) + rs_lds_entries(T, R) * R * T;  // corrections of the window's cells
   unsigned long long* x0w = glob(Q.x0w);
   unsigned long long* phw = glob(Q.phw);
   unsigned long long* r0w = glob(Q.r0w);
@@ -1066,6 +1093,47 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
     wc[w] = __builtin_amdgcn_readfirstlane((s < wn) ? wl[s] : -1);
     const int g = wc[w] * PS_CHUNK + l;
     wk[w] = (wc[w] >= 0 && g < n) ? cell[g] : -1;
+  }
+  // One row per thread: the level-1 corrections of the window's cells are formed
+  // here rather than by the cells' workgroups, which saves an exchange.  Thread
+  // t has cells t, t + T, ... of the window's; a window element keeps its
+  // cell's number (in wk).
+  constexpr int NC = rs_cells(R);
+  int uc[NC ? NC : 1];
+  if constexpr (NC > 0) {
+    int* slot_cnt = reinterpret_cast<int*>(X);                       // first rows per chunk
+    int* list = slot_cnt + RS_WCAP;                                  // the window's cells
+    bool first[W];
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+      const int before = __shfl_up(wk[w], 1, 64);
+      first[w] = wk[w] >= 0 && (l == 0 || before != wk[w]);
+      const unsigned long long m = __ballot(first[w]);
+      if (l == 0) slot_cnt[w * (T / PS_CHUNK) + t / PS_CHUNK] = (int)__popcll(m);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+      const int s = w * (T / PS_CHUNK) + t / PS_CHUNK;
+      int base = 0;
+      for (int k = 0; k < s; k++) base += slot_cnt[k];
+      const unsigned long long m = __ballot(first[w]);
+      const int u = base + (int)__popcll(m & (~0ull >> (63 - l))) - 1;
+      if (first[w]) list[u] = wk[w];
+      if (wk[w] >= 0) wk[w] = u;
+    }
+    if (t == 0) slot_cnt[0] = 0;
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < W; w++) total = max(total, wk[w] + 1);
+    atomicMax(&slot_cnt[0], total);
+    __syncthreads();
+    total = slot_cnt[0];
+#pragma unroll
+    for (int j = 0; j < NC; j++) uc[j] = (t + j * T < total) ? list[t + j * T] : -1;
+    __syncthreads();
   }
   // cells whose first row is here, with the empty ones up to the next
   // workgroup's first; rows of a cell begun earlier are sent to its workgroup
@@ -1116,6 +1184,8 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
       for (int q = 0; q < R; q++) asm volatile("" : "+v"(row[q]));
 #pragma unroll
       for (int w = 0; w < W; w++) asm volatile("" : "+v"(wk[w]));
+#pragma unroll
+      for (int j = 0; j < NC; j++) asm volatile("" : "+v"(uc[j]));
       const int l = t & 63;
       // ---- V-cycle of v = p (half 0) or s, which is in r (half 1)
       float v[R];
@@ -1132,17 +1202,14 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
         auto other = [&](int w) {
           return wc[w] >= 0 && (wc[w] < oc0 || wc[w] >= oc1) && wk[w] >= 0;
         };
+        float e[W];
+        rs_poll<W>(tag, bad, [&](int w) {
+          return other(w) ? ld_word(words + (int64_t)wc[w] * PS_CHUNK, l)
+                          : (unsigned long long)tag << 32;
+        }, e);
 #pragma unroll
-        for (int w0 = 0; w0 < W; w0 += 6) {
-          float e[6];
-          rs_poll<6>(tag, bad, [&](int w) {
-            return other(w0 + w) ? ld_word(words + (int64_t)wc[w0 + w] * PS_CHUNK, l)
-                                 : (unsigned long long)tag << 32;
-          }, e);
-#pragma unroll
-          for (int w = 0; w < 6; w++)
-            if (other(w0 + w)) X[(w0 + w) * T + t] = e[w];
-        }
+        for (int w = 0; w < W; w++)
+          if (other(w)) X[w * T + t] = e[w];
       };
       // x += alpha ph + omega sh of the iteration before, while x0 is on its
       // way (nothing of the iteration waits for it)
@@ -1196,20 +1263,31 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
         }
       }
       for (int lv = 1; lv <= Q.m; lv++) rs_down<T>(H, Q, wg, t, lv, tag, bad);
-      for (int lv = Q.m; lv >= 1; lv--) rs_up<T>(H, Q, wg, t, lv, tag, bad);
-      // x1 = x0 + c e1 over the window; one wavefront waits for the first
-      // corrections before the others read theirs
-      if (t < 64 && wk[0] >= 0) (void)rs_wait(ps_at(e1w, wk[0]), tag, bad, 0ull);
-      __syncthreads();
+      for (int lv = Q.m; lv > (NC ? 1 : 0); lv--) rs_up<T>(H, Q, wg, t, lv, tag, bad);
+      // x1 = x0 + c e1 over the window
+      if constexpr (NC > 0) {
+        const MgLevel C1 = rs_level(lev, Q.m ? 2 : 1);
 #pragma unroll
-      for (int w0 = 0; w0 < W; w0 += 6) {
-        float e[6];
-        rs_poll<6>(tag, bad, [&](int w) {
-          return wk[w0 + w] >= 0 ? ld_word(e1w, wk[w0 + w]) : (unsigned long long)tag << 32;
+        for (int j = 0; j < NC; j++)
+          if (uc[j] >= 0)
+            E1[t + j * T] = Q.m ? rs_up_cell(H, Q, L1, C1, uc[j], tag, bad)
+                                : rs_wait(ps_at(e1w, uc[j]), tag, bad, 0ull);
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < W; w++)
+          if (wk[w] >= 0) X[w * T + t] = X[w * T + t] + mc * E1[wk[w]];
+      } else {
+        // one wavefront waits for the first corrections before the others read
+        // theirs
+        if (t < 64 && wk[0] >= 0) (void)rs_wait(ps_at(e1w, wk[0]), tag, bad, 0ull);
+        __syncthreads();
+        float e[W];
+        rs_poll<W>(tag, bad, [&](int w) {
+          return wk[w] >= 0 ? ld_word(e1w, wk[w]) : (unsigned long long)tag << 32;
         }, e);
 #pragma unroll
-        for (int w = 0; w < 6; w++)
-          if (wk[w0 + w] >= 0) X[(w0 + w) * T + t] = X[(w0 + w) * T + t] + mc * e[w];
+        for (int w = 0; w < W; w++)
+          if (wk[w] >= 0) X[w * T + t] = X[w * T + t] + mc * e[w];
       }
       __syncthreads();
       // x = x1 + w (v - A x1) d
@@ -1299,7 +1377,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
 
 template <int T, int R>
 __host__ __device__ inline int64_t rs_row_lds() {
-  return 8 * 8 + 4 * (rs_work_words(T, R) + rs_lds_entries(T, R) * R * T);
+  return 8 * 8 + 4 * (rs_work_words(T, R) + rs_lds_entries(T, R) * R * T + rs_cells(R) * T);
 }
 // whether the coarse workgroup can take level l0 and those below
 __host__ __device__ inline bool rs_coarse_fits(const MgDev& G, int l0) {
