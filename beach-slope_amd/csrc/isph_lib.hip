@@ -1490,9 +1490,11 @@ static int bicg_loop(isph_ctx* c, const ResPlan* plan, int* iters_out, int* brk_
   return 0;
 }
 
-// the resident solve's flags
-__global__ void k_res_clear(Dev D) {
-  if (blockIdx.x == 0 && threadIdx.x < 4) D.sc->counter[threadIdx.x] = 0u;
+// ||b|| from its square, and the resident solve's flags
+__global__ void k_res_begin(Dev D, const double* bn2) {
+  if (blockIdx.x != 0) return;
+  if (threadIdx.x < 4) D.sc->counter[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) D.sc->bnorm = sqrt(*bn2);
 }
 
 static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
@@ -1510,21 +1512,31 @@ static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
     int rc = bh_solve(c->self_batch, &st);
     if (rc) return rc;
   } else {
-    {
-      long long nnz = 0;
-      HIPCHK(c, hipMemcpyAsync(&nnz, &c->D.sc->nnz, sizeof nnz, hipMemcpyDeviceToHost, c->stream));
-      HIPCHK(c, hipStreamSynchronize(c->stream));
-      st.nnz = (double)nnz;
-    }
-    // ||b||
+    // ||b||, the set-up and the start residual, read back together
     RLAUNCH(k_dot, n, c->D, c->D.b, c->D.b);
     FINALIZE_OUT(FIN_DOT, n, c->d_bn2);
-    double bn2 = 0;
-    HIPCHK(c, hipMemcpyAsync(&bn2, c->d_bn2, 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const double bnorm = std::sqrt(bn2);
+    hipLaunchKernelGGL(k_res_begin, dim3(1), dim3(64), 0, c->stream, c->D, c->d_bn2);
+    // kernel timing brackets launches, so it takes the launch-per-phase form
+    ResPlan plan;
+    bool resident = !c->prof && res_plan(c->D.nblk, &plan);
+    if (resident) {
+      PersArg& Q = c->ps;
+      auto words = [](double* p) { return reinterpret_cast<unsigned long long*>(p); };
+      Q.tlo = words(c->D.t1);
+      Q.thi = words(c->D.t2);
+      Q.rlo = words(c->D.sv);
+      Q.lidx = c->D.aoff;
+      Q.ls = c->D.cap;
+      HIPCHK(c, res_setup(plan, c->D, Q, c->stream));
+    }
+    RLAUNCH(k_bicg_init, n, c->D);
+    FINALIZE(FIN_INIT, n);
+    DevScalars s;
+    int rc = read_scalars(c, &s);
+    if (rc) return rc;
+    st.nnz = (double)s.nnz;
+    const double bnorm = s.bnorm;
     st.bnorm = bnorm;
-    HIPCHK(c, hipMemcpy(&c->D.sc->bnorm, &bnorm, 8, hipMemcpyHostToDevice));
     if (bnorm == 0.0 || !std::isfinite(bnorm)) {
       if (bnorm == 0.0) {
         HIPCHK(c, hipMemsetAsync(c->D.sol, 0, 8 * (size_t)c->cap, c->stream));
@@ -1532,25 +1544,6 @@ static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
       }
       st.rel_residual = (bnorm == 0.0) ? 0.0 : bnorm;
     } else {
-      // kernel timing brackets launches, so it takes the launch-per-phase form
-      ResPlan plan;
-      bool resident = !c->prof && res_plan(c->D.nblk, &plan);
-      hipLaunchKernelGGL(k_res_clear, dim3(1), dim3(64), 0, c->stream, c->D);
-      if (resident) {
-        PersArg& Q = c->ps;
-        auto words = [](double* p) { return reinterpret_cast<unsigned long long*>(p); };
-        Q.tlo = words(c->D.t1);
-        Q.thi = words(c->D.t2);
-        Q.rlo = words(c->D.sv);
-        Q.lidx = c->D.aoff;
-        Q.ls = c->D.cap;
-        HIPCHK(c, res_setup(plan, c->D, Q, c->stream));
-      }
-      RLAUNCH(k_bicg_init, n, c->D);
-      FINALIZE(FIN_INIT, n);
-      DevScalars s;
-      int rc = read_scalars(c, &s);
-      if (rc) return rc;
       if (s.counter[PS_FLAG_WIN]) resident = false;
       int it = 0, brk = 0, conv = s.conv, restarts = 0;
       double rel = s.rel;
