@@ -28,8 +28,9 @@ solver's kernels (the two SpMVs, the V-cycle's level-0 passes, level-1
 restriction, cell-level down and up passes and coarse workgroup, and the
 dot-product finalizes; together ~90% of a step's kernel time) are timed with
 HIP events on the context's stream over as many steps again, right after
-the timed region (the events cost ~10% of a step, so the timed region runs
-without them), and the kernel function with the most time per step (all
+the timed region (the timed region runs without them: its solves are one
+resident launch each, and with the events on they run as a launch per
+phase), and the kernel function with the most time per step (all
 its launches: both applications of the V-cycle, every cell level) is
 reported, with its algorithmic bytes per launch (bytes_model) over its mean
 launch time.  Its

@@ -284,7 +284,8 @@ int isph_load_system(isph_ctx *ctx, int32_t n, const int32_t *row_len,
  * No counterpart in the reference (a single-scenario program); this is the
  * batched configuration's entry.  The contexts keep their own state; while
  * they belong to a batch they share one stream, and the PPE solves of the
- * precision-form contexts run as one set of launches over all of them.  A
+ * precision-form contexts run as one set of launches over all of them (one
+ * resident launch up to some 780,000 rows together).  A
  * scenario's results are the same as when it is stepped alone.  Destroy the
  * batch before any of its contexts.  isph_batch_step returns the worst
  * non-fatal solve code (ISPH_ENOCONV) over the scenarios and steps;
@@ -311,7 +312,8 @@ int isph_batch_autotune(isph_batch *b, int32_t trials, int32_t *shape, double *u
 
 /* ---- kernel timing (HIP events on the context's stream) ----
  * When enabled, every launch of the solver's timed kernels is bracketed by
- * a pair of HIP events; isph_prof_read returns the summed event time and the
+ * a pair of HIP events (the solves then run as a launch per phase rather than
+ * as one resident launch; results are the same); isph_prof_read returns the summed event time and the
  * launch count per kernel (launches after the solve has finished are left
  * out).  kernel: "spmv_p" (t = A p), "spmv_s" (t = A s) of the FP64 form;
  * "spmv_p32", "spmv_s32" (t1 = A ph, t2 = A sh), "mg_pre0", "mg_post0" (the
@@ -327,7 +329,8 @@ int isph_prof_read(isph_ctx *ctx, const char *kernel, double *total_ms,
  * Times the particle kernels below on the context's current state in each
  * of their launch shapes (trials launches each, HIP events on its stream)
  * and launches each in its fastest shape from then on.  Shapes: 0, 1, 2 =
- * one thread per particle in blocks of 64, 128, 256 threads; for the
+ * one thread per particle (eight where there are few particles) in blocks of
+ * 64, 128, 256 threads; for the
  * neighbour search also 3, 4 = one workgroup per tile of 4 (8) cells of a
  * cell column on 128 (256) threads, the tile's neighbourhood staged in LDS.
  * Results do not depend on the shape.  Call it at a step boundary (after
