@@ -426,7 +426,7 @@ __device__ __forceinline__ void block_tree_n(double (&v)[N], double* lds) {
 // maxima over a block of two non-negative double bit patterns (valid in
 // thread 0); every thread of the block must call it
 __device__ __forceinline__ void block_max2_u64(unsigned long long& a, unsigned long long& b) {
-  __shared__ unsigned long long wa[RED_BLOCK / 64], wb[RED_BLOCK / 64];
+  __shared__ unsigned long long wa[16], wb[16];
 #pragma unroll
   for (int s = 32; s >= 1; s >>= 1) {
     const unsigned long long oa = __shfl_xor(a, s, 64), ob = __shfl_xor(b, s, 64);

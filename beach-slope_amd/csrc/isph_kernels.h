@@ -331,7 +331,7 @@ __global__ void k_rebin_finish(Dev D, int ncell) {
 }
 
 // ---------------------------------------------------------------------
-// exclusive scan of int32 (bins -> bin starts), three passes
+// exclusive scan of int32 (bins -> bin starts): tiles, then the tiles' offsets
 // ---------------------------------------------------------------------
 #define SCAN_ITEMS 4
 #define SCAN_TILE (256 * SCAN_ITEMS)
@@ -387,13 +387,26 @@ __device__ __forceinline__ void scan_sums_body(int32_t* tile_sums, int ntiles, i
   }
   if (t == 0 && total_out) *total_out = carry;
 }
-__global__ void k_scan_sums(int32_t* tile_sums, int ntiles, int32_t* total_out) {
-  scan_sums_body(tile_sums, ntiles, total_out);
-}
-
-__global__ void k_scan_add(int32_t* out, const int32_t* tile_sums, int len) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx < len) out[idx] += tile_sums[idx / SCAN_TILE];
+// Adds the sums of the tiles before it to a tile, which each workgroup sums for
+// itself: at 200 tiles (653k particles) that is one load a thread, and the scan
+// is a launch shorter (offsets and addition 2.6 + 2.4 us at 22k particles, 4.7 + 4.9
+// at 653k as two launches; 3.2 and 4.8 as one).
+__global__ void __launch_bounds__(256) k_scan_add(int32_t* out, const int32_t* tile_sums,
+                                                  int len) {
+  __shared__ int32_t s[4];
+  const int t = threadIdx.x, tile = blockIdx.x;
+  int32_t a = 0;
+  for (int k = t; k < tile; k += 256) a += tile_sums[k];
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) a += __shfl_xor(a, m, 64);
+  if ((t & 63) == 0) s[t >> 6] = a;
+  __syncthreads();
+  a = (s[0] + s[1]) + (s[2] + s[3]);
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; k++) {
+    const int idx = tile * SCAN_TILE + k * 256 + t;
+    if (idx < len) out[idx] += a;
+  }
 }
 
 // ---------------------------------------------------------------------
@@ -1314,29 +1327,33 @@ __global__ void __launch_bounds__(256) k_comp_vel(Dev D) {
 // buffer particle, whose slot the reference reads stale).  With init the
 // velocities count as 0 and empty cells are cleared: the state before the
 // first step.  Each block of 256 cells leaves the maxima over its cells for
-// timestep (one thread per cell; non-negative doubles compare as their bits).
-__device__ __forceinline__ void cell_max_cell(const Dev& D, int k, int ncell, int init,
-                                              int blk) {
+// timestep (non-negative doubles compare as their bits).  LPC lanes per cell:
+// with one, a cell's rows are two dependent trips of 32 loads on a chip nearly
+// empty (12 us at 22k particles, 16.5 at 653k; four lanes: 7 and 11).
+template <int LPC>
+__device__ __forceinline__ void cell_max_cell(const Dev& D, int ncell, int init, int blk) {
+  constexpr int U = LPC == 1 ? 8 : 4;
+  const int k = blk * 256 + threadIdx.x / LPC, sub = threadIdx.x % LPC;
   unsigned long long vb = 0ull, nb = 0ull;
   if (k < ncell) {
     const int i0 = D.cstart[k], i1 = D.cstart[k + 1];
     if (i1 > i0) {
-      // eight rows' fields requested before any is used (a maximum of
+      // U rows' fields requested before any is used (a maximum of
       // non-negative bit patterns does not depend on the order)
-      for (int b0 = i0; b0 < i1; b0 += 8) {
-        uint8_t tb[8], fb[8];
-        double vl[8], nt[8];
+      for (int b0 = i0 + sub; b0 < i1; b0 += U * LPC) {
+        uint8_t tb[U], fb[U];
+        double vl[U], nt[U];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int i = (b0 + u < i1) ? b0 + u : i0;
+        for (int u = 0; u < U; u++) {
+          const int i = (b0 + u * LPC < i1) ? b0 + u * LPC : i0;
           tb[u] = D.tid[i];
           fb[u] = D.flags[i];
           vl[u] = D.vel[i];
           nt[u] = D.nut[i];
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          if (b0 + u >= i1) break;
+        for (int u = 0; u < U; u++) {
+          if (b0 + u * LPC >= i1) break;
           if (!init && tb[u] == TID_FLUID && !(fb[u] & F_BUFFER)) {
             const unsigned long long b = max_bits(vl[u]);
             vb = (b > vb) ? b : vb;
@@ -1345,11 +1362,21 @@ __device__ __forceinline__ void cell_max_cell(const Dev& D, int k, int ncell, in
           nb = (b > nb) ? b : nb;
         }
       }
-      D.cmaxv[k] = vb;
-      D.cmaxn[k] = nb;
+#pragma unroll
+      for (int s = LPC / 2; s >= 1; s >>= 1) {
+        const unsigned long long ov = __shfl_xor(vb, s, 64), on = __shfl_xor(nb, s, 64);
+        vb = (ov > vb) ? ov : vb;
+        nb = (on > nb) ? on : nb;
+      }
+      if (sub == 0) {
+        D.cmaxv[k] = vb;
+        D.cmaxn[k] = nb;
+      }
     } else if (init) {
-      D.cmaxv[k] = 0ull;
-      D.cmaxn[k] = 0ull;
+      if (sub == 0) {
+        D.cmaxv[k] = 0ull;
+        D.cmaxn[k] = 0ull;
+      }
     } else {
       vb = D.cmaxv[k];
       nb = D.cmaxn[k];
@@ -1362,8 +1389,8 @@ __device__ __forceinline__ void cell_max_cell(const Dev& D, int k, int ncell, in
   }
 }
 
-__global__ void __launch_bounds__(256) k_cell_max(Dev D, int ncell, int init) {
-  cell_max_cell(D, blockIdx.x * blockDim.x + threadIdx.x, ncell, init, blockIdx.x);
+__global__ void __launch_bounds__(1024) k_cell_max(Dev D, int ncell, int init) {
+  cell_max_cell<4>(D, ncell, init, blockIdx.x);
 }
 
 // comp_pos, integrator.f90:845-883

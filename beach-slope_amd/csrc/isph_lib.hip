@@ -911,9 +911,7 @@ static int scan_bins(isph_ctx* c, int len) {
   const int ntiles = (len + SCAN_TILE - 1) / SCAN_TILE;
   hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(256), 0, c->stream, c->D.bincnt,
                      c->D.binstart, c->D.scan_tmp, len);
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(256), 0, c->stream, c->D.scan_tmp, ntiles,
-                     (int32_t*)nullptr);
-  hipLaunchKernelGGL(k_scan_add, dim3(grid_of(len)), dim3(256), 0, c->stream, c->D.binstart,
+  hipLaunchKernelGGL(k_scan_add, dim3(ntiles), dim3(256), 0, c->stream, c->D.binstart,
                      c->D.scan_tmp, len);
   HIPCHK(c, hipGetLastError());
   return 0;
@@ -1587,7 +1585,9 @@ extern "C" int isph_ppesolve(isph_ctx* c, isph_solve_stats* stats) {
 extern "C" int isph_comp_vel(isph_ctx* c) {
   if (!c) return ISPH_EARG;
   TLAUNCH(TK_COMPVEL, k_comp_vel);
-  LAUNCH(k_cell_max, c->ncell, c->D, c->ncell, 0);
+  hipLaunchKernelGGL(k_cell_max, dim3(grid_of(c->ncell)), dim3(1024), 0, c->stream, c->D,
+                     c->ncell, 0);
+  HIPCHK(c, hipGetLastError());
   return 0;
 }
 extern "C" int isph_comp_pos(isph_ctx* c) {
@@ -1637,7 +1637,9 @@ extern "C" int isph_init_state(isph_ctx* c) {
   if (rc) return rc;
   TLAUNCH(TK_EFFPOR, k_effpor);
   TLAUNCH(TK_EDDYVIS, k_eddyvis);
-  LAUNCH(k_cell_max, c->ncell, c->D, c->ncell, 1);
+  hipLaunchKernelGGL(k_cell_max, dim3(grid_of(c->ncell)), dim3(1024), 0, c->stream, c->D,
+                     c->ncell, 1);
+  HIPCHK(c, hipGetLastError());
   rc = isph_timestep(c);
   if (rc) return rc;
   return sync(c);
@@ -1913,7 +1915,9 @@ static int step_pre(isph_ctx* c) {
 // check: read the error bits now (else the next step_pre's scalar read does)
 static int step_post(isph_ctx* c, bool check) {
   TLAUNCH(TK_COMPVEL, k_comp_vel);
-  LAUNCH(k_cell_max, c->ncell, c->D, c->ncell, 0);
+  hipLaunchKernelGGL(k_cell_max, dim3(grid_of(c->ncell)), dim3(1024), 0, c->stream, c->D,
+                     c->ncell, 0);
+  HIPCHK(c, hipGetLastError());
   LAUNCH(k_comp_pos, c->n_hi, c->D);
   int rc = rebin(c, 1);
   if (rc) return rc;

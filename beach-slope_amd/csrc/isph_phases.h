@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(256) kb_comp_vel(PhaseBatch B) {
 }
 __global__ void __launch_bounds__(256) kb_cell_max(PhaseBatch B, int init) {
   PH_IDX(B, PH_CELL);
-  cell_max_cell(D, lb_ * 256 + threadIdx.x, D.P.cellx * D.P.celly, init, lb_);
+  cell_max_cell<1>(D, D.P.cellx * D.P.celly, init, lb_);
 }
 __global__ void kb_comp_pos(PhaseBatch B) {
   PH_PIDX(B);
