@@ -12,6 +12,9 @@
 // scenarios.  Finalize, coarse-level and dense kernels run one workgroup per
 // scenario.  A scenario's results do not depend on which other scenarios
 // share the launch: every sum is over its own rows, in its own block order.
+//
+// The iteration's kernels are the form of timed solves and of systems that the
+// resident form (isph_mgres.h) does not take; both give the same bits.
 #pragma once
 #include "isph_mg.h"
 

@@ -11,16 +11,21 @@
 // phase waits for more than the words it reads.
 //
 // Work split.  A scenario's row blocks (256 rows) lie in runs of nbw blocks on
-// its row workgroups (1024 threads, up to R rows per thread); one more
-// workgroup per scenario runs the coarse levels, with their stencils and the
-// dense inverse in LDS for the whole solve, and forms the dot products.
+// its row workgroups (512 threads with a row each, or 1,024 with up to three);
+// one more workgroup per scenario runs the coarse levels, with their stencils
+// and the dense inverse in registers and LDS for the whole solve, and forms
+// the dot products.  An iteration takes 38 us at 7,485 and 22k rows, 56 at
+// 137k, 66 at 207k and 133 at 653k: up to ~130k rows the chain of some 20
+// exchanges of 1.2 us with the work between them, above that half and more the
+// products' streaming.
 // Windows, row positions and the polling rules are those of isph_persist.h.
 //   level 0   x0 (and ph, sh) of the window's rows by words; the products
 //             gather from LDS
 //   restrict  a cell's rows are summed by the workgroup holding its first
 //             row; rows of the next workgroup arrive by words
 //   levels 1..m   aggregates (down) and cells (up) in equal runs per
-//             workgroup; right-hand sides and corrections by words
+//             workgroup; right-hand sides and corrections by words (with one
+//             row per thread every window forms its level-1 corrections)
 //   levels m+1..  the coarse workgroup
 // The arithmetic and its order are those of the launch-per-phase bodies, so
 // every iterate, scalar and count has the same bits.

@@ -6,7 +6,9 @@
 // What bounds the launch-per-phase form is not the rows but the seven
 // dependent launches of an iteration: at 7,485 rows an iteration took 39 us,
 // of which the two products' data need less than 2 us.  Here an iteration
-// has three grid-wide reductions of ~2 us each.
+// has three grid-wide reductions of ~2 us each and takes 9.7 us; at 22k rows
+// 12.0 (40 before), at 95k 14.8 (42), at 207k 20.9 (50.7), at 653k, where the
+// products' streaming is most of it, 59.0 (93.5).
 //
 // Rows and sums.  A workgroup of T threads holds up to R rows per thread: the
 // row blocks (256 rows) b0 .. b0 + nbw - 1, thread t row t & 255 of blocks

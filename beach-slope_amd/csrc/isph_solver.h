@@ -12,6 +12,9 @@
 // the device.  The kernel boundary makes the
 // partials visible, so no device-scope fence is needed inside the row
 // kernels.  The host only polls the `done` flag every few iterations.
+//
+// This is the form of timed solves and of systems that the resident form
+// (isph_persist.h) does not take; both give the same bits.
 #pragma once
 #include "isph_device.h"
 
