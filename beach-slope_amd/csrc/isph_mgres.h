@@ -34,6 +34,7 @@
 // collected partial sums that every reader published after its reads.
 #pragma once
 #include "isph_batch.h"
+#include "isph_cells.h"
 #include "isph_persist.h"
 
 #define RS_W 6                      // window elements per thread
@@ -1106,39 +1107,9 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
   constexpr int NC = rs_cells(R);
   int uc[NC ? NC : 1];
   if constexpr (NC > 0) {
-    int* slot_cnt = reinterpret_cast<int*>(X);                       // first rows per chunk
-    int* list = slot_cnt + RS_WCAP;                                  // the window's cells
-    bool first[W];
+    static_assert(rs_number_words<T, W, NC>() <= rs_work_words(T, R), "no room in the window");
     __syncthreads();
-#pragma unroll
-    for (int w = 0; w < W; w++) {
-      const int before = __shfl_up(wk[w], 1, 64);
-      first[w] = wk[w] >= 0 && (l == 0 || before != wk[w]);
-      const unsigned long long m = __ballot(first[w]);
-      if (l == 0) slot_cnt[w * (T / PS_CHUNK) + t / PS_CHUNK] = (int)__popcll(m);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < W; w++) {
-      const int s = w * (T / PS_CHUNK) + t / PS_CHUNK;
-      int base = 0;
-      for (int k = 0; k < s; k++) base += slot_cnt[k];
-      const unsigned long long m = __ballot(first[w]);
-      const int u = base + (int)__popcll(m & (~0ull >> (63 - l))) - 1;
-      if (first[w]) list[u] = wk[w];
-      if (wk[w] >= 0) wk[w] = u;
-    }
-    if (t == 0) slot_cnt[0] = 0;
-    __syncthreads();
-    int total = 0;
-#pragma unroll
-    for (int w = 0; w < W; w++) total = max(total, wk[w] + 1);
-    atomicMax(&slot_cnt[0], total);
-    __syncthreads();
-    total = slot_cnt[0];
-#pragma unroll
-    for (int j = 0; j < NC; j++) uc[j] = (t + j * T < total) ? list[t + j * T] : -1;
-    __syncthreads();
+    rs_number_cells<T, W, NC>(t, wk, uc, reinterpret_cast<int*>(X));
   }
   // cells whose first row is here, with the empty ones up to the next
   // workgroup's first; rows of a cell begun earlier are sent to its workgroup
