@@ -96,7 +96,7 @@ EXPORTS = ("isph_create", "isph_destroy", "isph_last_error", "isph_set_params",
            "isph_wavemaker_motion", "isph_set_wavemaker", "isph_wavemaker",
            "isph_ppe_solve_noalloc", "isph_batch_launches", "isph_batch_count",
            "isph_batch_set_graph", "isph_autotune", "isph_batch_autotune", "isph_set_shape",
-           "isph_batch_set_shape") + tuple("isph_" + p for p in PHASES)
+           "isph_batch_set_shape", "isph_set_resident", "isph_resident_counts") + tuple("isph_" + p for p in PHASES)
 
 _lib = None
 
@@ -158,6 +158,8 @@ def lib():
     L.isph_wavemaker.argtypes = [vp]
     L.isph_prof_enable.argtypes = [vp, i32]
     L.isph_prof_read.argtypes = [vp, C.c_char_p, C.POINTER(d), C.POINTER(i64)]
+    L.isph_set_resident.argtypes = [vp, i32, i32]
+    L.isph_resident_counts.argtypes = [vp, vp]
     L.isph_footprint_bytes.restype = i64
     L.isph_footprint_bytes.argtypes = [i64, i64, i32, i32, i32]
     L.isph_ppe_solve_noalloc.argtypes = [i32, i32] + [vp] * 5 + [d, i32, i32, vp,
@@ -173,6 +175,10 @@ def _ptr(a: np.ndarray):
 PART_FIELDS = ("x", "y", "u", "v", "p", "m", "rho", "rho0", "vol0", "c")
 PROP_FIELDS = ("porosity", "resist", "gradvx", "coff", "nut", "tke", "varts", "cdiff", "vel",
                "us", "vs", "xs", "ys")
+
+
+# what Scenario.resident_counts counts (ISPH_RESIDENT_N of them)
+RESIDENT_COUNTS = ("launches", "too_wide", "refused")
 
 
 class Scenario:
@@ -403,6 +409,15 @@ class Scenario:
         self._check(lib().isph_prof_read(self._ctx, kernel.encode(), C.byref(ms), C.byref(cnt)),
                     "isph_prof_read")
         return ms.value, cnt.value
+
+    def set_resident(self, launches: int = -1, iters: int = 0):
+        """Limits of the solves' resident launches (isph_set_resident)."""
+        self._check(lib().isph_set_resident(self._ctx, launches, iters), "isph_set_resident")
+
+    def resident_counts(self) -> dict:
+        k = np.zeros(len(RESIDENT_COUNTS), np.int64)
+        self._check(lib().isph_resident_counts(self._ctx, _ptr(k)), "isph_resident_counts")
+        return dict(zip(RESIDENT_COUNTS, k.tolist()))
 
     def solution(self) -> np.ndarray:
         x = np.empty(self.n)

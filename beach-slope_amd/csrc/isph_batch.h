@@ -150,6 +150,10 @@ __global__ void __launch_bounds__(256) kb_pb_resid(BatchDev B, int init) {
   BATCH_ROW(B);
   pb_resid_rows(D, B.mgs[s_], vb_, init, lds);
 }
+__global__ void __launch_bounds__(256) kb_pb_x0(BatchDev B) {
+  BATCH_ROW(B);
+  pb_x0_rows(D, B.mgs[s_], vb_);
+}
 __global__ void __launch_bounds__(256) kb_pb_bnorm(BatchDev B) {
   __shared__ double lds[RED_BLOCK];
   BATCH_ROW(B);

@@ -66,6 +66,16 @@ struct HostZone {
   int iter = 1;
 };
 
+#define RES_ITERS 1024          // iterations of one resident launch at most
+
+// Limits of a context's resident solves (isph_set_resident)
+struct ResLimits {
+  int launches = -1;       // of one solve (-1: no limit); the rest runs launch by launch
+  int iters = RES_ITERS;   // iterations of one launch
+};
+// What became of its solves' resident form (isph_resident_counts)
+enum { RC_LAUNCH = 0, RC_WINDOW = 1, RC_REFUSED = 2, RC_N = 3 };
+
 struct isph_ctx {
   isph_params P;
   HostZone zones[2];
@@ -98,6 +108,8 @@ struct isph_ctx {
   int pred_first = 0, pred_after = 0;
   PersArg ps{};            // resident FP64 solve: its exchange slots and windows
   ResDev rs{};             // resident precision solve: its words, slots and windows
+  ResLimits lim;
+  int64_t rcount[RC_N] = {};
   bool loaded = false;     // the system came from isph_load_system (no cells behind its rows)
   bool in_batch = false;   // a member of a batch: its form (precision, WCSPH) is fixed
   int tshape[TK_N] = {TS_P256, TS_P256, TS_P256, TS_P256, TS_P256,
@@ -196,7 +208,6 @@ static void fill_devparams(isph_ctx* c) {
 // ---------------------------------------------------------------------
 #define RES_MAX_WG 256          // workgroups of a launch, at most one per CU
 #define RES_WLIST (RES_MAX_WG * (8 * 1024 / PS_CHUNK))
-#define RES_ITERS 1024          // iterations of one launch at most
 
 // LDS of a resident workgroup at most; the kernels are allowed this much
 // whatever a launch needs, so contexts of several threads ask for the same
@@ -852,6 +863,23 @@ extern "C" int isph_prof_enable(isph_ctx* c, int32_t on) {
   return 0;
 }
 
+extern "C" int isph_set_resident(isph_ctx* c, int32_t launches, int32_t iters) {
+  if (!c) return ISPH_EARG;
+  if (iters < 0 || iters > RES_ITERS) {
+    set_err(c, "iterations of a resident launch %d outside [0, %d]", iters, RES_ITERS);
+    return ISPH_EARG;
+  }
+  c->lim.launches = launches < 0 ? -1 : launches;
+  c->lim.iters = iters ? iters : RES_ITERS;
+  return 0;
+}
+
+extern "C" int isph_resident_counts(isph_ctx* c, int64_t* counts) {
+  if (!c || !counts) return ISPH_EARG;
+  for (int k = 0; k < RC_N; k++) counts[k] = c->rcount[k];
+  return 0;
+}
+
 extern "C" int isph_prof_read(isph_ctx* c, const char* kernel, double* total_ms,
                               int64_t* launches) {
   if (!c || !kernel) return ISPH_EARG;
@@ -1304,17 +1332,24 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
       if (rc) return rc;
     }
   }
-  // the packed columns are window positions in the resident form; back to
-  // offsets where the solve cannot run resident after all
-  bool positions = resident;
+  // what the launches read and the resident form keeps otherwise, where the
+  // solve cannot run resident after all: the packed columns (there window
+  // positions) as offsets, and x0 of the iteration that comes next
   auto to_launches = [&]() -> int {
     resident = false;
-    if (positions) BLAUNCH(kb_mg_setup0, grow, 256, B);
-    positions = false;
+    BLAUNCH(kb_mg_setup0, grow, 256, B);
+    BLAUNCH(kb_pb_x0, grow, 256, B);
     return 0;
   };
-  for (int s = 0; s < S && resident; s++)
-    if (b->sc[s].counter[PS_FLAG_WIN] && (rc = to_launches())) return rc;
+  if (resident) {
+    bool wide = false;
+    for (int s = 0; s < S; s++)
+      if (b->sc[s].counter[PS_FLAG_WIN]) {
+        b->ctx[s]->rcount[RC_WINDOW]++;
+        wide = true;
+      }
+    if (wide && (rc = to_launches())) return rc;
+  }
   // packed 16-bit column offsets unless some scenario's rows need int32
   bool off16 = true;
   for (int s = 0; s < S; s++) off16 = off16 && !b->sc[s].far;
@@ -1345,6 +1380,12 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
   };
   int chunk = 4, seq = 0;
   unsigned vtag = 1, ep = 1;  // numbers of the resident form's V-cycles and reductions
+  // the tightest limits of the scenarios
+  int left = -1, riters = RES_ITERS;
+  for (const isph_ctx* q : b->ctx) {
+    if (q->lim.launches >= 0) left = left < 0 ? q->lim.launches : std::min(left, q->lim.launches);
+    riters = std::min(riters, q->lim.iters);
+  }
   bool guessed = false;  // the chunk just run was sized from the last solve
   if (const int p = predicted(false); p > 0) {
     chunk = p;
@@ -1356,11 +1397,14 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
       return ISPH_ENOCONV;
     }
     if (resident) {
-      if (bh_resident(b, B, RES_ITERS, vtag, ep) == hipSuccess) {
-        vtag += 2u * RES_ITERS;
-        ep += 2u * RES_ITERS;
+      if (left != 0 && bh_resident(b, B, riters, vtag, ep) == hipSuccess) {
+        for (isph_ctx* q : b->ctx) q->rcount[RC_LAUNCH]++;
+        if (left > 0) left--;
+        vtag += 2u * (unsigned)riters;
+        ep += 2u * (unsigned)riters;
       } else {  // refused (another process holds the cooperative queue): nothing ran
         (void)hipGetLastError();
+        for (isph_ctx* q : b->ctx) q->rcount[RC_REFUSED]++;
         rc = to_launches();
         if (rc) return rc;
       }
@@ -1429,16 +1473,21 @@ static int bicg_loop(isph_ctx* c, const ResPlan* plan, int* iters_out, int* brk_
   const int n = c->n_hi;
   int chunk = 4, restarts = 0, prev = 0;
   unsigned ep = 1;
+  int left = c->lim.launches;
   DevScalars s;
   for (int64_t it = 0;; ) {
     if (plan) {
       // a refused launch (another process holds the device's cooperative
       // queue) leaves the state as it was: the solve goes on launch by launch
-      if (res_launch(*plan, c->D, c->ps, RES_ITERS, ep, c->stream) == hipSuccess) {
-        chunk = RES_ITERS;
+      if (left != 0 &&
+          res_launch(*plan, c->D, c->ps, c->lim.iters, ep, c->stream) == hipSuccess) {
+        c->rcount[RC_LAUNCH]++;
+        if (left > 0) left--;
+        chunk = c->lim.iters;
         ep += 3u * (unsigned)chunk;
       } else {
         (void)hipGetLastError();
+        c->rcount[RC_REFUSED]++;
         plan = nullptr;
         chunk = 4;
       }
@@ -1542,7 +1591,10 @@ static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
       }
       st.rel_residual = (bnorm == 0.0) ? 0.0 : bnorm;
     } else {
-      if (s.counter[PS_FLAG_WIN]) resident = false;
+      if (resident && s.counter[PS_FLAG_WIN]) {
+        c->rcount[RC_WINDOW]++;
+        resident = false;
+      }
       int it = 0, brk = 0, conv = s.conv, restarts = 0;
       double rel = s.rel;
       if (!s.done) {

@@ -949,6 +949,13 @@ __device__ __forceinline__ void pb_resid_rows(const Dev& D, const MgDev& G, int 
   }
 }
 
+// x0 of the next V-cycle from the direction p, which the resident form does not
+// leave in memory: where its solve goes on launch by launch
+__device__ __forceinline__ void pb_x0_rows(const Dev& D, const MgDev& G, int vb) {
+  const int i = vb * RED_BLOCK + threadIdx.x;
+  if (!D.sc->done && i < D.sc->n) mg_scale0(G, D.pp32[i], i);
+}
+
 // partial (b . b)
 __device__ __forceinline__ void pb_bnorm_rows(const Dev& D, int vb, double* lds) {
   const int i = vb * RED_BLOCK + threadIdx.x;

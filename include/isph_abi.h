@@ -325,6 +325,20 @@ int isph_prof_enable(isph_ctx *ctx, int32_t on);
 int isph_prof_read(isph_ctx *ctx, const char *kernel, double *total_ms,
                    int64_t *launches);
 
+/* ---- resident solves (no counterpart in the reference) ----
+ * A solve whose system fits the device runs in launches of many iterations
+ * that keep it on the chip.  isph_set_resident limits them: `launches`
+ * resident launches per solve (negative: no limit, the default), after which
+ * the solve goes on in one launch per phase as it does when the device refuses
+ * one, and `iters` iterations per launch (0: the default, 1,024).  In a batch
+ * the tightest limits of its contexts hold.  Results do not depend on them.
+ * isph_resident_counts gives, since the context was created, the resident
+ * launches, the solves whose rows couple over too wide a range of rows for
+ * them, and the launches refused or beyond the limit. */
+#define ISPH_RESIDENT_N 3
+int isph_set_resident(isph_ctx *ctx, int32_t launches, int32_t iters);
+int isph_resident_counts(isph_ctx *ctx, int64_t *counts /* ISPH_RESIDENT_N */);
+
 /* ---- autotuner (no counterpart in the reference) ----
  * Times the particle kernels below on the context's current state in each
  * of their launch shapes (trials launches each, HIP events on its stream)
