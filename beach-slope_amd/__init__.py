@@ -96,7 +96,8 @@ EXPORTS = ("isph_create", "isph_destroy", "isph_last_error", "isph_set_params",
            "isph_wavemaker_motion", "isph_set_wavemaker", "isph_wavemaker",
            "isph_ppe_solve_noalloc", "isph_batch_launches", "isph_batch_count",
            "isph_batch_set_graph", "isph_autotune", "isph_batch_autotune", "isph_set_shape",
-           "isph_batch_set_shape", "isph_set_resident", "isph_resident_counts") + tuple("isph_" + p for p in PHASES)
+           "isph_batch_set_shape", "isph_set_resident", "isph_resident_counts",
+           "isph_ppe_solve_noalloc_limits") + tuple("isph_" + p for p in PHASES)
 
 _lib = None
 
@@ -158,12 +159,14 @@ def lib():
     L.isph_wavemaker.argtypes = [vp]
     L.isph_prof_enable.argtypes = [vp, i32]
     L.isph_prof_read.argtypes = [vp, C.c_char_p, C.POINTER(d), C.POINTER(i64)]
-    L.isph_set_resident.argtypes = [vp, i32, i32]
+    L.isph_set_resident.argtypes = [vp, i32, i32, i32]
     L.isph_resident_counts.argtypes = [vp, vp]
     L.isph_footprint_bytes.restype = i64
     L.isph_footprint_bytes.argtypes = [i64, i64, i32, i32, i32]
     L.isph_ppe_solve_noalloc.argtypes = [i32, i32] + [vp] * 5 + [d, i32, i32, vp,
                                                                 C.POINTER(SolveStats)]
+    L.isph_ppe_solve_noalloc_limits.argtypes = [i32, i32] + [vp] * 5 + [
+        d, i32, i32, i32, i32, i32, vp, vp, C.POINTER(SolveStats)]
     _lib = L
     return L
 
@@ -178,7 +181,7 @@ PROP_FIELDS = ("porosity", "resist", "gradvx", "coff", "nut", "tke", "varts", "c
 
 
 # what Scenario.resident_counts counts (ISPH_RESIDENT_N of them)
-RESIDENT_COUNTS = ("launches", "too_wide", "refused")
+RESIDENT_COUNTS = ("launches", "too_wide", "refused", "ran_out")
 
 
 class Scenario:
@@ -410,9 +413,10 @@ class Scenario:
                     "isph_prof_read")
         return ms.value, cnt.value
 
-    def set_resident(self, launches: int = -1, iters: int = 0):
+    def set_resident(self, launches: int = -1, iters: int = 0, ended: int = 0):
         """Limits of the solves' resident launches (isph_set_resident)."""
-        self._check(lib().isph_set_resident(self._ctx, launches, iters), "isph_set_resident")
+        self._check(lib().isph_set_resident(self._ctx, launches, iters, ended),
+                    "isph_set_resident")
 
     def resident_counts(self) -> dict:
         k = np.zeros(len(RESIDENT_COUNTS), np.int64)
@@ -526,15 +530,26 @@ def footprint_bytes(n_cap: int, n_solid_cap: int, cellx: int, celly: int,
 
 def ppe_solve_noalloc(n: int, ld: int, row_len: int, col: int, val: int, rhs: int, x: int,
                       tol: float, max_iter: int, max_outer: int = 0, stream: int | None = None,
-                      check: bool = True):
+                      check: bool = True, limits: tuple | None = None,
+                      counts: dict | None = None):
     """FP64 BiCGStab on a system already in device memory, with no allocation
     (isph_ppe_solve_noalloc).  row_len, col, val, rhs and x are device
     addresses (integers); col/val are ELL slot-major with leading dimension
-    ld; x holds the initial guess and receives the solution.  Returns
-    (return code, SolveStats)."""
+    ld; x holds the initial guess and receives the solution.  limits
+    (launches, iters, ended) and counts are those of Scenario.set_resident and
+    resident_counts (isph_ppe_solve_noalloc_limits).  Returns (return code,
+    SolveStats)."""
     st = SolveStats()
-    rc = lib().isph_ppe_solve_noalloc(int(n), int(ld), row_len, col, val, rhs, x, float(tol),
-                                      int(max_iter), int(max_outer), stream, C.byref(st))
+    args = [int(n), int(ld), row_len, col, val, rhs, x, float(tol), int(max_iter),
+            int(max_outer)]
+    if limits is None and counts is None:
+        rc = lib().isph_ppe_solve_noalloc(*args, stream, C.byref(st))
+    else:
+        k = np.zeros(len(RESIDENT_COUNTS), np.int64)
+        rc = lib().isph_ppe_solve_noalloc_limits(*args, *(limits or (-1, 0, 0)), _ptr(k),
+                                                 stream, C.byref(st))
+        if counts is not None:
+            counts.update(zip(RESIDENT_COUNTS, k.tolist()))
     if check and rc != 0:
         raise IsphError(rc, "isph_ppe_solve_noalloc",
                         (lib().isph_last_error(None) or b"").decode())

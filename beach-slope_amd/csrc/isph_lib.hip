@@ -72,9 +72,10 @@ struct HostZone {
 struct ResLimits {
   int launches = -1;       // of one solve (-1: no limit); the rest runs launch by launch
   int iters = RES_ITERS;   // iterations of one launch
+  int ended = 0;           // workgroups in it whose waits count as run out
 };
 // What became of its solves' resident form (isph_resident_counts)
-enum { RC_LAUNCH = 0, RC_WINDOW = 1, RC_REFUSED = 2, RC_N = 3 };
+enum { RC_LAUNCH = 0, RC_WINDOW = 1, RC_REFUSED = 2, RC_WAIT = 3, RC_N = 4 };
 
 struct isph_ctx {
   isph_params P;
@@ -296,7 +297,7 @@ extern "C" int64_t isph_footprint_bytes(int64_t n_cap, int64_t n_solid_cap, int3
   per += 4 + 4 * NBR_CAP;                       // neighbour list
   per += 4 * 3;                                 // bin, rank, scan scratch
   per += 4 + ROW_CAP * (4 + 8) + 2 * 8;         // PPE rows, rhs, solution
-  per += 7 * 8;                                 // FP64 solver vectors
+  per += 8 * 8;                                 // FP64 solver vectors
   per += 4 * ((ROW_CAP + 1) / 2);               // packed 16-bit columns
   // precision form: FP16 V-cycle matrix, FP32 vectors, level-0 multigrid
   // vectors, setup rows
@@ -388,6 +389,7 @@ extern "C" int isph_create(const isph_params* params, int64_t n_cap, int64_t n_s
   rc |= dalloc(c, &D.aoff, N * ((ROW_CAP + 1) / 2));
   rc |= dalloc(c, &c->ps.slots, 8 * (N / 256 + 2 + RES_MAX_WG));
   rc |= dalloc(c, &c->ps.rhi, N);
+  rc |= dalloc(c, &c->ps.x0, N);
   rc |= dalloc(c, &c->ps.wlist, RES_WLIST);
   rc |= dalloc(c, &c->ps.wcnt, 2 * RES_MAX_WG);
   if (params->precision) {
@@ -863,14 +865,22 @@ extern "C" int isph_prof_enable(isph_ctx* c, int32_t on) {
   return 0;
 }
 
-extern "C" int isph_set_resident(isph_ctx* c, int32_t launches, int32_t iters) {
+// limits as the caller gives them; false: out of range
+static bool res_limits(int32_t launches, int32_t iters, int32_t ended, ResLimits* out) {
+  if (iters < 0 || iters > RES_ITERS || ended < 0) return false;
+  out->launches = launches < 0 ? -1 : launches;
+  out->iters = iters ? iters : RES_ITERS;
+  out->ended = ended;
+  return true;
+}
+
+extern "C" int isph_set_resident(isph_ctx* c, int32_t launches, int32_t iters, int32_t ended) {
   if (!c) return ISPH_EARG;
-  if (iters < 0 || iters > RES_ITERS) {
-    set_err(c, "iterations of a resident launch %d outside [0, %d]", iters, RES_ITERS);
+  if (!res_limits(launches, iters, ended, &c->lim)) {
+    set_err(c, "resident launches: %d iterations outside [0, %d] or %d workgroups below 0", iters,
+            RES_ITERS, ended);
     return ISPH_EARG;
   }
-  c->lim.launches = launches < 0 ? -1 : launches;
-  c->lim.iters = iters ? iters : RES_ITERS;
   return 0;
 }
 
@@ -1182,6 +1192,7 @@ static void bh_plan(BatchHost* b) {
     q = c->rs;
     q.wg0 = wg0;
     q.nbw = nbw;
+    q.ended = c->lim.ended;
     q.G = (c->D.nblk + nbw - 1) / nbw;
     wg0 += q.G + 1;
     int l0 = 1;
@@ -1315,14 +1326,17 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
   for (int l = 1; l < b->max_nlev; l++)
     if (tot(BK_COARSEN + l - 1) > 0) BLAUNCH(kb_mg_coarsen, tot(BK_COARSEN + l - 1), 256, B, l);
   BLAUNCH(kb_mg_dense, S, MG_DENSE_THREADS, B);
-  // ||b||, then the FP64 start residual
-  BLAUNCH(kb_pb_bnorm, grow, 256, B);
-  BLAUNCH(kb_pfinalize, S, 256, B, (int)PFIN_BNORM, 0, 0);
   bool resident = b->rs_grid > 0;
-  if (resident) HIPCHK(c, bh_rs_setup(b, B));
-  BLAUNCH(kb_pb_resid, grow, 256, B, 1);
-  BLAUNCH(kb_pfinalize, S, 256, B, (int)PFIN_RESID, 1, 0);
-  rc = bh_gather(b);
+  // ||b||, then the FP64 start residual
+  auto start = [&]() -> int {
+    BLAUNCH(kb_pb_bnorm, grow, 256, B);
+    BLAUNCH(kb_pfinalize, S, 256, B, (int)PFIN_BNORM, 0, 0);
+    if (resident) HIPCHK(c, bh_rs_setup(b, B));
+    BLAUNCH(kb_pb_resid, grow, 256, B, 1);
+    BLAUNCH(kb_pfinalize, S, 256, B, (int)PFIN_RESID, 1, 0);
+    return bh_gather(b);
+  };
+  rc = start();
   if (rc) return rc;
   // error bits of the phases before the solve (neighbour capacity, PPE
   // diagonal) end the step, as the per-scenario check does
@@ -1353,7 +1367,7 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
   // packed 16-bit column offsets unless some scenario's rows need int32
   bool off16 = true;
   for (int s = 0; s < S; s++) off16 = off16 && !b->sc[s].far;
-  std::vector<int> it_prev(S), rs_prev(S), first_stop(S, -1);
+  std::vector<int> it_prev(S, 0), rs_prev(S, 0), first_stop(S, -1);
   auto all_fin = [&]() {
     for (int s = 0; s < S; s++)
       if (!b->sc[s].fin) return false;
@@ -1363,8 +1377,6 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
   for (int s = 0; s < S; s++) {
     max_iter = std::max(max_iter, b->ctx[s]->P.max_iter);
     max_outer = std::max(max_outer, b->ctx[s]->P.max_outer);
-    it_prev[s] = b->sc[s].iters;
-    rs_prev[s] = b->sc[s].restarts;
   }
   // every chunk either advances an unfinished scenario by at least one
   // iteration or ends it at the check, so this bound is never the exit
@@ -1419,11 +1431,22 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
     BLAUNCH(kb_pfinalize, S, 256, B, (int)PFIN_RESID, 2, 0);
     rc = bh_gather(b);
     if (rc) return rc;
+    bool ran_out = false;
     for (int s = 0; s < S; s++)
       if (resident && b->sc[s].counter[PS_FLAG_ABORT]) {
-        set_err(b->ctx[s], "resident PPE solve: a wait ran out");
-        return ISPH_EHIP;
+        b->ctx[s]->rcount[RC_WAIT]++;
+        ran_out = true;
       }
+    if (ran_out) {  // every solve again from its start, launch by launch
+      rc = to_launches();
+      if (!rc) rc = start();
+      if (rc) return rc;
+      it_prev.assign(S, 0);
+      rs_prev.assign(S, 0);
+      first_stop.assign(S, -1);
+      nchunks = -1;
+      continue;
+    }
     // the timed launches that did work: the chunk's leading iterations
     int worked = 0, restarted = 0;
     for (int s = 0; s < S; s++) {
@@ -1507,8 +1530,19 @@ static int bicg_loop(isph_ctx* c, const ResPlan* plan, int* iters_out, int* brk_
     int rc = read_scalars(c, &s);
     if (rc) return rc;
     if (plan && s.counter[PS_FLAG_ABORT]) {
-      set_err(c, "resident PPE solve: a grid-wide wait ran out");
-      return ISPH_EHIP;
+      // a wait ran out: the solve again from its start, launch by launch
+      c->rcount[RC_WAIT]++;
+      plan = nullptr;
+      HIPCHK(c, hipMemcpyAsync(c->D.sol, c->ps.x0, 8 * (size_t)s.n, hipMemcpyDeviceToDevice,
+                               c->stream));
+      RLAUNCH(k_bicg_init, n, c->D);
+      FINALIZE(FIN_INIT, n);
+      rc = read_scalars(c, &s);
+      if (rc) return rc;
+      it = prev = restarts = 0;
+      chunk = 4;
+      if (s.done) break;
+      continue;
     }
     // the timed launches that did work: the chunk's leading iterations
     if (c->prof) timers_collect(c, s.iters - prev);
@@ -1574,6 +1608,7 @@ static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
       Q.rlo = words(c->D.sv);
       Q.lidx = c->D.aoff;
       Q.ls = c->D.cap;
+      Q.ended = c->lim.ended;
       HIPCHK(c, res_setup(plan, c->D, Q, c->stream));
     }
     RLAUNCH(k_bicg_init, n, c->D);
@@ -2741,8 +2776,8 @@ extern "C" int isph_batch_destroy(isph_batch* b) {
 // Scratch of the allocation-free solve, one static device array per GPU: room
 // for six BiCGStab vectors of ISPH_NOALLOC_MAX_ROWS doubles (r, rh, p, t1, s,
 // t2; a smaller system's vectors, then what the resident form exchanges and
-// its window positions), the block partials of two dot products, then the solver scalars and
-// the squared right-hand-side norm.  Host code never uses the array's name
+// its window positions), the block partials of two dot products, the solver scalars and
+// the squared right-hand-side norm, then the start vector that the resident form keeps.  Host code never uses the array's name
 // as an address: scratch_base() looks up each device's own copy once, with
 // that device current, and every kernel argument is derived from it.
 #define NA_ROWS ((size_t)ISPH_NOALLOC_MAX_ROWS)
@@ -2750,7 +2785,11 @@ extern "C" int isph_batch_destroy(isph_batch* b) {
 #define NA_SC_DOUBLES 48
 static_assert(sizeof(DevScalars) + sizeof(double) <= NA_SC_DOUBLES * sizeof(double),
               "solver scalars do not fit their scratch slot");
-static __device__ __align__(256) double scratch[6 * NA_ROWS + NA_PART + NA_SC_DOUBLES];
+// rows of the largest system whose resident form fits the six vectors' room
+// (23.5 doubles a row), and a few more
+#define NA_START_ROWS ((size_t)270 * 1024)
+static __device__ __align__(256) double
+    scratch[6 * NA_ROWS + NA_PART + NA_SC_DOUBLES + NA_START_ROWS];
 
 #define NA_MAX_DEVICES 64
 static std::mutex g_na_mu;
@@ -2839,12 +2878,10 @@ static int na_read(hipStream_t st, const DevScalars* d_sc, DevScalars* s, double
   return 0;
 }
 
-extern "C" int isph_ppe_solve_noalloc(int32_t n, int32_t ld, const int32_t* row_len,
-                                      const int32_t* col, const double* val, const double* rhs,
-                                      double* x, double tol, int32_t max_iter,
-                                      int32_t max_outer, void* stream,
-                                      isph_solve_stats* stats) {
-  g_noctx_err.clear();
+static int na_solve(int32_t n, int32_t ld, const int32_t* row_len, const int32_t* col,
+                    const double* val, const double* rhs, double* x, double tol,
+                    int32_t max_iter, int32_t max_outer, const ResLimits& lim, int64_t* counts,
+                    void* stream, isph_solve_stats* stats) {
   if (n < 0 || (size_t)n > NA_ROWS)
     return na_fail(ISPH_EARG, "isph_ppe_solve_noalloc: %d rows outside [0, %d]", n,
                    ISPH_NOALLOC_MAX_ROWS);
@@ -2909,7 +2946,9 @@ extern "C" int isph_ppe_solve_noalloc(int32_t n, int32_t ld, const int32_t* row_
     Q.wcnt = reinterpret_cast<int32_t*>(take(RES_MAX_WG));
     Q.lidx = reinterpret_cast<uint32_t*>(take(((ROW_CAP + 1) / 2) * nv / 2));
     Q.ls = (int)nv;
-    resident = at <= 6 * NA_ROWS;
+    Q.ended = lim.ended;
+    Q.x0 = base + 6 * NA_ROWS + NA_PART + NA_SC_DOUBLES;
+    resident = at <= 6 * NA_ROWS && nv <= NA_START_ROWS;
   }
   double* d_bn2 = base + 6 * NA_ROWS + NA_PART + NA_SC_DOUBLES - 1;
   const int rg = row_grid(n), nb = grid_of(n);
@@ -2949,16 +2988,22 @@ extern "C" int isph_ppe_solve_noalloc(int32_t n, int32_t ld, const int32_t* row_
                        (double*)nullptr);
     rc = na_read(st, D.sc, &s, nullptr);
     if (rc) return rc;
-    if (s.counter[PS_FLAG_WIN]) resident = false;
-    int restarts = 0, chunk = 4;
+    if (resident && s.counter[PS_FLAG_WIN]) {
+      counts[RC_WINDOW]++;
+      resident = false;
+    }
+    int restarts = 0, chunk = 4, left = lim.launches;
     unsigned ep = 1;
     for (int64_t it = 0; !s.done;) {
       if (resident) {
-        if (res_launch(plan, D, Q, RES_ITERS, ep, st) == hipSuccess) {
-          chunk = RES_ITERS;
-          ep += 3u * RES_ITERS;
+        if (left != 0 && res_launch(plan, D, Q, lim.iters, ep, st) == hipSuccess) {
+          counts[RC_LAUNCH]++;
+          if (left > 0) left--;
+          chunk = lim.iters;
+          ep += 3u * (unsigned)chunk;
         } else {  // refused: nothing ran
           (void)hipGetLastError();
+          counts[RC_REFUSED]++;
           resident = false;
           chunk = 4;
         }
@@ -2978,8 +3023,22 @@ extern "C" int isph_ppe_solve_noalloc(int32_t n, int32_t ld, const int32_t* row_
       it += chunk;
       rc = na_read(st, D.sc, &s, nullptr);
       if (rc) return rc;
-      if (resident && s.counter[PS_FLAG_ABORT])
-        return na_fail(ISPH_EHIP, "isph_ppe_solve_noalloc: a grid-wide wait ran out");
+      if (resident && s.counter[PS_FLAG_ABORT]) {
+        // a wait ran out: the solve again from its start, launch by launch
+        counts[RC_WAIT]++;
+        resident = false;
+        const hipError_t e = hipMemcpyAsync(x, Q.x0, 8 * (size_t)n, hipMemcpyDeviceToDevice, st);
+        if (e != hipSuccess)
+          return na_fail(ISPH_EHIP, "isph_ppe_solve_noalloc: %s", hipGetErrorString(e));
+        NA_LAUNCH(k_bicg_init, rg, D);
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, st, D, (int)FIN_INIT, nb,
+                           (double*)nullptr);
+        rc = na_read(st, D.sc, &s, nullptr);
+        if (rc) return rc;
+        it = restarts = 0;
+        chunk = 4;
+        continue;
+      }
       if (s.done) {
         if (s.brk && !s.conv && s.iters < max_iter && restarts < max_outer) {
           restarts++;
@@ -3012,6 +3071,34 @@ extern "C" int isph_ppe_solve_noalloc(int32_t n, int32_t ld, const int32_t* row_
     return na_fail(ISPH_ENOCONV, "isph_ppe_solve_noalloc: %d iterations, rel residual %g",
                    out.iterations, out.rel_residual);
   return 0;
+}
+
+extern "C" int isph_ppe_solve_noalloc(int32_t n, int32_t ld, const int32_t* row_len,
+                                      const int32_t* col, const double* val, const double* rhs,
+                                      double* x, double tol, int32_t max_iter,
+                                      int32_t max_outer, void* stream,
+                                      isph_solve_stats* stats) {
+  g_noctx_err.clear();
+  int64_t counts[RC_N] = {};
+  return na_solve(n, ld, row_len, col, val, rhs, x, tol, max_iter, max_outer, ResLimits(),
+                  counts, stream, stats);
+}
+
+extern "C" int isph_ppe_solve_noalloc_limits(int32_t n, int32_t ld, const int32_t* row_len,
+                                             const int32_t* col, const double* val,
+                                             const double* rhs, double* x, double tol,
+                                             int32_t max_iter, int32_t max_outer,
+                                             int32_t launches, int32_t iters, int32_t ended,
+                                             int64_t* counts, void* stream,
+                                             isph_solve_stats* stats) {
+  g_noctx_err.clear();
+  ResLimits lim;
+  if (!counts || !res_limits(launches, iters, ended, &lim))
+    return na_fail(ISPH_EARG, "isph_ppe_solve_noalloc_limits: null counts, %d iterations "
+                   "outside [0, %d] or %d workgroups below 0", iters, RES_ITERS, ended);
+  for (int k = 0; k < RC_N; k++) counts[k] = 0;
+  return na_solve(n, ld, row_len, col, val, rhs, x, tol, max_iter, max_outer, lim, counts,
+                  stream, stats);
 }
 
 // ---------------------------------------------------------------------

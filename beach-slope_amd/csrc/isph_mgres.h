@@ -61,6 +61,7 @@ struct ResDev {
   int wg0, G;                 // first workgroup; row workgroups (the coarse one is wg0 + G)
   int nbw;                    // row blocks per workgroup
   int m;                      // cell levels 1..m on the row workgroups
+  int ended;                  // workgroups of the scenario whose waits count as run out
   unsigned long long* slots;  // 10 words per row block
   unsigned long long* mail;   // RS_MAIL words per workgroup
   unsigned long long *x0w, *phw, *r0w;  // a word per row: x0, V-cycle result, r0
@@ -851,7 +852,7 @@ __device__ __forceinline__ void rs_coarse_solve(const Dev& D, const MgDev& M, co
   const float* sten = glob(M.sten);
   const float* rdg = glob(M.rdg);
   const double* dinv = glob(M.dense_inv);
-  if (t0 == 0) *bad = 0;
+  if (t0 == 0) *bad = Q.G < Q.ended;
   if (t0 < 8) Bv[S + t0] = 0.0f;
   for (int e = t0; e < nd8 * LD.n; e += T) DI[e] = e < LD.n * LD.n ? dinv[e] : 0.0;
   for (int e = t0; e < nst; e += T) ST[e] = sten[9 * (size_t)stb + e];
@@ -1050,7 +1051,7 @@ __device__ __forceinline__ void rs_rows_solve(const Dev& D, const MgDev& M, cons
   double* area = res + 8;  // 5 S4 192 doubles, in the window's place
   float* X = reinterpret_cast<float*>(res + 8);  // the window
   float* r0s = X + W * T;                  // r0 of the workgroup's rows
-  if (t == 0) *bad = 0;
+  if (t == 0) *bad = wg < Q.ended;
   float* E1 = X + rs_work_words(T, R) + rs_lds_entries(T, R) * R * T;  // corrections of the window's cells
   unsigned long long* x0w = glob(Q.x0w);
   unsigned long long* phw = glob(Q.phw);

@@ -40,7 +40,10 @@
 //
 // Progress.  The launch is cooperative (all workgroups resident); every wait
 // is bounded (PS_SPIN polls) and a wait that ends without its data makes the
-// launch return with the abort flag set.
+// launch return with the abort flag set.  Other work that keeps CUs of the
+// device busy for that long does so; the host then solves the system again from
+// its start, launch by launch (what the others computed meanwhile may hang on
+// values that never came).  k_ps_setup keeps the start for that.
 #pragma once
 #include <type_traits>
 
@@ -48,7 +51,7 @@
 
 #define PS_CHUNK 64                 // rows per window chunk
 #define PS_MAX_CHUNKS 16384         // chunks of the largest system (2^20 rows)
-#define PS_SPIN (1 << 20)           // polls of one wait: about a second
+#define PS_SPIN (1 << 20)           // polls of one wait: some tenths of a second
 
 // DevScalars::counter slots of the resident solve
 #define PS_FLAG_WIN 0               // a window exceeds its capacity
@@ -65,6 +68,8 @@ struct PersArg {
   int32_t* wcnt;              // per workgroup: their count, and the slot of its own first chunk
   int wcap;                   // window capacity in chunks
   int nbw;                    // row blocks per workgroup
+  int ended;                  // workgroups whose waits count as run out (0 but in a test)
+  double* x0;                 // the solution vector at the start
 };
 
 template <typename V>
@@ -107,7 +112,10 @@ __global__ void __launch_bounds__(T) k_ps_setup(Dev D, PersArg Q) {
       Q.slots[4 * ((size_t)D.nblk + b) + q] = 0;
     }
   if (t < 8) Q.slots[8 * ((size_t)D.nblk + wg) + t] = 0;
-  for (int i = i0 + t; i < i1; i += T) Q.tlo[i] = Q.thi[i] = Q.rlo[i] = Q.rhi[i] = 0;
+  for (int i = i0 + t; i < i1; i += T) {
+    Q.tlo[i] = Q.thi[i] = Q.rlo[i] = Q.rhi[i] = 0;
+    Q.x0[i] = D.sol[i];
+  }
   for (int c = t; c < nch; c += T) map[c] = 0;
   __syncthreads();
   for (int i = i0 + t; i < i1; i += T) {
@@ -514,7 +522,7 @@ __global__ void __launch_bounds__(T) k_bicg_resident(Dev D, PersArg Q, int iters
   const int wn = Q.wcnt[2 * wg], s0 = Q.wcnt[2 * wg + 1];
   {
     const int t = threadIdx.x, sub = t >> 8, l = t & 63;
-    if (t == 0) *bad = 0;
+    if (t == 0) *bad = wg < Q.ended;
 #pragma unroll
     for (int q = 0; q < R; q++) {
       const int lb = q * S + sub, i = (b0 + lb) * RED_BLOCK + (t & 255);

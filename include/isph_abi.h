@@ -330,14 +330,26 @@ int isph_prof_read(isph_ctx *ctx, const char *kernel, double *total_ms,
  * that keep it on the chip.  isph_set_resident limits them: `launches`
  * resident launches per solve (negative: no limit, the default), after which
  * the solve goes on in one launch per phase as it does when the device refuses
- * one, and `iters` iterations per launch (0: the default, 1,024).  In a batch
- * the tightest limits of its contexts hold.  Results do not depend on them.
+ * one, and `iters` iterations per launch (0: the default, 1,024).  The
+ * workgroups of a launch wait for each other, some tenths of a second at most; a wait
+ * that runs out, since other work keeps CUs from the launch, makes the solve
+ * start over in one launch per phase.  `ended` workgroups of each launch act as
+ * if that had happened to them (0, the default, but in tests of it).  In a batch
+ * the tightest launches and iters of its contexts hold, and ended for the
+ * context's own workgroups.  Results depend on none of them.
  * isph_resident_counts gives, since the context was created, the resident
  * launches, the solves whose rows couple over too wide a range of rows for
- * them, and the launches refused or beyond the limit. */
-#define ISPH_RESIDENT_N 3
-int isph_set_resident(isph_ctx *ctx, int32_t launches, int32_t iters);
+ * them, the launches refused or beyond the limit, and the waits run out. */
+#define ISPH_RESIDENT_N 4
+int isph_set_resident(isph_ctx *ctx, int32_t launches, int32_t iters, int32_t ended);
 int isph_resident_counts(isph_ctx *ctx, int64_t *counts /* ISPH_RESIDENT_N */);
+/* isph_ppe_solve_noalloc with such limits, and its counts. */
+int isph_ppe_solve_noalloc_limits(int32_t n, int32_t ld, const int32_t *row_len,
+                                  const int32_t *col, const double *val, const double *rhs,
+                                  double *x, double tol, int32_t max_iter, int32_t max_outer,
+                                  int32_t launches, int32_t iters, int32_t ended,
+                                  int64_t *counts /* ISPH_RESIDENT_N */, void *stream,
+                                  isph_solve_stats *stats);
 
 /* ---- autotuner (no counterpart in the reference) ----
  * Times the particle kernels below on the context's current state in each
@@ -372,9 +384,9 @@ int64_t isph_footprint_bytes(int64_t n_cap, int64_t n_solid_cap,
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): the FP64 BiCGStab of isph_ppe_solve in the
- * ISPH_PPE_FP64 form (same kernels, same reduction order, same restarts: the
- * iterates equal those of isph_load_system + isph_ppe_solve bit for bit) on
- * a system the caller holds in device memory, with no context.
+ * ISPH_PPE_FP64 form (same reduction order, same restarts: the iterates equal
+ * those of isph_load_system + isph_ppe_solve bit for bit) on a system the
+ * caller holds in device memory, with no context.
  *   n rows (0 <= n <= ISPH_NOALLOC_MAX_ROWS), ELL slot-major with leading
  *   dimension ld >= n: entry k of row i is col[k*ld + i], val[k*ld + i] for
  *   k < row_len[i] <= ISPH_NBR_CAP + 2; rhs[n]; x[n] holds the initial guess
@@ -384,7 +396,7 @@ int64_t isph_footprint_bytes(int64_t n_cap, int64_t n_solid_cap,
  *   NULL for the null stream; the call returns after the stream has drained.
  * The BiCGStab vectors, the block partials and the solver scalars live in a
  * static device array of fixed size (6 * ISPH_NOALLOC_MAX_ROWS doubles plus
- * ~64 KB, about 50 MB, held on every GPU the library runs on until the
+ * ~2.3 MB, about 53 MB, held on every GPU the library runs on until the
  * process ends); the call makes no hipMalloc, hipFree or other allocation.
  * All calls on one GPU share that array, so calls that overlap in time on
  * one GPU (from two host threads, or on two streams) race and must not be
