@@ -74,6 +74,12 @@ struct ResLimits {
   int iters = RES_ITERS;   // iterations of one launch
   int ended = 0;           // workgroups in it whose waits count as run out
 };
+// Solves of a context that go launch by launch after one whose resident form
+// came to nothing (windows too wide, launch refused, wait run out) before it is
+// tried again.  Particles move little in as many steps, and a try costs what the
+// set-up takes and what it has overwritten: on a 580k basin 79 of a precision
+// solve's 7,640 us, on a splash of 113k particles 27 of 5,170.
+#define RES_RETRY 32
 // What became of its solves' resident form (isph_resident_counts)
 enum { RC_LAUNCH = 0, RC_WINDOW = 1, RC_REFUSED = 2, RC_WAIT = 3, RC_N = 4 };
 
@@ -111,6 +117,7 @@ struct isph_ctx {
   ResDev rs{};             // resident precision solve: its words, slots and windows
   ResLimits lim;
   int64_t rcount[RC_N] = {};
+  int res_skip = 0;        // solves to go launch by launch (RES_RETRY)
   bool loaded = false;     // the system came from isph_load_system (no cells behind its rows)
   bool in_batch = false;   // a member of a batch: its form (precision, WCSPH) is fixed
   int tshape[TK_N] = {TS_P256, TS_P256, TS_P256, TS_P256, TS_P256,
@@ -238,6 +245,13 @@ static int resident_capacity(const void* fn, int T) {
     (void)hipGetLastError();
   known[key] = n;
   return n;
+}
+
+// whether this solve of c tries the resident form (RES_RETRY)
+static bool res_tried(isph_ctx* c) {
+  if (c->res_skip == 0) return true;
+  c->res_skip--;
+  return false;
 }
 
 struct ResPlan {
@@ -631,6 +645,7 @@ extern "C" int isph_upload(isph_ctx* c, int64_t n, const double* x, const double
   s.umax_bits = 0;
   s.numax_bits = 0;
   HIPCHK(c, hipMemcpy(D.sc, &s, sizeof s, hipMemcpyHostToDevice));
+  c->res_skip = 0;
   set_nhi(c, (int)n);
   c->assembled = false;
   c->have_nbr = false;
@@ -1168,10 +1183,13 @@ static int64_t rs_shape(BatchHost* b) {
 // with which every scenario's row workgroups and its coarse one fit the
 // device at one per CU, and the coarse workgroups' first levels.  Leaves
 // rs_grid 0 where the solve has to run launch by launch: kernel timing on,
-// more than 12 row blocks per workgroup, a loaded system, or a device that
-// cannot hold the grid.
+// more than 12 row blocks per workgroup, a loaded system, a scenario whose
+// resident form lately came to nothing, or a device that cannot hold the grid.
 static void bh_plan(BatchHost* b) {
   b->rs_grid = 0;
+  bool tried = true;
+  for (isph_ctx* c : b->ctx) tried = res_tried(c) && tried;
+  if (!tried) return;
   for (isph_ctx* c : b->ctx)
     if (c->prof || c->loaded || c->D.nblk > PS_MAX_CHUNKS / 4) return;
   int nbw = 0, grid = 0;
@@ -1360,6 +1378,7 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
     for (int s = 0; s < S; s++)
       if (b->sc[s].counter[PS_FLAG_WIN]) {
         b->ctx[s]->rcount[RC_WINDOW]++;
+        b->ctx[s]->res_skip = RES_RETRY;
         wide = true;
       }
     if (wide && (rc = to_launches())) return rc;
@@ -1416,7 +1435,10 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
         ep += 2u * (unsigned)riters;
       } else {  // refused (another process holds the cooperative queue): nothing ran
         (void)hipGetLastError();
-        for (isph_ctx* q : b->ctx) q->rcount[RC_REFUSED]++;
+        for (isph_ctx* q : b->ctx) {
+          q->rcount[RC_REFUSED]++;
+          if (left != 0) q->res_skip = RES_RETRY;
+        }
         rc = to_launches();
         if (rc) return rc;
       }
@@ -1435,6 +1457,7 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
     for (int s = 0; s < S; s++)
       if (resident && b->sc[s].counter[PS_FLAG_ABORT]) {
         b->ctx[s]->rcount[RC_WAIT]++;
+        b->ctx[s]->res_skip = RES_RETRY;
         ran_out = true;
       }
     if (ran_out) {  // every solve again from its start, launch by launch
@@ -1511,6 +1534,7 @@ static int bicg_loop(isph_ctx* c, const ResPlan* plan, int* iters_out, int* brk_
       } else {
         (void)hipGetLastError();
         c->rcount[RC_REFUSED]++;
+        if (left != 0) c->res_skip = RES_RETRY;
         plan = nullptr;
         chunk = 4;
       }
@@ -1532,6 +1556,7 @@ static int bicg_loop(isph_ctx* c, const ResPlan* plan, int* iters_out, int* brk_
     if (plan && s.counter[PS_FLAG_ABORT]) {
       // a wait ran out: the solve again from its start, launch by launch
       c->rcount[RC_WAIT]++;
+      c->res_skip = RES_RETRY;
       plan = nullptr;
       HIPCHK(c, hipMemcpyAsync(c->D.sol, c->ps.x0, 8 * (size_t)s.n, hipMemcpyDeviceToDevice,
                                c->stream));
@@ -1599,7 +1624,7 @@ static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
     hipLaunchKernelGGL(k_res_begin, dim3(1), dim3(64), 0, c->stream, c->D, c->d_bn2);
     // kernel timing brackets launches, so it takes the launch-per-phase form
     ResPlan plan;
-    bool resident = !c->prof && res_plan(c->D.nblk, &plan);
+    bool resident = res_tried(c) && !c->prof && res_plan(c->D.nblk, &plan);
     if (resident) {
       PersArg& Q = c->ps;
       auto words = [](double* p) { return reinterpret_cast<unsigned long long*>(p); };
@@ -1628,6 +1653,7 @@ static int ppe_solve_impl(isph_ctx* c, isph_solve_stats* stats) {
     } else {
       if (resident && s.counter[PS_FLAG_WIN]) {
         c->rcount[RC_WINDOW]++;
+        c->res_skip = RES_RETRY;
         resident = false;
       }
       int it = 0, brk = 0, conv = s.conv, restarts = 0;
@@ -2179,6 +2205,7 @@ extern "C" int isph_load_system(isph_ctx* c, int32_t n, const int32_t* len, cons
   set_nhi(c, n);
   c->assembled = true;
   c->loaded = true;
+  c->res_skip = 0;
   return 0;
 }
 
