@@ -10,7 +10,6 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -221,29 +220,41 @@ static void fill_devparams(isph_ctx* c) {
 // whatever a launch needs, so contexts of several threads ask for the same
 #define RES_LDS_MAX (152 * 1024)
 
+// Device memory that has to be free before a kernel's first resident launch: the
+// runtime then sets up its cooperative queue and the kernel's private memory
+// (28 MiB over the FP64 shapes).  A fuller device keeps to the launches.
+#define RES_FREE_MIN ((size_t)256 << 20)
+
 // Workgroups of T threads and RES_LDS_MAX bytes of LDS of kernel fn that the
 // current device holds resident for a cooperative launch (0: none); asked
-// once per device and kernel
+// once per device and kernel (in a fixed table: the allocation-free solve asks)
 static int resident_capacity(const void* fn, int T) {
   static std::mutex mu;
-  static std::map<std::pair<int, const void*>, int> known;
+  static struct {
+    int dev;
+    const void* fn;
+    int n;
+  } known[128];
+  static int nknown = 0;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   std::lock_guard<std::mutex> lock(mu);
-  const auto key = std::make_pair(dev, fn);
-  const auto at = known.find(key);
-  if (at != known.end()) return at->second;
-  int cus = 0, coop = 0, per_cu = 0, n = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) == hipSuccess &&
-      coop &&
-      hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS_MAX) ==
-          hipSuccess &&
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, T, RES_LDS_MAX) == hipSuccess)
-    n = per_cu * cus;
-  else
+  for (int k = 0; k < nknown; k++)
+    if (known[k].dev == dev && known[k].fn == fn) return known[k].n;
+  int cus = 0, coop = 0, per_cu = 0;
+  size_t free = 0, total = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
+      hipMemGetInfo(&free, &total) != hipSuccess ||
+      hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS_MAX) !=
+          hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, T, RES_LDS_MAX) != hipSuccess) {
     (void)hipGetLastError();
-  known[key] = n;
+    return 0;  // asked again next time
+  }
+  if (free < RES_FREE_MIN) return 0;
+  const int n = coop ? per_cu * cus : 0;
+  if (nknown < (int)(sizeof known / sizeof known[0])) known[nknown++] = {dev, fn, n};
   return n;
 }
 

@@ -398,6 +398,11 @@ int64_t isph_footprint_bytes(int64_t n_cap, int64_t n_solid_cap,
  * static device array of fixed size (6 * ISPH_NOALLOC_MAX_ROWS doubles plus
  * ~2.3 MB, about 53 MB, held on every GPU the library runs on until the
  * process ends); the call makes no hipMalloc, hipFree or other allocation.
+ * The HIP runtime, though, sets up its queue for cooperative launches and the
+ * kernels' private memory at the first resident launch of each size class in a
+ * process (28 MiB in all, kept), as it loads code at a kernel's first launch.
+ * isph_ppe_solve_noalloc_limits with launches = 0 does without; so does a call
+ * that finds less than 256 MiB of device memory free.
  * All calls on one GPU share that array, so calls that overlap in time on
  * one GPU (from two host threads, or on two streams) race and must not be
  * made.  Rows longer than ISPH_NBR_CAP + 2 or columns outside [0, n) are

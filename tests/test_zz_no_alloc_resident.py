@@ -2,6 +2,8 @@
 launch-per-phase form (no resident launches allowed), bit for bit: at the edges
 of its launch shapes and of its scratch block, where its launches are refused
 half way, and where its waits run out."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -55,3 +57,33 @@ def test_noalloc_forms_agree(pkg):
             assert got == (k if fits else (0, 0, 0)), (n, name, c)
             assert out[name][0] == out["launches"][0], (n, name)
             assert np.array_equal(out[name][1], out["launches"][1]), (n, name)
+
+
+@pytest.mark.gpu
+def test_noalloc_takes_no_device_memory(pkg):
+    """Each launch shape's first resident launch apart, at which the runtime sets
+    up what it keeps; without resident launches, the first call apart."""
+    dv = DeviceArrays()
+
+    def free():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert dv.hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    for limits in ((0, 0, 0), (-1, 0, 0)):
+        for n in (3000, 65537, 131073, 262145):
+            ln, cs, vs, rhs, x0 = _system(pkg, n)
+            args = [dv.put(a) for a in (ln, cs, vs, rhs)]
+            xs = [dv.put(x0) for _ in range(3)]
+            taken = []
+            for d_x in xs:
+                before = free()
+                counts = {}
+                print(f"noalloc: n={n}, limits {limits}", flush=True)
+                pkg.ppe_solve_noalloc(n, n + 3, *args, d_x, 1e-12, 30, 2, check=False,
+                                      limits=limits, counts=counts)
+                taken.append(before - free())
+                assert counts["launches"] == (1 if limits[0] else 0)
+            assert taken[1:] == [0, 0], (n, limits, taken)
+            assert limits[0] or n == 3000 or taken[0] == 0, (n, taken)
+    dv.free()
