@@ -403,7 +403,9 @@ class Scenario:
         self._check(lib().isph_set_shape(self._ctx, TUNED_KERNELS.index(kernel),
                                          TUNE_SHAPES.index(shape)), "isph_set_shape")
 
-    def prof_enable(self, on: bool = True):
+    def prof_enable(self, on: bool | int = True):
+        """Kernel timers: True (1) of the launch-per-phase solves' kernels, 2 of
+        the resident launches (isph_prof_enable)."""
         self._check(lib().isph_prof_enable(self._ctx, int(on)), "isph_prof_enable")
 
     def prof_read(self, kernel: str):

@@ -1,4 +1,5 @@
-"""Algorithmic (compulsory) HBM bytes of the solver kernels.
+"""Algorithmic (compulsory) bytes of the solver kernels, launched phase by
+phase; of the resident solves (resident_iteration_bytes) below.
 
 Each kernel is charged for reading every input array once and writing every
 output once; values gathered at neighbour rows are assumed to come from cache
@@ -141,13 +142,47 @@ _ITER_PER_ROW = {"plain": 64 + 32, "precision": 4 * 16 + 32 + 72}
 _ITER_PER_NNZ = {"plain": 0, "precision": 4 * 4}
 
 
-def step_bytes(form: str, n: int, nnz: float, iters: float) -> float:
-    """Algorithmic HBM bytes of one step of `form` ("plain" or "precision")
-    over n particles with nnz stored PPE entries and `iters` iterations."""
+# Entries of each row that a resident solve keeps on the chip for the launch, by
+# row blocks (of 256 rows) per workgroup at most: (blocks, positions, and FP16
+# values in the precision form, FP64 values)
+_RESIDENT_KEPT = {"plain": ((1, 32, 32), (2, 32, 32), (4, 22, 7), (8, 22, 0), (12, 16, 0)),
+                  "precision": ((2, 24, 24), (4, 22, 0), (8, 14, 0), (12, 8, 0))}
+
+
+def resident_iteration_bytes(form: str, n: int, nnz: float) -> float | None:
+    """Bytes that one iteration of a resident solve of n rows reads and writes
+    beyond the chip's registers and LDS, each once: the entries that it does
+    not keep, the vectors of several rows per thread that it does not keep,
+    and the words of the exchanged vectors (8 B a value and half, written and
+    read).  They come from the caches between the chip and HBM where they fit
+    (the matrix of 653k rows is 163 MB; the memory-side cache 256 MB).  None
+    beyond the resident form's size."""
+    blocks = (n + 255) // 256
+    per = next((k for k in range(1, 13)
+                if (blocks + k - 1) // k + (1 if form == "precision" else 0) <= 256), None)
+    if per is None:
+        return None
+    pos, val = next(k[1:] for k in _RESIDENT_KEPT[form] if per <= k[0])
+    far_pos, far_val = max(0.0, nnz - pos * n), max(0.0, nnz - val * n)
+    several = per > 4
+    if form == "plain":
+        # two products; t1 and r, or p and s, as two words each; rh twice and x
+        return 2 * (2 * far_pos + 8 * far_val) + 2 * 32 * n + (32 * n if several else 0)
+    # four V-cycle passes (FP16) and two products (FP64); x0 and the V-cycle's
+    # result, twice an iteration, as a word each; x
+    return 4 * 4 * far_pos + 2 * (2 * far_pos + 8 * far_val) + 4 * 16 * n + 16 * n
+
+
+def step_bytes(form: str, n: int, nnz: float, iters: float, resident: bool = False) -> float:
+    """Algorithmic bytes of one step of `form` ("plain" or "precision") over n
+    particles with nnz stored PPE entries and `iters` iterations, of resident
+    solves or of the launch-per-phase ones."""
     particles = n * sum(_STEP_PER_PARTICLE.values()) + 12 * nnz
     if form == "plain":
         it = kernel_bytes("k_bicg_1", n, nnz) + kernel_bytes("k_bicg_2", n, nnz)
     else:
         it = kernel_bytes("kb_pb_1", n, nnz) + kernel_bytes("kb_pb_2", n, nnz)
     it += n * _ITER_PER_ROW[form] + nnz * _ITER_PER_NNZ[form]
+    if resident:
+        it = resident_iteration_bytes(form, n, nnz)
     return particles + iters * it

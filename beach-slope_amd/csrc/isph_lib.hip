@@ -89,12 +89,14 @@ struct isph_ctx {
   // piston wavemaker: stroke, period, ramp time and start time of the paddle motion
   bool wave = false;
   double wv_stroke = 0.0, wv_period = 1.0, wv_ramp = 0.0, wv_t0 = 0.0;
-  bool prof = false;
+  bool prof = false;      // kernel timers on (the solves run launch by launch)
+  bool prof_res = false;  // the timer of the resident launches on
   // per_iter of mg_down and mg_up (2 x the multi-workgroup cell levels) is
   // set by each solve
-  KTimer timers[11] = {{"spmv_p", 1},    {"spmv_s", 1},  {"spmv_p32", 1},     {"spmv_s32", 1},
+  KTimer timers[12] = {{"spmv_p", 1},    {"spmv_s", 1},  {"spmv_p32", 1},     {"spmv_s32", 1},
                        {"mg_coarse", 2}, {"mg_pre0", 2}, {"mg_post0", 2},     {"mg_down", 0},
-                       {"mg_up", 0},     {"pfinalize", 2}, {"mg_restrict0", 2}};
+                       {"mg_up", 0},     {"pfinalize", 2}, {"mg_restrict0", 2},
+                       {"resident", 0}};
   Dev D;
   hipStream_t stream = nullptr;
   int64_t cap = 0, scap = 0, ns = 0;  // particle and solid capacities, solids
@@ -859,6 +861,20 @@ static void timers_collect(isph_ctx* c, int64_t keep) {
   }
 }
 
+// launch() between two events of c's resident timer, when it is on; the caller
+// collects after it has waited for the launch
+template <typename F>
+static hipError_t timed_resident(isph_ctx* c, F launch) {
+  if (!c->prof_res) return launch();
+  KTimer& t = c->timers[11];
+  const std::pair<hipEvent_t, hipEvent_t> ev = timer_pair(t);
+  (void)hipEventRecord(ev.first, c->stream);
+  const hipError_t e = launch();
+  (void)hipEventRecord(ev.second, c->stream);
+  (e == hipSuccess ? t.pending : t.pool).push_back(ev);
+  return e;
+}
+
 // A timed launch of a row kernel: the two events are attached to the kernel's own dispatch
 // (hipExtLaunchKernelGGL), so their difference is the kernel's execution
 // time without the gaps around it.
@@ -883,7 +899,8 @@ extern "C" int isph_prof_enable(isph_ctx* c, int32_t on) {
   if (!c) return ISPH_EARG;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   timers_collect(c, -1);
-  c->prof = on != 0;
+  c->prof = on != 0 && on != 2;
+  c->prof_res = on == 2;
   for (KTimer& t : c->timers) {
     t.total_ms = 0;
     t.launches = 0;
@@ -1439,7 +1456,9 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
       return ISPH_ENOCONV;
     }
     if (resident) {
-      if (left != 0 && bh_resident(b, B, riters, vtag, ep) == hipSuccess) {
+      if (left != 0 && timed_resident(c, [&] {
+            return bh_resident(b, B, riters, vtag, ep);
+          }) == hipSuccess) {
         for (isph_ctx* q : b->ctx) q->rcount[RC_LAUNCH]++;
         if (left > 0) left--;
         vtag += 2u * (unsigned)riters;
@@ -1493,6 +1512,7 @@ static int bh_solve(BatchHost* b, isph_solve_stats* stats) {
       rs_prev[s] = b->sc[s].restarts;
     }
     if (c->prof) timers_collect(c, worked);
+    if (c->prof_res) timers_collect(c, -1);
     if (restarted) {
       const int p = predicted(true);
       guessed = p > 0;
@@ -1537,7 +1557,9 @@ static int bicg_loop(isph_ctx* c, const ResPlan* plan, int* iters_out, int* brk_
       // a refused launch (another process holds the device's cooperative
       // queue) leaves the state as it was: the solve goes on launch by launch
       if (left != 0 &&
-          res_launch(*plan, c->D, c->ps, c->lim.iters, ep, c->stream) == hipSuccess) {
+          timed_resident(c, [&] {
+            return res_launch(*plan, c->D, c->ps, c->lim.iters, ep, c->stream);
+          }) == hipSuccess) {
         c->rcount[RC_LAUNCH]++;
         if (left > 0) left--;
         chunk = c->lim.iters;
@@ -1582,6 +1604,7 @@ static int bicg_loop(isph_ctx* c, const ResPlan* plan, int* iters_out, int* brk_
     }
     // the timed launches that did work: the chunk's leading iterations
     if (c->prof) timers_collect(c, s.iters - prev);
+    if (c->prof_res) timers_collect(c, -1);
     prev = s.iters;
     if (s.done) {
       if (s.brk && !s.conv && s.iters < c->P.max_iter && restarts < c->P.max_outer) {

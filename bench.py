@@ -20,25 +20,23 @@ like for like.  `value` is the chosen form.
 
 Each form also reports the whole step against the HBM roofline: its
 algorithmic bytes per particle-step (bytes_model.step_bytes, at the measured
-iteration count), the rate that gives at the measured speed, and the
-fraction of the 8 TB/s peak.
+iteration count), the rate that gives at the measured speed, and its ratio to
+the 8 TB/s peak (of HBM; at this size part of the bytes come from the caches).
 
-The roofline object is for the headline form's dominant kernel: the
-solver's kernels (the two SpMVs, the V-cycle's level-0 passes, level-1
-restriction, cell-level down and up passes and coarse workgroup, and the
-dot-product finalizes; together ~90% of a step's kernel time) are timed with
-HIP events on the context's stream over as many steps again, right after
-the timed region (the timed region runs without them: its solves are one
-resident launch each, and with the events on they run as a launch per
-phase), and the kernel function with the most time per step (all
-its launches: both applications of the V-cycle, every cell level) is
-reported, with its algorithmic bytes per launch (bytes_model) over its mean
-launch time.  Its
-`traffic` (HBM bytes per launch) comes from the FETCH_SIZE / WRITE_SIZE
-counter passes summarised in profiles/traffic_flume_650k.md, when that file
-holds the kernel.  The CPU baseline is the oracle (a C/OpenMP restatement of
-the reference) on a bounded sample of the same workload: one untimed step,
-then three timed steps.
+The roofline object is for the headline form's dominant kernel in the timed
+steps, the resident solve: HIP events around its launch over as many steps
+again, right after the timed region, with the bytes of its iterations beyond
+the chip (bytes_model.resident_iteration_bytes) over its mean launch time.
+`traffic` is what a launch moves in and out of the L2s by the FETCH_SIZE /
+WRITE_SIZE counter passes summarised in profiles/traffic_flume_650k.md, when
+that file holds the kernel.  Where the solve does not run resident, the kernel
+is the launch-per-phase form's with the most time per step.  That form's
+kernels (the two SpMVs, the V-cycle's level-0 passes, level-1 restriction,
+cell-level down and up passes and coarse workgroup, and the dot-product
+finalizes) are timed over a third set of steps, launched phase by phase, and
+reported as `timed_kernels`.  The CPU baseline is the oracle (a C/OpenMP
+restatement of the reference) on a bounded sample of the same workload: one
+untimed step, then three timed steps.
 
 Three more legs run by default, at bounded sizes, and go into the same line:
   precision_errors  the jittered dam break, 200 steps in each form: pressure,
@@ -105,8 +103,7 @@ def run_gpu(pkg, case, precision: int, steps: int, warmup: int, tol: float, tune
         g.step(1)
     # launch shapes of the particle kernels, timed on the warmed-up state
     shapes = _shapes(g.autotune(trials=3)) if tune else None
-    # the timed region runs without the per-kernel HIP-event timers: their
-    # events cost ~10% of a precision-form step at 650k
+    # the timed region runs without the kernel timers
     iters, outer = [], []
     nnz = 0.0
     t0 = time.perf_counter()
@@ -116,8 +113,12 @@ def run_gpu(pkg, case, precision: int, steps: int, warmup: int, tol: float, tune
         outer.append(st.outer)
         nnz = st.nnz
     t1 = time.perf_counter()
-    # kernel durations: as many further steps with the timers on
-    g.prof_enable(True)
+    # the resident launches' durations, then those of the launch-per-phase
+    # form's kernels: as many further steps with each timer on
+    g.prof_enable(2)
+    res_iters = sum(g.step(1)[1].iterations for _ in range(steps))
+    res_ms, res_launches = g.prof_read("resident")
+    g.prof_enable(1)
     prof_iters = []
     for _ in range(steps):
         _, st = g.step(1)
@@ -141,21 +142,30 @@ def run_gpu(pkg, case, precision: int, steps: int, warmup: int, tol: float, tune
     g.prof_enable(False)
     g.close()
     wall = t1 - t0
-    # the dominant kernel: the most time per step
-    kname = max(timed, key=lambda k: timed[k]["ms_per_step"])
+    form = "precision" if precision else "plain"
+    resident = res_launches > 0
+    if resident:
+        kb = bytes_model.resident_iteration_bytes(form, n, nnz) * res_iters / res_launches
+        avg = 1e3 * res_ms / res_launches
+        timed["resident"] = dict(kernel=KERNEL_OF["resident"][precision],
+                                 ms_per_step=res_ms / steps, launches=res_launches, avg_us=avg,
+                                 bytes=kb, gbs=kb / (avg * 1e-6) / 1e9,
+                                 iterations_per_launch=res_iters / res_launches)
+    # the dominant kernel of the timed steps: the resident solve, else the one
+    # with the most time per step
+    kname = "resident" if resident else max(timed, key=lambda k: timed[k]["ms_per_step"])
     avg_us, launches = timed[kname]["avg_us"], timed[kname]["launches"]
     bytes_per, achieved = timed[kname]["bytes"], timed[kname]["gbs"]
     # the whole step against the HBM roofline: algorithmic bytes per step
     # (bytes_model.step_bytes) at the measured rate, over the 8 TB/s peak
-    step_b = bytes_model.step_bytes("precision" if precision else "plain", n, nnz,
-                                    float(np.mean(iters)))
+    step_b = bytes_model.step_bytes(form, n, nnz, float(np.mean(iters)), resident)
     step_gbs = step_b * steps / wall / 1e9
     return dict(
         n=n, seconds=wall, ms_per_step=1e3 * wall / steps,
         particle_steps_per_s=n * steps / wall, iters_mean=float(np.mean(iters)),
         outer_mean=float(np.mean(outer)), nnz_per_row=nnz / n,
         timer_steps_iters_mean=float(np.mean(prof_iters)),
-        kernel=kname, kernel_avg_us=avg_us, kernel_launches=launches,
+        kernel=timed[kname]["kernel"], kernel_timer=kname, kernel_avg_us=avg_us, kernel_launches=launches,
         kernel_bytes=bytes_per, kernel_gbs=achieved,
         timed_kernels={k: {kk: (round(vv, 4) if isinstance(vv, float) else vv)
                            for kk, vv in v.items()} for k, v in timed.items()},
@@ -446,7 +456,8 @@ def run_flume_full(pkg, cases, steps: int, tol: float) -> dict:
 KERNEL_OF = {"spmv_p": "k_bicg_1", "spmv_s": "k_bicg_2", "spmv_p32": "kb_pb_1",
              "spmv_s32": "kb_pb_2", "mg_pre0": "kb_mg_pre0", "mg_post0": "kb_mg_post0",
              "mg_coarse": "kb_mg_coarse", "mg_restrict0": "kb_mg_restrict0",
-             "mg_down": "kb_mg_down", "mg_up": "kb_mg_up", "pfinalize": "kb_pfinalize"}
+             "mg_down": "kb_mg_down", "mg_up": "kb_mg_up", "pfinalize": "kb_pfinalize",
+             "resident": ("k_bicg_resident", "kb_pb_resident")}
 TIMED_PLAIN = ("spmv_p", "spmv_s")
 TIMED_PRECISION = ("spmv_p32", "spmv_s32", "mg_pre0", "mg_post0", "mg_restrict0", "mg_down",
                    "mg_coarse", "mg_up", "pfinalize")
@@ -455,12 +466,13 @@ TRAFFIC_FILE = pathlib.Path(__file__).resolve().parent / "profiles" / "traffic_f
 
 
 def measured_traffic(kernel: str):
-    """HBM bytes per launch of `kernel` from the counter summary, or None."""
+    """Bytes per launch of `kernel` (per iteration of a resident one) from the
+    counter summary, or None."""
     if not TRAFFIC_FILE.exists():
         return None
     for line in TRAFFIC_FILE.read_text().splitlines():
         m = re.match(r"^traffic\s+(\S+)\s+([0-9.eE+]+)\s*$", line.strip())
-        if m and m.group(1) == KERNEL_OF.get(kernel, kernel):
+        if m and m.group(1) == kernel:
             return float(m.group(2))
     return None
 
@@ -585,6 +597,10 @@ def main() -> int:
     if not args.no_cpu:
         cpu = cpu_baseline(entry.load_oracle(), c, args.tol)
         print(f"bench: cpu {cpu}", file=sys.stderr, flush=True)
+    dominant = head["timed_kernels"][head["kernel_timer"]]
+    traffic = measured_traffic(head["kernel"])
+    if traffic is not None:
+        traffic *= dominant.get("iterations_per_launch", 1)
     out = {
         "metric": METRIC,
         "value": head["particle_steps_per_s"],
@@ -606,10 +622,10 @@ def main() -> int:
                    "form": "chosen" if "chosen" in res else "plain"},
         "roofline": {"bound": "hbm", "achieved": head["kernel_gbs"], "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": head["kernel_gbs"] / HBM_PEAK_GBS,
-                     "traffic": measured_traffic(head["kernel"]),
-                     "kernel": KERNEL_OF[head["kernel"]],
+                     "traffic": traffic,
+                     "kernel": head["kernel"],
                      "avg_launch_us": head["kernel_avg_us"],
-                     "ms_per_step": head["timed_kernels"][head["kernel"]]["ms_per_step"]},
+                     "ms_per_step": dominant["ms_per_step"]},
         "cpu_baseline": cpu,
         "precision_errors": errors,
         "batched": batched,

@@ -311,11 +311,13 @@ int isph_batch_set_graph(isph_batch *b, int32_t on);
 int isph_batch_autotune(isph_batch *b, int32_t trials, int32_t *shape, double *us);
 
 /* ---- kernel timing (HIP events on the context's stream) ----
- * When enabled, every launch of the solver's timed kernels is bracketed by
- * a pair of HIP events (the solves then run as a launch per phase rather than
- * as one resident launch; results are the same); isph_prof_read returns the summed event time and the
- * launch count per kernel (launches after the solve has finished are left
- * out).  kernel: "spmv_p" (t = A p), "spmv_s" (t = A s) of the FP64 form;
+ * on = 1: every launch of the solver's timed kernels is bracketed by a pair of
+ * HIP events; the solves then run as a launch per phase rather than as resident
+ * launches.  on = 2: the solves run as they do untimed, and their resident
+ * launches are bracketed.  Results are the same.  isph_prof_read returns the
+ * summed event time and the launch count per kernel (launches after the solve
+ * has finished are left out).  kernel: "resident" (on = 2; in a batch, of its
+ * first context); "spmv_p" (t = A p), "spmv_s" (t = A s) of the FP64 form;
  * "spmv_p32", "spmv_s32" (t1 = A ph, t2 = A sh), "mg_pre0", "mg_post0" (the
  * V-cycle's level-0 passes), "mg_restrict0" (the restriction to level 1),
  * "mg_down", "mg_up" (the multi-workgroup cell levels, every level),
