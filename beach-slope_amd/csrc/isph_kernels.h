@@ -366,7 +366,7 @@ __global__ void k_scan_tiles(const int32_t* in, int32_t* out, int32_t* tile_sums
   scan_tile_body(in, out, tile_sums, len, blockIdx.x);
 }
 
-__device__ __forceinline__ void scan_sums_body(int32_t* tile_sums, int ntiles, int32_t* total_out) {
+__device__ __forceinline__ void scan_sums_body(int32_t* tile_sums, int ntiles) {
   __shared__ int32_t s[256];
   const int t = threadIdx.x;
   int32_t carry = 0;
@@ -385,18 +385,25 @@ __device__ __forceinline__ void scan_sums_body(int32_t* tile_sums, int ntiles, i
     __syncthreads();
     carry += tot;
   }
-  if (t == 0 && total_out) *total_out = carry;
 }
+__global__ void k_scan_sums(int32_t* tile_sums, int ntiles) { scan_sums_body(tile_sums, ntiles); }
 // Adds the sums of the tiles before it to a tile, which each workgroup sums for
-// itself: at 200 tiles (653k particles) that is one load a thread, and the scan
-// is a launch shorter (offsets and addition 2.6 + 2.4 us at 22k particles, 4.7 + 4.9
-// at 653k as two launches; 3.2 and 4.8 as one).
-__global__ void __launch_bounds__(256) k_scan_add(int32_t* out, const int32_t* tile_sums,
-                                                  int len) {
+// itself up to SCAN_DIRECT tiles: at 200 tiles (653k particles) that is one load a
+// thread, and the scan is a launch shorter (offsets and addition 2.6 + 2.4 us at
+// 22k particles, 4.7 + 4.9 at 653k as two launches; 3.2 and 4.8 as one).  The
+// loads grow with the tiles' square: a rebin over 2.25M cells (22k tiles) takes
+// 256 us with the launch for the offsets and 243 without, over 9M 989 and 1,660,
+// over 36M 3.8 and 15.8 ms.
+#define SCAN_DIRECT 16384
+__global__ void __launch_bounds__(256) k_scan_add(int32_t* out, const int32_t* tile_sums, int len,
+                                                  int direct) {
   __shared__ int32_t s[4];
   const int t = threadIdx.x, tile = blockIdx.x;
   int32_t a = 0;
-  for (int k = t; k < tile; k += 256) a += tile_sums[k];
+  if (direct)
+    for (int k = t; k < tile; k += 256) a += tile_sums[k];
+  else if (t == 0)
+    a = tile_sums[tile];
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) a += __shfl_xor(a, m, 64);
   if ((t & 63) == 0) s[t >> 6] = a;

@@ -992,8 +992,11 @@ static int scan_bins(isph_ctx* c, int len) {
   const int ntiles = (len + SCAN_TILE - 1) / SCAN_TILE;
   hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(256), 0, c->stream, c->D.bincnt,
                      c->D.binstart, c->D.scan_tmp, len);
+  const int direct = ntiles <= SCAN_DIRECT;
+  if (!direct)
+    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(256), 0, c->stream, c->D.scan_tmp, ntiles);
   hipLaunchKernelGGL(k_scan_add, dim3(ntiles), dim3(256), 0, c->stream, c->D.binstart,
-                     c->D.scan_tmp, len);
+                     c->D.scan_tmp, len, direct);
   HIPCHK(c, hipGetLastError());
   return 0;
 }

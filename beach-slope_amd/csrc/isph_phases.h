@@ -145,7 +145,7 @@ __global__ void kb_scan_tiles(PhaseBatch B) {
 }
 __global__ void kb_scan_sums(PhaseBatch B) {
   const Dev& D = B.devs[blockIdx.x];
-  scan_sums_body(D.scan_tmp, (phase_nbins(D) + SCAN_TILE - 1) / SCAN_TILE, nullptr);
+  scan_sums_body(D.scan_tmp, (phase_nbins(D) + SCAN_TILE - 1) / SCAN_TILE);
 }
 __global__ void kb_scan_add(PhaseBatch B) {
   PH_IDX(B, PH_BIN);
