@@ -1210,12 +1210,36 @@ static int64_t rs_shape(BatchHost* b) {
   return rs_row_lds<T, R>();
 }
 
+// Whether the row workgroups of a resident launch of b (rs_T threads each, nbw
+// row blocks) get through the cells of level 1 as fast as the launches do, which
+// have a thread per cell: a cell here costs some thirty polled words a V-cycle.
+// Times of a solve of 40 iterations, launches / resident, in ms, on flumes (and
+// the dam of 25k) in ever wider domains:
+//   rows   threads       cells: ms
+//   25k    98 x 512      25k: 4.6/2.5   75k: 5.2/4.4   100k: 5.4/5.3   150k: 5.6/7.3
+//   119k   233 x 512     59k: 5.5/4.1   89k: 5.7/5.2   119k: 5.8/6.2   238k: 6.4/10.7
+//   171k   223 x 1,024   114k: 6.2/4.7  171k: 6.5/5.9  228k: 6.7/7.3   456k: 7.8/11.8
+//   327k   214 x 1,024   109k: 7.3/5.2  164k: 7.5/6.5  219k: 7.7/7.9   437k: 8.7/12.6
+//   621k   243 x 1,024   123k: 9.7/7.2  185k: 10.0/8.8 248k: 10.4/11.0 496k: 11.5/17.7
+// and with few workgroups from some four cells per thread on (7.5k rows, 30 x
+// 512: 4.6/4.0 at three).  A domain full of fluid has a cell for ~16 rows.
+static bool rs_cells_fit(const BatchHost* b, int nbw) {
+  int64_t cells = 0;
+  for (const isph_ctx* c : b->ctx) {
+    const int64_t n = c->G.lev[1].n, G = (c->D.nblk + nbw - 1) / nbw;
+    if (n > 4 * G * b->rs_T) return false;
+    cells += n;
+  }
+  return cells <= (int64_t)184 * b->rs_T;
+}
+
 // The resident launch of b's scenarios: the fewest row blocks per workgroup
 // with which every scenario's row workgroups and its coarse one fit the
 // device at one per CU, and the coarse workgroups' first levels.  Leaves
 // rs_grid 0 where the solve has to run launch by launch: kernel timing on,
 // more than 12 row blocks per workgroup, a loaded system, a scenario whose
-// resident form lately came to nothing, or a device that cannot hold the grid.
+// resident form lately came to nothing, too many cells (rs_cells_fit), or a
+// device that cannot hold the grid.
 static void bh_plan(BatchHost* b) {
   b->rs_grid = 0;
   bool tried = true;
@@ -1234,6 +1258,7 @@ static void bh_plan(BatchHost* b) {
                 : nbw <= 4 ? rs_shape<1024, 1>(b)
                 : nbw <= 8 ? rs_shape<1024, 2>(b)
                            : rs_shape<1024, 3>(b);
+  if (!rs_cells_fit(b, nbw)) return;
   int wg0 = 0;
   for (int s = 0; s < b->S; s++) {
     isph_ctx* c = b->ctx[s];

@@ -1,5 +1,7 @@
-"""The rebin's scan over cell grids on both sides of the size at which it takes
-a pass of its own for the tiles' offsets."""
+"""Domains with many more cells than their particles fill: the rebin's scan on
+both sides of the size at which it takes a pass of its own for the tiles'
+offsets, and the precision solve on both sides of the cells that its resident
+form takes on."""
 import numpy as np
 import pytest
 
@@ -32,3 +34,28 @@ def test_rebin_over_a_wide_grid(pkg, cases, cells):
         moved += int((before != cell).sum())
     s.close()
     assert moved > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dx,cells,resident", [
+    (0.0025, (290, 320), True), (0.0025, (300, 320), False),  # of 94,208 in all
+    (0.02, (80, 100), True), (0.02, (84, 100), False),        # of 4 per thread, 2,048 threads
+])
+def test_cells_of_a_resident_solve(pkg, cases, dx, cells, resident):
+    out = []
+    for timed in (True, False):
+        c = cases.dam_break(dx=dx)
+        c.params.update(cellx=cells[0], celly=cells[1], precision=1, tol=1e-9, max_iter=30,
+                        max_outer=1)
+        off = 4.0 * c.params["h"] * 5
+        c.parts["x"], c.parts["y"] = c.parts["x"] + off, c.parts["y"] + off
+        print(f"cells: {cells}, n={c.n}, timed {timed}", flush=True)
+        s = pkg.Scenario(c)
+        s.init_state()
+        s.prof_enable(timed)
+        rc, st = s.step(1, check=False)
+        out.append((rc, st.iterations, st.rel_residual, s.solution(), s.resident_counts()))
+        s.close()
+    assert out[1][4]["launches"] == int(resident) and out[1][4]["too_wide"] == 0
+    assert out[0][:3] == out[1][:3] and out[0][1] > 3
+    assert np.array_equal(out[0][3], out[1][3])
