@@ -1336,7 +1336,10 @@ __global__ void __launch_bounds__(256) k_comp_vel(Dev D) {
 // first step.  Each block of 256 cells leaves the maxima over its cells for
 // timestep (non-negative doubles compare as their bits).  LPC lanes per cell:
 // with one, a cell's rows are two dependent trips of 32 loads on a chip nearly
-// empty (12 us at 22k particles, 16.5 at 653k; four lanes: 7 and 11).
+// empty (12 us at 22k particles, 16.5 at 653k; four lanes: 7 and 11).  Empty cells
+// cost four times the lanes: comp_vel with its maxima took 48 us with one lane
+// and 37 with four over 243k cells, 81 and 83 over 478k, 91 and 180 over 4.8M.
+#define CELL_MAX_LANES4 (1 << 18)  // cells up to which four lanes take one
 template <int LPC>
 __device__ __forceinline__ void cell_max_cell(const Dev& D, int ncell, int init, int blk) {
   constexpr int U = LPC == 1 ? 8 : 4;
@@ -1396,8 +1399,9 @@ __device__ __forceinline__ void cell_max_cell(const Dev& D, int ncell, int init,
   }
 }
 
-__global__ void __launch_bounds__(1024) k_cell_max(Dev D, int ncell, int init) {
-  cell_max_cell<4>(D, ncell, init, blockIdx.x);
+template <int LPC>
+__global__ void __launch_bounds__(256 * LPC) k_cell_max(Dev D, int ncell, int init) {
+  cell_max_cell<LPC>(D, ncell, init, blockIdx.x);
 }
 
 // comp_pos, integrator.f90:845-883

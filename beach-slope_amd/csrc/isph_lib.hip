@@ -1757,12 +1757,19 @@ extern "C" int isph_ppesolve(isph_ctx* c, isph_solve_stats* stats) {
   return isph_ppe_solve(c, stats);
 }
 
+static hipError_t launch_cell_max(isph_ctx* c, int init) {
+  const dim3 grid(grid_of(c->ncell));
+  if (c->ncell <= CELL_MAX_LANES4)
+    hipLaunchKernelGGL(k_cell_max<4>, grid, dim3(1024), 0, c->stream, c->D, c->ncell, init);
+  else
+    hipLaunchKernelGGL(k_cell_max<1>, grid, dim3(256), 0, c->stream, c->D, c->ncell, init);
+  return hipGetLastError();
+}
+
 extern "C" int isph_comp_vel(isph_ctx* c) {
   if (!c) return ISPH_EARG;
   TLAUNCH(TK_COMPVEL, k_comp_vel);
-  hipLaunchKernelGGL(k_cell_max, dim3(grid_of(c->ncell)), dim3(1024), 0, c->stream, c->D,
-                     c->ncell, 0);
-  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, launch_cell_max(c, 0));
   return 0;
 }
 extern "C" int isph_comp_pos(isph_ctx* c) {
@@ -1812,9 +1819,7 @@ extern "C" int isph_init_state(isph_ctx* c) {
   if (rc) return rc;
   TLAUNCH(TK_EFFPOR, k_effpor);
   TLAUNCH(TK_EDDYVIS, k_eddyvis);
-  hipLaunchKernelGGL(k_cell_max, dim3(grid_of(c->ncell)), dim3(1024), 0, c->stream, c->D,
-                     c->ncell, 1);
-  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, launch_cell_max(c, 1));
   rc = isph_timestep(c);
   if (rc) return rc;
   return sync(c);
@@ -2090,9 +2095,7 @@ static int step_pre(isph_ctx* c) {
 // check: read the error bits now (else the next step_pre's scalar read does)
 static int step_post(isph_ctx* c, bool check) {
   TLAUNCH(TK_COMPVEL, k_comp_vel);
-  hipLaunchKernelGGL(k_cell_max, dim3(grid_of(c->ncell)), dim3(1024), 0, c->stream, c->D,
-                     c->ncell, 0);
-  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, launch_cell_max(c, 0));
   LAUNCH(k_comp_pos, c->n_hi, c->D);
   int rc = rebin(c, 1);
   if (rc) return rc;

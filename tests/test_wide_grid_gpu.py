@@ -1,7 +1,8 @@
 """Domains with many more cells than their particles fill: the rebin's scan on
 both sides of the size at which it takes a pass of its own for the tiles'
-offsets, and the precision solve on both sides of the cells that its resident
-form takes on."""
+offsets, the cell maxima on both sides of the size to which four lanes share a
+cell, and the precision solve on both sides of the cells that its resident form
+takes on."""
 import numpy as np
 import pytest
 
@@ -59,3 +60,31 @@ def test_cells_of_a_resident_solve(pkg, cases, dx, cells, resident):
     assert out[1][4]["launches"] == int(resident) and out[1][4]["too_wide"] == 0
     assert out[0][:3] == out[1][:3] and out[0][1] > 3
     assert np.array_equal(out[0][3], out[1][3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cells", [(512, 512), (513, 512)])
+def test_cell_maxima(pkg, cases, cells):
+    """umax is the largest pore velocity of the fluid whatever the grid."""
+    c = cases.dam_break(dx=0.005)
+    c.params.update(cellx=cells[0], celly=cells[1], tol=1e-6, max_iter=50, max_outer=0)
+    fl = c.parts["tid"] == 3
+    rng = np.random.default_rng(5)
+    c.parts["u"][fl] = rng.uniform(-0.3, 0.3, fl.sum())
+    off = 4.0 * c.params["h"] * 200
+    c.parts["x"], c.parts["y"] = c.parts["x"] + off, c.parts["y"] + off
+    print(f"cell maxima: {cells}", flush=True)
+    s = pkg.Scenario(c)
+    s.init_state()
+    for ph in ("projection", "cellshift", "neighbour", "effpor", "eddyvis", "int_vel"):
+        getattr(s, ph)()
+    s.ppe_assemble()
+    s.ppe_solve(check=False)
+    s.comp_vel()
+    d, p = s.download(), s.props()
+    s.timestep()
+    um = s.scalars().umax
+    fl = (d["tid"] == 3) & ((d["flags"] & 1) == 0)
+    want = np.sqrt(d["u"] * d["u"] + d["v"] * d["v"]) / p["porosity"]
+    assert um == want[fl].max() == p["vel"][fl].max() and um > 0.0
+    s.close()
