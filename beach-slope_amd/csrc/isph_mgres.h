@@ -177,32 +177,8 @@ __global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
     Q.bw[c] = 0;
     Q.ew[c] = 0;
   }
-  for (int c = t; c < nch; c += T) map[c] = 0;
-  __syncthreads();
-  for (int i = i0 + t; i < i1; i += T) {
-    const int L = alen[i];
-    map[i / PS_CHUNK] = 1;  // its own rows, in order, whatever the columns
-    for (int k0 = 0; k0 < L; k0 += 8) {
-      int c[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) c[u] = acol[((k0 + u < L) ? k0 + u : k0) * cap + i];
-#pragma unroll
-      for (int u = 0; u < 8; u++) map[c[u] / PS_CHUNK] = 1;
-    }
-  }
-  __syncthreads();
-  const int per = (nch + T - 1) / T, c0 = t * per, c1 = min(nch, c0 + per);
-  int own = 0;
-  for (int c = c0; c < c1; c++) own += map[c];
-  cnt[t] = own;
-  __syncthreads();
-  for (int off = 1; off < T; off <<= 1) {
-    const int a = (t >= off) ? cnt[t - off] : 0;
-    __syncthreads();
-    cnt[t] += a;
-    __syncthreads();
-  }
-  const int total = cnt[T - 1];
+  int own;
+  const int total = ps_window_chunks<T>(acol, alen, cap, i0, i1, nch, map, cnt, own);
   // rows of the last cell in later workgroups (rs_rows_solve's tail)
   int tail = 0;
   if (i1 > i0 && i1 < n) {
@@ -213,14 +189,8 @@ __global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
     if (t == 0) atomicOr(&D.sc->counter[PS_FLAG_WIN], 1u);
     return;
   }
-  int pos = cnt[t] - own;
-  for (int c = c0; c < c1; c++)
-    if (map[c]) {
-      Q.wlist[(size_t)wg * RS_WCAP + pos] = c;
-      if (c == i0 / PS_CHUNK) Q.wcnt[2 * wg + 1] = pos;
-      map[c] = (uint16_t)pos++;
-    }
-  if (t == 0) Q.wcnt[2 * wg] = total;
+  int32_t* wlist = Q.wlist + (size_t)wg * RS_WCAP;
+  ps_window_list<T>(i0, nch, own, total, map, cnt, wlist, Q.wcnt + 2 * wg);
   if (rs_cells(R) > 0) {
     // the window's cells (a chunk's rows lie in cell order), of which
     // rs_rows_solve takes rs_cells per thread
@@ -228,7 +198,7 @@ __global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
     __syncthreads();
     int mine = 0;
     for (int p = t; p < total * PS_CHUNK; p += T) {
-      const int g = Q.wlist[(size_t)wg * RS_WCAP + p / PS_CHUNK] * PS_CHUNK + p % PS_CHUNK;
+      const int g = wlist[p / PS_CHUNK] * PS_CHUNK + p % PS_CHUNK;
       if (g < n && (g % PS_CHUNK == 0 || D.cell[g] != D.cell[g - 1])) mine++;
     }
     atomicAdd(&cnt[0], mine);
@@ -236,21 +206,7 @@ __global__ void __launch_bounds__(T) kb_rs_setup(BatchDev B, const ResDev* rs) {
     if (cnt[0] > rs_cells(R) * T && t == 0) atomicOr(&D.sc->counter[PS_FLAG_WIN], 1u);
   }
   __syncthreads();
-  for (int i = i0 + t; i < i1; i += T) {
-    const int L = alen[i];
-    for (int k0 = 0; k0 < L; k0 += 8) {
-      int c[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) c[u] = acol[((k0 + u < L) ? k0 + u : k0) * cap + i];
-#pragma unroll
-      for (int u = 0; u < 8; u += 2) {
-        if (k0 + u >= L) break;
-        const uint32_t a = map[c[u] / PS_CHUNK] * PS_CHUNK + c[u] % PS_CHUNK;
-        const uint32_t b = map[c[u + 1] / PS_CHUNK] * PS_CHUNK + c[u + 1] % PS_CHUNK;
-        lidx[((k0 + u) >> 1) * cap + i] = a | (b << 16);
-      }
-    }
-  }
+  ps_window_positions<T>(acol, alen, cap, i0, i1, map, lidx, cap);
 }
 
 // ---------------------------------------------------------------------
@@ -579,15 +535,8 @@ struct RsScalars {
   int iters, conv, brk, done;
   bool update;  // the stopped iteration's x and r update still applies
 };
-// a value that is the same in every lane, out of the vector registers
-__device__ __forceinline__ double rs_uni(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readfirstlane((int)b);
-  const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
 __device__ __forceinline__ void rs_alpha(RsScalars& z, double s0) {
-  z.alpha = rs_uni(z.rho / s0);
+  z.alpha = lane0(z.rho / s0);
   if (!isfinite(z.alpha)) {
     z.brk = 1;
     z.done = 1;
@@ -595,7 +544,7 @@ __device__ __forceinline__ void rs_alpha(RsScalars& z, double s0) {
 }
 __device__ __forceinline__ void rs_omega(RsScalars& z, const double (&s)[5], double stop,
                                          double bnorm, int max_iter) {
-  const double om = rs_uni(s[0] / s[1]);
+  const double om = lane0(s[0] / s[1]);
   z.omega = om;
   z.update = false;
   if (!isfinite(om) || om == 0.0) {
@@ -616,8 +565,8 @@ __device__ __forceinline__ void rs_omega(RsScalars& z, const double (&s)[5], dou
     z.brk = 1;
     z.done = 1;
   } else {
-    z.beta = rs_uni((rhon / z.rho) * (z.alpha / om));
-    z.rho = rs_uni(rhon);
+    z.beta = lane0((rhon / z.rho) * (z.alpha / om));
+    z.rho = lane0(rhon);
     if (z.iters >= max_iter) z.done = 1;
   }
 }

@@ -21,12 +21,20 @@
 // 64-row chunks that its rows' columns fall into (its window: its own rows
 // and a strip on each side, since rows are sorted by cell) and rewrites each
 // column as a 16-bit position in that window.  The products gather from the
-// window in LDS.  A workgroup's threads keep r, t1 and p of the window's
-// elements in registers: t1 and r of other workgroups' rows are read while
-// the reduction after their production is under way, and
+// window in LDS.  With one row per thread a workgroup's threads keep r, t1 and p
+// of the window's elements in registers: t1 and r of other workgroups' rows are
+// read while the reduction after their production is under way, and
 // p = r + beta (p - omega t1) is formed for the window by the same expression
-// as at its owner, so p is never exchanged.  Rows whose window does not fit
-// (wlist's capacity) leave the flag set and the solve runs launch by launch.
+// as at its owner, so p is not exchanged.  With several rows per thread those
+// registers hold the rows' own vectors, and p and s themselves are exchanged.
+//
+// What fits.  The columns of a workgroup's rows lie in the cell columns on either
+// side, not further up or down than its own rows and a cell more.  Up to seven
+// row blocks per workgroup (~458k rows) that fits the window however high the
+// cell columns; beyond, they may have some (6,144 - own rows) / 2 - 250 rows:
+// basins 360 particles deep fit and 380 do not at eight blocks, 320 and 340 at
+// ten, 270 and 280 at twelve.  Other systems (wlist's capacity) leave a flag set,
+// and the solve runs launch by launch.
 //
 // Visibility between workgroups.  Exchanged values (r, t1, the partial sums)
 // are doubles in two 64-bit words, each with 32 bits of the value and the
@@ -96,13 +104,89 @@ __device__ __forceinline__ unsigned long long ld_word(const unsigned long long* 
   return ld_agent(ps_at(base, i));
 }
 
+// ---- the window of the rows i0 .. i1 - 1 of a workgroup of T threads ----
+// Its 64-row chunks: those that the rows are in and those that their columns fall
+// into.  map (nch entries) gets 1 for each, cnt the prefix sums of the threads'
+// shares of them; `own` is this thread's share.  Returns their number.
+template <int T>
+__device__ __forceinline__ int ps_window_chunks(const int32_t* acol, const int32_t* alen, int cap,
+                                                int i0, int i1, int nch, uint16_t* map, int* cnt,
+                                                int& own) {
+  const int t = threadIdx.x;
+  for (int c = t; c < nch; c += T) map[c] = 0;
+  __syncthreads();
+  for (int i = i0 + t; i < i1; i += T) {
+    const int L = alen[i];
+    map[i / PS_CHUNK] = 1;  // its own rows, in order, whatever the columns
+    for (int k0 = 0; k0 < L; k0 += 8) {
+      int c[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) c[u] = acol[((k0 + u < L) ? k0 + u : k0) * cap + i];
+#pragma unroll
+      for (int u = 0; u < 8; u++) map[c[u] / PS_CHUNK] = 1;  // every writer stores 1
+    }
+  }
+  __syncthreads();
+  // thread t counts a run of consecutive chunks, then the runs are scanned
+  const int per = (nch + T - 1) / T, c0 = t * per, c1 = min(nch, c0 + per);
+  own = 0;
+  for (int c = c0; c < c1; c++) own += map[c];
+  cnt[t] = own;
+  __syncthreads();
+  for (int off = 1; off < T; off <<= 1) {
+    const int a = (t >= off) ? cnt[t - off] : 0;
+    __syncthreads();
+    cnt[t] += a;
+    __syncthreads();
+  }
+  return cnt[T - 1];
+}
+// The chunks in ascending order (wlist), their count and the slot of the
+// workgroup's first own one (wcnt), and in map the slot of each
+template <int T>
+__device__ __forceinline__ void ps_window_list(int i0, int nch, int own, int total, uint16_t* map,
+                                               const int* cnt, int32_t* wlist, int32_t* wcnt) {
+  const int t = threadIdx.x;
+  const int per = (nch + T - 1) / T, c0 = t * per, c1 = min(nch, c0 + per);
+  int pos = cnt[t] - own;
+  for (int c = c0; c < c1; c++)
+    if (map[c]) {
+      wlist[pos] = c;
+      if (c == i0 / PS_CHUNK) wcnt[1] = pos;
+      map[c] = (uint16_t)pos++;
+    }
+  if (t == 0) wcnt[0] = total;
+}
+// The rows' columns as window positions, slots 2w and 2w + 1 of row i in word
+// [w * ls + i]; map holds the chunks' slots (after a barrier)
+template <int T>
+__device__ __forceinline__ void ps_window_positions(const int32_t* acol, const int32_t* alen,
+                                                    int cap, int i0, int i1, const uint16_t* map,
+                                                    uint32_t* lidx, int ls) {
+  for (int i = i0 + threadIdx.x; i < i1; i += T) {
+    const int L = alen[i];
+    for (int k0 = 0; k0 < L; k0 += 8) {
+      int c[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) c[u] = acol[((k0 + u < L) ? k0 + u : k0) * cap + i];
+#pragma unroll
+      for (int u = 0; u < 8; u += 2) {
+        if (k0 + u >= L) break;
+        const uint32_t a = map[c[u] / PS_CHUNK] * PS_CHUNK + c[u] % PS_CHUNK;
+        const uint32_t b = map[c[u + 1] / PS_CHUNK] * PS_CHUNK + c[u + 1] % PS_CHUNK;
+        lidx[(size_t)((k0 + u) >> 1) * ls + i] = a | (b << 16);
+      }
+    }
+  }
+}
+
 // Windows of the workgroups' rows (one workgroup each, as the solve), the
-// rows' columns as window positions, and the slots cleared.
+// rows' columns as window positions, the slots cleared and the start kept
 template <int T>
 __global__ void __launch_bounds__(T) k_ps_setup(Dev D, PersArg Q) {
   __shared__ uint16_t map[PS_MAX_CHUNKS];
   __shared__ int cnt[T];
-  const int t = threadIdx.x, wg = blockIdx.x, n = D.sc->n, cap = D.cap;
+  const int t = threadIdx.x, wg = blockIdx.x, n = D.sc->n;
   const int nch = (n + PS_CHUNK - 1) / PS_CHUNK;
   const int i0 = wg * Q.nbw * RED_BLOCK;
   const int i1 = min(n, min(D.nblk, (wg + 1) * Q.nbw) * RED_BLOCK);
@@ -116,34 +200,8 @@ __global__ void __launch_bounds__(T) k_ps_setup(Dev D, PersArg Q) {
     Q.tlo[i] = Q.thi[i] = Q.rlo[i] = Q.rhi[i] = 0;
     Q.x0[i] = D.sol[i];
   }
-  for (int c = t; c < nch; c += T) map[c] = 0;
-  __syncthreads();
-  for (int i = i0 + t; i < i1; i += T) {
-    const int L = D.alen[i];
-    map[i / PS_CHUNK] = 1;  // its own rows, in order, whatever the columns
-    for (int k0 = 0; k0 < L; k0 += 8) {
-      int c[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) c[u] = D.acol[((k0 + u < L) ? k0 + u : k0) * cap + i];
-#pragma unroll
-      for (int u = 0; u < 8; u++) map[c[u] / PS_CHUNK] = 1;  // every writer stores 1
-    }
-  }
-  __syncthreads();
-  // positions of the marked chunks in ascending order: thread t counts a
-  // run of consecutive chunks, then the runs are scanned
-  const int per = (nch + T - 1) / T, c0 = t * per, c1 = min(nch, c0 + per);
-  int own = 0;
-  for (int c = c0; c < c1; c++) own += map[c];
-  cnt[t] = own;
-  __syncthreads();
-  for (int off = 1; off < T; off <<= 1) {
-    const int a = (t >= off) ? cnt[t - off] : 0;
-    __syncthreads();
-    cnt[t] += a;
-    __syncthreads();
-  }
-  const int total = cnt[T - 1];
+  int own;
+  const int total = ps_window_chunks<T>(D.acol, D.alen, D.cap, i0, i1, nch, map, cnt, own);
   if (total > Q.wcap) {  // the whole workgroup
     if (t == 0) {
       atomicOr(&D.sc->counter[PS_FLAG_WIN], 1u);
@@ -151,32 +209,14 @@ __global__ void __launch_bounds__(T) k_ps_setup(Dev D, PersArg Q) {
     }
     return;
   }
-  int pos = cnt[t] - own;
-  for (int c = c0; c < c1; c++)
-    if (map[c]) {
-      Q.wlist[(size_t)wg * Q.wcap + pos] = c;
-      if (c == i0 / PS_CHUNK) Q.wcnt[2 * wg + 1] = pos;
-      map[c] = (uint16_t)pos++;
-    }
-  if (t == 0) Q.wcnt[2 * wg] = total;
+  ps_window_list<T>(i0, nch, own, total, map, cnt, Q.wlist + (size_t)wg * Q.wcap,
+                    Q.wcnt + 2 * wg);
   __syncthreads();
-  for (int i = i0 + t; i < i1; i += T) {
-    const int L = D.alen[i];
-    for (int k0 = 0; k0 < L; k0 += 8) {
-      int c[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) c[u] = D.acol[((k0 + u < L) ? k0 + u : k0) * cap + i];
-#pragma unroll
-      for (int u = 0; u < 8; u += 2) {
-        if (k0 + u >= L) break;
-        const uint32_t a = map[c[u] / PS_CHUNK] * PS_CHUNK + c[u] % PS_CHUNK;
-        const uint32_t b = map[c[u + 1] / PS_CHUNK] * PS_CHUNK + c[u + 1] % PS_CHUNK;
-        Q.lidx[(size_t)((k0 + u) >> 1) * Q.ls + i] = a | (b << 16);
-      }
-    }
-  }
+  ps_window_positions<T>(D.acol, D.alen, D.cap, i0, i1, map, Q.lidx, Q.ls);
 }
 
+// a value that is the same in every lane (that of the first), out of the vector
+// registers
 __device__ __forceinline__ double lane0(double v) {
   const long long b = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_readfirstlane((int)b);
