@@ -795,9 +795,9 @@ extern "C" int isph_set_scalars(isph_ctx* c, const isph_scalars* in) {
 // effpor's walk is over ~50 solids and the longest of them; without solids
 // there is no walk (4.8/6 at 40k, 5/7 at 80k).  varts, which skips all but the
 // free surface, and the assembly run eight lanes always.
-// The weakly compressible step keeps one lane: its dam break compresses past
-// the list's capacity after about a thousand steps, and a faster step reaches
-// that inside the run that it would have to be compared over.
+// The weakly compressible step runs one lane per particle (but for varts): the
+// eight-lane form is not carried over to it yet, its continuity pass has none,
+// and by one measurement its step would take some 2.5 times less at 29k.
 static bool lanes8(const isph_ctx* c, int tk) {
   if (c->wcsph) return false;
   switch (tk) {

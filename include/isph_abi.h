@@ -286,10 +286,10 @@ int isph_load_system(isph_ctx *ctx, int32_t n, const int32_t *row_len,
  * they belong to a batch they share one stream, and the PPE solves of the
  * precision-form contexts run as one set of launches over all of them: one
  * resident launch up to some 780,000 rows together, where every scenario's rows
- * couple over a narrow enough range of rows (up to 458,000 rows always, beyond
- * that in basins less than 270 to 360 particles deep) and has no more than a few
- * cells per row.  A scenario's results are the same as when it is stepped alone.  Destroy the
- * batch before any of its contexts.  isph_batch_step returns the worst
+ * couple over a narrow enough range of rows (so does fluid up to 458,000 rows,
+ * and beyond that in basins less than 270 to 360 particles deep) and its domain
+ * has no more than a few cells per row.  A scenario's results are the same as
+ * when it is stepped alone.  Destroy the batch before any of its contexts.  isph_batch_step returns the worst
  * non-fatal solve code (ISPH_ENOCONV) over the scenarios and steps;
  * isph_batch_stats gives scenario s's last solve. */
 typedef struct isph_batch isph_batch;

@@ -1,6 +1,8 @@
 """A resident solve that has to go on, or start over, launch by launch: the
 results are those of the launch-per-phase form (kernel timing on), bit for bit,
 whatever the iteration at which the resident form ends."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -111,3 +113,36 @@ def test_batch_leaves_the_resident_form(pkg, cases, limits):
     for a, b in zip(out[0][1], out[1][1]):
         for k in a:
             assert np.array_equal(a[k], b[k], equal_nan=True), k
+
+
+@pytest.mark.gpu
+def test_contexts_stepped_by_several_threads(pkg, cases):
+    """Resident launches of three threads' contexts, in either form and of
+    different shapes, at once: each gets the results that it has alone."""
+    shapes = [(200, 40, 1), (330, 61, 0), (1280, 100, 1)]
+
+    def make(nx, ny, precision):
+        c = _tank(cases, nx, ny)
+        c.params.update(precision=precision, tol=1e-9, max_iter=80, max_outer=2)
+        s = pkg.Scenario(c)
+        s.init_state()
+        return s
+
+    def run(s, out):
+        st = [_stats(s.step(1, check=False)[1]) for _ in range(6)]
+        out.append((st, s.solution(), s.resident_counts()))
+        s.close()
+
+    alone = []
+    for q in shapes:
+        run(make(*q), alone)
+    print("resident: three threads", flush=True)
+    scen, together = [make(*q) for q in shapes], [[] for _ in shapes]
+    th = [threading.Thread(target=run, args=a) for a in zip(scen, together)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for a, (b,) in zip(alone, together):
+        assert a[0] == b[0] and np.array_equal(a[1], b[1])
+        assert b[2]["launches"] + b[2]["refused"] >= 1
